@@ -62,21 +62,6 @@ __device__ __forceinline__ int64_t xcd_block(int64_t b, int64_t n) {
     return x * q + (x < r ? x : r) + b / kXcds;
 }
 
-
-// Moves inside groups of four lanes through DPP quad permutations (a VALU
-// operand modifier) instead of ds_bpermute (an LDS round trip). QP is the
-// quad_perm control: bits [2l+1:2l] name the source lane of lane l; every lane
-// of the quad must be active.
-template <int QP>
-__device__ __forceinline__ double quad_perm(double x) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), QP, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), QP, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-constexpr int kQuadXor1 = 0xB1;  // lanes (1, 0, 3, 2)
-constexpr int kQuadXor2 = 0x4E;  // lanes (2, 3, 0, 1)
-__host__ __device__ constexpr int quad_bcast(int l) { return l * 0x55; }  // lanes (l, l, l, l)
-
 // The RK update of a step, fused into its last stage's kernel:
 // y_new = u + sum_j c_j x_j, the terms added one after another in FP64 (the
 // operations of multi_axpy, so the result is bitwise the same), where term
@@ -159,7 +144,7 @@ __device__ __forceinline__ void rk_update_run(const RkUpdate& q, int64_t o, cons
     for (int j = 0; j < kRkPre; ++j)
         if (j < q.n_x) {
 #pragma unroll
-            for (int a = 0; a < N; ++a) y[a] += q.c[j] * xs[j][a];
+            for (int a = 0; a < N; ++a) y[a] = fma(q.c[j], xs[j][a], y[a]);
         }
 #pragma unroll
     for (int j = kRkPre; j < kMaxIn; ++j) {
@@ -167,7 +152,7 @@ __device__ __forceinline__ void rk_update_run(const RkUpdate& q, int64_t o, cons
         double x[N];
         rk_term<N>(q, j, o, own, x);
 #pragma unroll
-        for (int a = 0; a < N; ++a) y[a] += q.c[j] * x[a];
+        for (int a = 0; a < N; ++a) y[a] = fma(q.c[j], x[a], y[a]);
     }
     if constexpr (N % 2 == 0) {
 #pragma unroll
@@ -193,10 +178,10 @@ __device__ __forceinline__ double combine(const StageIO& p, int64_t idx) {
     double x1 = 0;
     if (p.n_in > 1) x1 = load_in(p, 1, idx);
     double s = p.coef[0] * x0;
-    if (p.n_in > 1) s += p.coef[1] * x1;
+    if (p.n_in > 1) s = fma(p.coef[1], x1, s);
 #pragma unroll
     for (int i = 2; i < kMaxIn; ++i)
-        if (i < p.n_in) s += p.coef[i] * load_in(p, i, idx);
+        if (i < p.n_in) s = fma(p.coef[i], load_in(p, i, idx), s);
     return s;
 }
 
@@ -225,14 +210,14 @@ __device__ __forceinline__ void combine_n(const StageIO& p, const int64_t (&idx)
     for (int k = 0; k < K; ++k) s[k] = p.coef[0] * x0[k];
     if (p.n_in > 1) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) s[k] += p.coef[1] * x1[k];
+        for (int k = 0; k < K; ++k) s[k] = fma(p.coef[1], x1[k], s[k]);
     }
 #pragma unroll
     for (int i = 2; i < kMaxIn; ++i) {
         if (i >= p.n_in) break;
         load_n(p, i, idx, x0);
 #pragma unroll
-        for (int k = 0; k < K; ++k) s[k] += p.coef[i] * x0[k];
+        for (int k = 0; k < K; ++k) s[k] = fma(p.coef[i], x0[k], s[k]);
     }
 }
 

@@ -54,11 +54,11 @@ __device__ __forceinline__ double axpy_value(const A& p, int64_t i) {
         if (j < p.n_x) x[j] = term(j);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-        if (j < p.n_x) y += p.c[j] * x[j];
+        if (j < p.n_x) y = fma(p.c[j], x[j], y);
 #pragma unroll
     for (int j = 4; j < kMaxIn; ++j) {
         if (j >= p.n_x) break;
-        y += p.c[j] * term(j);
+        y = fma(p.c[j], term(j), y);
     }
     return y;
 }

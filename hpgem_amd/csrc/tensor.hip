@@ -113,109 +113,14 @@ __device__ __forceinline__ void combine_pencil(const StageIO& p, int64_t base, d
     for (int a = 0; a < N1; ++a) w[a] = p.coef[0] * x[a];
     if (p.n_in > 1) {
 #pragma unroll
-        for (int a = 0; a < N1; ++a) w[a] += p.coef[1] * y[a];
+        for (int a = 0; a < N1; ++a) w[a] = fma(p.coef[1], y[a], w[a]);
     }
 #pragma unroll
     for (int i = 2; i < kMaxIn; ++i) {
         if (i >= p.n_in) break;
         load_pencil<N1>(p, i, base, x);
 #pragma unroll
-        for (int a = 0; a < N1; ++a) w[a] += p.coef[i] * x[a];
-    }
-}
-
-// Stage input at the traces of all 2 DIM faces of a pencil: x faces (f < 2)
-// one value at at[f], y/z faces the pencil [at[f], at[f] + N1). PAIR: the
-// first two input vectors' loads all issue before any value is used (twice
-// the registers); otherwise, and for further inputs, one input vector at a
-// time. Same rounding as combine().
-template <int DIM, int N1>
-__device__ __forceinline__ void load_traces(const StageIO& p, int i, const int64_t (&at)[2 * DIM],
-                                            double (&x)[2 * DIM][N1]) {
-    if ((p.in_f32 >> i) & 1u) {
-        const float* v = static_cast<const float*>(p.in[i]);
-#pragma unroll
-        for (int f = 0; f < 2; ++f) x[f][0] = v[at[f]];
-#pragma unroll
-        for (int f = 2; f < 2 * DIM; ++f) {
-            const float* q = v + at[f];
-            if constexpr (N1 % 4 == 0) {
-#pragma unroll
-                for (int a = 0; a < N1; a += 4) {
-                    const float4 t = *reinterpret_cast<const float4*>(q + a);
-                    x[f][a] = t.x; x[f][a + 1] = t.y; x[f][a + 2] = t.z; x[f][a + 3] = t.w;
-                }
-            } else if constexpr (N1 % 2 == 0) {
-#pragma unroll
-                for (int a = 0; a < N1; a += 2) {
-                    const float2 t = *reinterpret_cast<const float2*>(q + a);
-                    x[f][a] = t.x; x[f][a + 1] = t.y;
-                }
-            } else {
-#pragma unroll
-                for (int a = 0; a < N1; ++a) x[f][a] = q[a];
-            }
-        }
-    } else {
-        const double* v = static_cast<const double*>(p.in[i]);
-#pragma unroll
-        for (int f = 0; f < 2; ++f) x[f][0] = v[at[f]];
-#pragma unroll
-        for (int f = 2; f < 2 * DIM; ++f) {
-            const double* q = v + at[f];
-            if constexpr (N1 % 2 == 0) {
-#pragma unroll
-                for (int a = 0; a < N1; a += 2) {
-                    const double2 t = *reinterpret_cast<const double2*>(q + a);
-                    x[f][a] = t.x; x[f][a + 1] = t.y;
-                }
-            } else {
-#pragma unroll
-                for (int a = 0; a < N1; ++a) x[f][a] = q[a];
-            }
-        }
-    }
-}
-
-template <int DIM, int N1, bool PAIR = true>
-__device__ __forceinline__ void combine_traces(const StageIO& p, const int64_t (&at)[2 * DIM],
-                                               double (&w)[2 * DIM][N1]) {
-    double x[2 * DIM][N1];
-    load_traces<DIM, N1>(p, 0, at, x);
-    if constexpr (PAIR) {
-        double y[2 * DIM][N1];
-        if (p.n_in > 1) load_traces<DIM, N1>(p, 1, at, y);
-#pragma unroll
-        for (int f = 0; f < 2 * DIM; ++f)
-#pragma unroll
-            for (int a = 0; a < (f < 2 ? 1 : N1); ++a) w[f][a] = p.coef[0] * x[f][a];
-        if (p.n_in > 1) {
-#pragma unroll
-            for (int f = 0; f < 2 * DIM; ++f)
-#pragma unroll
-                for (int a = 0; a < (f < 2 ? 1 : N1); ++a) w[f][a] += p.coef[1] * y[f][a];
-        }
-    } else {
-#pragma unroll
-        for (int f = 0; f < 2 * DIM; ++f)
-#pragma unroll
-            for (int a = 0; a < (f < 2 ? 1 : N1); ++a) w[f][a] = p.coef[0] * x[f][a];
-        if (p.n_in > 1) {
-            load_traces<DIM, N1>(p, 1, at, x);
-#pragma unroll
-            for (int f = 0; f < 2 * DIM; ++f)
-#pragma unroll
-                for (int a = 0; a < (f < 2 ? 1 : N1); ++a) w[f][a] += p.coef[1] * x[f][a];
-        }
-    }
-#pragma unroll
-    for (int i = 2; i < kMaxIn; ++i) {
-        if (i >= p.n_in) break;
-        load_traces<DIM, N1>(p, i, at, x);
-#pragma unroll
-        for (int f = 0; f < 2 * DIM; ++f)
-#pragma unroll
-            for (int a = 0; a < (f < 2 ? 1 : N1); ++a) w[f][a] += p.coef[i] * x[f][a];
+        for (int a = 0; a < N1; ++a) w[a] = fma(p.coef[i], x[a], w[a]);
     }
 }
 
@@ -585,13 +490,17 @@ __global__ __launch_bounds__(kBlock) void tensor_advection_rhs_batched(const Rhs
 
 // Acoustic wave system on tensor elements (AcousticWaveLinear_Impl.h:102-283):
 // fields v, s_1..s_dim stored field-major per element. With g_r = sum_d
-// (J^{-1})_{r,d} s_d,
-//   k_v   = sum_r (Dr along r) g_r + sum_faces Mi(:,s) (x) C_v
-//   k_s_d = (1/c_inv) [ sum_r (J^{-1})_{r,d} (Dr along r) v + sum_faces Mi(:,s) (x) C_d ]
-// where, on face (d_f, s) with w_k = (2s-1) (J^{-1})_{d_f,k} (= outward normal
-// times face area over element volume), C_v = -1/2 w.(s_own - s_nbr) and
-// C_d = -1/2 w_d (v_own - v_nbr) on internal faces, C_v = -w.s_own and C_d = 0
-// on reflecting walls. Jumps are formed in FP64.
+// (J^{-1})_{r,d} s_d, the element's own J throughout, and per face (r, s)
+//   F_v = -1/2 (2s-1) (g_r,own - sum_d (J^{-1})_{r,d} s_d,nbr),
+//   F_s = -1/2 (2s-1) (v_own - v_nbr)
+// on internal faces, F_v = -(2s-1) g_r,own and F_s = 0 on reflecting walls,
+//   k_v   =             sum_r [ (Dr along r) g_r + sum_s Mi(:,s) (x) F_v(r,s) ]
+//   k_s_d = (1/c_inv) sum_r (J^{-1})_{r,d} [ (Dr along r) v + sum_s Mi(:,s) (x) F_s(r,s) ].
+// Both brackets are the same one-dimensional operator, applied to g_r and to
+// v; the s fields are only combined from the second at the end. The
+// arithmetic is FP64 in both precisions (an FP64 multiply-add issues at the
+// FP32 rate here); the mixed path differs in the storage of its stage
+// derivatives.
 struct AcousticParams {
     int64_t n_elem;
     StageIO io;
@@ -602,481 +511,458 @@ struct AcousticParams {
     const double* Mi;
 };
 
-// Four lanes per pencil, one per field (v, s_1 .. s_3; in 2D the fourth lane
-// idles), so a lane carries one field's N1 values. Both equations then
-// run the same instructions:
-//   volume: acc = sum_r scale_r (Dr along r) src_r, with src_r = g_r =
-//     sum_d (J^{-1})_{r,d} s_d and scale_r = 1 on the v lane, src_r = v and
-//     scale_r = (J^{-1})_{r,d} on the s_d lane;
-//   faces: each lane forms its own field's jump; the v lane gets
-//     sum_k w_k [s_k] by a reduction over the pencil's four lanes, the s
-//     lanes get [v] from the v lane, both by lane shuffles within the quad.
-constexpr int kQuad2DMinN1 = 3;  // 2D orders whose pencils take the four-lane layout: N1 >= this
-
+// One thread owns one x-pencil of an element with all its fields; v, g_y and
+// g_z go to LDS for the y and z contractions, and each y or z face pencil's
+// fluxes are formed once, by one of the element's threads (NQ face pencils),
+// and shared through LDS. Nothing but an element's own threads meets at a
+// barrier, so a workgroup is the smallest of 64, 128 and 256 threads that
+// leaves at most one lane in sixteen idle: one wavefront where it can.
+// Sums are explicit multiply-adds: every instance (with and without the
+// update, batched) rounds alike.
+// Bound by memory: 32^3 p = 3 in FP64 reads and writes 201 MB at 4.3 TB/s
+// (a copy of that size reaches 5.4 - 6.9 TB/s). One lane per field and pencil,
+// which applies the derivative of v once per s field and forms every face
+// pencil's flux N1 times, took 104 us FP64 / 80 mixed there against 47 / 36;
+// 30^3 p = 2 42 against 23, 23x19x21 p = 4 66 against 37 (FP64).
+// kAhead: the first face pencil's neighbour values are loaded together with
+// the own ones, one memory round trip less (32^3 p = 3 53 -> 47 us, 256^2
+// p = 3 20.1 -> 17.7); at orders 4 and 5 in 3D, and with the update's terms
+// held too, its registers cost as much as that gains (20^3 p = 5 60 -> 64 us).
+// kEarly: all of the update's sum but the own term is formed before the
+// volume terms, from u and k as they are loaded anyway (RK4 step of 30^3 p = 2
+// 107 -> 103 us, 256^2 p = 1 34.8 -> 32.3); at orders 4 and 5 the 4 N1 sums do
+// not fit beside the rest (20^3 p = 5 276 -> 288 us), so there it comes last.
 template <int DIM, int N1>
 struct AcousticShape {
     static constexpr int NF = DIM + 1;
     static constexpr int NP = Pencil<DIM, N1>::NP;
     static constexpr int NB = Pencil<DIM, N1>::NB;
-    static constexpr bool QUAD = DIM == 3 || N1 >= kQuad2DMinN1;
-    static constexpr int TPE = QUAD ? 4 * NP : NP;  // threads per element
-    static constexpr int EPB = kBlock / TPE;
+    static constexpr int NQ = 2 * (DIM - 1) * (DIM == 3 ? N1 : 1);
+    static constexpr int THREADS = (64 % NP) * 16 <= 64 ? 64 : (128 % NP) * 16 <= 128 ? 128 : 256;
+    static constexpr int EPB = THREADS / NP;
+    // LDS strides (doubles) of a plane and an element: even orders' planes
+    // are a multiple of the 64 banks' period apart without the padding
+    static constexpr int PS = N1 * N1 + (N1 % 2 == 0 ? 2 : 0);
+    static constexpr int ES = (DIM == 3 ? N1 : 1) * PS;
 };
 
-template <int DIM, int N1, typename T, bool UPD>
-__device__ __forceinline__ void acoustic_block_quad(const AcousticParams& p, int64_t blk) {
-    using S = AcousticShape<DIM, N1>;
-    constexpr int NF = S::NF;
-    constexpr int NB = S::NB;
-    __shared__ double s_w[S::EPB * NF * NB];      // FP64 stage input
-    __shared__ T s_g[S::EPB * (DIM + 1) * NB];    // v, then g_r, in T
-    __shared__ double s_J[S::EPB * DIM * DIM];    // J^{-1}
-    __shared__ T s_D[N1 * N1];
-    __shared__ T s_Mi[2 * N1];
-    const int tid = threadIdx.x;
-    if (tid < N1 * N1) s_D[tid] = T(p.Dr[tid]);
-    if (tid < 2 * N1) s_Mi[tid] = T(p.Mi[(tid % N1) * N1 + tid / N1]);
-    const int le = tid / S::TPE;
-    const int pc = (tid % S::TPE) / 4;
-    const int fld = tid % 4;
-    const int64_t e = blk * S::EPB + le;
-    const bool active = (le < S::EPB) && (e < p.n_elem);
-    const bool lane = active && fld < NF;
-    const int ib = pc % N1;
-    const int ic = DIM == 3 ? pc / N1 : 0;
-    double* sw = s_w + le * NF * NB;
-    T* sg = s_g + le * (DIM + 1) * NB;
-    double* sJ = s_J + le * DIM * DIM;
-    const int64_t base = e * NF * NB;
-    const int d = fld - 1;  // s lanes: the component
-
-    // ---- stage input, v and g_r into LDS
-    double w[N1];
+// Pencils of one input vector as loaded: FP32 values stay as their bits in the
+// doubles' low words until they are used (raw_value), so nothing waits for a
+// load where it is issued.
+template <int NR, int N1>
+__device__ __forceinline__ void load_raw(const void* v, bool f32, int64_t base, int64_t stride, double (&x)[NR][N1]) {
+    if (f32) {
+        const float* f = static_cast<const float*>(v) + base;
 #pragma unroll
-    for (int a = 0; a < N1; ++a) w[a] = 0.0;
-    if (lane) {
-        combine_pencil<N1>(p.io, base + fld * NB + pc * N1, w);
+        for (int r = 0; r < NR; ++r) {
+            float t[N1];
+            if constexpr (N1 % 4 == 0) {
 #pragma unroll
-        for (int a = 0; a < N1; ++a) sw[fld * NB + pc * N1 + a] = w[a];
-        if (pc == 0 && fld == 0)
-#pragma unroll
-            for (int k = 0; k < DIM * DIM; ++k) sJ[k] = p.jinv[k * p.n_elem + e];
-    }
-    {
-        // lane 1 + r of the quad forms g_r at the pencil's nodes, lane 0 writes v
-        double Jr[DIM];
-        const int r = fld - 1;
-#pragma unroll
-        for (int k = 0; k < DIM; ++k) Jr[k] = (active && r >= 0 && r < DIM) ? p.jinv[(r * DIM + k) * p.n_elem + e] : 0.0;
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            double g = 0;
-#pragma unroll
-            for (int k = 0; k < DIM; ++k) {
-                const double wk = k == 0 ? quad_perm<quad_bcast(1)>(w[a])
-                                : k == 1 ? quad_perm<quad_bcast(2)>(w[a]) : quad_perm<quad_bcast(3)>(w[a]);
-                g += Jr[k] * wk;
-            }
-            if (lane) sg[(r + 1) * NB + pc * N1 + a] = fld == 0 ? T(w[a]) : T(g);
-        }
-    }
-    const double cinv = active ? p.cinv[e] : 1.0;
-    int32_t nbi[2 * DIM];  // the face neighbours, loaded with the stage input
-#pragma unroll
-    for (int f = 0; f < 2 * DIM; ++f) nbi[f] = active ? p.nbr[f * p.n_elem + e] : -1;
-    __syncthreads();
-
-    // ---- volume
-    Acc<T> acc[N1];
-    if (lane) {
-#pragma unroll
-        for (int a = 0; a < N1; ++a) acc[a] = Acc<T>(T(0));
-        T vol[N1];
-#pragma unroll
-        for (int a = 0; a < N1; ++a) vol[a] = T(0);
-#pragma unroll
-        for (int r = 0; r < DIM; ++r) {
-            const T* src = fld == 0 ? sg + (1 + r) * NB : sg;
-            const T scale = fld == 0 ? T(1) : T(sJ[r * DIM + d]);
-            T t[N1];
-            if (r == 0) {  // along this pencil
-#pragma unroll
-                for (int a = 0; a < N1; ++a) {
-                    T sv = T(0);
-#pragma unroll
-                    for (int j = 0; j < N1; ++j) sv += s_D[a * N1 + j] * src[pc * N1 + j];
-                    t[a] = sv;
+                for (int a = 0; a < N1; a += 4) {
+                    const float4 q = *reinterpret_cast<const float4*>(f + r * stride + a);
+                    t[a] = q.x; t[a + 1] = q.y; t[a + 2] = q.z; t[a + 3] = q.w;
                 }
-            } else {  // across the element's other pencils
-                const int my = r == 1 ? ib : ic;
+            } else if constexpr (N1 % 2 == 0) {
 #pragma unroll
-                for (int a = 0; a < N1; ++a) t[a] = T(0);
-#pragma unroll
-                for (int j = 0; j < N1; ++j) {
-                    const int opc = r == 1 ? j + N1 * ic : ib + N1 * j;
-                    const T dr = s_D[my * N1 + j];
-#pragma unroll
-                    for (int a = 0; a < N1; ++a) t[a] += dr * src[opc * N1 + a];
+                for (int a = 0; a < N1; a += 2) {
+                    const float2 q = *reinterpret_cast<const float2*>(f + r * stride + a);
+                    t[a] = q.x; t[a + 1] = q.y;
                 }
+            } else {
+#pragma unroll
+                for (int a = 0; a < N1; ++a) t[a] = f[r * stride + a];
             }
 #pragma unroll
-            for (int a = 0; a < N1; ++a) vol[a] += scale * t[a];
-        }
-#pragma unroll
-        for (int a = 0; a < N1; ++a) acc[a] = Acc<T>(vol[a]);
-    }
-
-    // ---- faces: x faces one value per pencil, y/z faces a whole pencil.
-    // The neighbours' traces of all faces first, every global load issued
-    // before any is used (a neighbour in the block is read from LDS; a face
-    // that loads nothing points at the thread's own pencil). At p = 3
-    // (N1 = 4) the registers that holds cost more than the shorter wait
-    // gains (measured in both precisions), so there each face loads its own.
-    constexpr bool kHoist = N1 != 4;
-    double oth[2 * DIM][N1];
-    if constexpr (kHoist) {
-        int64_t at[2 * DIM];
-#pragma unroll
-        for (int f = 0; f < 2 * DIM; ++f) {
-            const int df = f / 2, s = f % 2;
-            const int nbr_pc = df == 0 ? pc : df == 1 ? (1 - s) + N1 * ic : ib + N1 * (1 - s);
-            const int noff = df == 0 ? 1 - s : 0;
-            const int64_t lnb = int64_t(nbi[f]) - blk * S::EPB;
-            const bool glob = lane && nbi[f] >= 0 && !(lnb >= 0 && lnb < S::EPB);
-            at[f] = glob ? int64_t(nbi[f]) * NF * NB + fld * NB + nbr_pc * N1 + noff : base + fld * NB + pc * N1;
-        }
-        // (at order 4 in FP32 holding two inputs' traces costs an occupancy step)
-        constexpr bool kPair = !(N1 >= 5 && std::is_same<T, float>::value);
-        if (lane) combine_traces<DIM, N1, kPair>(p.io, at, oth);  // (an inactive thread's own pencil may lie past the end)
-#pragma unroll
-        for (int f = 0; f < 2 * DIM; ++f) {
-            const int df = f / 2, s = f % 2;
-            const int nbr_pc = df == 0 ? pc : df == 1 ? (1 - s) + N1 * ic : ib + N1 * (1 - s);
-            const int noff = df == 0 ? 1 - s : 0;
-            const int64_t lnb = int64_t(nbi[f]) - blk * S::EPB;
-            if (lane && nbi[f] >= 0 && lnb >= 0 && lnb < S::EPB) {
-#pragma unroll
-                for (int a = 0; a < (df == 0 ? 1 : N1); ++a)
-                    oth[f][a] = s_w[(lnb * NF + fld) * NB + nbr_pc * N1 + noff + a];
-            }
-        }
-    }
-#pragma unroll
-    for (int f = 0; f < 2 * DIM; ++f) {
-        const int df = f / 2, s = f % 2;
-        const bool inner = nbi[f] >= 0;
-        const int own_pc = df == 0 ? pc : df == 1 ? s + N1 * ic : ib + N1 * s;
-        const int na = df == 0 ? 1 : N1;  // trace values per pencil
-        const int off = df == 0 ? s : 0;  // own node of an x face
-        double jmp[N1];
-#pragma unroll
-        for (int a = 0; a < N1; ++a) jmp[a] = 0.0;
-        if constexpr (!kHoist) {
-            if (lane && inner) {
-                const int nbr_pc = df == 0 ? pc : df == 1 ? (1 - s) + N1 * ic : ib + N1 * (1 - s);
-                const int noff = df == 0 ? 1 - s : 0;
-                const int64_t lnb = int64_t(nbi[f]) - blk * S::EPB;
-                if (lnb >= 0 && lnb < S::EPB) {
-#pragma unroll
-                    for (int a = 0; a < N1; ++a)
-                        if (a < na) oth[f][a] = s_w[(lnb * NF + fld) * NB + nbr_pc * N1 + noff + a];
-                } else if (df == 0) {
-                    oth[f][0] = combine(p.io, int64_t(nbi[f]) * NF * NB + fld * NB + nbr_pc * N1 + noff);
-                } else {
-                    combine_pencil<N1>(p.io, int64_t(nbi[f]) * NF * NB + fld * NB + nbr_pc * N1, oth[f]);
-                }
-            }
-        }
-        if (lane) {
-#pragma unroll
-            for (int a = 0; a < N1; ++a)
-                if (a < na) jmp[a] = sw[fld * NB + own_pc * N1 + off + a] - (inner ? oth[f][a] : 0.0);
-        }
-        const double wd = (2 * s - 1) * (lane && fld > 0 ? sJ[df * DIM + d] : 0.0);  // w_d on the s_d lane
-        const int my = df == 1 ? ib : ic;
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            if (a >= na) break;
-            // v lane: sum_k w_k [s_k] over the quad; s lanes: [v] from the v lane
-            double x = wd * jmp[a];
-            x += quad_perm<kQuadXor1>(x);
-            x += quad_perm<kQuadXor2>(x);
-            const double jv = quad_perm<quad_bcast(0)>(jmp[a]);
-            double c;
-            if (fld == 0) c = inner ? -0.5 * x : -x;
-            else c = inner ? wd * (-0.5 * jv) : 0.0;
-            if (lane) {
-                if (df == 0) {
-#pragma unroll
-                    for (int b = 0; b < N1; ++b) acc[b].add(s_Mi[s * N1 + b] * T(c));
-                } else {
-                    acc[a].add(s_Mi[s * N1 + my] * T(c));
-                }
-            }
-        }
-    }
-    if (!lane) return;
-    const T ci = T(1.0 / cinv);
-    const int64_t o = base + fld * NB + pc * N1;
-    double kv[N1];  // the values as stored
-    if (p.io.out_f32) {
-        float* out = static_cast<float*>(p.io.out);
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            const float v = float(fld == 0 ? acc[a].value() : ci * acc[a].value());
-            out[o + a] = v;
-            kv[a] = double(v);
+            for (int a = 0; a < N1; ++a) x[r][a] = __hiloint2double(0, __float_as_int(t[a]));
         }
     } else {
-        double* out = static_cast<double*>(p.io.out);
+        const double* d = static_cast<const double*>(v) + base;
 #pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            const double v = double(fld == 0 ? acc[a].value() : ci * acc[a].value());
-            out[o + a] = v;
-            kv[a] = v;
-        }
+        for (int r = 0; r < NR; ++r) load_run<N1>(d + r * stride, x[r]);
     }
-    if constexpr (UPD) rk_update_run<N1>(p.io.upd, o, kv);
 }
 
-// In 2D at order 1 (three fields, little work per pencil) one thread per
-// pencil does all fields; from order 2 on the four-lane layout above is
-// faster (the one-thread form needs up to 256 registers there: one wave per
-// SIMD at orders 4 and 5).
-template <int DIM, int N1, typename T, bool UPD>
-__device__ __forceinline__ void acoustic_block_pencil(const AcousticParams& p, int64_t blk) {
-    using S = Pencil<DIM, N1>;
-    static_assert(AcousticShape<DIM, N1>::EPB == S::EPB, "launch geometry");
-    constexpr int NF = DIM + 1;
-    constexpr int NB = S::NB;
-    __shared__ double s_w[S::EPB * NF * NB];
-    __shared__ T s_D[N1 * N1];
-    __shared__ T s_Mi[2 * N1];
+__device__ __forceinline__ double raw_value(double x, bool f32) {
+    return f32 ? double(__int_as_float(__double2loint(x))) : x;
+}
+
+// y += c x for NR pencils as load_raw left them
+template <int NR, int N1>
+__device__ __forceinline__ void add_raw(double c, const double (&x)[NR][N1], bool f32, double (&y)[NR][N1]) {
+    if (f32) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int a = 0; a < N1; ++a) y[r][a] = fma(c, raw_value(x[r][a], true), y[r][a]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int a = 0; a < N1; ++a) y[r][a] = fma(c, x[r][a], y[r][a]);
+    }
+}
+
+// Stage input of NR pencils at [base + r stride, + N1), in two halves:
+// load_pencils issues the first two input vectors' loads (u, x), mix_pencils
+// forms combine()'s sums from them in u and adds further inputs one by one.
+template <int NR, int N1>
+__device__ __forceinline__ void load_pencils(const StageIO& p, int64_t base, int64_t stride, double (&u)[NR][N1],
+                                             double (&x)[NR][N1]) {
+    load_raw<NR, N1>(p.in[0], p.in_f32 & 1u, base, stride, u);
+    if (p.n_in > 1) load_raw<NR, N1>(p.in[1], p.in_f32 & 2u, base, stride, x);
+}
+
+template <int NR, int N1>
+__device__ __forceinline__ void mix_pencils(const StageIO& p, int64_t base, int64_t stride, double (&u)[NR][N1],
+                                            double (&x)[NR][N1]) {
+    const bool u32 = p.in_f32 & 1u;
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int a = 0; a < N1; ++a) u[r][a] = p.coef[0] * raw_value(u[r][a], u32);
+    if (p.n_in > 1) add_raw<NR, N1>(p.coef[1], x, p.in_f32 & 2u, u);
+#pragma unroll
+    for (int i = 2; i < kMaxIn; ++i) {
+        if (i >= p.n_in) break;
+        load_raw<NR, N1>(p.in[i], (p.in_f32 >> i) & 1u, base, stride, x);
+        add_raw<NR, N1>(p.coef[i], x, (p.in_f32 >> i) & 1u, u);
+    }
+}
+
+// The fused RK update of NR pencils but for this kernel's own term, which is
+// the last of its sum (RkUpdate::self): y = u + sum_{j != self} c_j x_j in
+// rk_update_run's order. u and x are the stage input's first two vectors as
+// load_raw left them (not yet mixed): the update reads those two again, so
+// they are taken from registers; the first two other terms are loaded
+// together, further ones one by one.
+template <int NR, int N1>
+__device__ __forceinline__ void update_partial(const StageIO& p, int64_t base, int64_t stride,
+                                               const double (&u)[NR][N1], const double (&x)[NR][N1],
+                                               double (&y)[NR][N1]) {
+    const RkUpdate& q = p.upd;
+    double t[2][NR][N1];
+    auto from_x = [&](int j) { return p.n_in > 1 && q.x[j] == p.in[1]; };
+    auto fetch = [&](int j, double (&d)[NR][N1]) {
+        if (j < q.n_x && j != q.self && !from_x(j)) load_raw<NR, N1>(q.x[j], (q.x_f32 >> j) & 1u, base, stride, d);
+    };
+    auto add = [&](int j, const double (&d)[NR][N1]) {
+        if (j >= q.n_x || j == q.self) return;
+        if (from_x(j)) add_raw<NR, N1>(q.c[j], x, p.in_f32 & 2u, y);
+        else add_raw<NR, N1>(q.c[j], d, (q.x_f32 >> j) & 1u, y);
+    };
+    fetch(0, t[0]);
+    fetch(1, t[1]);
+    if (q.u == p.in[0]) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int a = 0; a < N1; ++a) y[r][a] = u[r][a];
+    } else {
+        load_raw<NR, N1>(q.u, false, base, stride, y);
+    }
+    add(0, t[0]);
+    add(1, t[1]);
+#pragma unroll
+    for (int j = 2; j < kMaxIn; ++j) {
+        if (j >= q.n_x) break;
+        fetch(j, t[0]);
+        add(j, t[0]);
+    }
+}
+
+// The rest of that update: the own term (k as stored), then y_new.
+template <int N1>
+__device__ __forceinline__ void update_store(const RkUpdate& q, int64_t o, const double (&k)[N1], double (&y)[N1]) {
+    if (q.self >= 0) {
+#pragma unroll
+        for (int a = 0; a < N1; ++a) y[a] = fma(q.c[q.self], k[a], y[a]);
+    }
+    if constexpr (N1 % 2 == 0) {
+#pragma unroll
+        for (int a = 0; a < N1; a += 2) *reinterpret_cast<double2*>(q.y_new + o + a) = make_double2(y[a], y[a + 1]);
+    } else {
+#pragma unroll
+        for (int a = 0; a < N1; ++a) q.y_new[o + a] = y[a];
+    }
+}
+
+// The output pencil at o, in the output's storage type; v becomes the values
+// as stored.
+template <int N1>
+__device__ __forceinline__ void store_pencil(const StageIO& p, int64_t o, double (&v)[N1]) {
+    if (p.out_f32) {
+        float* out = static_cast<float*>(p.out) + o;
+        float f[N1];
+#pragma unroll
+        for (int a = 0; a < N1; ++a) {
+            f[a] = float(v[a]);
+            v[a] = double(f[a]);
+        }
+        if constexpr (N1 % 4 == 0) {
+#pragma unroll
+            for (int a = 0; a < N1; a += 4)
+                *reinterpret_cast<float4*>(out + a) = make_float4(f[a], f[a + 1], f[a + 2], f[a + 3]);
+        } else if constexpr (N1 % 2 == 0) {
+#pragma unroll
+            for (int a = 0; a < N1; a += 2) *reinterpret_cast<float2*>(out + a) = make_float2(f[a], f[a + 1]);
+        } else {
+#pragma unroll
+            for (int a = 0; a < N1; ++a) out[a] = f[a];
+        }
+    } else {
+        double* out = static_cast<double*>(p.out) + o;
+        if constexpr (N1 % 2 == 0) {
+#pragma unroll
+            for (int a = 0; a < N1; a += 2) *reinterpret_cast<double2*>(out + a) = make_double2(v[a], v[a + 1]);
+        } else {
+#pragma unroll
+            for (int a = 0; a < N1; ++a) out[a] = v[a];
+        }
+    }
+}
+
+template <int DIM, int N1, bool UPD>
+__device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t blk) {
+    using S = AcousticShape<DIM, N1>;
+    constexpr int NF = S::NF, NB = S::NB, NP = S::NP, NQ = S::NQ;
+    __shared__ double s_v[S::EPB * S::ES];                  // v
+    __shared__ double s_g[(DIM - 1) * S::EPB * S::ES];      // g_y, g_z
+    __shared__ double s_f[S::EPB * NQ * 2 * N1];            // per y/z face pencil: F_v, F_s
     const int tid = threadIdx.x;
-    if (tid < N1 * N1) s_D[tid] = T(p.Dr[tid]);
-    if (tid < 2 * N1) s_Mi[tid] = T(p.Mi[(tid % N1) * N1 + tid / N1]);
-    const int le = tid / S::NP;
-    const int pc = tid % S::NP;
+    const int le = tid / NP, pc = tid % NP;
     const int64_t e = blk * S::EPB + le;
     const bool active = (le < S::EPB) && (e < p.n_elem);
     const int ib = pc % N1;
     const int ic = DIM == 3 ? pc / N1 : 0;
-    double* sw = s_w + le * NF * NB;
+    auto row = [](int b, int c) { return c * S::PS + b * N1; };
     const int64_t base = e * NF * NB;
-    double w[NF][N1];
+    // face pencil q: face (r, s) with (r - 1) * 2 + s = q / N1 (2D: q), pencil
+    // q % N1 of it; where its values start in neighbour nb
+    auto face_pencil = [](int q, int32_t nb) {
+        const int fi = DIM == 3 ? q / N1 : q, k = DIM == 3 ? q % N1 : 0, s = fi % 2;
+        return int64_t(nb) * NF * NB + (fi / 2 ? k + N1 * (1 - s) : (1 - s) + N1 * k) * N1;
+    };
+
+    // ---- own pencil of every field; g_r
+    // (kAhead: and the neighbour's pencils of the first face pencil: all loads of
+    // both are in flight before any is used)
+    constexpr bool kAhead = !UPD && (DIM == 2 || N1 <= 4);
+    double w[NF][N1], J[DIM][DIM], wq[NF][N1];
+    constexpr bool kEarly = UPD && N1 <= 4;
+    double y[NF][N1];  // kEarly: the update's sum but for this stage's own term
+    int32_t nbx[2] = {-1, -1}, nbq = -1;
+    if (active) {
+        if (pc < NQ) nbq = p.nbr[(2 + (DIM == 3 ? pc / N1 : pc)) * p.n_elem + e];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) nbx[s] = p.nbr[s * p.n_elem + e];
+#pragma unroll
+        for (int r = 0; r < DIM; ++r)
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) J[r][d] = p.jinv[(r * DIM + d) * p.n_elem + e];
+        double x[NF][N1];
+        load_pencils<NF, N1>(p.io, base + pc * N1, NB, w, x);
+        if constexpr (kEarly) update_partial<NF, N1>(p.io, base + pc * N1, NB, w, x, y);
+        if constexpr (kAhead) {
+            double xq[NF][N1];
+            const int64_t bq = face_pencil(pc, nbq);
+            if (nbq >= 0) load_pencils<NF, N1>(p.io, bq, NB, wq, xq);
+            mix_pencils<NF, N1>(p.io, base + pc * N1, NB, w, x);
+            if (nbq >= 0) mix_pencils<NF, N1>(p.io, bq, NB, wq, xq);
+        } else {
+            mix_pencils<NF, N1>(p.io, base + pc * N1, NB, w, x);
+        }
+    } else {
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int a = 0; a < N1; ++a) w[f][a] = 0.0;
+#pragma unroll
+        for (int r = 0; r < DIM; ++r)
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) J[r][d] = 0.0;
+    }
+    double gx[N1];
     if (active) {
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            combine_pencil<N1>(p.io, base + f * NB + pc * N1, w[f]);
+        for (int r = 0; r < DIM; ++r) {
+            double g[N1];
 #pragma unroll
-            for (int a = 0; a < N1; ++a) sw[f * NB + pc * N1 + a] = w[f][a];
+            for (int a = 0; a < N1; ++a) {
+                g[a] = 0.0;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) g[a] = fma(J[r][d], w[1 + d][a], g[a]);
+            }
+#pragma unroll
+            for (int a = 0; a < N1; ++a) {
+                if (r == 0) gx[a] = g[a];
+                else s_g[((r - 1) * S::EPB + le) * S::ES + row(ib, ic) + a] = g[a];
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < N1; ++a) s_v[le * S::ES + row(ib, ic) + a] = w[0][a];
+    }
+
+    // ---- x faces: one trace value per pencil; a neighbour whose pencil lies
+    // in this wavefront hands it over by a lane shuffle
+    double fvx[2], fsx[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const int64_t ln = int64_t(nbx[s]) - blk * S::EPB;
+        const bool here = ln >= 0 && ln < S::EPB && (int(ln) * NP + pc) / 64 == tid / 64;
+        const int src = here ? (int(ln) * NP + pc) % 64 : tid % 64;
+        double o[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) o[f] = __shfl(w[f][1 - s], src, 64);
+        fvx[s] = fsx[s] = 0.0;
+        if (active && nbx[s] >= 0) {
+            if (!here) {
+                int64_t at[NF];
+#pragma unroll
+                for (int f = 0; f < NF; ++f) at[f] = (int64_t(nbx[s]) * NF + f) * NB + pc * N1 + (1 - s);
+                combine_n<NF>(p.io, at, o);
+            }
+            double gn = 0.0;
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) gn = fma(J[0][d], o[1 + d], gn);
+            fvx[s] = (s ? -0.5 : 0.5) * (gx[s] - gn);
+            fsx[s] = (s ? -0.5 : 0.5) * (w[0][s] - o[0]);
+        } else if (active) {
+            fvx[s] = (s ? -1.0 : 1.0) * gx[s];
+        }
+    }
+    double v[N1];
+#pragma unroll
+    for (int a = 0; a < N1; ++a) v[a] = w[0][a];
+    __syncthreads();
+
+    // ---- y and z faces: each face pencil's fluxes once, into LDS
+#pragma unroll
+    for (int q0 = 0; q0 < NQ; q0 += NP) {
+        const int q = q0 + pc;
+        if (!active || q >= NQ) continue;
+        const int fi = DIM == 3 ? q / N1 : q;     // (r - 1) * 2 + s
+        const int k = DIM == 3 ? q % N1 : 0;
+        const int s = fi % 2, z = fi / 2;          // z: 0 a y face, 1 a z face
+        const int32_t nb = q0 == 0 ? nbq : p.nbr[(2 + fi) * p.n_elem + e];
+        double Jr[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) Jr[d] = z ? J[DIM - 1][d] : J[1][d];
+        const double* vo = s_v + le * S::ES + (z ? row(k, s) : row(s, k));
+        const double* go = s_g + (z * S::EPB + le) * S::ES + (z ? row(k, s) : row(s, k));
+        double* out = s_f + (le * NQ + q) * 2 * N1;
+        if (nb >= 0) {
+            double o[NF][N1];
+            if (kAhead && q0 == 0) {
+#pragma unroll
+                for (int f = 0; f < NF; ++f)
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) o[f][a] = wq[f][a];
+            } else {
+                double x[NF][N1];
+                load_pencils<NF, N1>(p.io, face_pencil(q, nb), NB, o, x);
+                mix_pencils<NF, N1>(p.io, face_pencil(q, nb), NB, o, x);
+            }
+            const double h = s ? -0.5 : 0.5;
+#pragma unroll
+            for (int a = 0; a < N1; ++a) {
+                double gn = 0.0;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) gn = fma(Jr[d], o[1 + d][a], gn);
+                out[a] = h * (go[a] - gn);
+                out[N1 + a] = h * (vo[a] - o[0][a]);
+            }
+        } else {
+            const double h = s ? -1.0 : 1.0;
+#pragma unroll
+            for (int a = 0; a < N1; ++a) {
+                out[a] = h * go[a];
+                out[N1 + a] = 0.0;
+            }
         }
     }
     __syncthreads();
     if (!active) return;
 
-    double Ji[DIM][DIM];
-#pragma unroll
-    for (int r = 0; r < DIM; ++r)
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) Ji[r][d] = p.jinv[(r * DIM + d) * p.n_elem + e];
-    const double cinv = p.cinv[e];
-
-    // g_r of a pencil from its s values
-    auto g_of = [&](const double* sv_base, int r, int a) {
-        double g = 0;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) g += Ji[r][d] * sv_base[(1 + d) * NB + a];
-        return g;
-    };
-    T kv[N1], t[DIM][N1];
+    // ---- per direction: the one-dimensional operator on g_r and on v
+    double kv[N1], ks[DIM][N1];
 #pragma unroll
     for (int a = 0; a < N1; ++a) {
-        kv[a] = T(0);
-#pragma unroll
-        for (int r = 0; r < DIM; ++r) t[r][a] = T(0);
-    }
-    // x direction (own pencil, registers)
-#pragma unroll
-    for (int a = 0; a < N1; ++a) {
-        T sg = T(0), sv = T(0);
+        double x = 0.0, t = 0.0;
 #pragma unroll
         for (int j = 0; j < N1; ++j) {
-            double g0 = 0;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) g0 += Ji[0][d] * w[1 + d][j];
-            sg += s_D[a * N1 + j] * T(g0);
-            sv += s_D[a * N1 + j] * T(w[0][j]);
+            x = fma(p.Dr[a * N1 + j], gx[j], x);
+            t = fma(p.Dr[a * N1 + j], v[j], t);
         }
-        kv[a] += sg;
-        t[0][a] += sv;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            x = fma(p.Mi[a * N1 + s], fvx[s], x);
+            t = fma(p.Mi[a * N1 + s], fsx[s], t);
+        }
+        kv[a] = x;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) ks[d][a] = J[0][d] * t;
     }
-    // y (and z) directions from the element's other pencils
 #pragma unroll
     for (int r = 1; r < DIM; ++r) {
         const int my = r == 1 ? ib : ic;
+        const double* sv = s_v + le * S::ES;
+        const double* sg = s_g + ((r - 1) * S::EPB + le) * S::ES;
+        double t[N1];
+#pragma unroll
+        for (int a = 0; a < N1; ++a) t[a] = 0.0;
 #pragma unroll
         for (int j = 0; j < N1; ++j) {
-            const int opc = r == 1 ? j + N1 * ic : ib + N1 * j;
-            const double* ob = sw + opc * N1;
-            const T dr = s_D[my * N1 + j];
+            const double dr = p.Dr[my * N1 + j];
+            const int at = r == 1 ? row(j, ic) : row(ib, j);
 #pragma unroll
             for (int a = 0; a < N1; ++a) {
-                kv[a] += dr * T(g_of(ob, r, a));
-                t[r][a] += dr * T(ob[a]);
+                kv[a] = fma(dr, sg[at + a], kv[a]);
+                t[a] = fma(dr, sv[at + a], t[a]);
             }
         }
-    }
-    Acc<T> av[N1], as[DIM][N1];
-#pragma unroll
-    for (int a = 0; a < N1; ++a) {
-        av[a] = Acc<T>(kv[a]);
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            T v = T(0);
-#pragma unroll
-            for (int r = 0; r < DIM; ++r) v += T(Ji[r][d]) * t[r][a];
-            as[d][a] = Acc<T>(v);
-        }
-    }
-
-    // faces
-#pragma unroll
-    for (int df = 0; df < DIM; ++df) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            const int f = 2 * df + s;
-            const int64_t nb = p.nbr[f * p.n_elem + e];
-            double wk[DIM];
+            const double mi = p.Mi[my * N1 + s];
+            const int q = DIM == 3 ? ((r - 1) * 2 + s) * N1 + (r == 1 ? ic : ib) : s;
+            const double* f = s_f + (le * NQ + q) * 2 * N1;
 #pragma unroll
-            for (int k = 0; k < DIM; ++k) wk[k] = (2 * s - 1) * Ji[df][k];
-            if (df == 0) {
-                // one trace value per field for this pencil
-                double own[NF], oth[NF];
-#pragma unroll
-                for (int q = 0; q < NF; ++q) own[q] = w[q][s];
-                if (nb >= 0) {
-                    const int64_t lnb = nb - blk * S::EPB;
-                    if (lnb >= 0 && lnb < S::EPB) {  // neighbour in this block
-#pragma unroll
-                        for (int q = 0; q < NF; ++q) oth[q] = s_w[(lnb * NF + q) * NB + pc * N1 + (1 - s)];
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < NF; ++q) oth[q] = combine(p.io, nb * NF * NB + q * NB + pc * N1 + (1 - s));
-                    }
-                }
-                double cv = 0, cd = 0;
-                if (nb >= 0) {
-#pragma unroll
-                    for (int k = 0; k < DIM; ++k) cv += wk[k] * (own[1 + k] - oth[1 + k]);
-                    cv *= -0.5;
-                    cd = -0.5 * (own[0] - oth[0]);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < DIM; ++k) cv -= wk[k] * own[1 + k];
-                }
-#pragma unroll
-                for (int a = 0; a < N1; ++a) {
-                    av[a].add(s_Mi[s * N1 + a] * T(cv));
-                    if (nb >= 0)
-#pragma unroll
-                        for (int d = 0; d < DIM; ++d) as[d][a].add(s_Mi[s * N1 + a] * T(wk[d] * cd));
-                }
-            } else {
-                const int own_pc = df == 1 ? s + N1 * ic : ib + N1 * s;
-                const int nbr_pc = df == 1 ? (1 - s) + N1 * ic : ib + N1 * (1 - s);
-                const int my = df == 1 ? ib : ic;
-                double oth[NF][N1];
-                if (nb >= 0) {
-                    const int64_t lnb = nb - blk * S::EPB;
-                    if (lnb >= 0 && lnb < S::EPB) {
-#pragma unroll
-                        for (int q = 0; q < NF; ++q)
-#pragma unroll
-                            for (int a = 0; a < N1; ++a) oth[q][a] = s_w[(lnb * NF + q) * NB + nbr_pc * N1 + a];
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < NF; ++q)
-                            combine_pencil<N1>(p.io, nb * NF * NB + q * NB + nbr_pc * N1, oth[q]);
-                    }
-                }
-                const T m = s_Mi[s * N1 + my];
-#pragma unroll
-                for (int a = 0; a < N1; ++a) {
-                    double cv = 0, cd = 0;
-                    if (nb >= 0) {
-#pragma unroll
-                        for (int k = 0; k < DIM; ++k) cv += wk[k] * (sw[(1 + k) * NB + own_pc * N1 + a] - oth[1 + k][a]);
-                        cv *= -0.5;
-                        cd = -0.5 * (sw[own_pc * N1 + a] - oth[0][a]);
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < DIM; ++k) cv -= wk[k] * sw[(1 + k) * NB + own_pc * N1 + a];
-                    }
-                    av[a].add(m * T(cv));
-                    if (nb >= 0)
-#pragma unroll
-                        for (int d = 0; d < DIM; ++d) as[d][a].add(m * T(wk[d] * cd));
-                }
+            for (int a = 0; a < N1; ++a) {
+                kv[a] = fma(mi, f[a], kv[a]);
+                t[a] = fma(mi, f[N1 + a], t[a]);
             }
         }
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+#pragma unroll
+            for (int a = 0; a < N1; ++a) ks[d][a] = fma(J[r][d], t[a], ks[d][a]);
     }
+    const double ci = 1.0 / p.cinv[e];
     const int64_t o = base + pc * N1;
-    const T ci = T(1.0 / cinv);
-    double ks_out[NF][N1];  // the values as stored
-    if (p.io.out_f32) {
-        float* out = static_cast<float*>(p.io.out);
+    store_pencil<N1>(p.io, o, kv);
+    if constexpr (kEarly) update_store<N1>(p.io.upd, o, kv, y[0]);
+    else if constexpr (UPD) rk_update_run<N1>(p.io.upd, o, kv);
 #pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            const float v = float(av[a].value());
-            out[o + a] = v;
-            ks_out[0][a] = double(v);
+    for (int d = 0; d < DIM; ++d) {
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                const float vs = float(ci * as[d][a].value());
-                out[o + (1 + d) * NB + a] = vs;
-                ks_out[1 + d][a] = double(vs);
-            }
-        }
-    } else {
-        double* out = static_cast<double*>(p.io.out);
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            const double v = double(av[a].value());
-            out[o + a] = v;
-            ks_out[0][a] = v;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                const double vs = double(ci * as[d][a].value());
-                out[o + (1 + d) * NB + a] = vs;
-                ks_out[1 + d][a] = vs;
-            }
-        }
-    }
-    if constexpr (UPD) {
-#pragma unroll
-        for (int f = 0; f < NF; ++f) rk_update_run<N1>(p.io.upd, o + f * NB, ks_out[f]);
+        for (int a = 0; a < N1; ++a) ks[d][a] *= ci;
+        store_pencil<N1>(p.io, o + (1 + d) * NB, ks[d]);
+        if constexpr (kEarly) update_store<N1>(p.io.upd, o + (1 + d) * NB, ks[d], y[1 + d]);
+        else if constexpr (UPD) rk_update_run<N1>(p.io.upd, o + (1 + d) * NB, ks[d]);
     }
 }
 
 // UPD: the RK update fused into this (last) stage, StageIO::upd.
-template <int DIM, int N1, typename T, bool UPD = false>
-__device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t blk) {
-    if constexpr (AcousticShape<DIM, N1>::QUAD) acoustic_block_quad<DIM, N1, T, UPD>(p, blk);
-    else acoustic_block_pencil<DIM, N1, T, UPD>(p, blk);
+template <int DIM, int N1, bool UPD = false>
+__global__ __launch_bounds__((AcousticShape<DIM, N1>::THREADS)) void tensor_acoustic_rhs(const AcousticParams p) {
+    acoustic_block<DIM, N1, UPD>(p, xcd_block(blockIdx.x, gridDim.x));
 }
 
-template <int DIM, int N1, typename T, bool UPD = false>
-__global__ __launch_bounds__(kBlock) void tensor_acoustic_rhs(const AcousticParams p) {
-    acoustic_block<DIM, N1, T, UPD>(p, xcd_block(blockIdx.x, gridDim.x));
-}
-
-template <int DIM, int N1, typename T, bool UPD = false>
-__global__ __launch_bounds__(kBlock) void tensor_acoustic_rhs_batched(const AcousticParams* ps, const int64_t* off,
-                                                                      int n) {
+template <int DIM, int N1, bool UPD = false>
+__global__ __launch_bounds__((AcousticShape<DIM, N1>::THREADS)) void tensor_acoustic_rhs_batched(
+    const AcousticParams* __restrict__ ps, const int64_t* __restrict__ off, int n) {
     const int64_t b = xcd_block(blockIdx.x, gridDim.x);
-    const int s = find_problem(off, n, b);
-    acoustic_block<DIM, N1, T, UPD>(ps[s], b - off[s]);
+    const int s = __builtin_amdgcn_readfirstlane(find_problem(off, n, b));
+    acoustic_block<DIM, N1, UPD>(ps[s], b - off[s]);
 }
 
 // L2 projection of f(x) = sum_m amp_m sin(2 pi k_m . x) on affine tensor
@@ -1893,7 +1779,6 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
         tensor_general_rhs(c, io);
         return;
     }
-    const bool mixed = c->op.precision == HGDG_PREC_MIXED_FP32;
     if (c->op.kind == HGDG_OP_ACOUSTIC_CENTRAL) {
         AcousticParams a{};
         a.n_elem = c->n_elem;
@@ -1907,18 +1792,11 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
             constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
             using S = AcousticShape<DIMc, N1c>;
             const int64_t grid = (c->n_elem + S::EPB - 1) / S::EPB;
-            const bool upd = io.upd.u != nullptr;  // the fused RK update of a step's last stage
-            if (mixed && upd)
-                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, float, true>), dim3(unsigned(grid)), dim3(kBlock),
-                                   0, c->stream, a);
-            else if (mixed)
-                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, float>), dim3(unsigned(grid)), dim3(kBlock), 0,
+            if (io.upd.u != nullptr)  // the fused RK update of a step's last stage
+                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, true>), dim3(unsigned(grid)), dim3(S::THREADS), 0,
                                    c->stream, a);
-            else if (upd)
-                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, double, true>), dim3(unsigned(grid)),
-                                   dim3(kBlock), 0, c->stream, a);
             else
-                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, double>), dim3(unsigned(grid)), dim3(kBlock), 0,
+                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c>), dim3(unsigned(grid)), dim3(S::THREADS), 0,
                                    c->stream, a);
         });
         HGDG_HIP(hipGetLastError());
@@ -2128,11 +2006,12 @@ void tensor_batch_launch(hipStream_t stream, int kind, int dim, int n1, bool mix
     dispatch_tensor(dim, n1, [&](auto D, auto N) {
         constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
         const dim3 grid{unsigned(blocks), 1, 1}, block{unsigned(kBlock), 1, 1};
+        const dim3 acoustic_block{unsigned(AcousticShape<DIMc, N1c>::THREADS), 1, 1};
         auto go = [&](auto T_, auto U_) {
             using Tc = decltype(T_);
             constexpr bool Uc = decltype(U_)::value;
             if (kind == HGDG_OP_ACOUSTIC_CENTRAL)
-                hipLaunchKernelGGL((tensor_acoustic_rhs_batched<DIMc, N1c, Tc, Uc>), grid, block, 0, stream,
+                hipLaunchKernelGGL((tensor_acoustic_rhs_batched<DIMc, N1c, Uc>), grid, acoustic_block, 0, stream,
                                    static_cast<const AcousticParams*>(params), off, n);
             else
                 hipLaunchKernelGGL((tensor_advection_rhs_batched<DIMc, N1c, Tc, Uc>), grid, block, 0, stream,

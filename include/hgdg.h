@@ -61,9 +61,10 @@ enum {
 /* ---- arithmetic of the bulk contractions ------------------------------- */
 enum {
     HGDG_PREC_FP64 = 0,       /* everything FP64 (the parity path)                  */
-    HGDG_PREC_MIXED_FP32 = 1  /* FP32 contractions, FP32 stage derivatives,
-                                 compensated FP32 face sums; FP64 geometry, state
-                                 and RK update                                      */
+    HGDG_PREC_MIXED_FP32 = 1  /* FP32 stage derivatives; FP32 contractions with
+                                 compensated FP32 face sums where they are faster
+                                 (tensor advection, tetrahedra), FP64 elsewhere;
+                                 FP64 geometry, state and RK update                 */
 };
 
 /*
