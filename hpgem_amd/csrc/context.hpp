@@ -41,11 +41,11 @@ struct TensorMesh {
 // layout, per element row a diagonal block and one block per face neighbour.
 struct MatrixOp {
     bool on = false;
-    int max_rows = 0;
-    std::vector<int64_t> elem_off, sq_off, row_ptr, blk_off;
-    std::vector<int32_t> blk_col;
-    DevBuf<int64_t> d_elem_off, d_sq_off, d_row_ptr, d_blk_off;
-    DevBuf<int32_t> d_blk_col;
+    int max_rows = 0;      // largest element block
+    int64_t max_cols = 0;  // most columns of an element row
+    std::vector<int64_t> elem_off, sq_off;
+    DevBuf<int64_t> d_elem_off, d_sq_off, d_col_ptr, d_row_off;
+    DevBuf<uint32_t> d_col;  // per column of an element row: the unknown it multiplies
     DevBuf<double> d_pool, d_minv, d_mass;
 };
 

@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "context.hpp"
@@ -32,78 +33,129 @@ namespace {
 
 constexpr int kMatThreads = 256;
 constexpr int kMatMaxRows = 4 * kMatThreads;  // rows per element a workgroup takes
+constexpr int kMatCols = 2048;                // columns of an element row staged in LDS at a time
+constexpr int kMatAhead = 8;                  // matrix loads a thread keeps in flight
 
 struct MatParams {
     int64_t n_elem;
     StageIO io;
     const int64_t* elem_off;  // [E + 1]
-    const int64_t* row_ptr;   // [E + 1] block entries of each element row
-    const int64_t* blk_off;   // [entries] offset of the block in pool
-    const int32_t* blk_col;   // [entries] trial element
+    const int64_t* col_ptr;   // [E + 1] columns of each element row
+    const uint32_t* col;      // [columns] the unknown each column multiplies
+    const int64_t* row_off;   // [E] offset of the element row's first block in pool
     const double* pool;
     const int64_t* sq_off;    // [E] offset of element e's n_e x n_e matrices in minv / mass
     const double* minv;       // NULL: no mass solve
+    int32_t cols;             // columns the LDS stage holds
 };
 
+// a += sum over this thread's columns j = g, g + G, .. < nc of B[i + n j] x[j],
+// B column-major with n rows: consecutive threads (i fast, g slow) read
+// consecutive values.
+__device__ __forceinline__ double mat_columns(const double* __restrict__ B, int n, int i, int g, int G, int nc,
+                                              const double* x, double a) {
+    for (int j0 = g; j0 < nc; j0 += kMatAhead * G) {
+        double b[kMatAhead];
+#pragma unroll
+        for (int u = 0; u < kMatAhead; ++u) {
+            const int j = j0 + u * G;
+            b[u] = j < nc ? __builtin_nontemporal_load(B + (i + int64_t(n) * j)) : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kMatAhead; ++u) {
+            const int j = j0 + u * G;
+            if (j < nc) a = fma(b[u], x[j], a);
+        }
+    }
+    return a;
+}
+
 // r_e = sum over the element row's blocks of B w_trial (w = the stage
-// combination), then k_e = M_e^{-1} r_e when minv is set. One workgroup per
-// element; rows over threads, trial values through LDS.
-__global__ __launch_bounds__(kMatThreads) void matrix_rhs(const MatParams p) {
+// combination), then k_e = M_e^{-1} r_e when minv is set. One workgroup of T
+// threads per element. The blocks of an element row lie one after another in
+// the pool, column-major, so they are one n x N matrix: its N trial values go
+// to LDS, and with n <= T the threads take G = T / n columns at once, n rows
+// each, so that every thread streams matrix values and consecutive threads
+// read consecutive ones; the G partial sums of a row meet in LDS. With n > T a
+// thread takes up to four rows of every column.
+// Bound by HBM: every matrix value is read once, with eight loads in flight per
+// thread (non-temporal: nothing of a matrix is read twice). One block at a time
+// behind its own barriers, with n threads of 256, read 1.8 TB/s at n = 27 and
+// 7 blocks a row (5760 elements, 268 MB: 148 us); this form takes 47 us, 5.7
+// TB/s (n = 8: 51 -> 8 us; n = 64, 1680 elements: 151 -> 75).
+template <int T>
+__global__ __launch_bounds__(T) void matrix_rhs(const MatParams p) {
     extern __shared__ double sh[];
-    const int64_t e = blockIdx.x;
+    double* red = sh + p.cols;  // [max(T, n)]
+    constexpr int R = T == kMatThreads ? kMatMaxRows / T : 1;  // smaller workgroups only take n <= T
+    const int64_t e = xcd_block(blockIdx.x, gridDim.x);
     const int64_t o = p.elem_off[e];
     const int n = int(p.elem_off[e + 1] - o);
-    double acc[4] = {0, 0, 0, 0};
-    for (int64_t k = p.row_ptr[e]; k < p.row_ptr[e + 1]; ++k) {
-        const int64_t t = p.blk_col[k];
-        const int64_t ot = p.elem_off[t];
-        const int nt = int(p.elem_off[t + 1] - ot);
-        for (int j = threadIdx.x; j < nt; j += kMatThreads) sh[j] = combine(p.io, ot + j);
+    const int64_t c0 = p.col_ptr[e], nc = p.col_ptr[e + 1] - c0;
+    const double* B = p.pool + p.row_off[e];
+    const int t = threadIdx.x;
+    const bool narrow = n <= T;
+    const int G = narrow ? T / n : 1, i = narrow ? t % n : t, g = narrow ? t / n : 0;
+    double acc[R] = {};
+    for (int64_t j0 = 0; j0 < nc; j0 += p.cols) {
+        const int m = int(nc - j0 < p.cols ? nc - j0 : p.cols);
+        if (j0 > 0) __syncthreads();  // the previous columns' readers are done
+        for (int j = t; j < m; j += T) sh[j] = combine(p.io, p.col[c0 + j0 + j]);
         __syncthreads();
-        const double* B = p.pool + p.blk_off[k];
+        const double* Bj = B + int64_t(n) * j0;
+        if (narrow) {
+            if (g < G) acc[0] = mat_columns(Bj, n, i, g, G, m, sh, acc[0]);
+        } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int i = threadIdx.x + s * kMatThreads;
-            if (i >= n) break;
-            double a = acc[s];
-            for (int j = 0; j < nt; ++j) a += B[i + int64_t(n) * j] * sh[j];
-            acc[s] = a;
+            for (int s = 0; s < R; ++s)
+                if (t + s * T < n) acc[s] = mat_columns(Bj, n, t + s * T, 0, 1, m, sh, acc[s]);
         }
-        __syncthreads();
     }
+    // the partial sums of a row; afterwards thread t (+ s T) holds row t (+ s T)
+    auto gather = [&] {
+        red[t] = acc[0];
+        __syncthreads();
+        if (t < n) {
+            double a = red[t];
+            for (int q = 1; q < G; ++q) a += red[t + n * q];
+            acc[0] = a;
+        }
+    };
+    if (narrow) gather();
     if (p.minv) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int i = threadIdx.x + s * kMatThreads;
-            if (i < n) sh[i] = acc[s];
-        }
-        __syncthreads();
         const double* Mi = p.minv + p.sq_off[e];
+        if (narrow) {
+            if (t < n) sh[t] = acc[0];  // every reader of the stage passed gather()'s barrier
+            __syncthreads();
+            acc[0] = 0.0;
+            if (g < G) acc[0] = mat_columns(Mi, n, i, g, G, n, sh, 0.0);
+            gather();
+        } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int i = threadIdx.x + s * kMatThreads;
-            if (i >= n) break;
-            double a = 0;
-            for (int j = 0; j < n; ++j) a += Mi[i + int64_t(n) * j] * sh[j];
-            acc[s] = a;
+            for (int s = 0; s < R; ++s)
+                if (t + s * T < n) red[t + s * T] = acc[s];
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+                if (t + s * T < n) acc[s] = mat_columns(Mi, n, t + s * T, 0, 1, n, red, 0.0);
         }
     }
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const int i = threadIdx.x + s * kMatThreads;
-        if (i >= n) break;
+    for (int s = 0; s < R; ++s) {
+        const int r = t + s * T;
+        if (r >= n) break;
         double kept;  // the value as stored
         if (p.io.out_f32) {
             const float v = float(acc[s]);
-            static_cast<float*>(p.io.out)[o + i] = v;
+            static_cast<float*>(p.io.out)[o + r] = v;
             kept = double(v);
         } else {
-            static_cast<double*>(p.io.out)[o + i] = acc[s];
+            static_cast<double*>(p.io.out)[o + r] = acc[s];
             kept = acc[s];
         }
         if (p.io.upd.u != nullptr) {  // the RK update fused into a step's last stage (StageIO::upd)
             const double own[1] = {kept};
-            rk_update_run<1>(p.io.upd, o + i, own);
+            rk_update_run<1>(p.io.upd, o + r, own);
         }
     }
 }
@@ -257,22 +309,26 @@ void matrix_operator_set(hgdg_ctx* c, const hgdg_matrix_desc* d, int precision) 
     }
     std::stable_sort(cross.begin(), cross.end(), [](const Cross& a, const Cross& b) { return a.row < b.row; });
     std::vector<double> pool;
-    m.row_ptr.assign(size_t(ne) + 1, 0);
+    std::vector<int64_t> col_ptr(size_t(ne) + 1, 0), row_off(static_cast<size_t>(ne));
+    std::vector<uint32_t> col;
+    auto columns = [&](int64_t t) {
+        for (int64_t j = m.elem_off[size_t(t)]; j < m.elem_off[size_t(t) + 1]; ++j) col.push_back(uint32_t(j));
+    };
     size_t ci = 0;
     for (int64_t e = 0; e < ne; ++e) {
-        m.blk_off.push_back(int64_t(pool.size()));
-        m.blk_col.push_back(int32_t(e));
+        row_off[size_t(e)] = int64_t(pool.size());
+        columns(e);
         pool.insert(pool.end(), diag[size_t(e)].begin(), diag[size_t(e)].end());
         diag[size_t(e)].clear();
         diag[size_t(e)].shrink_to_fit();
         for (; ci < cross.size() && cross[ci].row == e; ++ci) {
             const Cross& x = cross[ci];
             const int64_t n = d->block_size[e], nt = d->block_size[x.col];
-            m.blk_off.push_back(int64_t(pool.size()));
-            m.blk_col.push_back(int32_t(x.col));
+            columns(x.col);
             pool.insert(pool.end(), d->face_blocks + x.at, d->face_blocks + x.at + n * nt);
         }
-        m.row_ptr[size_t(e) + 1] = int64_t(m.blk_off.size());
+        col_ptr[size_t(e) + 1] = int64_t(col.size());
+        m.max_cols = std::max(m.max_cols, col_ptr[size_t(e) + 1] - col_ptr[size_t(e)]);
     }
     std::vector<double> minv(static_cast<size_t>(sq));
     for (int64_t e = 0; e < ne; ++e) {
@@ -284,9 +340,9 @@ void matrix_operator_set(hgdg_ctx* c, const hgdg_matrix_desc* d, int precision) 
     c->vecs.clear();
     m.d_elem_off.upload(m.elem_off, c->stream);
     m.d_sq_off.upload(m.sq_off, c->stream);
-    m.d_row_ptr.upload(m.row_ptr, c->stream);
-    m.d_blk_off.upload(m.blk_off, c->stream);
-    m.d_blk_col.upload(m.blk_col, c->stream);
+    m.d_col_ptr.upload(col_ptr, c->stream);
+    m.d_col.upload(col, c->stream);
+    m.d_row_off.upload(row_off, c->stream);
     m.d_pool.upload(pool, c->stream);
     m.d_minv.upload(minv, c->stream);
     m.d_mass.upload(std::vector<double>(d->mass, d->mass + sq), c->stream);
@@ -310,15 +366,26 @@ void matrix_rhs(hgdg_ctx* c, const StageIO& io, bool solve) {
     p.n_elem = c->n_elem;
     p.io = io;
     p.elem_off = c->mat.d_elem_off.ptr;
-    p.row_ptr = c->mat.d_row_ptr.ptr;
-    p.blk_off = c->mat.d_blk_off.ptr;
-    p.blk_col = c->mat.d_blk_col.ptr;
+    p.col_ptr = c->mat.d_col_ptr.ptr;
+    p.col = c->mat.d_col.ptr;
+    p.row_off = c->mat.d_row_off.ptr;
     p.pool = c->mat.d_pool.ptr;
     p.sq_off = c->mat.d_sq_off.ptr;
     p.minv = solve ? c->mat.d_minv.ptr : nullptr;
-    // LDS: the largest trial block (any element's size) and the row values
-    const size_t lds = sizeof(double) * size_t(c->mat.max_rows);
-    hipLaunchKernelGGL(matrix_rhs, dim3(unsigned(c->n_elem)), dim3(kMatThreads), lds, c->stream, p);
+    p.cols = int32_t(std::max<int64_t>(std::min<int64_t>(c->mat.max_cols, kMatCols), c->mat.max_rows));
+    auto launch = [&](auto T_) {
+        constexpr int T = decltype(T_)::value;
+        const size_t lds = sizeof(double) * size_t(p.cols + std::max(T, c->mat.max_rows));
+        hipLaunchKernelGGL((matrix_rhs<T>), dim3(unsigned(c->n_elem)), dim3(T), lds, c->stream, p);
+    };
+    // By the largest block: a workgroup of 64 threads keeps more element rows
+    // in flight where they are short (5760 elements of n = 10: 11.8, 13.9 and
+    // 22.6 us with 64, 128 and 256 threads; n = 27: 47.4, 49.3, 47.9), 128 is
+    // best from there (1680 elements of n = 40: 33.3, 30.3, 33.5; n = 64 alike);
+    // beyond 128 rows the widest form has the most threads on rows.
+    if (c->mat.max_rows <= 32) launch(std::integral_constant<int, 64>{});
+    else if (c->mat.max_rows <= 128) launch(std::integral_constant<int, 128>{});
+    else launch(std::integral_constant<int, kMatThreads>{});
     HGDG_HIP(hipGetLastError());
 }
 
