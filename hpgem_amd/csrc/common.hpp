@@ -62,6 +62,11 @@ __device__ __forceinline__ int64_t xcd_block(int64_t b, int64_t n) {
     return x * q + (x < r ? x : r) + b / kXcds;
 }
 
+// Has x formed here. A value used only after a barrier is otherwise free to be
+// formed there, and then every operand it is made of (loads from LDS and
+// memory cannot move) holds its registers until then.
+__device__ __forceinline__ void form_here(double& x) { asm volatile("" : "+v"(x)); }
+
 // The RK update of a step, fused into its last stage's kernel:
 // y_new = u + sum_j c_j x_j, the terms added one after another in FP64 (the
 // operations of multi_axpy, so the result is bitwise the same), where term

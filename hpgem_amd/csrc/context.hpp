@@ -34,6 +34,7 @@ struct TensorMesh {
     std::vector<int32_t> gnbr;       // [2 dim][e] neighbour per local face (hpGEM numbering) or -1
     std::vector<int32_t> ginfo;      // [2 dim][e] neighbour's face, point map, left flag
     DevBuf<double> d_gX, d_gtab, d_gcinv;
+    DevBuf<double> d_ggeo, d_gfgeo;  // the RHS kernel's geometry per point and per face point
     DevBuf<int32_t> d_gface;         // gnbr then ginfo
 };
 

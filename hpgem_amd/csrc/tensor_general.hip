@@ -185,7 +185,7 @@ __device__ inline double along_val(const double* M, int ax, int t, const double*
     const int t0 = t - i * st;
     double s = 0;
 #pragma unroll
-    for (int m = 0; m < N1; ++m) s += (TRANSPOSE ? M[m * N1 + i] : M[i * N1 + m]) * in[t0 + m * st];
+    for (int m = 0; m < N1; ++m) s = fma(TRANSPOSE ? M[m * N1 + i] : M[i * N1 + m], in[t0 + m * st], s);
     return s;
 }
 
@@ -210,289 +210,338 @@ __host__ __device__ __forceinline__ void partner_point(int code, int ka, int kb,
 struct GenParams {
     int64_t n_elem;
     StageIO io;
-    const double* X;       // [E][NV][DIM] vertex coordinates
     const int32_t* nbr;    // [NFACE][E]
     const int32_t* info;   // [NFACE][E]
     const double* tab;     // NodalOps of the order, packed
+    const double* geo;     // per point, GenRhs::GP numbers [E][GP][NP]
+    const double* fgeo;    // per face point, GenRhs::GF numbers [E][NFACE][GF][NFP]
     const double* cinv;    // [E] (acoustic)
-    double a[3];           // advection velocity
 };
 
+// One thread per point. Threads of a workgroup: the smallest of 64, 128 and
+// 256 that whole elements fill to 15/16, or as many elements as 256 hold.
 template <int DIM, int N1, bool ACOUSTIC>
-struct GenLds {
+struct GenRhs {
     using S = GenShape<DIM, N1>;
     static constexpr int NF = ACOUSTIC ? DIM + 1 : 1;
-    // per element, in doubles
-    static constexpr int XV = 0;                                    // [NV][DIM] own vertices
-    static constexpr int XN = XV + S::NV * DIM;                     // [NFACE][NV][DIM] left neighbours' vertices
-    static constexpr int U = XN + S::NFACE * S::NV * DIM;           // [NF][NP] stage input (coefficients)
-    static constexpr int A = U + NF * S::NP;                        // [NF][NP] work
-    static constexpr int B = A + NF * S::NP;                        // [NF][NP] work
-    static constexpr int F = B + NF * S::NP;                        // [DIM][NP] advection fluxes at the points
-    static constexpr int NB = F + (ACOUSTIC ? 0 : DIM * S::NP);     // [NFACE][NF][NFP] neighbours' face coefficients
-    static constexpr int FC = NB + S::NFACE * NF * S::NFP;          // [NFACE][NF][NFP] face integrands
-    static constexpr int PER = FC + S::NFACE * NF * S::NFP;
+    static constexpr int NP = S::NP, NFP = S::NFP, NFACE = S::NFACE;
+    static constexpr int EPB = (64 % NP) * 16 <= 64 ? 64 / NP : (128 % NP) * 16 <= 128 ? 128 / NP : 256 / NP;
+    static constexpr int THREADS = EPB * NP;
+    // stored geometry. Per point: acoustic J^{-1} and 1/W; advection W ahat_r
+    // and 1/W (W the point's weight times |det J|). Per face point: acoustic
+    // the own outward normal times the face's weight and area element;
+    // advection the two factors of the own and the neighbour's trace in the
+    // flux, upwinding included.
+    static constexpr int GP = (ACOUSTIC ? DIM * DIM : DIM) + 1;
+    static constexpr int GF = ACOUSTIC ? DIM : 2;
+    // face values of all fields per element, and how many a thread loads
+    static constexpr int NI = NFACE * NF * NFP;
+    static constexpr int KI = (NI + NP - 1) / NP;
+    static constexpr int KF = (NFACE * NFP + NP - 1) / NP;  // face points per thread
+    // LDS per element, in doubles: two work arrays, the advection fluxes, the
+    // neighbours' face coefficients, and (3D) those with the first face
+    // coordinate at points; the face integrands overlay the coefficients in 3D
+    static constexpr int A = 0, B = NF * NP, F = 2 * NF * NP, NBC = F + (ACOUSTIC ? 0 : DIM * NP), NBT = NBC + NI,
+                         PER = NBT + NI;
+    static constexpr int FC = DIM == 3 ? NBC : NBT;
+};
+
+// The geometry a mesh and an operator fix, once per operator: thread t of
+// element e takes point t and the face points t, t + NP, ..
+struct GenGeoParams {
+    int64_t n_elem;
+    const double* X;       // [E][NV][DIM] vertex coordinates
+    const int32_t* nbr;
+    const int32_t* info;
+    const double* tab;
+    double a[3];           // advection velocity
+    double* geo;
+    double* fgeo;
 };
 
 template <int DIM, int N1, bool ACOUSTIC>
-__global__ __launch_bounds__(kGenTarget) void tensor_general_rhs(const GenParams p) {
-    using S = GenShape<DIM, N1>;
-    using L = GenLds<DIM, N1, ACOUSTIC>;
+__global__ __launch_bounds__(kGenTarget) void tensor_general_geometry(const GenGeoParams p) {
+    using G = GenRhs<DIM, N1, ACOUSTIC>;
     using T = NodalTab<N1>;
-    constexpr int NP = S::NP, NFP = S::NFP, NV = S::NV, NFACE = S::NFACE, NF = L::NF;
-    __shared__ double lds[S::EPB * L::PER];
+    constexpr int NP = G::NP, NFP = G::NFP, NV = G::S::NV, NFACE = G::NFACE;
+    const int t = threadIdx.x % NP;
+    const int64_t e = int64_t(blockIdx.x) * G::EPB + threadIdx.x / NP;
+    if (e >= p.n_elem) return;
+    const double* tab = p.tab;
+    const double* X = p.X + e * NV * DIM;
+    const int ii[3] = {t % N1, (t / N1) % N1, DIM == 3 ? t / (N1 * N1) : 0};
+    double xi[DIM], J[DIM][DIM], Ji[DIM][DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) xi[d] = tab[T::X + ii[d]];
+    multilinear<DIM>(X, xi, J, nullptr);
+    double W = fabs(det_inv<DIM>(J, Ji));
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) W *= tab[T::W + ii[d]];
+    double* geo = p.geo + e * G::GP * NP + t;
+#pragma unroll
+    for (int r = 0; r < DIM; ++r) {
+        double ah = 0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            if constexpr (ACOUSTIC) geo[(r * DIM + d) * NP] = Ji[r][d];
+            else ah += Ji[r][d] * p.a[d];
+        }
+        if constexpr (!ACOUSTIC) geo[r * NP] = W * ah;
+    }
+    geo[(G::GP - 1) * NP] = 1.0 / W;
+    for (int it = t; it < NFACE * NFP; it += NP) {
+        const int f = it / NFP, k = it % NFP;
+        const int ka = k % N1, kb = DIM == 3 ? k / N1 : 0;
+        const int32_t nb = p.nbr[f * p.n_elem + e];
+        const int32_t info = p.info[f * p.n_elem + e];
+        const bool inner = nb >= 0;
+        const bool left = !inner || ((info >> 6) & 1);
+        // the left element's normal and area element at its point
+        int qa = ka, qb = kb;
+        if (!left) partner_point((info >> 3) & 7, ka, kb, N1, qa, qb);
+        double n[DIM];
+        face_normal<DIM, N1>(left ? X : p.X + int64_t(nb) * NV * DIM, left ? f : (info & 7), qa, qb, tab, n);
+        double area = 0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) area += n[d] * n[d];
+        area = sqrt(area);
+        double wf = tab[T::W + qa];
+        if constexpr (DIM == 3) wf *= tab[T::W + qb];
+        const double sgn = left ? 1.0 : -1.0;  // own normal = sgn n
+        double* out = p.fgeo + ((e * NFACE + f) * G::GF) * NFP + k;
+        if constexpr (ACOUSTIC) {
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) out[d * NFP] = sgn * n[d] * wf;
+        } else {
+            double An = 0;
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) An += p.a[d] * (n[d] / area);
+            // the trace of the flux: left, right (none on a boundary), or half of each
+            double cl = 0, cr = 0;
+            if (An > 1e-12) cl = 1;
+            else if (An < -1e-12) cr = 1;
+            else if (fabs(An) < 1e-12) cl = cr = 0.5;
+            const double flux = -(An * sgn) * (wf * area);
+            out[0] = flux * (left ? cl : cr);
+            out[NFP] = inner ? flux * (left ? cr : cl) : 0.0;
+        }
+    }
+}
+
+// Bound by the LDS reads and barriers of its one-dimensional contractions:
+// every operand but a row of the matrix comes from LDS. The geometry comes
+// from memory (3.5 KB an element at p = 2 in 3D, beside 2.6 KB of state): formed
+// from the vertices at every point and face point of every launch, it took 256
+// registers, a third of the LDS for the vertices and most of the time (FP64
+// acoustic, 22x18x20 p = 2: 114 us then, 24 now; 14x12x13 p = 3 70 and 14;
+// advection 22x18x20 p = 2 31.5 and 8.1). A face's traces at its points cost
+// N1 products each: the own one from the point values, the neighbour's one
+// face coordinate after the other. form_here on the volume sums takes the
+// acoustic p = 2 kernel from 208 to 108 registers.
+template <int DIM, int N1, bool ACOUSTIC>
+__global__ __launch_bounds__((GenRhs<DIM, N1, ACOUSTIC>::THREADS)) void tensor_general_rhs(const GenParams p) {
+    using G = GenRhs<DIM, N1, ACOUSTIC>;
+    using T = NodalTab<N1>;
+    constexpr int NP = G::NP, NFP = G::NFP, NFACE = G::NFACE, NF = G::NF;
+    __shared__ double lds[G::EPB * G::PER];
     __shared__ double tab[T::SIZE];
-    __shared__ int32_t s_nbr[S::EPB][NFACE], s_info[S::EPB][NFACE];
     const int tid = threadIdx.x;
     const int le = tid / NP;
     const int t = tid % NP;
-    const int64_t e = int64_t(blockIdx.x) * S::EPB + le;
+    const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t e = blk * G::EPB + le;
     const bool ok = e < p.n_elem;
     const int64_t E = p.n_elem;
-    double* sX = lds + le * L::PER + L::XV;
-    double* sXn = lds + le * L::PER + L::XN;
-    double* su = lds + le * L::PER + L::U;
-    double* sA = lds + le * L::PER + L::A;
-    double* sB = lds + le * L::PER + L::B;
-    double* sF = lds + le * L::PER + L::F;
-    double* snb = lds + le * L::PER + L::NB;
-    double* sc = lds + le * L::PER + L::FC;
-    for (int k = tid; k < T::SIZE; k += blockDim.x) tab[k] = p.tab[k];
+    double* sA = lds + le * G::PER + G::A;
+    double* sB = lds + le * G::PER + G::B;
+    double* snb = lds + le * G::PER + G::NBC;
+    double* sc = lds + le * G::PER + G::FC;
+    for (int k = tid; k < T::SIZE; k += G::THREADS) tab[k] = p.tab[k];
 
-    // ---- stage input, own vertices, faces; neighbours' face coefficients and,
-    // where this element is the right one, the left neighbour's vertices
+    // ---- stage input, neighbours' face coefficients, geometry
+    const int64_t base = e * NF * NP;
+    double gp[G::GP], gf[G::KF][G::GF];
+    int32_t fnb[G::KF], finfo[G::KF];
     if (ok) {
-        for (int k = t; k < NV * DIM; k += NP) sX[k] = p.X[e * NV * DIM + k];  // NP may be below NV * DIM
-        for (int k = t; k < NFACE; k += NP) {
-            s_nbr[le][k] = p.nbr[k * E + e];
-            s_info[le][k] = p.info[k * E + e];
-        }
-        const int64_t base = e * NF * NP;
+        int64_t at[G::KI];
 #pragma unroll
-        for (int fld = 0; fld < NF; ++fld) su[fld * NP + t] = combine(p.io, base + fld * NP + t);
-        constexpr int PERF = NV * DIM + NF * NFP;
-        for (int it = t; it < NFACE * PERF; it += NP) {
-            const int f = it / PERF;
-            int r = it % PERF;
+        for (int i = 0; i < G::KI; ++i) {
+            const int it = t + i * NP < G::NI ? t + i * NP : 0;
+            const int f = it / (NF * NFP), r = it % (NF * NFP), fld = r / NFP, k = r % NFP;
             const int32_t nb = p.nbr[f * E + e];
-            if (nb < 0) continue;
-            const int32_t info = p.info[f * E + e];
-            if (r < NV * DIM) {
-                if (!((info >> 6) & 1)) sXn[f * NV * DIM + r] = p.X[int64_t(nb) * NV * DIM + r];
-                continue;
+            const int fn = p.info[f * E + e] & 7;
+            int idx = face_side(DIM, fn) * ipow(N1, face_axis(DIM, fn)) +
+                      (k % N1) * ipow(N1, face_coord_axis(DIM, fn, 0));
+            if constexpr (DIM == 3) idx += (k / N1) * ipow(N1, face_coord_axis(DIM, fn, 1));
+            at[i] = (nb >= 0 ? int64_t(nb) * NF * NP : base) + fld * NP + idx;
+        }
+        int64_t own[NF];
+#pragma unroll
+        for (int fld = 0; fld < NF; ++fld) own[fld] = base + fld * NP + t;
+        double u[NF], v[G::KI];
+        combine_n<NF>(p.io, own, u);
+        combine_n<G::KI>(p.io, at, v);
+#pragma unroll
+        for (int c = 0; c < G::GP; ++c) gp[c] = p.geo[(e * G::GP + c) * NP + t];
+#pragma unroll
+        for (int i = 0; i < G::KF; ++i) {
+            const int it = t + i * NP < NFACE * NFP ? t + i * NP : 0;
+            const int f = it / NFP;
+            fnb[i] = p.nbr[f * E + e];
+            finfo[i] = p.info[f * E + e];
+#pragma unroll
+            for (int c = 0; c < G::GF; ++c)
+                gf[i][c] = p.fgeo[((e * NFACE + f) * G::GF + c) * NFP + it % NFP];
+        }
+#pragma unroll
+        for (int fld = 0; fld < NF; ++fld) sA[fld * NP + t] = u[fld];
+#pragma unroll
+        for (int i = 0; i < G::KI; ++i)
+            if (t + i * NP < G::NI) snb[t + i * NP] = v[i];
+    }
+    __syncthreads();
+
+    // ---- point values U = B u, one direction after the other; the first face
+    // coordinate of the neighbours' traces with the first of them
+    along<N1, NP, NF, false>(tab + T::B, 0, t, sA, sB);
+    if constexpr (DIM == 3) {
+        double* st = lds + le * G::PER + G::NBT;
+#pragma unroll
+        for (int i = 0; i < G::KI; ++i) {
+            const int it = t + i * NP;
+            if (it < G::NI) {
+                const int q = it % N1, row = it - q;
+                double s = 0;
+#pragma unroll
+                for (int a = 0; a < N1; ++a) s = fma(tab[T::B + q * N1 + a], snb[row + a], s);
+                st[it] = s;
             }
-            r -= NV * DIM;
-            const int fld = r / NFP, k = r % NFP;
-            const int fn = info & 7;
-            const int ka = k % N1, kb = k / N1;
-            int idx = face_side(DIM, fn) * ipow(N1, face_axis(DIM, fn)) + ka * ipow(N1, face_coord_axis(DIM, fn, 0));
-            if constexpr (DIM == 3) idx += kb * ipow(N1, face_coord_axis(DIM, fn, 1));
-            snb[(f * NF + fld) * NFP + k] = combine(p.io, int64_t(nb) * NF * NP + fld * NP + idx);
         }
     }
     __syncthreads();
-
-    // ---- point values U = B u (three passes through LDS) and the geometry at
-    // this thread's point
-    const int ii[3] = {t % N1, (t / N1) % N1, DIM == 3 ? t / (N1 * N1) : 0};
-    double Wq, Ji[DIM][DIM];
-    {
-        double xi[DIM], J[DIM][DIM];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) xi[d] = tab[T::X + ii[d]];
-        multilinear<DIM>(sX, xi, J, nullptr);
-        const double det = det_inv<DIM>(J, Ji);
-        Wq = fabs(det);
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) Wq *= tab[T::W + ii[d]];
-    }
-    along<N1, NP, NF, false>(tab + T::B, 0, t, su, sA);
+    along<N1, NP, NF, false>(tab + T::B, 1, t, sB, sA);
     __syncthreads();
-    along<N1, NP, NF, false>(tab + T::B, 1, t, sA, sB);
-    __syncthreads();
-    const double* Up = sB;
+    const double* Up = sA;
     if constexpr (DIM == 3) {
-        along<N1, NP, NF, false>(tab + T::B, 2, t, sB, sA);
+        along<N1, NP, NF, false>(tab + T::B, 2, t, sA, sB);
         __syncthreads();
-        Up = sA;
+        Up = sB;
     }
 
-    // ---- volume terms, as point residuals (W times the integrand's point value)
+    // ---- volume terms at the point
     double res[NF];
     if constexpr (!ACOUSTIC) {
-        double ah[DIM];
-#pragma unroll
-        for (int r = 0; r < DIM; ++r) {
-            ah[r] = 0;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) ah[r] += Ji[r][d] * p.a[d];
-        }
+        double* sF = lds + le * G::PER + G::F;
         const double u = Up[t];
 #pragma unroll
-        for (int r = 0; r < DIM; ++r) sF[r * NP + t] = Wq * ah[r] * u;
-        __syncthreads();
-        double v = 0;
-#pragma unroll
-        for (int r = 0; r < DIM; ++r) v += along_val<N1, true>(tab + T::C, r, t, sF + r * NP);
-        res[0] = v;
+        for (int r = 0; r < DIM; ++r) sF[r * NP + t] = gp[r] * u;
     } else {
-        // reference-coordinate derivatives of every field at this point
-        double g[NF][DIM];
 #pragma unroll
-        for (int fld = 0; fld < NF; ++fld)
+        for (int fld = 0; fld < NF; ++fld) res[fld] = 0.0;
 #pragma unroll
-            for (int r = 0; r < DIM; ++r) g[fld][r] = along_val<N1, false>(tab + T::C, r, t, Up + fld * NP);
-        double div = 0;
+        for (int r = 0; r < DIM; ++r) {
+            const double gv = along_val<N1, false>(tab + T::C, r, t, Up);
 #pragma unroll
-        for (int d = 0; d < DIM; ++d)
-#pragma unroll
-            for (int r = 0; r < DIM; ++r) div += Ji[r][d] * g[1 + d][r];
-        res[0] = Wq * div;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            double gv = 0;
-#pragma unroll
-            for (int r = 0; r < DIM; ++r) gv += Ji[r][d] * g[0][r];
-            res[1 + d] = Wq * gv;
+            for (int d = 0; d < DIM; ++d) {
+                const double Jrd = gp[r * DIM + d];
+                res[1 + d] = fma(Jrd, gv, res[1 + d]);
+                res[0] = fma(Jrd, along_val<N1, false>(tab + T::C, r, t, Up + (1 + d) * NP), res[0]);
+            }
         }
+#pragma unroll
+        for (int fld = 0; fld < NF; ++fld) form_here(res[fld]);
     }
 
-    // ---- face integrands at the face points: items (face, point)
+    // ---- face integrands at the face points
     if (ok) {
-        for (int it = t; it < NFACE * NFP; it += NP) {
+#pragma unroll
+        for (int i = 0; i < G::KF; ++i) {
+            const int it = t + i * NP;
+            if (it >= NFACE * NFP) continue;
             const int f = it / NFP, k = it % NFP;
-            const int ax = face_axis(DIM, f), side = face_side(DIM, f);
-            const int a0 = face_coord_axis(DIM, f, 0), a1 = DIM == 3 ? face_coord_axis(DIM, f, 1) : 0;
             const int ka = k % N1, kb = DIM == 3 ? k / N1 : 0;
-            const int stf = ipow(N1, 0) * (ax == 0 ? 1 : ax == 1 ? N1 : N1 * N1);
-            const int st0 = a0 == 0 ? 1 : a0 == 1 ? N1 : N1 * N1;
-            const int st1 = a1 == 0 ? 1 : a1 == 1 ? N1 : N1 * N1;
-            // own trace: the coefficients with index `side` along ax, at (ka, kb)
+            const int ax = face_axis(DIM, f), a0 = face_coord_axis(DIM, f, 0);
+            const int stf = ax == 0 ? 1 : ax == 1 ? N1 : N1 * N1;
+            const int st0 = a0 == 0 ? 1 : N1;  // the first face coordinate is x or y,
+            const int st1 = face_coord_axis(DIM, f, 1) == 1 ? N1 : N1 * N1;  // the second y or z
+            const double* lam = tab + (face_side(DIM, f) ? T::LAM1 : T::LAM0);
+            const double* uf = Up + ka * st0 + (DIM == 3 ? kb * st1 : 0);
+            const bool inner = fnb[i] >= 0;
+            int pa = ka, pb = kb;
+            if (inner) partner_point((finfo[i] >> 3) & 7, ka, kb, N1, pa, pb);
             double own[NF], nbv[NF];
 #pragma unroll
             for (int fld = 0; fld < NF; ++fld) {
-                double s = 0;
+                double s = 0, q = 0;
 #pragma unroll
-                for (int b = 0; b < (DIM == 3 ? N1 : 1); ++b) {
-                    double sa = 0;
-#pragma unroll
-                    for (int a = 0; a < N1; ++a) sa += tab[T::B + ka * N1 + a] * su[fld * NP + side * stf + a * st0 + b * st1];
-                    s += DIM == 3 ? tab[T::B + kb * N1 + b] * sa : sa;
+                for (int m = 0; m < N1; ++m) {
+                    s = fma(lam[m], uf[fld * NP + m * stf], s);
+                    const double* nf = lds + le * G::PER + (DIM == 3 ? G::NBT : G::NBC) + (f * NF + fld) * NFP;
+                    q = DIM == 3 ? fma(tab[T::B + pb * N1 + m], nf[pa + N1 * m], q)
+                                 : fma(tab[T::B + pa * N1 + m], nf[m], q);
                 }
                 own[fld] = s;
+                nbv[fld] = q;
             }
-            const int32_t nb = s_nbr[le][f];
-            const int32_t info = s_info[le][f];
-            const bool inner = nb >= 0;
-            const bool left = !inner || ((info >> 6) & 1);
-            int pa = ka, pb = kb;
-            if (inner) {
-                partner_point((info >> 3) & 7, ka, kb, N1, pa, pb);
-#pragma unroll
-                for (int fld = 0; fld < NF; ++fld) {
-                    const double* cf = snb + (f * NF + fld) * NFP;
-                    double s = 0;
-#pragma unroll
-                    for (int b = 0; b < (DIM == 3 ? N1 : 1); ++b) {
-                        double sa = 0;
-#pragma unroll
-                        for (int a = 0; a < N1; ++a) sa += tab[T::B + pa * N1 + a] * cf[a + N1 * b];
-                        s += DIM == 3 ? tab[T::B + pb * N1 + b] * sa : sa;
-                    }
-                    nbv[fld] = s;
-                }
-            }
-            // the left element's normal and area element at its point
-            double n[DIM];
-            int qa = ka, qb = kb;
-            if (left) {
-                face_normal<DIM, N1>(sX, f, ka, kb, tab, n);
-            } else {
-                qa = pa;
-                qb = pb;
-                face_normal<DIM, N1>(sXn + f * NV * DIM, info & 7, pa, pb, tab, n);
-            }
-            double area = 0;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) area += n[d] * n[d];
-            area = sqrt(area);
-            double wf = tab[T::W + qa];
-            if constexpr (DIM == 3) wf *= tab[T::W + qb];
-            wf *= area;
-            double nu[DIM];  // the left element's unit normal
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) nu[d] = n[d] / area;
-            const double sgn = left ? 1.0 : -1.0;  // own normal = sgn * nu
             double* out = sc + f * NF * NFP + k;
             if constexpr (!ACOUSTIC) {
-                double A = 0;
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) A += p.a[d] * nu[d];
-                const double uL = left ? own[0] : nbv[0];
-                const double uR = left ? (inner ? nbv[0] : 0.0) : own[0];
-                double up = 0;
-                if (A > 1e-12) up = uL;
-                else if (A < -1e-12) up = inner ? uR : 0.0;
-                else if (fabs(A) < 1e-12) up = inner ? 0.5 * uL + 0.5 * uR : 0.5 * uL;
-                out[0] = -(A * sgn) * up * wf;
+                out[0] = inner ? fma(gf[i][0], own[0], gf[i][1] * nbv[0]) : gf[i][0] * own[0];
             } else {
-                if (inner) {
-                    double jn = 0;
+                // -1/2 n.(s_own - s_nbr) and -1/2 n (v_own - v_nbr), n the own
+                // normal; -n.s_own and nothing on a wall
+                double jn = 0;
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) jn += nu[d] * (own[1 + d] - nbv[1 + d]);
-                    // -1/2 n_own . (s_own - s_nbr) and -1/2 n_own (v_own - v_nbr),
-                    // n_own = sgn * nu (both sides see L's normal, negated on R)
-                    out[0] = -0.5 * (sgn * jn) * wf;
-                    const double jv = own[0] - nbv[0];
+                for (int d = 0; d < DIM; ++d) jn = fma(gf[i][d], inner ? own[1 + d] - nbv[1 + d] : own[1 + d], jn);
+                out[0] = inner ? -0.5 * jn : -jn;
+                const double jv = inner ? -0.5 * (own[0] - nbv[0]) : 0.0;
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) out[(1 + d) * NFP] = -0.5 * (sgn * nu[d]) * jv * wf;
-                } else {
-                    double ns = 0;
-#pragma unroll
-                    for (int d = 0; d < DIM; ++d) ns += nu[d] * own[1 + d];
-                    out[0] = -ns * wf;
-#pragma unroll
-                    for (int d = 0; d < DIM; ++d) out[(1 + d) * NFP] = 0.0;
-                }
+                for (int d = 0; d < DIM; ++d) out[(1 + d) * NFP] = inner ? gf[i][d] * jv : 0.0;
             }
         }
     }
     __syncthreads();
 
     // ---- lift the face integrands to the points, divide by the point weight
-    double ci = 1.0;
-    if constexpr (ACOUSTIC) {
-        if (ok) ci = 1.0 / p.cinv[e];
-    }
+    const int ii[3] = {t % N1, (t / N1) % N1, DIM == 3 ? t / (N1 * N1) : 0};
+    const double wi = gp[G::GP - 1];
+    const double ci = ACOUSTIC && ok ? 1.0 / p.cinv[e] : 1.0;
+    double lift[NF];
+#pragma unroll
+    for (int fld = 0; fld < NF; ++fld) lift[fld] = 0.0;
 #pragma unroll
     for (int f = 0; f < NFACE; ++f) {
-        const int ax = face_axis(DIM, f);
         const int a0 = face_coord_axis(DIM, f, 0), a1 = DIM == 3 ? face_coord_axis(DIM, f, 1) : 0;
         const int k = ii[a0] + (DIM == 3 ? N1 * ii[a1] : 0);
-        const double lam = tab[(face_side(DIM, f) ? T::LAM1 : T::LAM0) + ii[ax]];
+        const double lam = tab[(face_side(DIM, f) ? T::LAM1 : T::LAM0) + ii[face_axis(DIM, f)]];
 #pragma unroll
-        for (int fld = 0; fld < NF; ++fld) res[fld] += lam * sc[(f * NF + fld) * NFP + k];
+        for (int fld = 0; fld < NF; ++fld) lift[fld] = fma(lam, sc[(f * NF + fld) * NFP + k], lift[fld]);
     }
+    if constexpr (!ACOUSTIC) {
+        const double* sF = lds + le * G::PER + G::F;
+        double v = lift[0];
 #pragma unroll
-    for (int fld = 0; fld < NF; ++fld) sA[fld * NP + t] = res[fld] / Wq * (fld > 0 ? ci : 1.0);
+        for (int r = 0; r < DIM; ++r) v += along_val<N1, true>(tab + T::C, r, t, sF + r * NP);
+        sA[t] = v * wi;
+    } else {
+#pragma unroll
+        for (int fld = 0; fld < NF; ++fld) sA[fld * NP + t] = fma(lift[fld], wi, res[fld]) * (fld > 0 ? ci : 1.0);
+    }
     __syncthreads();
 
     // ---- back to coefficients: k = B^{-1} (point values)
     along<N1, NP, NF, false>(tab + T::BINV, 0, t, sA, sB);
     __syncthreads();
-    const double* Kp = sA;
-    along<N1, NP, NF, false>(tab + T::BINV, 1, t, sB, sA);
+    const double* Kp = sB;
     if constexpr (DIM == 3) {
+        along<N1, NP, NF, false>(tab + T::BINV, 1, t, sB, sA);
         __syncthreads();
-        along<N1, NP, NF, false>(tab + T::BINV, 2, t, sA, sB);
-        Kp = sB;
+        Kp = sA;
     }
     if (ok) {
-        const int64_t base = e * NF * NP;
         double kept[NF];  // the values as stored
 #pragma unroll
         for (int fld = 0; fld < NF; ++fld) {
-            const double v = Kp[fld * NP + t];
+            const double v = along_val<N1, false>(tab + T::BINV, DIM - 1, t, Kp + fld * NP);
             if (p.io.out_f32) {
                 const float vf = float(v);
                 static_cast<float*>(p.io.out)[base + fld * NP + t] = vf;
@@ -916,6 +965,29 @@ void tensor_general_operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
         c->n_fields = 1;
     }
     c->dof = ne * c->tm.nb * c->n_fields;
+    const bool acoustic = op->kind == HGDG_OP_ACOUSTIC_CENTRAL;
+    GenGeoParams p{};
+    p.n_elem = ne;
+    p.X = c->tm.d_gX.ptr;
+    p.nbr = c->tm.d_gface.ptr;
+    p.info = c->tm.d_gface.ptr + size_t(2 * c->dim) * ne;
+    p.tab = c->tm.d_gtab.ptr;
+    for (int d = 0; d < 3; ++d) p.a[d] = !acoustic && d < c->dim ? op->velocity[d] : 0.0;
+    dispatch_general(c->dim, c->tm.n1, [&](auto D, auto N) {
+        auto build = [&](auto A) {
+            constexpr bool kAc = decltype(A)::value;
+            using G = GenRhs<decltype(D)::value, decltype(N)::value, kAc>;
+            c->tm.d_ggeo.alloc(size_t(ne) * G::GP * G::NP);
+            c->tm.d_gfgeo.alloc(size_t(ne) * G::NFACE * G::GF * G::NFP);
+            p.geo = c->tm.d_ggeo.ptr;
+            p.fgeo = c->tm.d_gfgeo.ptr;
+            hipLaunchKernelGGL((tensor_general_geometry<decltype(D)::value, decltype(N)::value, kAc>),
+                               dim3(unsigned((ne + G::EPB - 1) / G::EPB)), dim3(G::THREADS), 0, c->stream, p);
+        };
+        if (acoustic) build(std::true_type{});
+        else build(std::false_type{});
+    });
+    HGDG_HIP(hipGetLastError());
     HGDG_HIP(hipStreamSynchronize(c->stream));
 }
 
@@ -923,23 +995,22 @@ void tensor_general_rhs(hgdg_ctx* c, const StageIO& io) {
     GenParams p{};
     p.n_elem = c->n_elem;
     p.io = io;
-    p.X = c->tm.d_gX.ptr;
     p.nbr = c->tm.d_gface.ptr;
     p.info = c->tm.d_gface.ptr + size_t(2 * c->dim) * c->n_elem;
     p.tab = c->tm.d_gtab.ptr;
+    p.geo = c->tm.d_ggeo.ptr;
+    p.fgeo = c->tm.d_gfgeo.ptr;
     const bool acoustic = c->op.kind == HGDG_OP_ACOUSTIC_CENTRAL;
     p.cinv = acoustic ? c->tm.d_gcinv.ptr : nullptr;
-    for (int d = 0; d < 3; ++d) p.a[d] = d < c->dim ? c->op.velocity[d] : 0.0;
     dispatch_general(c->dim, c->tm.n1, [&](auto D, auto N) {
-        constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
-        using S = GenShape<DIMc, N1c>;
-        const int64_t grid = (c->n_elem + S::EPB - 1) / S::EPB;
-        if (acoustic)
-            hipLaunchKernelGGL((tensor_general_rhs<DIMc, N1c, true>), dim3(unsigned(grid)), dim3(S::THREADS), 0,
-                               c->stream, p);
-        else
-            hipLaunchKernelGGL((tensor_general_rhs<DIMc, N1c, false>), dim3(unsigned(grid)), dim3(S::THREADS), 0,
-                               c->stream, p);
+        auto launch = [&](auto A) {
+            constexpr bool kAc = decltype(A)::value;
+            using G = GenRhs<decltype(D)::value, decltype(N)::value, kAc>;
+            hipLaunchKernelGGL((tensor_general_rhs<decltype(D)::value, decltype(N)::value, kAc>),
+                               dim3(unsigned((c->n_elem + G::EPB - 1) / G::EPB)), dim3(G::THREADS), 0, c->stream, p);
+        };
+        if (acoustic) launch(std::true_type{});
+        else launch(std::false_type{});
     });
     HGDG_HIP(hipGetLastError());
 }
