@@ -21,7 +21,7 @@ struct TensorMesh {
     std::vector<double> absdet;     // [e]
     std::vector<int32_t> nbr;       // [2 dim][e]
     TensorOps ops;
-    DevBuf<int32_t> d_nbr;
+    DevBuf<int32_t> d_nbr, d_perm;   // d_perm: perm on the device (built on first use)
     DevBuf<double> d_absdet, d_ops;  // d_ops: Dr, Mi, M1 (n1 x n1 each)
     DevBuf<double> d_geo;            // advection: ahat [dim][e]; acoustic: J^{-1} [dim*dim][e], then c_inv [e]
     DevBuf<uint32_t> d_mode;         // advection: upwind mode, 3 bits per face
@@ -61,6 +61,8 @@ struct SimplexMesh {
     std::vector<int64_t> rank;                   // mesh element -> processing (locality) rank
     std::vector<int32_t> order;                  // per device element
     std::vector<int64_t> dof_off;                // per device element: first DOF
+    std::vector<int64_t> host_off;               // [E + 1] per mesh element: first DOF in hpGEM's vector
+    DevBuf<int64_t> d_io_off;                    // host_off, then the device DOF of each mesh element (on first use)
     std::vector<SimplexOps> ops;                 // per order (index p-1), built on demand
     DevBuf<double> d_tables;                     // Dr, proj, lift of every order
     DevBuf<float> d_tables32;                    // the same in FP32 (mixed path)
@@ -179,8 +181,6 @@ void tensor_state_diff(hgdg_ctx* c, const Vec& x, const Vec& y, double* l2, doub
 void tensor_mass_apply(hgdg_ctx* c, Vec& v, bool inverse);
 void tensor_error_modes(hgdg_ctx* c, const Vec& v, int field, int n_modes, const double* amp, const double* k,
                         const double* shift, double* l2, double* max_abs);
-void tensor_to_device(hgdg_ctx* c, const double* host, std::vector<double>& dev);
-void tensor_from_device(hgdg_ctx* c, const std::vector<double>& dev, double* host);
 
 // tensor_general.hip: the Gauss-point path (non-affine elements, unaligned faces)
 void tensor_general_upload(hgdg_ctx* c, const hgdg_mesh_desc* m);
@@ -204,8 +204,10 @@ void tensor_batch_launch(hipStream_t stream, int kind, int dim, int n1, bool mix
 void set_storage(hgdg_ctx* c, Vec& v, bool f32);
 void mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m);
 void operator_set(hgdg_ctx* c, const hgdg_op_desc* op);
-void upload_vector(hgdg_ctx* c, Vec& v, const std::vector<double>& dev);
-void download_vector(hgdg_ctx* c, Vec& v, std::vector<double>& dev);
+// Contexts and servers count as users of the process's pinned chunks.
+void pinned_user(int change);
+void host_get(hgdg_ctx* c, Vec& v, double* host);        // host = v in hpGEM's layout
+void host_set(hgdg_ctx* c, Vec& v, const double* host);  // v = host
 void state_diff(hgdg_ctx* c, int x, int y, double* l2, double* max_abs);
 
 // matrix_op.hip
@@ -231,7 +233,5 @@ void simplex_error_modes(hgdg_ctx* c, const Vec& v, int field, int n_modes, cons
                          const double* shift, double* l2, double* max_abs);
 void simplex_project(hgdg_ctx* c, Vec& v, int field, int n_modes, const double* amp, const double* k,
                      const double* gauss = nullptr);
-void simplex_to_device(hgdg_ctx* c, const double* host, std::vector<double>& dev);
-void simplex_from_device(hgdg_ctx* c, const std::vector<double>& dev, double* host);
 
 }  // namespace hgdg

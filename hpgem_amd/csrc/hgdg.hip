@@ -9,11 +9,15 @@
 #include <fstream>
 #include <sstream>
 #include <cmath>
+#include <cstring>
+#include <exception>
 #include <functional>
 #include <limits>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "context.hpp"
@@ -98,32 +102,223 @@ void set_storage(hgdg_ctx* c, Vec& v, bool f32) {
     v.is_f32 = f32;
 }
 
-void upload_vector(hgdg_ctx* c, Vec& v, const std::vector<double>& dev) {
-    require(dev.size() == size_t(c->n_dof()), HGDG_ERR_ARG, "vector size mismatch");
-    if (v.is_f32) {
-        std::vector<float> f(dev.begin(), dev.end());
-        HGDG_HIP(hipMemcpyAsync(v.f32->ptr, f.data(), f.size() * sizeof(float), hipMemcpyHostToDevice, c->stream));
-        HGDG_HIP(hipStreamSynchronize(c->stream));
+// ---- vectors to and from the caller, in hpGEM's layout ----------------------
+// A chunk of unknowns goes through pinned host memory: one kernel permutes (and
+// converts FP32 storage) between the vector and the chunk across PCIe, the host
+// copies between the chunk and the caller's memory. Large vectors are shared by
+// up to kCopyThreads host threads with a chunk of their own each, so that the
+// transfers run beside the copies, most of whose time is the caller's pages
+// being touched for the first time. 67 MB (32^3 p = 3 acoustic): 100 RK4 steps
+// and reading the state took 34.1 ms with a permutation on the host around a
+// pageable copy, 25.8 so; the copy to fresh memory alone takes 4.9 ms with one
+// thread and 1.6 with four, the transfer 1.3.
+constexpr int64_t kChunk = int64_t(1) << 18;  // doubles per chunk
+constexpr int kCopyThreads = 4;
+constexpr int64_t kThreadedFrom = int64_t(1) << 20;  // doubles: below, one thread is as fast
+
+// The pinned chunks are the process's: allocating one takes about 0.3 ms, too
+// much for a context of its own small vectors. At most kPinnedKept are kept for
+// the next call, and none once the last context and server are gone. A call
+// takes what it needs (never waiting for another call's) and gives it back
+// after its last use on the GPU has ended.
+constexpr size_t kPinnedKept = 2 * kCopyThreads;
+struct PinnedPool {
+    std::mutex mu;
+    std::vector<double*> kept;
+    int64_t users = 0;
+};
+PinnedPool& pinned_pool() {
+    static PinnedPool* pool = new PinnedPool;  // never destroyed: the HIP runtime may end before statics do
+    return *pool;
+}
+
+void pinned_user(int change) {
+    PinnedPool& pool = pinned_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    pool.users += change;
+    if (pool.users > 0) return;
+    for (double* p : pool.kept) (void)hipHostFree(p);
+    pool.kept.clear();
+}
+
+struct PinnedChunk {
+    double* ptr = nullptr;
+    PinnedChunk() {
+        PinnedPool& pool = pinned_pool();
+        {
+            std::lock_guard<std::mutex> lk(pool.mu);
+            if (!pool.kept.empty()) {
+                ptr = pool.kept.back();
+                pool.kept.pop_back();
+                return;
+            }
+        }
+        void* p = nullptr;
+        HGDG_HIP(hipHostMalloc(&p, size_t(kChunk) * sizeof(double), hipHostMallocPortable));
+        ptr = static_cast<double*>(p);
+    }
+    ~PinnedChunk() {
+        PinnedPool& pool = pinned_pool();
+        std::lock_guard<std::mutex> lk(pool.mu);
+        if (pool.users > 0 && pool.kept.size() < kPinnedKept) pool.kept.push_back(ptr);
+        else (void)hipHostFree(ptr);
+    }
+    PinnedChunk(const PinnedChunk&) = delete;
+    PinnedChunk& operator=(const PinnedChunk&) = delete;
+};
+
+struct HostCopyParams {
+    void* v;
+    int32_t v_f32;
+    int32_t get;           // 1: chunk = v, 0: v = chunk
+    double* chunk;         // hpGEM's unknowns from lo on
+    int64_t lo, n;         // unknowns lo .. lo + n
+    const int32_t* perm;   // tensor elements: position of hpGEM function i among a field's nb
+    uint32_t nb;
+    const int64_t* off;    // tetrahedra: first unknown of each mesh element in hpGEM's vector
+    const int64_t* dev;    //             and in v
+    int64_t e0, e1;        // the chunk's elements
+};
+
+__device__ __forceinline__ void host_copy_one(const HostCopyParams& p, int64_t at, int64_t j) {
+    if (p.get) {
+        p.chunk[j] = p.v_f32 ? double(static_cast<const float*>(p.v)[at]) : static_cast<const double*>(p.v)[at];
+    } else if (p.v_f32) {
+        static_cast<float*>(p.v)[at] = float(p.chunk[j]);
     } else {
-        HGDG_HIP(hipMemcpyAsync(v.f64->ptr, dev.data(), dev.size() * sizeof(double), hipMemcpyHostToDevice,
-                                c->stream));
-        HGDG_HIP(hipStreamSynchronize(c->stream));
+        static_cast<double*>(p.v)[at] = p.chunk[j];
     }
 }
 
-void download_vector(hgdg_ctx* c, Vec& v, std::vector<double>& dev) {
-    const size_t n = size_t(c->n_dof());
-    dev.assign(n, 0.0);
-    if (v.is_f32) {
-        std::vector<float> f(n);
-        HGDG_HIP(hipMemcpyAsync(f.data(), v.f32->ptr, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-        HGDG_HIP(hipStreamSynchronize(c->stream));
-        std::copy(f.begin(), f.end(), dev.begin());
-    } else {
-        HGDG_HIP(hipMemcpyAsync(dev.data(), v.f64->ptr, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        HGDG_HIP(hipStreamSynchronize(c->stream));
+__global__ __launch_bounds__(kBlock) void host_copy_flat(const HostCopyParams p) {
+    const uint32_t j = blockIdx.x * kBlock + threadIdx.x;  // a chunk has fewer than 2^32 unknowns
+    if (j >= p.n) return;
+    int64_t at = p.lo + j;
+    if (p.perm) {  // lo is a multiple of nb
+        const uint32_t b = j / p.nb;
+        at = p.lo + int64_t(b) * p.nb + p.perm[j - b * p.nb];
     }
+    host_copy_one(p, at, j);
 }
+
+// one wavefront per element
+__global__ __launch_bounds__(kBlock) void host_copy_elements(const HostCopyParams p) {
+    const int64_t e = p.e0 + int64_t(blockIdx.x) * (kBlock / 64) + threadIdx.x / 64;
+    if (e >= p.e1) return;
+    const int64_t h = p.off[e], n = p.off[e + 1] - h;
+    for (int64_t i = threadIdx.x % 64; i < n; i += 64) host_copy_one(p, p.dev[e] + i, h - p.lo + i);
+}
+
+static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
+    const int64_t n = c->n_dof();
+    HostCopyParams base{};
+    base.v = v.ptr();
+    base.v_f32 = v.is_f32 ? 1 : 0;
+    base.get = out != nullptr ? 1 : 0;
+    int64_t unit = 1;  // chunks are whole multiples of it (tensor elements' functions)
+    if (c->simplex()) {
+        SimplexMesh& sm = c->sm;
+        if (sm.d_io_off.n == 0) {
+            sm.host_off.assign(1, 0);
+            std::vector<int64_t> dev(static_cast<size_t>(c->n_elem));
+            for (int64_t e = 0; e < c->n_elem; ++e) {
+                const int64_t d = sm.dev_of[size_t(e)];
+                dev[size_t(e)] = sm.dof_off[size_t(d)];
+                sm.host_off.push_back(sm.host_off.back() + int64_t(c->n_fields) * tet_nb(sm.order[size_t(d)]));
+            }
+            std::vector<int64_t> both(sm.host_off);
+            both.insert(both.end(), dev.begin(), dev.end());
+            sm.d_io_off.upload(both, c->stream);
+            HGDG_HIP(hipStreamSynchronize(c->stream));
+        }
+        base.off = sm.d_io_off.ptr;
+        base.dev = sm.d_io_off.ptr + c->n_elem + 1;
+    } else if (!c->matrix()) {
+        TensorMesh& tm = c->tm;
+        if (tm.d_perm.n == 0) {
+            tm.d_perm.upload(std::vector<int32_t>(tm.perm.begin(), tm.perm.end()), c->stream);
+            HGDG_HIP(hipStreamSynchronize(c->stream));
+        }
+        base.perm = tm.d_perm.ptr;
+        base.nb = uint32_t(tm.nb);
+        unit = tm.nb;
+    }
+    // chunk k: unknowns [cut[k], cut[k + 1]); tetrahedra: elements [ecut[k], ecut[k + 1])
+    std::vector<int64_t> cut{0}, ecut{0};
+    while (cut.back() < n) {
+        const int64_t lo = cut.back();
+        int64_t hi = std::min(n, lo + kChunk / unit * unit);  // an element has far fewer unknowns than a chunk
+        if (c->simplex()) {
+            const std::vector<int64_t>& off = c->sm.host_off;
+            const int64_t e = std::upper_bound(off.begin(), off.end(), hi) - off.begin() - 1;
+            ecut.push_back(e);
+            hi = off[size_t(e)];
+        }
+        cut.push_back(hi);
+    }
+    const int64_t chunks = int64_t(cut.size()) - 1;
+    const int workers = int(n < kThreadedFrom ? 1 : std::min<int64_t>(kCopyThreads, chunks));
+    auto work = [&](int w) {
+        HGDG_HIP(hipSetDevice(c->device));
+        HostCopyParams p = base;
+        const PinnedChunk chunk;
+        p.chunk = chunk.ptr;
+        hipEvent_t done = nullptr;
+        if (workers > 1) HGDG_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+        try {
+            for (int64_t k = w; k < chunks; k += workers) {
+                p.lo = cut[size_t(k)];
+                p.n = cut[size_t(k) + 1] - p.lo;
+                if (in) std::memcpy(p.chunk, in + p.lo, size_t(p.n) * sizeof(double));
+                if (p.off) {
+                    p.e0 = ecut[size_t(k)];
+                    p.e1 = ecut[size_t(k) + 1];
+                    hipLaunchKernelGGL(host_copy_elements, dim3(unsigned((p.e1 - p.e0 + kBlock / 64 - 1) / (kBlock / 64))),
+                                       dim3(kBlock), 0, c->stream, p);
+                } else {
+                    hipLaunchKernelGGL(host_copy_flat, dim3(unsigned((p.n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                                       c->stream, p);
+                }
+                HGDG_HIP(hipGetLastError());
+                if (done) {
+                    HGDG_HIP(hipEventRecord(done, c->stream));
+                    HGDG_HIP(hipEventSynchronize(done));
+                } else {
+                    HGDG_HIP(hipStreamSynchronize(c->stream));
+                }
+                if (out) std::memcpy(out + p.lo, p.chunk, size_t(p.n) * sizeof(double));
+            }
+        } catch (...) {
+            (void)hipStreamSynchronize(c->stream);  // nothing may still use the chunk
+            if (done) (void)hipEventDestroy(done);
+            throw;
+        }
+        if (done) (void)hipEventDestroy(done);
+    };
+    std::vector<std::exception_ptr> failed(static_cast<size_t>(workers));
+    auto guarded = [&](int w) {
+        try {
+            work(w);
+        } catch (...) {
+            failed[size_t(w)] = std::current_exception();
+        }
+    };
+    std::vector<std::thread> threads;
+    threads.reserve(size_t(workers));
+    int started = 1;  // worker 0 is the calling thread
+    try {
+        for (; started < workers; ++started) threads.emplace_back(guarded, started);
+    } catch (const std::system_error&) {  // no more threads: this one does their chunks too
+    }
+    guarded(0);
+    for (int w = started; w < workers; ++w) guarded(w);
+    for (std::thread& t : threads) t.join();
+    for (const std::exception_ptr& f : failed)
+        if (f) std::rethrow_exception(f);
+}
+
+void host_get(hgdg_ctx* c, Vec& v, double* host) { host_copy(c, v, host, nullptr); }
+void host_set(hgdg_ctx* c, Vec& v, const double* host) { host_copy(c, v, nullptr, host); }
 
 void mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     require(m != nullptr, HGDG_ERR_ARG, "mesh descriptor is NULL");
@@ -638,6 +833,7 @@ int hgdg_ctx_create(hgdg_ctx** out, int device) {
         std::unique_ptr<hgdg_ctx> c(new hgdg_ctx);
         c->device = device;
         HGDG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+        hgdg::pinned_user(1);
         *out = c.release();
     });
 }
@@ -652,6 +848,7 @@ int hgdg_ctx_destroy(hgdg_ctx* ctx) {
         hipStream_t s = ctx->stream;
         delete ctx;
         if (s) (void)hipStreamDestroy(s);
+        hgdg::pinned_user(-1);
     });
 }
 
@@ -810,11 +1007,7 @@ int hgdg_state_set(hgdg_ctx* ctx, int vec, const double* host) {
         require(ctx != nullptr && host != nullptr, HGDG_ERR_ARG, "NULL argument");
         HGDG_HIP(hipSetDevice(ctx->device));
         hgdg::Vec& v = hgdg::vec_at(ctx, vec);
-        std::vector<double> dev;
-        if (ctx->matrix()) dev.assign(host, host + ctx->n_dof());
-        else if (ctx->simplex()) hgdg::simplex_to_device(ctx, host, dev);
-        else hgdg::tensor_to_device(ctx, host, dev);
-        hgdg::upload_vector(ctx, v, dev);
+        hgdg::host_set(ctx, v, host);
     });
 }
 
@@ -823,11 +1016,7 @@ int hgdg_state_get(hgdg_ctx* ctx, int vec, double* host) {
         require(ctx != nullptr && host != nullptr, HGDG_ERR_ARG, "NULL argument");
         HGDG_HIP(hipSetDevice(ctx->device));
         hgdg::Vec& v = hgdg::vec_at(ctx, vec);
-        std::vector<double> dev;
-        hgdg::download_vector(ctx, v, dev);
-        if (ctx->matrix()) std::copy(dev.begin(), dev.end(), host);
-        else if (ctx->simplex()) hgdg::simplex_from_device(ctx, dev, host);
-        else hgdg::tensor_from_device(ctx, dev, host);
+        hgdg::host_get(ctx, v, host);
     });
 }
 

@@ -482,17 +482,14 @@ void hgdg_server::worker_loop() {
                 try {
                     hgdg_ctx* c = s->ctx;
                     n_dof = c->n_dof();
-                    std::vector<double> dev;
                     if (s->cur)  // the last step left the solution in the ping-pong copy
                         HGDG_HIP(hipMemcpyAsync(c->vecs[0].f64->ptr, c->u_spare.ptr, size_t(n_dof) * sizeof(double),
                                                 hipMemcpyDeviceToDevice, c->stream));
-                    hgdg::download_vector(c, c->vecs[0], dev);
-                    for (double v : dev) norm += v * v;
+                    state.resize(size_t(n_dof));
+                    hgdg::host_get(c, c->vecs[0], state.data());
+                    for (double v : state) norm += v * v;
                     norm = std::sqrt(norm);
-                    if (s->req.d.keep_state) {
-                        state.resize(size_t(n_dof));
-                        hgdg::tensor_from_device(c, dev, state.data());
-                    }
+                    if (!s->req.d.keep_state) std::vector<double>().swap(state);
                 } catch (const std::exception& ex) {
                     serr = ex.what();
                 }
@@ -556,6 +553,7 @@ int hgdg_server_create(hgdg_server** out, int device, int precision, int64_t hbm
         s->max_active = max_active;
         HGDG_HIP(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
         HGDG_HIP(hipStreamCreateWithFlags(&s->prep_stream, hipStreamNonBlocking));
+        hgdg::pinned_user(1);
         hgdg_server* raw = s.get();
         s->preparer = std::thread([raw] { raw->prepare_loop(); });
         s->worker = std::thread([raw] { raw->worker_loop(); });
@@ -720,6 +718,7 @@ int hgdg_server_destroy(hgdg_server* s) {
         if (s->stream) (void)hipStreamDestroy(s->stream);
         if (s->prep_stream) (void)hipStreamDestroy(s->prep_stream);
         delete s;
+        hgdg::pinned_user(-1);
     });
 }
 

@@ -941,6 +941,7 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     sm.group_dof[0] = 0;
     for (int g = 0; g < 4; ++g) sm.group_dof[g + 1] = sm.group_dof[g] + counts[g] * nf * tet_nb(g + 1);
     sm.dof_off.assign(ne, 0);
+    sm.d_io_off.reset();
     for (int64_t d = 0; d < ne; ++d) {
         const int g = sm.order[d] - 1;
         sm.dof_off[d] = sm.group_dof[g] + (d - sm.group_start[g]) * nf * tet_nb(g + 1);
@@ -1609,29 +1610,6 @@ void simplex_error_modes(hgdg_ctx* c, const Vec& v, int field, int n_modes, cons
     }
     *l2 = std::sqrt(sum);
     *max_abs = mx;
-}
-
-void simplex_to_device(hgdg_ctx* c, const double* host, std::vector<double>& dev) {
-    const SimplexMesh& sm = c->sm;
-    dev.assign(size_t(c->n_dof()), 0.0);
-    int64_t off = 0;
-    for (int64_t e = 0; e < c->n_elem; ++e) {
-        const int64_t d = sm.dev_of[e];
-        const int64_t n = int64_t(c->n_fields) * tet_nb(sm.order[d]);
-        std::copy(host + off, host + off + n, dev.begin() + sm.dof_off[d]);
-        off += n;
-    }
-}
-
-void simplex_from_device(hgdg_ctx* c, const std::vector<double>& dev, double* host) {
-    const SimplexMesh& sm = c->sm;
-    int64_t off = 0;
-    for (int64_t e = 0; e < c->n_elem; ++e) {
-        const int64_t d = sm.dev_of[e];
-        const int64_t n = int64_t(c->n_fields) * tet_nb(sm.order[d]);
-        std::copy(dev.begin() + sm.dof_off[d], dev.begin() + sm.dof_off[d] + n, host + off);
-        off += n;
-    }
 }
 
 }  // namespace hgdg

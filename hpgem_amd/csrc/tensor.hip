@@ -1942,21 +1942,6 @@ void tensor_error_modes(hgdg_ctx* c, const Vec& v, int field, int n_modes, const
     *max_abs = m;
 }
 
-void tensor_to_device(hgdg_ctx* c, const double* host, std::vector<double>& dev) {
-    const int nb = c->tm.nb;
-    const int64_t blocks = c->n_elem * c->n_fields;  // field-major blocks of nb per element
-    dev.assign(size_t(c->n_dof()), 0.0);
-    for (int64_t b = 0; b < blocks; ++b)
-        for (int i = 0; i < nb; ++i) dev[size_t(b) * nb + c->tm.perm[i]] = host[size_t(b) * nb + i];
-}
-
-void tensor_from_device(hgdg_ctx* c, const std::vector<double>& dev, double* host) {
-    const int nb = c->tm.nb;
-    const int64_t blocks = c->n_elem * c->n_fields;
-    for (int64_t b = 0; b < blocks; ++b)
-        for (int i = 0; i < nb; ++i) host[size_t(b) * nb + i] = dev[size_t(b) * nb + c->tm.perm[i]];
-}
-
 // ---------------------------------------------------------------- batched launches
 // Problems of one family (kind, dim, order) advance together: their per-problem
 // parameter blocks go into `params` (device, written by the caller beforehand
