@@ -245,10 +245,10 @@ class HpgemAPIDevice:
 
     # ---- threads per element of the tetrahedral kernel ---------------------
     def setSimplexThreads(self, threads):
-        """Threads per element for orders 1..4 (four values): each 0 to time
-        both candidates of that order and keep the faster (done by default
-        when the operator is set), or one of the candidates (16/32, 32/64,
-        32/64, 35/64)."""
+        """Elements per workgroup for orders 1..4, named by threads per element
+        (four values): each 0 to time both candidates of that order and keep
+        the faster (done by default when the operator is set), or one of the
+        candidates (8/16, 12/32, 32/64, 35/64; the first fills a workgroup)."""
         t = np.ascontiguousarray(threads, dtype=np.int32)
         if t.shape != (4,):
             raise ValueError("four values, orders 1..4")

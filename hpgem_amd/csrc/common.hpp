@@ -226,6 +226,109 @@ __device__ __forceinline__ void combine_n(const StageIO& p, const int64_t (&idx)
     }
 }
 
+// K values of a vector as loaded: FP32 values stay as their bits in the
+// doubles' low words until they are used (raw_value), so nothing waits for a
+// load where it is issued.
+__device__ __forceinline__ double raw_value(double x, bool f32) {
+    return f32 ? double(__int_as_float(__double2loint(x))) : x;
+}
+
+template <int K>
+__device__ __forceinline__ void load_raw_n(const void* v, bool f32, const int64_t (&idx)[K], double (&x)[K]) {
+    if (f32) {
+        const float* f = static_cast<const float*>(v);
+#pragma unroll
+        for (int k = 0; k < K; ++k) x[k] = __hiloint2double(0, __float_as_int(f[idx[k]]));
+    } else {
+        const double* d = static_cast<const double*>(v);
+#pragma unroll
+        for (int k = 0; k < K; ++k) x[k] = d[idx[k]];
+    }
+}
+
+// y += c x for values as load_raw_n left them
+template <int K>
+__device__ __forceinline__ void add_raw_n(double c, const double (&x)[K], bool f32, double (&y)[K]) {
+    if (f32) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) y[k] = fma(c, raw_value(x[k], true), y[k]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) y[k] = fma(c, x[k], y[k]);
+    }
+}
+
+// What a stage's inputs are, where a kernel is instantiated for it: the RK
+// stages' own combinations without a branch between their loads, or any.
+enum StageKind : int {
+    STAGE_ANY = 0,
+    STAGE_ONE = 1,        // one input, FP64
+    STAGE_TWO = 2,        // two, both FP64
+    STAGE_TWO_MIXED = 3,  // two, FP64 and FP32
+};
+inline int stage_kind(const StageIO& p) {
+    if (p.n_in == 1 && p.in_f32 == 0) return STAGE_ONE;
+    if (p.n_in == 2 && p.in_f32 == 0) return STAGE_TWO;
+    if (p.n_in == 2 && p.in_f32 == 2) return STAGE_TWO_MIXED;
+    return STAGE_ANY;
+}
+
+// combine_n in two halves: the first two inputs' loads, then the sums (in a)
+template <int KIND, int K>
+__device__ __forceinline__ void load_two(const StageIO& p, const int64_t (&idx)[K], double (&a)[K], double (&b)[K]) {
+    load_raw_n(p.in[0], KIND == STAGE_ANY && (p.in_f32 & 1u), idx, a);
+    if (KIND == STAGE_ANY ? p.n_in > 1 : KIND != STAGE_ONE)
+        load_raw_n(p.in[1], KIND == STAGE_ANY ? (p.in_f32 & 2u) != 0 : KIND == STAGE_TWO_MIXED, idx, b);
+}
+
+template <int KIND, int K>
+__device__ __forceinline__ void mix_two(const StageIO& p, const int64_t (&idx)[K], double (&a)[K], double (&b)[K]) {
+    if (KIND == STAGE_ANY && (p.in_f32 & 1u)) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) a[k] = raw_value(a[k], true);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) a[k] = p.coef[0] * a[k];
+    if (KIND == STAGE_ANY ? p.n_in > 1 : KIND != STAGE_ONE)
+        add_raw_n(p.coef[1], b, KIND == STAGE_ANY ? (p.in_f32 & 2u) != 0 : KIND == STAGE_TWO_MIXED, a);
+    if (KIND == STAGE_ANY) {
+#pragma unroll 1
+        for (int i = 2; i < p.n_in; ++i) {
+            load_raw_n(p.in[i], (p.in_f32 >> i) & 1u, idx, b);
+            add_raw_n(p.coef[i], b, (p.in_f32 >> i) & 1u, a);
+        }
+    }
+}
+
+// The fused update at K indices, `own` the values of this kernel's output
+// there (as stored): rk_update_run's sums, the solution and the first kRkPre
+// terms of all K in flight together.
+template <int K>
+__device__ __forceinline__ void rk_update_n(const RkUpdate& q, const int64_t (&idx)[K], const double (&own)[K]) {
+    double y[K], xs[kRkPre][K];
+    auto fetch = [&](int j, double (&x)[K]) {
+        if (j != q.self) load_raw_n(q.x[j], (q.x_f32 >> j) & 1u, idx, x);
+    };
+    auto add = [&](int j, const double (&x)[K]) {
+        if (j == q.self) add_raw_n(q.c[j], own, false, y);
+        else add_raw_n(q.c[j], x, (q.x_f32 >> j) & 1u, y);
+    };
+    load_raw_n(q.u, false, idx, y);
+#pragma unroll
+    for (int j = 0; j < kRkPre; ++j)
+        if (j < q.n_x) fetch(j, xs[j]);
+#pragma unroll
+    for (int j = 0; j < kRkPre; ++j)
+        if (j < q.n_x) add(j, xs[j]);
+#pragma unroll 1
+    for (int j = kRkPre; j < q.n_x; ++j) {
+        fetch(j, xs[0]);
+        add(j, xs[0]);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) q.y_new[idx[k]] = y[k];
+}
+
 // Residual accumulation: FP64 plainly; FP32 with a compensated (TwoSum)
 // running sum for the face contributions.
 template <typename T>

@@ -54,8 +54,6 @@ struct MatrixOp {
 struct SimplexMesh {
     int64_t group_start[5] = {0, 0, 0, 0, 0};    // device elements of order g+1: [start[g], start[g+1])
     int64_t group_dof[5] = {0, 0, 0, 0, 0};      // first DOF of each group
-    int64_t group_tr[5] = {0, 0, 0, 0, 0};       // first face trace of each group (4 (p+1)(p+2)/2 per element)
-    DevBuf<double> d_trace;                      // face traces of the stage input, double2 per coefficient
     std::vector<int64_t> dev_of;                 // mesh element -> device element
     std::vector<int64_t> mesh_of;                // device element -> mesh element
     std::vector<int64_t> rank;                   // mesh element -> processing (locality) rank
@@ -64,29 +62,31 @@ struct SimplexMesh {
     std::vector<int64_t> host_off;               // [E + 1] per mesh element: first DOF in hpGEM's vector
     DevBuf<int64_t> d_io_off;                    // host_off, then the device DOF of each mesh element (on first use)
     std::vector<SimplexOps> ops;                 // per order (index p-1), built on demand
-    DevBuf<double> d_tables;                     // Dr, proj, lift of every order
-    DevBuf<float> d_tables32;                    // the same in FP32 (mixed path)
-    DevBuf<int32_t> d_blocks;                    // RHS block schedule: [n_blocks][4] order, first, count, variant
+    DevBuf<double> d_tables;                     // M_ref, Dr, lift of every order
+    DevBuf<int32_t> d_blocks;                    // RHS block schedule: [n_blocks][4] order, first, count, face functions
     int64_t n_blocks = 0;
-    int32_t tpe_variant[4] = {0, 0, 0, 0};       // per order: threads-per-element candidate in use (0 or 1)
+    int32_t tpe_variant[4] = {0, 0, 0, 0};       // per order: block size candidate in use (0 or 1)
     int32_t tpe_fixed[4] = {0, 0, 0, 0};         // per order: 0 = timed choice, else the fixed threads per element
     double tpe_ms[4][2] = {};                    // per order and candidate: timed RHS launch (ms), 0 if not timed
-    DevBuf<int32_t> d_tab_index;                 // offsets and column lists into d_tables
+    int32_t tab_dr[4] = {0, 0, 0, 0}, tab_lift[4] = {0, 0, 0, 0};  // per order: offsets in d_tables
+    DevBuf<int32_t> d_tab_index;                 // offsets into d_tables, face functions and how neighbours' match
     DevBuf<double> d_mass;                       // per order: M_ref [nb][nb], then M_ref^{-1}
     DevBuf<double> d_qtab;                       // projection / error-norm quadrature tables (built on first use)
     std::vector<int32_t> qtab_index;             // their offsets and sizes per order
     DevBuf<double> d_xj;                         // [E][12]: vertex 0 and J (row-major), device order
     DevBuf<int32_t> d_order;                     // per device element: its order
     DevBuf<int64_t> d_elem_off;                  // [E + 1] first DOF of each device element
-    DevBuf<double> d_geo;                        // J^{-1} [9][E], then c_inv [E], sigma [4][E], normal [3][4][E]
+    DevBuf<double> d_geo;                        // J^{-1} [9][E], then c_inv [E]
     DevBuf<int32_t> d_face;                      // [4][E]: neighbour device element or -1, then packed info [4][E]
+    DevBuf<uint32_t> d_frec;                     // [E][4][2]: the faces' neighbours (simplex_faces)
+    DevBuf<uint8_t> d_fcode;                     // [E][4][16]: their face functions
     DevBuf<double> d_absdet;                     // [E]
     std::vector<double> absdet;
     std::vector<double> jinv;                    // [E][9]
     std::vector<double> X;                       // mesh order [E][4][3]
     std::vector<int32_t> nbr_dev;                // [4][E]
     std::vector<int32_t> info;                   // [4][E]
-    std::vector<double> sigma, normal;           // [4][E], [3][4][E]
+    std::vector<double> sigma, normal;           // [4][E], [3][4][E] (Maxwell assembly)
     std::vector<double> x0, jac;                 // device order: vertex 0 [E][3], J [E][3][3] (row-major)
 };
 

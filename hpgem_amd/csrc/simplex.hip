@@ -8,15 +8,13 @@
 //
 // On an affine tetrahedron the inverse-mass apply turns the volume terms into
 // exact reference derivative matrices Dr_e (d/dxi_e in P_p) combined with
-// J^{-1}, and each face term into a lifting of the flux's face-polynomial
-// coefficients: face traces are projected (exactly: everything is a
-// polynomial of degree <= 4) onto an orthonormal basis of P_4 on the reference
-// triangle, the flux is formed coefficient by coefficient, and
-// Lift = M_ref^{-1} P^T scaled by area/volume brings it back. Both sides of a
-// face are evaluated in the left element's face coordinates, the right side
-// through hpGEM's orientation map (FaceGeometry.h:372-393). Elements are
-// grouped by order on the device; one launch covers all groups, each block
-// working on elements of one order.
+// J^{-1}, and each face term into a lifting, M_ref^{-1} int_f phi psi_m, of the
+// flux's coefficients in the face functions psi_m: the traces of the
+// hierarchical element functions that do not vanish on the face. A neighbour's
+// traces are the same functions up to order and signs, through hpGEM's
+// orientation map (FaceGeometry.h:372-393), so both sides are gathered from the
+// stage input itself and one launch does the whole stage: elements are grouped
+// by order on the device, each block working on elements of one order.
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -31,26 +29,20 @@ namespace hgdg {
 
 namespace {
 
-// int32 table index per order (p-1): offsets into the FP64 (and the FP32)
-// table arrays and, per local face, the offset of its list of face columns
-// (the basis functions whose trace on that face does not vanish). Face terms
-// work with an orthonormal hierarchical basis chi_m of P_4 on the reference
-// triangle (degree by degree): the trace tables give the chi-coefficients of
-// each face column's trace when the face is parametrised through orientation
-// o, the lift tables map flux coefficients back to the element.
-constexpr int kTixDrT = 0;           // [3][nb][nb]: DrT[r][j][i] = Dr_r(i, j)
-constexpr int kTixM = 1;             // [nb][nb]: M_ref
-constexpr int kTixCols = 2;          // + f
-constexpr int kTixProj = 6;          // [4 f][6 o][ncol][15 m]: chi_m-coefficients of the face columns' traces
-constexpr int kTixLift = 7;          // [4 f][ncol m][nb i]: (M_ref^{-1} int_f phi chi_m)_i, own face coordinates
-constexpr int kTixProjId = 8;        // [4 f][ncol c][ncol m]: the trace table at the identity orientation, m < ncol
-constexpr int kTixDrP = 9;           // orders >= 3: [3][4 ceil(nb/4) k][16 ceil(nb/16) i] DrT padded with zeros
-constexpr int kTixStride = 10;
-constexpr int kTixRel = 4 * kTixStride;  // [6 own][6 neighbour]: orientation of the neighbour's face seen from ours
-constexpr int kTixIdent = kTixRel + 36;  // the identity orientation
-constexpr int kTixRot = kTixIdent + 1;   // [6 o][55]: the orientation maps on face-basis coefficients, by degree block
-constexpr int kMaxCols = 15;         // face columns of an order-4 element
-constexpr int kTixMax = kTixRot + 1 + 4 * 4 * kMaxCols;  // whole index table
+// int32 table index: per order (p-1) the offsets of its tables in the table
+// array; then, of the order-4 set (whose first functions are those of the
+// lower orders), the face functions of each local face (the element functions
+// whose trace there does not vanish) and how a neighbour's meet ours.
+constexpr int kTixM = 0;       // [nb][nb]: M_ref
+constexpr int kTixDrP = 1;     // [3][4 ceil(nb/4) k][16 ceil(nb/16) i]: Dr_r(i, k), zeros outside nb x nb
+constexpr int kTixLift = 2;    // [4 f][16 m][16 ceil(nb/16) i]: (M_ref^{-1} int_f phi psi_m)_i, zeros for m = 15
+constexpr int kTixStride = 3;
+constexpr int kTixCols = 4 * kTixStride;  // [4 f][16 m]: the element function of face function m
+// [4 f][4 neighbour's face][6 relative orientation][16 m]: bits 0-5 the
+// neighbour's function loaded for m, bits 6-7 its coefficient in ours, bits
+// 8-9 the coefficient of the one loaded for 27 - m (0: none, 1: +1, 2: -1)
+constexpr int kTixFace = kTixCols + 4 * 16;
+constexpr int kTixSize = kTixFace + 4 * 4 * 6 * 16;
 
 // packed per-face info
 __host__ __device__ constexpr int info_lf(int v) { return v & 3; }
@@ -68,8 +60,6 @@ struct RefTetRule {
     const double* w;
 };
 #include "tet_rules.inc"
-static_assert(kFaceQ == 16, "the table index reserves 16 face points");
-
 }  // namespace
 
 struct SimplexParams {
@@ -77,544 +67,399 @@ struct SimplexParams {
     int64_t n_elem;
     int64_t group_start[5];
     int64_t group_dof[5];
-    int32_t group_block[5];
-    const double* jinv;    // [9][E]: (J^{-1})_{e,d} at [(3e + d) E + elem]
-    const double* cinv;    // [E]
-    const double* sigma;   // [4][E]: face area ratio / |det J|
-    const double* normal;  // [3][4][E]: outward unit normal
-    const int32_t* nbr;    // [4][E]: neighbour device element, -1 on walls
-    const int32_t* info;   // [4][E]
+    const double* jinv;       // [9][E]: (J^{-1})_{e,d} at [(3e + d) E + elem]
+    const double* cinv;       // [E]
+    const uint2* frec;        // [E][4]: the neighbours (simplex_faces)
+    const uint8_t* fcode;     // [E][4][16]: their face functions
     const double* tab;
-    const float* tab32;    // the same tables in FP32 (mixed path), same offsets
-    const int32_t* tix;
-    int32_t n_tix;
-    const int4* blocks;    // per block: order, first device element, element count, threads-per-element variant (informative)
-    double2* trace;        // face traces of the stage input: [element][4 f][ncol(p) m] (n.s, v), own face coordinates
-    int64_t group_tr[5];   // first trace of each order group
+    int32_t tab_dr[4], tab_lift[4];  // per order: offsets in tab
+    const int32_t* cols;      // [4 f][16]: the element function of each face function
+    const int4* blocks;       // per block: order, first device element, element count, face functions met
 };
 
 __host__ __device__ constexpr int simplex_nb(int p) { return (p + 1) * (p + 2) * (p + 3) / 6; }
 __host__ __device__ constexpr int simplex_ncol(int p) { return (p + 1) * (p + 2) / 2; }
-// Threads per element of the RHS kernel, two candidates per order (a row
-// phase needs at least nb threads): variant 0 = 8 at order 1 (32 elements per
-// block), 12 at order 2 (21), 32 at order 3 (8), nb = 35 at order 4 (7);
-// variant 1 = 16 at order 1, 32 at order 2, 64 (one element per wavefront)
-// above. Small orders gain from many elements per block (fewer blocks, each
-// with its barriers and table staging). The library times both per order
-// when the operator is set and keeps the faster; results do not depend on
-// the choice (every row and item is computed by the same instructions
-// whichever thread takes it).
+// Elements per workgroup of the RHS kernel, two candidates per order, for met =
+// the face functions the order's elements meet (their own or a neighbour's).
+// The first fills a workgroup: one basis function per thread, and LDS for five
+// workgroups a CU; the second makes more workgroups, which small meshes need.
+// The library times both per order when the operator is set; results do not
+// depend on the choice (a column's sums do not depend on its tile). The
+// interface names the choices by thread counts per element.
 __host__ __device__ constexpr int simplex_tpe(int p) { return p == 1 ? 8 : p == 2 ? 12 : p == 3 ? 32 : simplex_nb(p); }
 __host__ __device__ constexpr int simplex_tpe_alt(int p) { return p == 1 ? 16 : p == 2 ? 32 : 64; }
 __host__ __device__ constexpr int simplex_tpe_of(int p, int variant) { return variant ? simplex_tpe_alt(p) : simplex_tpe(p); }
+__host__ __device__ constexpr int simplex_face_lanes(int met) { return met <= 3 ? 4 : met <= 6 ? 8 : 16; }
+constexpr int kSimplexLds = 3968;  // doubles
+constexpr int kTile = 8;           // elements per column tile of the matrix cores
 
-template <int P, int TPE_ = simplex_tpe(P), int TB = 8>
+template <int P>
 struct SimplexShape {
-    static_assert(TPE_ >= simplex_nb(P) && TPE_ <= 256, "a row phase needs one thread per basis function");
     static constexpr int NB = simplex_nb(P);
-    static constexpr int NCOL = simplex_ncol(P);
-    static constexpr int TPE = TPE_;  // threads per element
-    static constexpr int EPB = kBlock / TPE;
-    // doubles taken by n values of the arithmetic type (TB bytes), rounded
-    // up to an even count (regions start double2-aligned)
-    static constexpr int tw(int n) { return (n * TB + 15) / 16 * 2; }
-    // LDS carve-up of the RHS kernel, in doubles. FM and SF live through the
-    // whole kernel; the work area W holds the volume data (G, DR) and, at
-    // order 4 in FP64, afterwards one face's lift table; LIFT follows.
-    static constexpr int FM = 0;                            // [EPB][4 faces][4]: unit normal, sigma
-    static constexpr int SF = FM + EPB * 16;                // [EPB][4 faces][NCOL] (T pairs): flux coefficients
-    static constexpr int W = SF + tw(EPB * 8 * NCOL);
-    static constexpr int G = W;                             // [EPB][4][NB] (T): v, then g_r = sum_d (J^{-1})_{r,d} s_d
-    // DrT: read through the caches by the matrix-core tiles (orders 3 and 4,
-    // from a zero-padded copy of the table); otherwise staged in LDS
-    static constexpr bool DR_GLOBAL = P >= 3;
-    static constexpr int DR = G + tw(EPB * 4 * NB);         // [3][NB][NB] (T): DrT
-    static constexpr int VOL_END = DR + (DR_GLOBAL ? 0 : tw(3 * NB * NB));
-    static constexpr bool LIFT_LDS = P < 4;                 // lift table staged in LDS for the whole kernel
-    // order 4: the lift tables pass through the work area once the volume
-    // terms are done, LIFT_CHUNK faces at a time
-    static constexpr bool LIFT_ONE = !LIFT_LDS;
-    static constexpr int LIFT_CHUNK = 2;                    // faces per pass through the work area
-    static constexpr int LIFT = VOL_END;                    // [4 f][NCOL m][NB i] (T), the whole kernel
-    static constexpr int W_END = LIFT_ONE && W + tw(LIFT_CHUNK * NCOL * NB) > VOL_END ? W + tw(LIFT_CHUNK * NCOL * NB) : VOL_END;
-    static constexpr int TOTAL = LIFT_LDS ? LIFT + tw(4 * NCOL * NB) : W_END;
-    static_assert(SF % 2 == 0 && W % 2 == 0 && DR % 2 == 0 && LIFT % 2 == 0, "double2 alignment");
+    static constexpr int NC = simplex_ncol(P);
+    static constexpr int NTM = (NB + 15) / 16;           // row tiles
+    static constexpr int KS = (NB + 3) / 4;              // steps of a derivative
+    static constexpr int NBP = 16 * NTM, KP = 4 * KS;    // padded tables: [3][KP][NBP] and [4][16][NBP]
+    // LDS per element, in doubles: v and g_r ([4][NB]); the face integrands
+    // ([4 f][v, s][lanes]); J^{-1} and minus the sum of its rows ([4][3]) and
+    // 1/c_inv. The first two strides are odd multiples of four doubles, so that
+    // the eight elements of a tile lie in different banks.
+    static constexpr int ES = NB % 2 ? 4 * NB : 4 * NB + 4;
+    static constexpr int JS = 13;
+    static constexpr int fs(int lanes) { return 8 * lanes + 4; }
 };
 
-// Face-basis degree of coefficient m < 15 (degree d holds m in
-// [d(d+1)/2, (d+1)(d+2)/2)).
-__host__ __device__ constexpr int face_degree(int m) { return (m >= 1) + (m >= 3) + (m >= 6) + (m >= 10); }
+__host__ __device__ constexpr int simplex_elem_lds(int p, int lanes) {
+    return 4 * simplex_nb(p) + (simplex_nb(p) % 2 ? 0 : 4) + 8 * lanes + 4 + 13;
+}
+__host__ __device__ constexpr int simplex_epb(int p, int variant, int met) {
+    const int full = kBlock / simplex_nb(p), room = kSimplexLds / simplex_elem_lds(p, simplex_face_lanes(met));
+    const int n = full < room ? full : room;
+    return variant == 0 ? (n > kTile ? n / 4 * 4 : n) : p == 4 ? 4 : kTile;
+}
 
 typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ mfma_d4 mfma_step(double a, double b, mfma_d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
-typedef float mfma_f4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ mfma_f4 mfma_step(float a, float b, mfma_f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
-template <typename T>
-struct FluxPair {
-    T v, s;  // flux coefficient of the v equation, of the s equations
-};
-
-// ---- face traces (the first kernel of a right-hand side)
-// Every element writes, for each local face f, the chi_m-coefficients
-// (m < (p+1)(p+2)/2, degree <= p) of n_f.s and of v on that face in its own
-// face coordinates, n_f its own outward unit normal, into the trace buffer;
-// the element's neighbours read them in the RHS kernel. One block takes EPB
-// elements of one order, TPE threads each: stage input, normals and the
-// identity-orientation trace table into LDS; items (face, column): n.s and v
-// at the face columns; items (face, m): their projections.
-template <int P>
-struct TraceShape {
-    static constexpr int NB = simplex_nb(P), NC = simplex_ncol(P), TPE = simplex_tpe(P), EPB = kBlock / TPE;
-    static constexpr int FM = 0;                    // [EPB][4 f][3] unit normals
-    static constexpr int U = FM + EPB * 12;         // [EPB][4][NB] stage input
-    static constexpr int SO = U + EPB * 4 * NB;     // [EPB][4 f][NC] (double2): n.s and v at the face columns
-    static constexpr int PR = SO + EPB * 8 * NC;    // [4 f][NC c][NC m]: identity-orientation trace table
-    static constexpr int CL = PR + 4 * NC * NC;     // [4 f][NC] (int32, as NC * 2 doubles): the face column lists
-    static constexpr int TOTAL = CL + 2 * NC;
-    static_assert(SO % 2 == 0, "double2 alignment");
-};
-
-constexpr int trace_lds_doubles() {
-    constexpr int t[4] = {TraceShape<1>::TOTAL, TraceShape<2>::TOTAL, TraceShape<3>::TOTAL, TraceShape<4>::TOTAL};
-    int m = 0;
-    for (int k = 0; k < 4; ++k) m = t[k] > m ? t[k] : m;
-    return m;
-}
-
-template <int P>
-__device__ __forceinline__ void simplex_trace_block(const SimplexParams& p, int64_t first, int count, double* lds) {
-    using S = TraceShape<P>;
-    constexpr int NB = S::NB, NC = S::NC;
-    const int tid = threadIdx.x;
-    const int le = tid / S::TPE;
-    const int i = tid % S::TPE;
-    const int64_t e = first + le;
-    const bool elem_ok = le < count;
-    const int64_t E = p.n_elem;
-    const int32_t* tx = p.tix + (P - 1) * kTixStride;
-    double* fm = lds + S::FM + le * 12;
-    double* su = lds + S::U + le * 4 * NB;
-    if (elem_ok) {
-        for (int k = i; k < 12; k += S::TPE) fm[k] = p.normal[((k % 3) * 4 + k / 3) * E + e];  // fm[3 f + c]
-        if (i < NB) {
-            const int64_t base = p.group_dof[P - 1] + (e - p.group_start[P - 1]) * 4 * NB;
-            const int64_t at[4] = {base + i, base + NB + i, base + 2 * NB + i, base + 3 * NB + i};
-            double sv[4];
-            combine_n(p.io, at, sv);
-#pragma unroll
-            for (int f = 0; f < 4; ++f) su[f * NB + i] = sv[f];
-        }
-    }
-    {
-        const double* gP = p.tab + tx[kTixProjId];
-        double* sP = lds + S::PR;
-#pragma unroll 4
-        for (int k = tid; k < 4 * NC * NC; k += kBlock) sP[k] = gP[k];
-        int32_t* sc = reinterpret_cast<int32_t*>(lds + S::CL);
-        for (int k = tid; k < 4 * NC; k += kBlock) sc[k] = p.tix[tx[kTixCols + k / NC] + k % NC];
-    }
-    __syncthreads();
-    double2* so = reinterpret_cast<double2*>(lds + S::SO) + le * 4 * NC;
-    if (elem_ok) {
-        for (int it = i; it < 4 * NC; it += S::TPE) {
-            const int f = it / NC;
-            const int col = reinterpret_cast<const int32_t*>(lds + S::CL)[it];
-            so[it] = make_double2(fm[f * 3] * su[NB + col] + fm[f * 3 + 1] * su[2 * NB + col] +
-                                      fm[f * 3 + 2] * su[3 * NB + col],
-                                  su[col]);
-        }
-    }
-    __syncthreads();
-    if (elem_ok) {
-        double2* out = p.trace + p.group_tr[P - 1] + (e - p.group_start[P - 1]) * 4 * NC;
-        for (int it = i; it < 4 * NC; it += S::TPE) {
-            const int f = it / NC, m = it % NC;
-            const double* col = lds + S::PR + f * NC * NC + m;
-            const double2* x = so + f * NC;
-            double a = 0, b = 0;
-#pragma unroll 5
-            for (int c = 0; c < NC; ++c) {
-                const double r = col[c * NC];
-                const double2 v = x[c];
-                a += r * v.x;
-                b += r * v.y;
-            }
-            out[it] = make_double2(a, b);
-        }
-    }
-}
-
-// Blocks in order-group order: group g takes blocks [group_block[g],
-// group_block[g + 1]) of 256 / simplex_tpe(g + 1) elements each.
-__global__ __launch_bounds__(kBlock) void simplex_trace(const SimplexParams p) {
-    __shared__ __align__(16) double lds[trace_lds_doubles()];
-    const int b = int(blockIdx.x);
-    int g = 0;
-    while (g < 3 && b >= p.group_block[g + 1]) ++g;
-    const int epb = kBlock / simplex_tpe(g + 1);
-    const int64_t first = p.group_start[g] + int64_t(b - p.group_block[g]) * epb;
-    const int64_t left = p.group_start[g + 1] - first;
-    const int count = left < epb ? int(left) : epb;
-    switch (g) {
-        case 0: simplex_trace_block<1>(p, first, count, lds); break;
-        case 1: simplex_trace_block<2>(p, first, count, lds); break;
-        case 2: simplex_trace_block<3>(p, first, count, lds); break;
-        default: simplex_trace_block<4>(p, first, count, lds); break;
-    }
-}
-
-// ---- the right-hand side (the second kernel)
-// Tetrahedral elements of order P: a block takes EPB consecutive device
-// elements of that order, TPE threads per element, in phases separated by
-// barriers:
-//  1. the stage input (all four fields) as v and g_r = sum_d (J^{-1})_{r,d}
-//     s_d per basis function, the faces' normals and area ratios, and the
-//     order's derivative and lift tables into LDS; items (face, m): the flux
-//     coefficients from the element's own traces and its neighbours' (in the
-//     neighbour's face coordinates, brought into ours by the orientation
-//     map's degree block, R_o; the neighbour's n.s is with its own normal,
-//     the negative of ours), central on internal faces, the wall flux on
-//     reflecting walls;
-//  2. threads of a row: the volume terms;
-//  3. threads of a row: the lift of the flux coefficients.
-// Every face term is a polynomial of degree <= 4 in the face coordinates and
-// chi spans P_4, so the coefficients represent it exactly; only chi_m of
-// degree <= p reach the lift (chi_m of higher degree are orthogonal to the
-// element's traces), so a face of an order-p element carries (p+1)(p+2)/2
-// coefficients, and the orientation maps keep degrees apart, so a neighbour of
-// order p_n contributes to degrees <= min(p, p_n) only. T = double: FP64;
-// T = float: the volume contractions and the lifts in FP32 on FP32 tables,
-// compensated per-row sums, traces and flux coefficients in FP64.
-template <int P, int TPE, typename T>
-__device__ __forceinline__ void simplex_block(const SimplexParams& p, int64_t first, int count, double* lds) {
-    using S = SimplexShape<P, TPE, int(sizeof(T))>;
+// One workgroup takes `count` consecutive device elements of order P.
+//
+// With g_r = sum_d (J^{-1})_{r,d} s_d, and grad lambda_o the gradient of the
+// barycentric coordinate of the vertex opposite face f (rows of J^{-1}; for
+// vertex 0 minus their sum), sigma_f n_f = -grad lambda_o (n_f the outward
+// normal, sigma_f area over volume). The first three local faces are opposite
+// vertices 1..3, so both equations share one operator per direction r:
+//   k_v   =             sum_r [ Dr_r g_r + L_r A_r ] + L_3 A_3
+//   k_s_d = (1/c_inv) sum_r (J^{-1})_{r,d} [ Dr_r v + L_r B_r + L_3 B_3 ]
+// with the face integrands (sigma_f times the flux of the v equation, and
+// minus / plus half the jump of v) as coefficients of the face functions,
+//   A_f = 1/2 grad lambda_o.(s_own - s_nbr),  B_f = 1/2 (v_own - v_nbr)  (f < 3; minus that for f = 3)
+// on internal faces and A_f = grad lambda_o.s_own, B_f = 0 on walls.
+//
+// The face functions of f are the traces of the order-4 element functions
+// that do not vanish there (hierarchical: order p has the first (p+1)(p+2)/2
+// of them), so an own trace is the element's coefficients of those functions,
+// and L_f = M_ref^{-1} int_f phi_i psi_m lifts them. A neighbour's traces in
+// our face coordinates are its coefficients of its face's functions, up to
+// their order and signs: the vertex, edge and degree-3 face functions of the
+// two sides match one to one, and the two degree-4 face functions are
+// combinations with coefficients 0, +-1 of the other side's two (checked when
+// the table is built). So a face function m needs one of the neighbour's
+// functions, of every field, gathered from the stage input itself.
+//
+// Phases: (1) own stage input as v and g_r to LDS, the neighbours' values in
+// registers, one face function per lane; (2) face integrands to LDS; (3) on
+// the matrix cores, per row tile and tile of eight elements, four
+// accumulators (r = 0..2 and the fourth face) over 16 columns [g_r or A | v
+// or B]: A(i, k) from lane i + 16 k, B(k, j) from lane j + 16 k, output q of
+// lane l holds D(4 q + l / 16, l % 16). A lane then holds k_v, or the brackets
+// of k_s, of its element and rows; (4) k goes back through LDS, so that stores
+// and the fused update's reads are in order.
+//
+// Bound by latency, not by a unit: at 24^3 x 5 elements of order 1..4 a launch
+// takes 71.5 us in FP64 (100.7 before: a launch of 28 us that wrote projected
+// traces of every face, and one of 73 that gathered them, with the matrix units
+// for the derivatives of orders 3 and 4 alone), 69.7 with FP32 stage values (81.1); the bytes of one launch, 92 MB,
+// take 19 us and the matrix instructions keep their units busy for 15 us.
+// Whole orders: 31.8 -> 23.3, 53 -> 39.7, 113 -> 66.2 and 179 -> 102.8 us for
+// p = 1..4; 13 x 11 x 9 cells of order 2 (launch-bound, two before) 14.7 ->
+// 10.1 us. Arithmetic is FP64 whatever the stage values' type: the matrix units
+// are not what bounds this, and it leaves the FP32 path the rounding of its
+// stored values as its only error. Five workgroups a CU, at the price of a few spilled
+// registers, beat four without (77.9 us) and three (102 registers and 32
+// accumulation registers, 78.4).
+template <int P, int KIND, bool UPD>
+__device__ __forceinline__ void simplex_block(const SimplexParams& p, int64_t first, int count, int met, double* lds) {
+    using S = SimplexShape<P>;
     constexpr int NB = S::NB;
-    constexpr int NC = S::NCOL;
+    constexpr int NI = 2;  // face functions a thread has in flight
     const int tid = threadIdx.x;
-    const int le = tid / S::TPE;
-    const int i = tid % S::TPE;
-    const int64_t e = first + le;
-    const bool elem_ok = le < count;
-    const bool row_ok = elem_ok && (i < NB);
     const int64_t E = p.n_elem;
-    const int64_t base = p.group_dof[P - 1] + (e - p.group_start[P - 1]) * 4 * NB;
-    double* fm = lds + S::FM + le * 16;
-    FluxPair<T>* sf = reinterpret_cast<FluxPair<T>*>(lds + S::SF) + le * 4 * NC;
-    T* sg = reinterpret_cast<T*>(lds + S::G) + le * 4 * NB;
-    T* sDr = reinterpret_cast<T*>(lds + S::DR);
-    const T* tabT = std::is_same<T, float>::value ? reinterpret_cast<const T*>(p.tab32)
-                                                  : reinterpret_cast<const T*>(p.tab);
+    const int64_t base0 = p.group_dof[P - 1] + (first - p.group_start[P - 1]) * 4 * NB;
+    const int lg = met <= 3 ? 2 : met <= 6 ? 3 : 4;  // lanes per face: 4, 8 or 16
+    const int FL = 1 << lg, FS = S::fs(FL);
+    double* sG = lds;
+    double* sF = sG + count * S::ES;
+    double* sJ = sF + count * FS;
+    const int lane = tid % 64, wave = tid / 64;
 
-    // ---- phase 1: geometry, stage input as v and g, flux coefficients, tables
-    double cinv = 1.0;
-    if (elem_ok) {
-        cinv = p.cinv[e];
-        for (int k = i; k < 16; k += S::TPE) {
-            const int f = k / 4, c = k % 4;
-            fm[k] = c < 3 ? p.normal[(c * 4 + f) * E + e] : p.sigma[f * E + e];
+    // ---- phase 1: geometry, own values and what the faces meet; then the
+    // neighbours' values
+    const int n_items = count << (2 + lg);
+    const int f = (tid >> lg) & 3, m = tid & (FL - 1);  // the same for all of a thread's items
+    uint2 rec[NI];
+    int code[NI];
+    auto fetch_faces = [&](int i0) {
+#pragma unroll
+        for (int k = 0; k < NI; ++k) {
+            const int it = i0 + tid + k * kBlock;
+            rec[k] = make_uint2(0, 0);
+            code[k] = 0;
+            if (it < n_items) {
+                rec[k] = p.frec[first * 4 + (it >> lg)];
+                code[k] = p.fcode[(first * 4 + (it >> lg)) * 16 + m];
+            }
         }
+    };
+    int64_t nbr_at[4 * NI];
+    double w[4 * NI], w1[4 * NI];  // per face function the neighbour's v and s
+    auto fetch_neighbours = [&] {
+#pragma unroll
+        for (int k = 0; k < NI; ++k) {
+            const int nbn = rec[k].y & 63;
+            const int64_t b = code[k] != 0 ? int64_t(rec[k].x) * 4 + (code[k] & 63) : base0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) nbr_at[4 * k + q] = b + (code[k] != 0 ? q * nbn : 0);
+        }
+        load_two<KIND>(p.io, nbr_at, w, w1);
+    };
+    fetch_faces(0);
+    const int own_fn = p.cols[f * 16 + m];
+    const bool row_ok = tid < count * NB;
+    const int row_le = tid / NB;
+    int64_t own_at[4];
+    double u[4], u1[4];
+    {
+        const int64_t b = base0 + (row_ok ? row_le * 4 * NB + tid % NB : 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) own_at[q] = b + q * NB;
     }
+    load_two<KIND>(p.io, own_at, u, u1);
+    for (int k = tid; k < count * S::JS; k += kBlock) {
+        const int le = k / S::JS, c = k % S::JS;
+        const double* Jp = p.jinv + first + le;
+        sJ[k] = c < 9 ? Jp[c * E] : c < 12 ? -(Jp[(c - 9) * E] + Jp[(c - 6) * E] + Jp[(c - 3) * E])
+                                  : 1.0 / p.cinv[first + le];
+    }
+    __syncthreads();
+    fetch_neighbours();
+    mix_two<KIND>(p.io, own_at, u, u1);
     if (row_ok) {
-        double Ji[9];
+        double* g = sG + row_le * S::ES + tid % NB;
+        const double* J = sJ + row_le * S::JS;
+        g[0] = u[0];
 #pragma unroll
-        for (int q = 0; q < 9; ++q) Ji[q] = p.jinv[q * E + e];
-        const int64_t at[4] = {base + i, base + NB + i, base + 2 * NB + i, base + 3 * NB + i};
-        double sv[4];
-        combine_n(p.io, at, sv);
-        sg[i] = T(sv[0]);
-#pragma unroll
-        for (int r = 0; r < 3; ++r) sg[(1 + r) * NB + i] = T(Ji[r * 3] * sv[1] + Ji[r * 3 + 1] * sv[2] + Ji[r * 3 + 2] * sv[3]);
+        for (int r = 0; r < 3; ++r) g[(1 + r) * NB] = fma(J[3 * r + 2], u[3], fma(J[3 * r + 1], u[2], J[3 * r] * u[1]));
     }
-    if (elem_ok) {
-        const double2* own = p.trace + p.group_tr[P - 1] + (e - p.group_start[P - 1]) * 4 * NC;
-        const double* rot = p.tab + p.tix[kTixRot];
-        // every item's own trace and face data first, then the neighbours'
-        // coefficients (their addresses need the face data)
-        constexpr int NIT = (4 * NC + S::TPE - 1) / S::TPE;  // items per thread
-        int nb_[NIT], inf_[NIT];
-        double2 a_[NIT];
+
+    // ---- the matrix cores' first task of this wave (phase 3) and its first
+    // table values: the values of one direction, or of two faces, are loaded
+    // while the previous ones are multiplied
+    const int col = lane % 16, kk = lane / 16;
+    const bool vcol = col >= kTile;
+    const int tasks = S::NTM * ((count + kTile - 1) / kTile);  // (row tile fast, column tile slow)
+    const int rt = wave % S::NTM;
+    const double* Dr = p.tab + p.tab_dr[P - 1] + kk * S::NBP + 16 * rt + col;
+    const double* L = p.tab + p.tab_lift[P - 1] + kk * S::NBP + 16 * rt + col;
+    constexpr int AG = S::KS > 8 ? S::KS : 8;
+    double av[2][AG];
+    auto fetch = [&](int g, double (&a)[AG]) {
+        if (g < 3) {
 #pragma unroll
-        for (int k = 0; k < NIT; ++k) {
-            const int it = i + k * S::TPE;
-            nb_[k] = -1; inf_[k] = 0; a_[k] = make_double2(0, 0);
-            if (it < 4 * NC) {
-                const int f = it / NC;
-                nb_[k] = p.nbr[f * E + e];
-                inf_[k] = p.info[f * E + e];
-                a_[k] = own[it];
-            }
+            for (int s = 0; s < S::KS; ++s) a[s] = Dr[(g * S::KP + 4 * s) * S::NBP];
+        } else {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) a[s] = L[(((g - 3) * 2 + s / 4) * 16 + 4 * (s % 4)) * S::NBP];
         }
+    };
+    fetch(0, av[0]);
+    mix_two<KIND>(p.io, nbr_at, w, w1);
+    __syncthreads();
+
+    // ---- phase 2: the face integrands
+    for (int i0 = 0;;) {
 #pragma unroll
-        for (int k = 0; k < NIT; ++k) {
-            const int it = i + k * S::TPE;
-            if (it >= 4 * NC) continue;
-            const int m = it % NC;
-            const int nbr = nb_[k];
-            const double2 a = a_[k];
-            double Fv, Fs;
-            if (nbr >= 0) {
-                const int inf = inf_[k];
-                const int pn = info_pn(inf);
-                const int d = face_degree(m);
-                double bns = 0, bv = 0;
-                if (d <= pn) {
-                    const int o = info_rel(inf);
-                    const int m0 = d * (d + 1) / 2, ncn = simplex_ncol(pn);
-                    const double* R = rot + o * 55 + d * (d + 1) * (2 * d + 1) / 6 + (m - m0) * (d + 1);
-                    const double2* x = p.trace + p.group_tr[pn - 1] + (nbr - p.group_start[pn - 1]) * 4 * ncn +
-                                       info_lf(inf) * ncn + m0;
-                    double rr[5];
-                    double2 xv[5];
+        for (int k = 0; k < NI; ++k) {
+            const int it = i0 + tid + k * kBlock, le = it >> (lg + 2);
+            const bool in = it < n_items;
+            double Jf[3] = {0, 0, 0};
+            if (in) {
 #pragma unroll
-                    for (int b = 0; b < 5; ++b)
-                        if (b <= d) {
-                            rr[b] = R[b];
-                            xv[b] = x[b];
-                        }
-#pragma unroll
-                    for (int b = 0; b < 5; ++b)
-                        if (b <= d) {
-                            bns += rr[b] * xv[b].x;
-                            bv += rr[b] * xv[b].y;
-                        }
-                }
-                Fv = -0.5 * (a.x + bns);  // n.(s_own - s_nbr), the neighbour's traces with n_nbr = -n
-                Fs = -0.5 * (a.y - bv);
-            } else {
-                Fv = -a.x;
-                Fs = 0;
+                for (int d = 0; d < 3; ++d) Jf[d] = sJ[le * S::JS + 3 * f + d];
             }
-            sf[it] = FluxPair<T>{T(Fv), T(Fs)};
+            const double nv = w[4 * k], ng = fma(Jf[2], w[4 * k + 3], fma(Jf[1], w[4 * k + 2], Jf[0] * w[4 * k + 1]));
+            // the other of the two degree-4 face functions sits in the lane of 27 - m
+            const int partner = m >= 13 && m < 15 ? lane + 27 - 2 * m : lane;
+            const double pv = __shfl(nv, partner, 64), pg = __shfl(ng, partner, 64);
+            if (!in) continue;
+            double bv = 0, bg = 0;
+            const int c1 = code[k] >> 6, c2 = m >= 13 ? (rec[k].y >> (m == 13 ? 8 : 10)) & 3 : 0;  // 1: +, 2: -
+            if (c1 == 1 || c1 == 2) {
+                bv = c1 == 1 ? nv : -nv;
+                bg = c1 == 1 ? ng : -ng;
+            }
+            if (c2 != 0) {
+                bv += c2 == 1 ? pv : -pv;
+                bg += c2 == 1 ? pg : -pg;
+            }
+            double ov = 0, og = 0;
+            if (m < S::NC) {
+                const double* g = sG + le * S::ES + own_fn;
+                ov = g[0];
+                og = f < 3 ? g[(1 + f) * NB] : -(g[NB] + g[2 * NB] + g[3 * NB]);
+            }
+            const bool inner = (rec[k].y & 64) != 0;
+            double* out = sF + le * FS + f * 2 * FL + m;
+            out[0] = inner ? 0.5 * (og - bg) : og;
+            out[FL] = inner ? (f < 3 ? 0.5 : -0.5) * (ov - bv) : 0.0;
         }
-    }
-    const T* gDr = tabT + p.tix[(P - 1) * kTixStride + kTixDrT];
-    if constexpr (!S::DR_GLOBAL) {
-#pragma unroll 4
-        for (int k = tid; k < 3 * NB * NB; k += kBlock) sDr[k] = gDr[k];
-    }
-    const T* gLift = tabT + p.tix[(P - 1) * kTixStride + kTixLift];
-    T* sLift = reinterpret_cast<T*>(lds + S::LIFT);
-    if constexpr (S::LIFT_LDS) {
-#pragma unroll 4
-        for (int k = tid; k < 4 * NC * NB; k += kBlock) sLift[k] = gLift[k];
+        i0 += NI * kBlock;
+        if (i0 >= n_items) break;
+        fetch_faces(i0);
+        fetch_neighbours();
+        mix_two<KIND>(p.io, nbr_at, w, w1);
     }
     __syncthreads();
 
-    // ---- phase 2: volume, k_v = sum_r Dr_r g_r ; k_s_d = (1/c_inv) sum_r (J^{-1})_{r,d} Dr_r v
-    // Orders 3 and 4 on the matrix cores: per direction r, Dr_r times the
-    // block's columns [g_r of elements 0..7 | v of elements 0..7] in
-    // 16 x 16 x 4 tiles, one row tile per wavefront (A(i, k) from lane
-    // i + 16 k, B(k, j) from lane j + 16 k; output q of lane l holds
-    // D(4 q + l / 16, l % 16) for v_mfma_f64_16x16x4f64 and
-    // D(4 (l / 16) + q, l % 16) for v_mfma_f32_16x16x4f32). In FP64 each
-    // output accumulates its products in k order, one fused multiply-add
-    // after another, as the row loop below does: the results are bitwise
-    // those of the VALU form (checked on the 24^3 x 5 workload); in FP32 the
-    // 100-step RK4 run of that workload gives the row loop's error against
-    // FP64 to every digit. Orders 1 and 2: the row loop.
-    Acc<T> kv, ks[3];
-    // order 4: the first lift chunk is loaded into registers while the
-    // volume terms finish, and stored to LDS once they are done
-    constexpr int LPRE = S::LIFT_ONE ? (S::LIFT_CHUNK * NC * NB + kBlock - 1) / kBlock : 1;
-    T lpre[LPRE];
-    if constexpr (P >= 3) {
-        static_assert(S::EPB <= 8, "16 columns");
-        static_assert(S::DR_GLOBAL, "the tiles read the padded table through the caches");
-        constexpr int NTM = (NB + 15) / 16, KS = (NB + 3) / 4;
-        constexpr int NBP = 16 * NTM, KP = 4 * KS;  // the padded table: [3][KP][NBP]
-        using V4 = typename std::conditional<std::is_same<T, double>::value, mfma_d4, mfma_f4>::type;
-        const int lane = tid % 64, wave = tid / 64;
-        const int col = lane % 16, kk = lane / 16;
-        const int ce = col % 8, cv = col / 8;
-        T* sG0 = reinterpret_cast<T*>(lds + S::G);
-        V4 acc[3];
+    // ---- phase 3: derivatives and lifts on the matrix cores; the results
+    // take the place of v and g_r. Orders 1 and 2 have one row tile: the wave
+    // is the only reader of its column tile's values. Orders 3 and 4 have one
+    // task per wave, whose results wait for the other waves' reads.
+    const int fsteps = (met + 3) / 4;
+    static_assert(S::NTM == 1 || S::NTM * 2 <= 4 || P == 4, "one task per wave");
+    mfma_d4 acc[4];
+    auto multiply = [&](int ct) {
 #pragma unroll
-        for (int r = 0; r < 3; ++r) acc[r] = V4{T(0), T(0), T(0), T(0)};
-        if (wave < NTM) {
-            // per direction the A operands first (zeros outside nb x nb come
-            // from the table, so every load is unconditional), then the
-            // accumulation chain
-            const T* Dr = tabT + p.tix[(P - 1) * kTixStride + kTixDrP] + kk * NBP +
-                          16 * wave + col;
+        for (int r = 0; r < 4; ++r) acc[r] = mfma_d4{0, 0, 0, 0};
+        const int le = ct * kTile + col % kTile < count ? ct * kTile + col % kTile : count - 1;
+        const double* gB = sG + le * S::ES + kk;
+        const double* fB = sF + le * FS + (vcol ? FL : 0) + kk;
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                T av[KS];
+        for (int g = 0; g < 5; ++g) {
+            if (g < 4) fetch(g + 1, av[(g + 1) % 2]);
+            const double (&a)[AG] = av[g % 2];
+            if (g < 3) {
 #pragma unroll
-                for (int s = 0; s < KS; ++s) av[s] = Dr[(r * KP + 4 * s) * NBP];
+                for (int s = 0; s < S::KS; ++s) {
+                    // (the table is zero beyond NB, but zero times a stray infinity is not)
+                    const double b = 4 * s + 3 < NB || 4 * s + kk < NB ? gB[(vcol ? 0 : 1 + g) * NB + 4 * s] : 0.0;
+                    acc[g] = mfma_step(a[s], b, acc[g]);
+                }
+            } else {
 #pragma unroll
-                for (int s = 0; s < KS; ++s) {
-                    const int k = 4 * s + kk;
-                    const T bv = (ce < count && k < NB) ? sG0[ce * 4 * NB + (cv ? 0 : 1 + r) * NB + k] : T(0);
-                    acc[r] = mfma_step(av[s], bv, acc[r]);
+                for (int s = 0; s < 8; ++s) {
+                    const int q = (g - 3) * 2 + s / 4;
+                    if (s % 4 < fsteps) acc[q] = mfma_step(a[s], fB[q * 2 * FL + 4 * (s % 4)], acc[q]);
                 }
             }
         }
-        if constexpr (S::LIFT_ONE) {
+    };
+    auto keep = [&](int ct) {
+        const int le = ct * kTile + col % kTile;
+        if (le >= count) return;
+        const double* J = sJ + le * S::JS;
+        const double ci = J[12];
+        double* out = sG + le * S::ES;
 #pragma unroll
-            for (int j = 0; j < LPRE; ++j) {
-                const int k = tid + j * kBlock;
-                lpre[j] = k < S::LIFT_CHUNK * NC * NB ? gLift[k] : T(0);
+        for (int q = 0; q < 4; ++q) {
+            const int row = 16 * rt + 4 * q + kk;
+            if (row >= NB) continue;
+            if (!vcol) {
+                out[row] = acc[0][q] + acc[1][q] + acc[2][q] + acc[3][q];
+            } else {
+                double b[3];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) b[r] = acc[r][q] + acc[3][q];
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    out[(1 + d) * NB + row] = fma(J[6 + d], b[2], fma(J[3 + d], b[1], J[d] * b[0])) * ci;
             }
         }
-        __syncthreads();  // every wave has read the inputs
-        if (wave < NTM) {
-#pragma unroll
-            for (int ri = 0; ri < 4; ++ri) {
-                const int row = 16 * wave + (std::is_same<T, double>::value ? 4 * ri + lane / 16 : 4 * (lane / 16) + ri);
-                if (row < NB && ce < count) {
-                    T* o = sG0 + ce * 4 * NB;
-                    if (cv == 0) o[row] = acc[0][ri] + acc[1][ri] + acc[2][ri];
-                    else {
-#pragma unroll
-                        for (int r = 0; r < 3; ++r) o[(1 + r) * NB + row] = acc[r][ri];
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        if (row_ok) {
-            T Jt[9];
-#pragma unroll
-            for (int q = 0; q < 9; ++q) Jt[q] = T(p.jinv[q * E + e]);
-            kv = Acc<T>(sg[i]);
-            const T ci = T(1.0 / cinv);
-            const T bb[3] = {sg[NB + i], sg[2 * NB + i], sg[3 * NB + i]};
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                ks[d] = Acc<T>((Jt[d] * bb[0] + Jt[3 + d] * bb[1] + Jt[6 + d] * bb[2]) * ci);
+    };
+    if constexpr (S::NTM == 1) {
+        for (int t = wave; t < tasks; t += kBlock / 64) {
+            if (t != wave) fetch(0, av[0]);
+            multiply(t);
+            keep(t);
         }
     } else {
-        T a[3] = {T(0), T(0), T(0)}, b[3] = {T(0), T(0), T(0)};
-        if (row_ok) {
-#pragma unroll 4
-            for (int j = 0; j < NB; ++j) {
-                const T v = sg[j];
-#pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    const T d = sDr[(r * NB + j) * NB + i];
-                    a[r] += d * sg[(1 + r) * NB + j];
-                    b[r] += d * v;
-                }
-            }
-        }
-        if (row_ok) {
-            T Jt[9];  // J^{-1} again (not kept in registers across the barrier)
-#pragma unroll
-            for (int q = 0; q < 9; ++q) Jt[q] = T(p.jinv[q * E + e]);
-            kv = Acc<T>(a[0] + a[1] + a[2]);
-            const T ci = T(1.0 / cinv);
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                ks[d] = Acc<T>((Jt[d] * b[0] + Jt[3 + d] * b[1] + Jt[6 + d] * b[2]) * ci);
-        }
-    }
-
-    // ---- phase 3: k += sigma_f sum_m (M_ref^{-1} int_f phi chi_m)_i F_m
-    // (order 4: the lift table passes through the work area, dead once the
-    // volume terms are done, LIFT_CHUNK faces at a time)
-    T* sL1 = reinterpret_cast<T*>(lds + S::W);
-    constexpr int LC = S::LIFT_CHUNK;
-    if constexpr (S::LIFT_ONE) {
-        __syncthreads();  // the volume data give way to the first faces' lift tables
-#pragma unroll
-        for (int j = 0; j < LPRE; ++j) {
-            const int k = tid + j * kBlock;
-            if (k < LC * NC * NB) sL1[k] = lpre[j];
-        }
+        if (wave < tasks) multiply(wave / S::NTM);
         __syncthreads();
+        if (wave < tasks) keep(wave / S::NTM);
     }
-    const T ci = T(1.0 / cinv);
-#pragma unroll 1
-    for (int f = 0; f < 4; ++f) {
-        const T* lift;
-        if constexpr (S::LIFT_LDS) {
-            lift = sLift + f * NC * NB + i;
-        } else if constexpr (!S::LIFT_ONE) {
-            lift = gLift + f * NC * NB + i;
-        } else {
-            if (f > 0 && f % LC == 0) {
-                __syncthreads();  // the block is done with the previous faces
-                for (int k = tid; k < LC * NC * NB; k += kBlock) sL1[k] = gLift[f * NC * NB + k];
-                __syncthreads();
-            }
-            lift = sL1 + (f % LC) * NC * NB + i;
-        }
-        if (row_ok) {
-            const FluxPair<T>* fl = sf + f * NC;
-            T lv = T(0), ls = T(0);
-#pragma unroll 5
-            for (int m = 0; m < NC; ++m) {
-                const T l = lift[m * NB];
-                const FluxPair<T> x = fl[m];
-                lv += l * x.v;
-                ls += l * x.s;
-            }
-            const T sig = T(fm[f * 4 + 3]);
-            kv.add(sig * lv);
-            const T c = sig * ls * ci;
-            ks[0].add(c * T(fm[f * 4]));
-            ks[1].add(c * T(fm[f * 4 + 1]));
-            ks[2].add(c * T(fm[f * 4 + 2]));
-        }
-    }
-    if (row_ok) {
-        const double vals[4] = {double(kv.value()), double(ks[0].value()), double(ks[1].value()),
-                                double(ks[2].value())};
-        double kept[4];  // the values as stored
+    __syncthreads();
+
+    // ---- phase 4: the block's values are stored (and the update read) in order
+    constexpr int NO = 4;  // outputs a thread has in flight
+    const int n_out = count * 4 * NB;
+    for (int i0 = tid; i0 < n_out; i0 += NO * kBlock) {
+        int64_t at[NO];
+        double k[NO];
 #pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            const int64_t o = base + f * NB + i;
+        for (int j = 0; j < NO; ++j) {
+            const int i = i0 + j * kBlock < n_out ? i0 + j * kBlock : i0;  // (past the end: the first once more)
+            at[j] = base0 + i;
+            k[j] = sG[i / (4 * NB) * S::ES + i % (4 * NB)];
             if (p.io.out_f32) {
-                const float v = float(vals[f]);
-                static_cast<float*>(p.io.out)[o] = v;
-                kept[f] = double(v);
+                const float v = float(k[j]);
+                static_cast<float*>(p.io.out)[at[j]] = v;
+                k[j] = double(v);
             } else {
-                static_cast<double*>(p.io.out)[o] = vals[f];
-                kept[f] = vals[f];
+                static_cast<double*>(p.io.out)[at[j]] = k[j];
             }
         }
-        if (p.io.upd.u != nullptr) {  // the RK update fused into a step's last stage (StageIO::upd)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                const double own[1] = {kept[f]};
-                rk_update_run<1>(p.io.upd, base + f * NB + i, own);
-            }
-        }
+        if constexpr (UPD) rk_update_n(p.io.upd, at, k);  // the RK update fused into a step's last stage
     }
 }
 
-template <int TB>
-constexpr int simplex_lds_doubles() {
-    constexpr int t[8] = {SimplexShape<1, simplex_tpe(1), TB>::TOTAL,     SimplexShape<2, simplex_tpe(2), TB>::TOTAL,
-                          SimplexShape<3, simplex_tpe(3), TB>::TOTAL,     SimplexShape<4, simplex_tpe(4), TB>::TOTAL,
-                          SimplexShape<1, simplex_tpe_alt(1), TB>::TOTAL, SimplexShape<2, simplex_tpe_alt(2), TB>::TOTAL,
-                          SimplexShape<3, simplex_tpe_alt(3), TB>::TOTAL, SimplexShape<4, simplex_tpe_alt(4), TB>::TOTAL};
-    int m = 0;
-    for (int k = 0; k < 8; ++k) m = t[k] > m ? t[k] : m;
-    return m;
+// What a face's lanes need of its neighbour, from the faces and the matching
+// table, once per mesh: per (element, face) the neighbour's first DOF / 4 and,
+// packed, its functions (bits 0-5), whether there is one (6) and the
+// coefficients of the partners of face functions 13 (8-9) and 14 (10-11); per
+// face function a byte: the neighbour's function (bits 0-5) and 64 times its
+// coefficient's code, or 192 if only the partner takes it; 0: nothing there.
+struct SimplexFaceParams {
+    int64_t n_elem;
+    const int32_t* nbr;
+    const int32_t* info;
+    const int64_t* elem_off;
+    const int32_t* tix;
+    uint2* frec;
+    uint8_t* fcode;
+};
+
+__global__ __launch_bounds__(kBlock) void simplex_faces(const SimplexFaceParams p) {
+    const int64_t it = int64_t(blockIdx.x) * kBlock + threadIdx.x;  // (element, face)
+    if (it >= 4 * p.n_elem) return;
+    const int64_t e = it / 4;
+    const int f = int(it % 4);
+    const int32_t nb = p.nbr[f * p.n_elem + e], info = p.info[f * p.n_elem + e];
+    uint2 rec = make_uint2(0, 0);
+    for (int m = 0; m < 16; ++m) {
+        int byte = 0;
+        if (nb >= 0) {
+            const int nbn = simplex_nb(info_pn(info));
+            rec.x = uint32_t(p.elem_off[nb] / 4);
+            rec.y |= uint32_t(nbn) | 64u;
+            const int code = p.tix[kTixFace + ((f * 4 + info_lf(info)) * 6 + info_rel(info)) * 16 + m];
+            if (m < kFaceBasis && (code & 63) < nbn) {
+                const int c1 = (code >> 6) & 3;
+                byte = (code & 63) | ((c1 == 0 ? 3 : c1) << 6);
+                if (m >= 13) rec.y |= uint32_t((code >> 8) & 3) << (m == 13 ? 8 : 10);
+            }
+        }
+        p.fcode[it * 16 + m] = uint8_t(byte);
+    }
+    p.frec[it] = rec;
 }
 
-// All orders in one launch. Blocks follow a schedule built on the host: the
+// All orders in one launch, one kernel for each way the stage values are stored
+// and counted (StageKind): deciding that inside costs registers. Blocks follow a schedule built on the host: the
 // mesh is cut into slabs of consecutive elements and, slab after slab, each
 // order's elements of the slab fill blocks of that order. With the XCD
-// renumbering an XCD works through neighbouring slabs, so the face columns an
+// renumbering an XCD works through neighbouring slabs, so the values an
 // element gathers from neighbours of every order are read while they are
-// still in that XCD's L2. The LDS carve-up of the largest order leaves room
-// for five blocks per CU; the register budget is set to match.
-template <typename T, int V>
+// still in that XCD's L2.
+template <int KIND, bool UPD>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void simplex_acoustic_rhs(const SimplexParams p) {
-    __shared__ __align__(16) double lds[simplex_lds_doubles<int(sizeof(T))>()];  // regions start at even doubles
+    __shared__ double lds[kSimplexLds];
     const int4 bl = p.blocks[xcd_block(blockIdx.x, gridDim.x)];
-    switch (bl.x) {  // the same order for the whole block; bit p-1 of V: the order's threads-per-element variant
-        case 1: simplex_block<1, simplex_tpe_of(1, V & 1), T>(p, bl.y, bl.z, lds); break;
-        case 2: simplex_block<2, simplex_tpe_of(2, (V >> 1) & 1), T>(p, bl.y, bl.z, lds); break;
-        case 3: simplex_block<3, simplex_tpe_of(3, (V >> 2) & 1), T>(p, bl.y, bl.z, lds); break;
-        default: simplex_block<4, simplex_tpe_of(4, (V >> 3) & 1), T>(p, bl.y, bl.z, lds); break;
+    switch (bl.x) {  // the same order for the whole block
+        case 1: simplex_block<1, KIND, UPD>(p, bl.y, bl.z, bl.w, lds); break;
+        case 2: simplex_block<2, KIND, UPD>(p, bl.y, bl.z, bl.w, lds); break;
+        case 3: simplex_block<3, KIND, UPD>(p, bl.y, bl.z, bl.w, lds); break;
+        default: simplex_block<4, KIND, UPD>(p, bl.y, bl.z, bl.w, lds); break;
     }
 }
 
@@ -635,8 +480,13 @@ struct SimplexDiffParams {
 };
 
 template <int P>
+struct SimplexRows {
+    static constexpr int NB = simplex_nb(P), TPE = simplex_tpe(P), EPB = kBlock / TPE;
+};
+
+template <int P>
 __device__ void simplex_diff_block(const SimplexDiffParams& p, int blk, double* sd, double* red) {
-    using S = SimplexShape<P>;
+    using S = SimplexRows<P>;
     constexpr int NB = S::NB;
     const int tid = threadIdx.x;
     const int le = tid / S::TPE;
@@ -677,8 +527,8 @@ __device__ void simplex_diff_block(const SimplexDiffParams& p, int blk, double* 
 }
 
 __global__ __launch_bounds__(kBlock) void simplex_diff_norm(const SimplexDiffParams p) {
-    constexpr int n1 = SimplexShape<1>::EPB * 4 * SimplexShape<1>::NB, n2 = SimplexShape<2>::EPB * 4 * SimplexShape<2>::NB;
-    constexpr int n3 = SimplexShape<3>::EPB * 4 * SimplexShape<3>::NB, n4 = SimplexShape<4>::EPB * 4 * SimplexShape<4>::NB;
+    constexpr int n1 = SimplexRows<1>::EPB * 4 * SimplexRows<1>::NB, n2 = SimplexRows<2>::EPB * 4 * SimplexRows<2>::NB;
+    constexpr int n3 = SimplexRows<3>::EPB * 4 * SimplexRows<3>::NB, n4 = SimplexRows<4>::EPB * 4 * SimplexRows<4>::NB;
     constexpr int n12 = n1 > n2 ? n1 : n2, n34 = n3 > n4 ? n3 : n4;
     __shared__ double sd[n12 > n34 ? n12 : n34];  // [EPB][4][NB] of the largest order group
     __shared__ double red[2 * kBlock];
@@ -910,6 +760,40 @@ std::vector<int64_t> locality_rank(const hgdg_mesh_desc* m) {
 
 }  // namespace
 
+namespace {
+
+// P^{-1} Q of two kFaceBasis x kFaceBasis matrices, row-major (Gauss-Jordan in
+// long double, partial pivoting).
+std::vector<double> face_match(const std::vector<double>& P, const std::vector<double>& Q) {
+    constexpr int n = kFaceBasis;
+    std::vector<long double> a(P.begin(), P.end()), b(Q.begin(), Q.end());
+    for (int k = 0; k < n; ++k) {
+        int piv = k;
+        for (int i = k + 1; i < n; ++i)
+            if (std::fabs(a[i * n + k]) > std::fabs(a[piv * n + k])) piv = i;
+        for (int j = 0; j < n; ++j) {
+            std::swap(a[k * n + j], a[piv * n + j]);
+            std::swap(b[k * n + j], b[piv * n + j]);
+        }
+        const long double d = a[k * n + k];
+        for (int j = 0; j < n; ++j) {
+            a[k * n + j] /= d;
+            b[k * n + j] /= d;
+        }
+        for (int i = 0; i < n; ++i) {
+            const long double f = a[i * n + k];
+            if (i == k || f == 0) continue;
+            for (int j = 0; j < n; ++j) {
+                a[i * n + j] -= f * a[k * n + j];
+                b[i * n + j] -= f * b[k * n + j];
+            }
+        }
+    }
+    return std::vector<double>(b.begin(), b.end());
+}
+
+}  // namespace
+
 void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     SimplexMesh& sm = c->sm;
     const int64_t ne = m->n_elements;
@@ -948,9 +832,6 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     }
     c->n_fields = nf;
     c->dof = sm.group_dof[4];
-    sm.group_tr[0] = 0;
-    for (int g = 0; g < 4; ++g) sm.group_tr[g + 1] = sm.group_tr[g] + counts[g] * 4 * simplex_ncol(g + 1);
-    sm.d_trace.alloc(size_t(2 * sm.group_tr[4]));
     std::vector<int64_t> elem_off(sm.dof_off);  // lives until the synchronize at the end
     elem_off.push_back(c->dof);
     sm.d_elem_off.upload(elem_off, c->stream);
@@ -991,12 +872,12 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     // faces: sorted node triples; the lower mesh index is hpGEM's left element
     sm.nbr_dev.assign(4 * size_t(ne), -1);
     sm.info.assign(4 * size_t(ne), 0);
-    sm.sigma.assign(4 * size_t(ne), 0.0);
-    sm.normal.assign(12 * size_t(ne), 0.0);
     struct Open { int64_t e; int f; };
     std::unordered_map<std::string, Open> open;
     open.reserve(size_t(ne) * 2);
     int64_t n_internal = 0, n_total = 0;
+    sm.sigma.assign(4 * size_t(ne), 0.0);
+    sm.normal.assign(12 * size_t(ne), 0.0);
     static const double V[4][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
     for (int64_t e = 0; e < ne; ++e) {
         const int64_t* nid = m->node_ids + size_t(e) * 4;
@@ -1054,9 +935,6 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     c->n_faces = n_total;
     c->n_internal = n_internal;
 
-    // reference tables of every order (see the kernel): DrT, M_ref, the face
-    // columns, the chi-coefficients of the face columns' traces per local face
-    // and orientation, and the lift in the element's own face coordinates
     int perm[6][kFaceQ];  // face point q after orientation o of the reference triangle
     for (int o = 0; o < 6; ++o)
         for (int qq = 0; qq < kFaceQ; ++qq) {
@@ -1074,7 +952,8 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     // the neighbour's face coordinates are o_nbr(o_own^{-1}(s)), itself one
     // of the six orientation maps (they form a group), identified here by
     // its action on the (symmetric) face rule points.
-    std::vector<int32_t> tix(size_t(kTixRot) + 1, 0);
+    std::vector<int32_t> tix(size_t(kTixSize), 0);
+    int rel_of[6][6];
     int ident = -1;
     for (int o = 0; o < 6 && ident < 0; ++o) {
         bool id = true;
@@ -1082,7 +961,6 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
         if (id) ident = o;
     }
     require(ident >= 0, HGDG_ERR_ARG, "no identity among the face orientation maps");
-    tix[kTixIdent] = ident;
     for (int oo = 0; oo < 6; ++oo) {
         int inv[kFaceQ];
         for (int qq = 0; qq < kFaceQ; ++qq) inv[perm[oo][qq]] = qq;
@@ -1094,66 +972,78 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
                 if (same) rel = o;
             }
             require(rel >= 0, HGDG_ERR_ARG, "face orientation maps do not compose");
-            tix[size_t(kTixRel) + oo * 6 + on] = rel;
+            rel_of[oo][on] = rel;
         }
     }
     for (size_t k = 0; k < sm.info.size(); ++k)
         if (sm.nbr_dev[k] >= 0)
-            sm.info[k] |= tix[size_t(kTixRel) + info_oown(sm.info[k]) * 6 + info_onbr(sm.info[k])] << 11;
+            sm.info[k] |= rel_of[info_oown(sm.info[k])][info_onbr(sm.info[k])] << 11;
     sm.ops.clear();
     for (int q = 1; q <= kMaxSimplexOrder; ++q) sm.ops.push_back(simplex_ops(q));
+    // reference tables of every order (see the kernel)
     std::vector<double> tab;
-    std::vector<int32_t> cols;
+    const SimplexOps& top = sm.ops[kMaxSimplexOrder - 1];
     for (int q = 1; q <= kMaxSimplexOrder; ++q) {
         const SimplexOps& ops = sm.ops[q - 1];
-        const int nb = ops.nb, nc = simplex_ncol(q);
+        const int nb = ops.nb, kp = 4 * ((nb + 3) / 4), ip = 16 * ((nb + 15) / 16);
         int32_t* t = tix.data() + (q - 1) * kTixStride;
-        t[kTixDrT] = int32_t(tab.size());
-        for (int r = 0; r < 3; ++r)
-            for (int j = 0; j < nb; ++j)
-                for (int i = 0; i < nb; ++i) tab.push_back(ops.Dr[(size_t(r) * nb + i) * nb + j]);
         t[kTixM] = int32_t(tab.size());
         tab.insert(tab.end(), ops.Mref.begin(), ops.Mref.end());
+        t[kTixDrP] = int32_t(tab.size());
+        for (int r = 0; r < 3; ++r)
+            for (int k = 0; k < kp; ++k)
+                for (int i = 0; i < ip; ++i)
+                    tab.push_back(k < nb && i < nb ? ops.Dr[(size_t(r) * nb + i) * nb + k] : 0.0);
+        t[kTixLift] = int32_t(tab.size());
         for (int f = 0; f < 4; ++f) {
-            require(int(ops.cols[f].size()) == nc, HGDG_ERR_ARG, "unexpected face column count");
-            t[kTixCols + f] = int32_t(cols.size());  // relative, fixed below
-            cols.insert(cols.end(), ops.cols[f].begin(), ops.cols[f].end());
+            // hierarchical: the order's face functions are the first of the order-4 ones
+            const int nc = simplex_ncol(q);
+            require(int(ops.cols[f].size()) == nc && int(top.cols[f].size()) == kFaceBasis &&
+                        std::equal(ops.cols[f].begin(), ops.cols[f].end(), top.cols[f].begin()),
+                    HGDG_ERR_ARG, "unexpected face functions");
+            for (int m = 0; m < 16; ++m)
+                for (int i = 0; i < ip; ++i) {
+                    long double v = 0;
+                    if (m < kFaceBasis && i < nb)
+                        for (int k = 0; k < kFaceBasis; ++k)
+                            v += (long double)ops.lift[f][ident][size_t(i) * kFaceBasis + k] *
+                                 top.proj[f][ident][size_t(k) * kFaceBasis + m];
+                    tab.push_back(double(v));
+                }
         }
-        t[kTixDrP] = int32_t(tab.size());  // [r][k < 4 ceil(nb/4)][i < 16 ceil(nb/16)], zeros outside nb x nb
-        if (q >= 3) {
-            const int kp = 4 * ((nb + 3) / 4), ip = 16 * ((nb + 15) / 16);
-            for (int r = 0; r < 3; ++r)
-                for (int k = 0; k < kp; ++k)
-                    for (int i = 0; i < ip; ++i)
-                        tab.push_back(k < nb && i < nb ? ops.Dr[(size_t(r) * nb + i) * nb + k] : 0.0);
-        }
-        t[kTixProjId] = int32_t(tab.size());  // [f][c < nc][m < nc]
-        for (int f = 0; f < 4; ++f)
-            for (int c = 0; c < nc; ++c)
-                for (int m = 0; m < nc; ++m) tab.push_back(ops.proj[f][ident][size_t(m) * nc + c]);
-        t[kTixProj] = int32_t(tab.size());  // [f][o][c < nc][m < kFaceBasis]
-        for (int f = 0; f < 4; ++f)
+    }
+    for (int g = 0; g < 4; ++g) {
+        sm.tab_dr[g] = tix[size_t(g) * kTixStride + kTixDrP];
+        sm.tab_lift[g] = tix[size_t(g) * kTixStride + kTixLift];
+    }
+    for (int f = 0; f < 4; ++f)
+        for (int m = 0; m < kFaceBasis; ++m) tix[size_t(kTixCols) + f * 16 + m] = top.cols[f][size_t(m)];
+    // neighbour's face functions in ours: P_f O = P_lf,rel (face-basis coefficients)
+    for (int f = 0; f < 4; ++f)
+        for (int lf = 0; lf < 4; ++lf)
             for (int o = 0; o < 6; ++o) {
-                require(ops.proj[f][o].size() == size_t(kFaceBasis) * nc, HGDG_ERR_ARG, "face trace table size");
-                for (int c = 0; c < nc; ++c)
-                    for (int m = 0; m < kFaceBasis; ++m) tab.push_back(ops.proj[f][o][size_t(m) * nc + c]);
+                const std::vector<double> O = face_match(top.proj[f][ident], top.proj[lf][o]);
+                for (int m = 0; m < kFaceBasis; ++m) {
+                    int from = m >= 13 ? m : -1, c1 = 0, c2 = 0;
+                    for (int q = 0; q < kFaceBasis; ++q) {
+                        const double v = O[size_t(m) * kFaceBasis + q];
+                        const int r = int(std::lround(v));
+                        require(std::fabs(v - r) < 1e-9 && std::abs(r) <= 1, HGDG_ERR_ARG, "face functions do not match");
+                        if (r == 0) continue;
+                        const int code = r > 0 ? 1 : 2;
+                        if (m < 13) {
+                            require(from < 0 && q < 13, HGDG_ERR_ARG, "face functions do not match one to one");
+                            from = q;
+                            c1 = code;
+                        } else {
+                            require(q >= 13, HGDG_ERR_ARG, "degree-4 face functions mix with others");
+                            (q == m ? c1 : c2) = code;
+                        }
+                    }
+                    require(from >= 0, HGDG_ERR_ARG, "a face function without match");
+                    tix[size_t(kTixFace) + ((f * 4 + lf) * 6 + o) * 16 + m] = top.cols[lf][size_t(from)] | (c1 << 6) | (c2 << 8);
+                }
             }
-        t[kTixLift] = int32_t(tab.size());  // [f][m < nc][i]: only chi_m of degree <= q meet the element's traces
-        for (int f = 0; f < 4; ++f)
-            for (int m = 0; m < nc; ++m)
-                for (int i = 0; i < nb; ++i) tab.push_back(ops.lift[f][ident][size_t(i) * kFaceBasis + m]);
-    }
-    {
-        const std::vector<double> rot = face_orientation_blocks();
-        require(rot.size() == 6 * size_t(kFaceRotBlock) && kFaceRotBlock == 55, HGDG_ERR_ARG, "orientation block table size");
-        tix[kTixRot] = int32_t(tab.size());
-        tab.insert(tab.end(), rot.begin(), rot.end());
-    }
-    const int32_t col_base = int32_t(tix.size());
-    for (int q = 0; q < kMaxSimplexOrder; ++q)
-        for (int f = 0; f < 4; ++f) tix[q * kTixStride + kTixCols + f] += col_base;
-    tix.insert(tix.end(), cols.begin(), cols.end());
-    require(tix.size() <= size_t(kTixMax), HGDG_ERR_ARG, "table index larger than its LDS copy");
 
     for (int g = 0; g < 4; ++g) {
         sm.tpe_variant[g] = sm.tpe_fixed[g] == simplex_tpe_alt(g + 1) ? 1 : 0;
@@ -1167,18 +1057,21 @@ void simplex_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     for (int q = 1; q <= kMaxSimplexOrder; ++q) mass.insert(mass.end(), sm.ops[q - 1].Minv.begin(), sm.ops[q - 1].Minv.end());
     sm.d_mass.upload(mass, c->stream);
     sm.d_order.upload(sm.order, c->stream);
-    const std::vector<float> tab32(tab.begin(), tab.end());  // lives until the synchronize below
-    sm.d_tables32.upload(tab32, c->stream);
     sm.d_tab_index.upload(tix, c->stream);
     sm.d_absdet.upload(sm.absdet, c->stream);
     std::vector<double> geo(jinv_soa);
     geo.resize(geo.size() + size_t(ne), 1.0);  // c_inv, set with the operator
-    geo.insert(geo.end(), sm.sigma.begin(), sm.sigma.end());
-    geo.insert(geo.end(), sm.normal.begin(), sm.normal.end());
     sm.d_geo.upload(geo, c->stream);
     std::vector<int32_t> face(sm.nbr_dev);
     face.insert(face.end(), sm.info.begin(), sm.info.end());
     sm.d_face.upload(face, c->stream);
+    require(c->dof / 4 <= int64_t(UINT32_MAX), HGDG_ERR_UNSUPPORTED, "more than 2^34 degrees of freedom");
+    sm.d_frec.alloc(8 * size_t(ne));
+    sm.d_fcode.alloc(64 * size_t(ne));
+    SimplexFaceParams fp{ne, sm.d_face.ptr, sm.d_face.ptr + 4 * ne, sm.d_elem_off.ptr, sm.d_tab_index.ptr,
+                         reinterpret_cast<uint2*>(sm.d_frec.ptr), sm.d_fcode.ptr};
+    hipLaunchKernelGGL(simplex_faces, dim3(unsigned((4 * ne + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->stream, fp);
+    HGDG_HIP(hipGetLastError());
     HGDG_HIP(hipStreamSynchronize(c->stream));
 }
 
@@ -1198,13 +1091,19 @@ int simplex_threads(int order, int variant) { return simplex_tpe_of(order, varia
 
 // Block schedule: the mesh is cut into slabs of consecutive elements and, slab
 // after slab, each order's elements of the slab fill blocks of that order's
-// size (256 / threads per element of the order's variant in use).
+// size in use. With each block goes the number of face functions its elements
+// meet: those of the highest order among them and their neighbours.
 void simplex_schedule(hgdg_ctx* c) {
     SimplexMesh& sm = c->sm;
     const int64_t ne = c->n_elem;
     const int64_t slab = std::max<int64_t>(1024, (ne + 255) / 256);  // in locality ranks
     int epb[4];
-    for (int g = 0; g < 4; ++g) epb[g] = kBlock / simplex_tpe_of(g + 1, sm.tpe_variant[g]);
+    for (int g = 0; g < 4; ++g) {
+        int top = g + 1;  // the highest order the order's elements meet
+        for (int64_t e = sm.group_start[g]; e < sm.group_start[g + 1] && top < kMaxSimplexOrder; ++e)
+            for (int f = 0; f < 4; ++f) top = std::max(top, info_pn(sm.info[size_t(f) * ne + e]));
+        epb[g] = simplex_epb(g + 1, sm.tpe_variant[g], simplex_ncol(top));
+    }
     std::vector<int32_t> blocks;
     int64_t cursor[4] = {sm.group_start[0], sm.group_start[1], sm.group_start[2], sm.group_start[3]};
     for (int64_t lo = 0; lo < ne; lo += slab) {
@@ -1214,10 +1113,14 @@ void simplex_schedule(hgdg_ctx* c) {
             int64_t end = cursor[g];
             while (end < sm.group_start[g + 1] && sm.rank[size_t(sm.mesh_of[end])] < hi) ++end;
             for (int64_t b = cursor[g]; b < end; b += epb[g]) {
+                const int64_t last = std::min<int64_t>(b + epb[g], end);
+                int top = g + 1;
+                for (int64_t e = b; e < last; ++e)
+                    for (int f = 0; f < 4; ++f) top = std::max(top, info_pn(sm.info[size_t(f) * ne + e]));
                 blocks.push_back(g + 1);
                 blocks.push_back(int32_t(b));
-                blocks.push_back(int32_t(std::min<int64_t>(epb[g], end - b)));
-                blocks.push_back(sm.tpe_variant[g]);
+                blocks.push_back(int32_t(last - b));
+                blocks.push_back(simplex_ncol(top));
             }
             cursor[g] = end;
         }
@@ -1239,44 +1142,32 @@ SimplexParams simplex_params(hgdg_ctx* c, const StageIO& io) {
         p.group_start[g] = sm.group_start[g];
         p.group_dof[g] = sm.group_dof[g];
     }
-    group_blocks(sm, p.group_block);
     p.jinv = sm.d_geo.ptr;
     p.cinv = sm.d_geo.ptr + 9 * ne;
-    p.sigma = sm.d_geo.ptr + 10 * ne;
-    p.normal = sm.d_geo.ptr + 14 * ne;
-    p.nbr = sm.d_face.ptr;
-    p.info = sm.d_face.ptr + 4 * ne;
+    p.frec = reinterpret_cast<const uint2*>(sm.d_frec.ptr);
+    p.fcode = sm.d_fcode.ptr;
     p.tab = sm.d_tables.ptr;
-    p.tab32 = sm.d_tables32.ptr;
-    p.tix = sm.d_tab_index.ptr;
-    p.n_tix = int32_t(sm.d_tab_index.n);
+    for (int g = 0; g < 4; ++g) {
+        p.tab_dr[g] = sm.tab_dr[g];
+        p.tab_lift[g] = sm.tab_lift[g];
+    }
+    p.cols = sm.d_tab_index.ptr + kTixCols;
     p.blocks = reinterpret_cast<const int4*>(sm.d_blocks.ptr);
-    p.trace = reinterpret_cast<double2*>(sm.d_trace.ptr);
-    for (int g = 0; g < 5; ++g) p.group_tr[g] = sm.group_tr[g];
     return p;
 }
 
 using SimplexKernel = void (*)(SimplexParams);
 
-template <typename T, int... V>
-constexpr std::array<SimplexKernel, sizeof...(V)> simplex_kernels(std::integer_sequence<int, V...>) {
-    return {&simplex_acoustic_rhs<T, V>...};
-}
-
 void launch_simplex(hgdg_ctx* c, const SimplexParams& p) {
-    // one kernel per combination of the orders' threads-per-element variants
-    static const auto k64 = simplex_kernels<double>(std::make_integer_sequence<int, 16>{});
-    static const auto k32 = simplex_kernels<float>(std::make_integer_sequence<int, 16>{});
-    const SimplexMesh& sm = c->sm;
-    int v = 0;
-    for (int g = 0; g < 4; ++g) v |= (sm.tpe_variant[g] & 1) << g;
-    const int grid = int(sm.n_blocks);
-    if (grid > 0) {
-        // the face traces of every element, then the right-hand side
-        hipLaunchKernelGGL(simplex_trace, dim3(unsigned(p.group_block[4])), dim3(kBlock), 0, c->stream, p);
-        const SimplexKernel k = c->op.precision == HGDG_PREC_MIXED_FP32 ? k32[size_t(v)] : k64[size_t(v)];
-        hipLaunchKernelGGL(k, dim3(unsigned(grid)), dim3(kBlock), 0, c->stream, p);
-    }
+    static constexpr SimplexKernel kernels[4][2] = {
+        {&simplex_acoustic_rhs<STAGE_ANY, false>, &simplex_acoustic_rhs<STAGE_ANY, true>},
+        {&simplex_acoustic_rhs<STAGE_ONE, false>, &simplex_acoustic_rhs<STAGE_ONE, true>},
+        {&simplex_acoustic_rhs<STAGE_TWO, false>, &simplex_acoustic_rhs<STAGE_TWO, true>},
+        {&simplex_acoustic_rhs<STAGE_TWO_MIXED, false>, &simplex_acoustic_rhs<STAGE_TWO_MIXED, true>}};
+    const int64_t grid = c->sm.n_blocks;
+    if (grid > 0)
+        hipLaunchKernelGGL(kernels[stage_kind(p.io)][p.io.upd.u != nullptr], dim3(unsigned(grid)), dim3(kBlock), 0,
+                           c->stream, p);
     HGDG_HIP(hipGetLastError());
 }
 

@@ -546,9 +546,7 @@ struct AcousticShape {
     static constexpr int ES = (DIM == 3 ? N1 : 1) * PS;
 };
 
-// Pencils of one input vector as loaded: FP32 values stay as their bits in the
-// doubles' low words until they are used (raw_value), so nothing waits for a
-// load where it is issued.
+// Pencils of one input vector as loaded (load_raw_n's form).
 template <int NR, int N1>
 __device__ __forceinline__ void load_raw(const void* v, bool f32, int64_t base, int64_t stride, double (&x)[NR][N1]) {
     if (f32) {
@@ -580,10 +578,6 @@ __device__ __forceinline__ void load_raw(const void* v, bool f32, int64_t base, 
 #pragma unroll
         for (int r = 0; r < NR; ++r) load_run<N1>(d + r * stride, x[r]);
     }
-}
-
-__device__ __forceinline__ double raw_value(double x, bool f32) {
-    return f32 ? double(__int_as_float(__double2loint(x))) : x;
 }
 
 // y += c x for NR pencils as load_raw left them

@@ -63,7 +63,7 @@ enum {
     HGDG_PREC_FP64 = 0,       /* everything FP64 (the parity path)                  */
     HGDG_PREC_MIXED_FP32 = 1  /* FP32 stage derivatives; FP32 contractions with
                                  compensated FP32 face sums where they are faster
-                                 (tensor advection, tetrahedra), FP64 elsewhere;
+                                 (tensor advection), FP64 elsewhere;
                                  FP64 geometry, state and RK update                 */
 };
 
@@ -188,11 +188,12 @@ int hgdg_set_tensor_general(hgdg_ctx* ctx, int force);
  * family (1) or the sum-factorised one (0; also for tetrahedra). */
 int hgdg_get_tensor_general(hgdg_ctx* ctx, int* force, int* in_use);
 
-/* Threads per element of the tetrahedral RHS kernel, per order 1..4
- * (threads[p-1]): 0 (the default) lets hgdg_operator_set time both candidates
- * of that order on the mesh and keep the faster; otherwise one of the two
- * candidates, 8 or 16 (order 1), 12 or 32 (order 2), 32 or 64 (order 3),
- * 35 or 64 (order 4). Results are bitwise the same for every choice. No
+/* Elements per workgroup of the tetrahedral RHS kernel, per order 1..4, named
+ * by threads per element (threads[p-1]): 0 (the default) lets
+ * hgdg_operator_set time both candidates of that order on the mesh and keep
+ * the faster; otherwise one of the two candidates, 8 or 16 (order 1), 12 or 32
+ * (order 2), 32 or 64 (order 3), 35 or 64 (order 4); the first fills a
+ * workgroup, the second makes more workgroups. Results are bitwise the same for every choice. No
  * counterpart in the reference (a launch parameter of this implementation);
  * applies to the next hgdg_operator_set, or at once if an operator is set. */
 int hgdg_set_simplex_threads(hgdg_ctx* ctx, const int32_t* threads);
