@@ -8,8 +8,8 @@ p = 3 (64 basis functions, 2,097,152 DOF), upwind flux, RK4; initial data:
 One timed step = one RHS evaluation as an RK stage performs it: the stage
 input u + (dt/2) k, the volume and face integrals and the inverse-mass apply
 (hpGEM's computeTimeDerivative), one fused kernel launch on state resident in
-HBM. Both arithmetic paths are timed: FP64 and mixed (FP32 contractions and
-stage derivatives, FP64 state, geometry and RK update); the mixed path's L2
+HBM. Both arithmetic paths are timed: FP64 and mixed (FP32
+stage derivatives, FP64 state, arithmetic, geometry and RK update); the mixed path's L2
 error against the FP64 path after the full 50-step RK4 run is measured in the
 same run. The CPU baseline is the FP64 oracle (a plain restatement of hpGEM's
 HpgemAPILinear algorithm) timed on a bounded sample on the host.

@@ -1,5 +1,5 @@
 // Shared pieces of the hgdg library: error type, HIP checks, stage-input
-// loads, compensated accumulation, device buffers.
+// loads, device buffers.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -273,24 +273,38 @@ inline int stage_kind(const StageIO& p) {
     return STAGE_ANY;
 }
 
-// combine_n in two halves: the first two inputs' loads, then the sums (in a)
+// Whether there is a second input, and whether it is FP32.
+template <int KIND>
+__device__ __forceinline__ bool stage_two(const StageIO& p) {
+    return KIND == STAGE_ANY ? p.n_in > 1 : KIND != STAGE_ONE;
+}
+template <int KIND>
+__device__ __forceinline__ bool stage_second_f32(const StageIO& p) {
+    return KIND == STAGE_ANY ? (p.in_f32 & 2u) != 0 : KIND == STAGE_TWO_MIXED;
+}
+
+// combine_n in parts: the first two inputs' loads, their sums (in a)
 template <int KIND, int K>
 __device__ __forceinline__ void load_two(const StageIO& p, const int64_t (&idx)[K], double (&a)[K], double (&b)[K]) {
     load_raw_n(p.in[0], KIND == STAGE_ANY && (p.in_f32 & 1u), idx, a);
-    if (KIND == STAGE_ANY ? p.n_in > 1 : KIND != STAGE_ONE)
-        load_raw_n(p.in[1], KIND == STAGE_ANY ? (p.in_f32 & 2u) != 0 : KIND == STAGE_TWO_MIXED, idx, b);
+    if (stage_two<KIND>(p)) load_raw_n(p.in[1], stage_second_f32<KIND>(p), idx, b);
 }
 
 template <int KIND, int K>
-__device__ __forceinline__ void mix_two(const StageIO& p, const int64_t (&idx)[K], double (&a)[K], double (&b)[K]) {
+__device__ __forceinline__ void mix_first(const StageIO& p, double (&a)[K], const double (&b)[K]) {
     if (KIND == STAGE_ANY && (p.in_f32 & 1u)) {
 #pragma unroll
         for (int k = 0; k < K; ++k) a[k] = raw_value(a[k], true);
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) a[k] = p.coef[0] * a[k];
-    if (KIND == STAGE_ANY ? p.n_in > 1 : KIND != STAGE_ONE)
-        add_raw_n(p.coef[1], b, KIND == STAGE_ANY ? (p.in_f32 & 2u) != 0 : KIND == STAGE_TWO_MIXED, a);
+    if (stage_two<KIND>(p)) add_raw_n(p.coef[1], b, stage_second_f32<KIND>(p), a);
+}
+
+// and any further inputs, one by one
+template <int KIND, int K>
+__device__ __forceinline__ void mix_two(const StageIO& p, const int64_t (&idx)[K], double (&a)[K], double (&b)[K]) {
+    mix_first<KIND>(p, a, b);
     if (KIND == STAGE_ANY) {
 #pragma unroll 1
         for (int i = 2; i < p.n_in; ++i) {
@@ -328,30 +342,6 @@ __device__ __forceinline__ void rk_update_n(const RkUpdate& q, const int64_t (&i
 #pragma unroll
     for (int k = 0; k < K; ++k) q.y_new[idx[k]] = y[k];
 }
-
-// Residual accumulation: FP64 plainly; FP32 with a compensated (TwoSum)
-// running sum for the face contributions.
-template <typename T>
-struct Acc {
-    T s;
-    __device__ Acc() : s(T(0)) {}
-    __device__ explicit Acc(T v) : s(v) {}
-    __device__ void add(T v) { s += v; }
-    __device__ T value() const { return s; }
-};
-template <>
-struct Acc<float> {
-    float s, c;
-    __device__ Acc() : s(0.f), c(0.f) {}
-    __device__ explicit Acc(float v) : s(v), c(0.f) {}
-    __device__ void add(float v) {
-        float t = s + v;
-        float bp = t - s;
-        c += (s - (t - bp)) + (v - bp);
-        s = t;
-    }
-    __device__ float value() const { return s + c; }
-};
 
 void require(bool ok, int code, const std::string& msg);
 

@@ -25,6 +25,7 @@ struct TensorMesh {
     DevBuf<double> d_absdet, d_ops;  // d_ops: Dr, Mi, M1 (n1 x n1 each)
     DevBuf<double> d_geo;            // advection: ahat [dim][e]; acoustic: J^{-1} [dim*dim][e], then c_inv [e]
     DevBuf<uint32_t> d_mode;         // advection: upwind mode, 3 bits per face
+    DevBuf<uint2> d_face;            // advection: [e][face] the neighbour met and the flux's coefficients
     bool structured = false;         // periodic unit box built by tensor_structured_upload
     int32_t cells[3] = {1, 1, 1};
     // Gauss-point path (tensor_general.hip): meshes with non-affine elements

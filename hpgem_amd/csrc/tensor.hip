@@ -17,12 +17,11 @@
 //
 // with Dr = M1^{-1} K the exact 1D derivative matrix (K(a,b) = int psi_a psi_b')
 // and own_{d,s} the element's own trace. Outflow faces drop out, and the face
-// terms only carry jumps, which are formed in FP64 from the FP64 stage input:
-// no large terms cancel, so the FP32 variant keeps ~1e-7 relative accuracy.
-// The 1D operators are built once on the host in long double by exact Gauss
+// terms only carry jumps: no large terms cancel. The arithmetic is FP64 in both
+// precisions, which differ in the storage of the stage derivatives. The 1D operators are built once on the host in long double by exact Gauss
 // quadrature; each element needs its stage input, `dim` numbers of geometry
-// and the traces of its inflow neighbours. One thread owns one coefficient;
-// an element's stage input sits in LDS for the 1D contractions.
+// and the traces of its inflow neighbours. One thread owns one x-pencil; an
+// element's stage input sits in LDS for the other 1D contractions.
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -37,12 +36,23 @@ namespace hgdg {
 // Per-face upwind modes, 3 bits per tensor face f = 2d + s.
 enum : uint32_t { MODE_NONE = 0, MODE_OWN = 1, MODE_NBR = 2, MODE_AVG = 3, MODE_HALF_OWN = 4 };
 
+// A face's flux (2s-1) (c_n other - c_o own): the upper halves of the two
+// coefficients' upper words (0, 1/2 and 1 need no more bits).
+inline uint32_t face_coef(uint32_t mode, int s) {
+    const uint32_t sign = s ? 0u : 0x8000u;
+    const uint32_t one = 0x3ff0u, half = 0x3fe0u;
+    const uint32_t cn = mode == MODE_NBR ? one : mode == MODE_AVG ? half : 0u;
+    const uint32_t co = mode == MODE_NBR || mode == MODE_NONE ? one : mode == MODE_OWN ? 0u : half;
+    return (cn ? (cn | sign) << 16 : 0u) | (co ? co | sign : 0u);
+}
+
 struct RhsParams {
     int64_t n_elem;
     StageIO io;
     const double* ahat;    // [dim][n_elem]
     const int32_t* nbr;    // [2 dim][n_elem]
     const uint32_t* mode;  // [n_elem]
+    const uint2* face;     // [n_elem][2 dim]: the neighbour (the element itself where none is met) and face_coef()
     const double* Dr;      // [n1][n1] exact derivative matrix
     const double* Mi;      // [n1][n1] inverse 1D mass
 };
@@ -57,493 +67,12 @@ struct Tensor {
 // One thread owns one x-pencil of an element (the N1 coefficients with fixed
 // y/z indices): the x-contraction and the x-face terms stay in registers, the
 // y/z contractions read the other pencils of the element from LDS, and the
-// y/z inflow traces arrive as whole pencils of the neighbour (vector loads).
+// y/z traces arrive as whole pencils of the neighbour.
 template <int DIM, int N1>
 struct Pencil {
     static constexpr int NP = DIM == 3 ? N1 * N1 : N1;  // pencils per element
     static constexpr int NB = NP * N1;                   // coefficients per element
     static constexpr int EPB = kBlock / NP;              // elements per block
-};
-
-// x[a] = vector i at [base, base + N1), as double
-template <int N1>
-__device__ __forceinline__ void load_pencil(const StageIO& p, int i, int64_t base, double (&x)[N1]) {
-    if ((p.in_f32 >> i) & 1u) {
-        const float* f = static_cast<const float*>(p.in[i]) + base;
-        if constexpr (N1 % 4 == 0) {
-#pragma unroll
-            for (int a = 0; a < N1; a += 4) {
-                const float4 v = *reinterpret_cast<const float4*>(f + a);
-                x[a] = v.x; x[a + 1] = v.y; x[a + 2] = v.z; x[a + 3] = v.w;
-            }
-        } else if constexpr (N1 % 2 == 0) {
-#pragma unroll
-            for (int a = 0; a < N1; a += 2) {
-                const float2 v = *reinterpret_cast<const float2*>(f + a);
-                x[a] = v.x; x[a + 1] = v.y;
-            }
-        } else {
-#pragma unroll
-            for (int a = 0; a < N1; ++a) x[a] = f[a];
-        }
-    } else {
-        const double* d = static_cast<const double*>(p.in[i]) + base;
-        if constexpr (N1 % 2 == 0) {
-#pragma unroll
-            for (int a = 0; a < N1; a += 2) {
-                const double2 v = *reinterpret_cast<const double2*>(d + a);
-                x[a] = v.x; x[a + 1] = v.y;
-            }
-        } else {
-#pragma unroll
-            for (int a = 0; a < N1; ++a) x[a] = d[a];
-        }
-    }
-}
-
-// Stage input pencil sum_i coef_i vec_i (getLinearCombinationOfVectors).
-// The first two inputs are loaded before either is used (their loads are in
-// flight together); the arithmetic and its order are those of the plain sum.
-template <int N1>
-__device__ __forceinline__ void combine_pencil(const StageIO& p, int64_t base, double (&w)[N1]) {
-    double x[N1], y[N1];
-    load_pencil<N1>(p, 0, base, x);
-    if (p.n_in > 1) load_pencil<N1>(p, 1, base, y);
-#pragma unroll
-    for (int a = 0; a < N1; ++a) w[a] = p.coef[0] * x[a];
-    if (p.n_in > 1) {
-#pragma unroll
-        for (int a = 0; a < N1; ++a) w[a] = fma(p.coef[1], y[a], w[a]);
-    }
-#pragma unroll
-    for (int i = 2; i < kMaxIn; ++i) {
-        if (i >= p.n_in) break;
-        load_pencil<N1>(p, i, base, x);
-#pragma unroll
-        for (int a = 0; a < N1; ++a) w[a] = fma(p.coef[i], x[a], w[a]);
-    }
-}
-
-__device__ __forceinline__ double face_jump(uint32_t m, double own, double other) {
-    if (m == MODE_NONE) return -own;
-    if (m == MODE_HALF_OWN) return -0.5 * own;
-    return (m == MODE_NBR) ? other - own : 0.5 * (other - own);
-}
-
-// Per-element data of the face terms: upwind modes, scaled velocity, and the
-// neighbour of every face. It is loaded together with the stage input, so
-// after the block's barrier only the neighbours' traces are still to come.
-template <int DIM>
-struct ElemMeta {
-    uint32_t md;
-    double ah[DIM];
-    int32_t nb[2 * DIM];
-};
-
-template <int DIM, int N1>
-__device__ __forceinline__ bool advection_load(const RhsParams& p, int64_t blk, double (&w)[N1], ElemMeta<DIM>& m) {
-    using S = Pencil<DIM, N1>;
-    const int le = threadIdx.x / S::NP, pc = threadIdx.x % S::NP;
-    const int64_t e = blk * S::EPB + le;
-    const bool active = (le < S::EPB) && (e < p.n_elem);
-    if (active) {
-        m.md = p.mode[e];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) m.ah[d] = p.ahat[d * p.n_elem + e];
-#pragma unroll
-        for (int f = 0; f < 2 * DIM; ++f) m.nb[f] = p.nbr[f * p.n_elem + e];
-        combine_pencil<N1>(p.io, e * S::NB + pc * N1, w);
-    }
-    return active;
-}
-
-// The arithmetic of one pencil once the block's stage input is in LDS (sw:
-// this element's coefficients; w: this thread's pencil, also in registers):
-// volume, upwind face jumps in FP64, lift, store. The neighbours' traces come
-// from xo(s) (x face s, this pencil's value) and yz(d, s, f, nbr_pc, other)
-// (y/z face: the neighbour's pencil nbr_pc), called only for faces whose mode
-// needs the neighbour; every kernel variant shares this code, so they agree
-// bit for bit.
-template <int DIM, int N1, typename T, bool UPD, typename XO, typename YZ>
-__device__ __forceinline__ void advection_compute(const RhsParams& p, int64_t e, int pc, const double (&w)[N1],
-                                                  uint32_t md, const double* ahd, const double* sw, const T* s_D,
-                                                  const T* s_Mi, XO xo, YZ yz) {
-    using S = Pencil<DIM, N1>;
-    const int ib = pc % N1;                    // y index of this pencil
-    const int ic = DIM == 3 ? pc / N1 : 0;     // z index of this pencil
-    T ah[DIM];
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) ah[d] = T(ahd[d]);
-
-    // volume (strong form): -sum_d ahat_d (Dr along d) w
-    T vol[N1];
-#pragma unroll
-    for (int a = 0; a < N1; ++a) {
-        T s = T(0);
-#pragma unroll
-        for (int j = 0; j < N1; ++j) s += s_D[a * N1 + j] * T(w[j]);
-        vol[a] = -ah[0] * s;
-    }
-#pragma unroll
-    for (int j = 0; j < N1; ++j) {
-        const T cy = -ah[1] * s_D[ib * N1 + j];
-        const double* row = sw + (j + N1 * ic) * N1;  // pencil (j, ic)
-#pragma unroll
-        for (int a = 0; a < N1; ++a) vol[a] += cy * T(row[a]);
-    }
-    if constexpr (DIM == 3) {
-#pragma unroll
-        for (int j = 0; j < N1; ++j) {
-            const T cz = -ah[2] * s_D[ic * N1 + j];
-            const double* row = sw + (ib + N1 * j) * N1;  // pencil (ib, j)
-#pragma unroll
-            for (int a = 0; a < N1; ++a) vol[a] += cz * T(row[a]);
-        }
-    }
-    Acc<T> acc[N1] = {};
-#pragma unroll
-    for (int a = 0; a < N1; ++a) acc[a] = Acc<T>(vol[a]);
-
-    // faces: -(2s-1) ahat_d Mi(idx_d, s) (T_{d,s} - own_{d,s}); jumps in FP64
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {  // x faces: one trace value per pencil
-        const uint32_t m = (md >> (3 * s)) & 7u;
-        if (m == MODE_OWN) continue;
-        const double other = (m == MODE_NBR || m == MODE_AVG) ? xo(s) : 0.0;
-        const T jump = T(face_jump(m, w[s], other));
-        const T sc = (s ? T(-1) : T(1)) * ah[0] * jump;
-#pragma unroll
-        for (int a = 0; a < N1; ++a) acc[a].add(sc * s_Mi[s * N1 + a]);
-    }
-#pragma unroll
-    for (int d = 1; d < DIM; ++d) {  // y (and z) faces: a whole pencil of traces
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int f = 2 * d + s;
-            const uint32_t m = (md >> (3 * f)) & 7u;
-            if (m == MODE_OWN) continue;
-            const int own_pc = d == 1 ? s + N1 * ic : ib + N1 * s;
-            const int nbr_pc = d == 1 ? (1 - s) + N1 * ic : ib + N1 * (1 - s);
-            double other[N1];
-            if (m == MODE_NBR || m == MODE_AVG) {
-                yz(d, s, f, nbr_pc, other);
-            } else {
-#pragma unroll
-                for (int a = 0; a < N1; ++a) other[a] = 0.0;
-            }
-            const int my = d == 1 ? ib : ic;
-            const T sc = (s ? T(-1) : T(1)) * ah[d] * s_Mi[s * N1 + my];
-#pragma unroll
-            for (int a = 0; a < N1; ++a) acc[a].add(sc * T(face_jump(m, sw[own_pc * N1 + a], other[a])));
-        }
-    }
-    const int64_t o = e * S::NB + pc * N1;
-    double kv[N1];
-    if (p.io.out_f32) {
-        float* out = static_cast<float*>(p.io.out) + o;
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            const float v = float(acc[a].value());
-            out[a] = v;
-            kv[a] = double(v);
-        }
-    } else {
-        double* out = static_cast<double*>(p.io.out) + o;
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-            const double v = double(acc[a].value());
-            out[a] = v;
-            kv[a] = v;
-        }
-    }
-    if constexpr (UPD) rk_update_run<N1>(p.io.upd, o, kv);
-}
-
-// General meshes: neighbour ids from the per-element face data; a neighbour
-// inside the block is read from LDS, any other from HBM.
-template <int DIM, int N1, typename T, bool UPD = false>
-__device__ __forceinline__ void advection_finish(const RhsParams& p, int64_t blk, const double (&w)[N1],
-                                                 const ElemMeta<DIM>& meta, const double* s_w, const T* s_D,
-                                                 const T* s_Mi) {
-    using S = Pencil<DIM, N1>;
-    const int tid = threadIdx.x;
-    const int le = tid / S::NP;
-    const int pc = tid % S::NP;
-    const int64_t e = blk * S::EPB + le;
-    const bool active = (le < S::EPB) && (e < p.n_elem);
-    if (!active) return;
-    auto xo = [&](int s) -> double {
-        const int64_t nb = meta.nb[s];
-        const int64_t lnb = nb - blk * S::EPB;
-        if (lnb >= 0 && lnb < S::EPB) return s_w[lnb * S::NB + pc * N1 + (1 - s)];  // neighbour in this block
-        return combine(p.io, nb * S::NB + pc * N1 + (1 - s));
-    };
-    auto yz = [&](int, int, int f, int nbr_pc, double (&other)[N1]) {
-        const int64_t nb = meta.nb[f];
-        const int64_t lnb = nb - blk * S::EPB;
-        if (lnb >= 0 && lnb < S::EPB) {
-#pragma unroll
-            for (int a = 0; a < N1; ++a) other[a] = s_w[lnb * S::NB + nbr_pc * N1 + a];
-        } else {
-            combine_pencil<N1>(p.io, nb * S::NB + nbr_pc * N1, other);
-        }
-    };
-    advection_compute<DIM, N1, T, UPD>(p, e, pc, w, meta.md, meta.ah, s_w + le * S::NB, s_D, s_Mi, xo, yz);
-}
-
-template <int DIM, int N1, typename T>
-__device__ __forceinline__ void advection_tables(const RhsParams& p, T* s_D, T* s_Mi) {
-    const int tid = threadIdx.x;
-    if (tid < N1 * N1) s_D[tid] = T(p.Dr[tid]);
-    if (tid < 2 * N1) s_Mi[tid] = T(p.Mi[(tid % N1) * N1 + tid / N1]);  // s_Mi[s * N1 + a] = Mi(a, s)
-}
-
-template <int DIM, int N1, typename T, bool UPD = false>
-__device__ __forceinline__ void advection_block(const RhsParams& p, int64_t blk) {
-    using S = Pencil<DIM, N1>;
-    __shared__ double s_w[S::EPB * S::NB];  // FP64 stage input of the block's elements
-    __shared__ T s_D[N1 * N1];
-    __shared__ T s_Mi[2 * N1];
-    advection_tables<DIM, N1, T>(p, s_D, s_Mi);
-    double w[N1];
-    ElemMeta<DIM> meta;
-    if (advection_load<DIM, N1>(p, blk, w, meta)) {
-        const int le = threadIdx.x / S::NP, pc = threadIdx.x % S::NP;
-#pragma unroll
-        for (int a = 0; a < N1; ++a) s_w[le * S::NB + pc * N1 + a] = w[a];
-    }
-    __syncthreads();
-    advection_finish<DIM, N1, T, UPD>(p, blk, w, meta, s_w, s_D, s_Mi);
-}
-
-// Whole RK steps of a small advection mesh in one workgroup: the solution,
-// the stage input, every stage derivative and the per-element face data stay
-// in LDS for all n_steps steps, with workgroup barriers between the phases,
-// so one launch replaces 5 n_steps launches (meshes this small are bound by
-// launch latency, not by HBM). The arithmetic is the graph path's, operation
-// for operation: the stage input as combine() forms it, the RHS through
-// advection_compute with the neighbour traces read from LDS, the update as
-// multi_axpy forms it; results are bitwise the same (tested).
-// The one workgroup: 16 wavefronts where the kernel fits in 128 registers,
-// else 8 (256 registers).
-template <int DIM, int N1>
-constexpr int rk_tiny_block() {
-    return (DIM == 2 ? N1 <= 4 : N1 <= 3) ? 1024 : 512;
-}
-
-struct RkTinyParams {
-    RhsParams rhs;          // geometry, tables; io unused
-    double* u;              // [n_dof] solution (read, then written after the last step)
-    void* k[kMaxIn];        // stage vectors (written with the last step's derivatives)
-    int32_t stages;
-    int32_t n_steps;
-    double ca[kMaxIn * kMaxIn];  // dt a_ij, row i
-    double cb[kMaxIn];           // dt b_j
-    uint32_t amask[kMaxIn];      // bit j of row i: a_ij != 0 (the graph path skips zero entries)
-    uint32_t bmask;              // bit j: b_j != 0
-};
-
-template <int DIM, int N1, typename T>
-__global__ __launch_bounds__((rk_tiny_block<DIM, N1>())) void tensor_advection_rk_tiny(const RkTinyParams p) {
-    constexpr int kTinyBlock = rk_tiny_block<DIM, N1>();
-    using S = Pencil<DIM, N1>;
-    extern __shared__ __align__(16) double dyn[];
-    __shared__ T s_D[N1 * N1];
-    __shared__ T s_Mi[2 * N1];
-    const int64_t E = p.rhs.n_elem, n = E * S::NB;
-    const int st = p.stages;
-    double* su = dyn;                                  // [n] solution
-    double* sw = su + n;                               // [n] stage input
-    uint32_t* smd = reinterpret_cast<uint32_t*>(sw + n);  // [E] upwind modes
-    int32_t* snb = reinterpret_cast<int32_t*>(smd + E);   // [2 DIM][E] neighbours
-    double* sah = reinterpret_cast<double*>(snb + 2 * DIM * E + ((E * (1 + 2 * DIM)) & 1));  // [DIM][E]
-    T* sk = reinterpret_cast<T*>(sah + DIM * E);       // [stages][n] stage derivatives
-    advection_tables<DIM, N1, T>(p.rhs, s_D, s_Mi);
-    for (int64_t i = threadIdx.x; i < n; i += kTinyBlock) su[i] = p.u[i];
-    for (int64_t e = threadIdx.x; e < E; e += kTinyBlock) {
-        smd[e] = p.rhs.mode[e];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) sah[d * E + e] = p.rhs.ahat[d * E + e];
-#pragma unroll
-        for (int f = 0; f < 2 * DIM; ++f) snb[f * E + e] = p.rhs.nbr[f * E + e];
-    }
-    __syncthreads();
-    RhsParams pp = p.rhs;
-    pp.io.out_f32 = sizeof(T) == 4 ? 1 : 0;
-    for (int step = 0; step < p.n_steps; ++step) {
-        for (int i = 0; i < st; ++i) {
-            // stage input: 1 * u, then + (dt a_ij) k_j in order of j
-            for (int64_t q = threadIdx.x; q < n; q += kTinyBlock) {
-                double v = 1.0 * su[q];
-                for (int j = 0; j < i; ++j)
-                    if ((p.amask[i] >> j) & 1u) v += p.ca[i * kMaxIn + j] * double(sk[int64_t(j) * n + q]);
-                sw[q] = v;
-            }
-            __syncthreads();
-            pp.io.out = sk + int64_t(i) * n;
-            for (int64_t q = threadIdx.x; q < E * S::NP; q += kTinyBlock) {
-                const int64_t e = q / S::NP;
-                const int pc = int(q % S::NP);
-                double w[N1];
-#pragma unroll
-                for (int a = 0; a < N1; ++a) w[a] = sw[e * S::NB + pc * N1 + a];
-                double ah[DIM];
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) ah[d] = sah[d * E + e];
-                auto xo = [&](int s) -> double { return sw[int64_t(snb[s * E + e]) * S::NB + pc * N1 + (1 - s)]; };
-                auto yz = [&](int, int, int f, int nbr_pc, double (&other)[N1]) {
-                    const int64_t nb = snb[f * E + e];
-#pragma unroll
-                    for (int a = 0; a < N1; ++a) other[a] = sw[nb * S::NB + nbr_pc * N1 + a];
-                };
-                advection_compute<DIM, N1, T, false>(pp, e, pc, w, smd[e], ah, sw + e * S::NB, s_D, s_Mi, xo, yz);
-            }
-            __syncthreads();
-        }
-        // update: u + (dt b_j) k_j in order of j
-        for (int64_t q = threadIdx.x; q < n; q += kTinyBlock) {
-            double y = su[q];
-            for (int j = 0; j < st; ++j)
-                if ((p.bmask >> j) & 1u) y += p.cb[j] * double(sk[int64_t(j) * n + q]);
-            su[q] = y;
-        }
-        __syncthreads();
-    }
-    for (int64_t q = threadIdx.x; q < n; q += kTinyBlock) {
-        p.u[q] = su[q];
-        for (int j = 0; j < st; ++j) static_cast<T*>(p.k[j])[q] = sk[int64_t(j) * n + q];
-    }
-}
-
-// Minimum waves per SIMD the compiler is asked to keep for the one-tile
-// kernel: 3D p=3 in FP64 needs a few registers beyond the 72 of seven waves
-// otherwise, and fits them without spilling.
-template <int DIM, int N1, typename T>
-constexpr int adv_min_waves() {
-    return (DIM == 3 && N1 == 4 && sizeof(T) == 8) ? 7 : 1;
-}
-
-// UPD: the RK update fused into this (last) stage, StageIO::upd.
-template <int DIM, int N1, typename T, bool UPD = false>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(adv_min_waves<DIM, N1, T>())))
-void tensor_advection_rhs(const RhsParams p) {
-    advection_block<DIM, N1, T, UPD>(p, xcd_block(blockIdx.x, gridDim.x));
-}
-
-// The same work with each block taking `tiles` consecutive tiles of EPB
-// elements: while a tile is computed, the next tile's stage input is already
-// being loaded into registers, so the loads of one tile overlap the
-// arithmetic and neighbour reads of the previous one, and a launch can be
-// sized to fill the GPU in one round. Per element the arithmetic is exactly
-// that of tensor_advection_rhs.
-template <int DIM, int N1, typename T>
-__global__ __launch_bounds__(kBlock) void tensor_advection_rhs_tiled(const RhsParams p, int tiles) {
-    using S = Pencil<DIM, N1>;
-    __shared__ double s_w[S::EPB * S::NB];
-    __shared__ T s_D[N1 * N1];
-    __shared__ T s_Mi[2 * N1];
-    advection_tables<DIM, N1, T>(p, s_D, s_Mi);
-    const int64_t n_tiles = (p.n_elem + S::EPB - 1) / S::EPB;
-    const int64_t t0 = xcd_block(blockIdx.x, gridDim.x) * tiles;
-    const int64_t t1 = t0 + tiles < n_tiles ? t0 + tiles : n_tiles;
-    const int le = threadIdx.x / S::NP, pc = threadIdx.x % S::NP;
-    double wn[N1];
-    ElemMeta<DIM> mn;
-    bool act_n = t0 < t1 && advection_load<DIM, N1>(p, t0, wn, mn);
-    for (int64_t t = t0; t < t1; ++t) {
-        double w[N1];
-#pragma unroll
-        for (int a = 0; a < N1; ++a) w[a] = wn[a];
-        const ElemMeta<DIM> meta = mn;
-        const bool act = act_n;
-        __syncthreads();  // the previous tile's readers of s_w are done
-        if (act)
-#pragma unroll
-            for (int a = 0; a < N1; ++a) s_w[le * S::NB + pc * N1 + a] = w[a];
-        __syncthreads();
-        act_n = t + 1 < t1 && advection_load<DIM, N1>(p, t + 1, wn, mn);
-        advection_finish<DIM, N1, T>(p, t, w, meta, s_w, s_D, s_Mi);
-    }
-}
-
-// Block b of a batched launch belongs to problem s with off[s] <= b < off[s+1].
-__device__ __forceinline__ int find_problem(const int64_t* off, int n, int64_t b) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) / 2;
-        if (off[mid] <= b) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-// Many independent problems of one kind in one launch: every block runs the
-// exact code of the single-problem kernel on its own problem's data (UPD:
-// with each problem's fused RK update, StageIO::upd).
-template <int DIM, int N1, typename T, bool UPD = false>
-__global__ __launch_bounds__(kBlock) void tensor_advection_rhs_batched(const RhsParams* ps, const int64_t* off,
-                                                                       int n) {
-    const int64_t b = xcd_block(blockIdx.x, gridDim.x);
-    const int s = find_problem(off, n, b);
-    advection_block<DIM, N1, T, UPD>(ps[s], b - off[s]);
-}
-
-// Acoustic wave system on tensor elements (AcousticWaveLinear_Impl.h:102-283):
-// fields v, s_1..s_dim stored field-major per element. With g_r = sum_d
-// (J^{-1})_{r,d} s_d, the element's own J throughout, and per face (r, s)
-//   F_v = -1/2 (2s-1) (g_r,own - sum_d (J^{-1})_{r,d} s_d,nbr),
-//   F_s = -1/2 (2s-1) (v_own - v_nbr)
-// on internal faces, F_v = -(2s-1) g_r,own and F_s = 0 on reflecting walls,
-//   k_v   =             sum_r [ (Dr along r) g_r + sum_s Mi(:,s) (x) F_v(r,s) ]
-//   k_s_d = (1/c_inv) sum_r (J^{-1})_{r,d} [ (Dr along r) v + sum_s Mi(:,s) (x) F_s(r,s) ].
-// Both brackets are the same one-dimensional operator, applied to g_r and to
-// v; the s fields are only combined from the second at the end. The
-// arithmetic is FP64 in both precisions (an FP64 multiply-add issues at the
-// FP32 rate here); the mixed path differs in the storage of its stage
-// derivatives.
-struct AcousticParams {
-    int64_t n_elem;
-    StageIO io;
-    const double* jinv;   // [dim*dim][n_elem]: (J^{-1})_{r,d} at [(r dim + d) n_elem + e]
-    const double* cinv;   // [n_elem]
-    const int32_t* nbr;   // [2 dim][n_elem], -1 on walls
-    const double* Dr;
-    const double* Mi;
-};
-
-// One thread owns one x-pencil of an element with all its fields; v, g_y and
-// g_z go to LDS for the y and z contractions, and each y or z face pencil's
-// fluxes are formed once, by one of the element's threads (NQ face pencils),
-// and shared through LDS. Nothing but an element's own threads meets at a
-// barrier, so a workgroup is the smallest of 64, 128 and 256 threads that
-// leaves at most one lane in sixteen idle: one wavefront where it can.
-// Sums are explicit multiply-adds: every instance (with and without the
-// update, batched) rounds alike.
-// Bound by memory: 32^3 p = 3 in FP64 reads and writes 201 MB at 4.3 TB/s
-// (a copy of that size reaches 5.4 - 6.9 TB/s). One lane per field and pencil,
-// which applies the derivative of v once per s field and forms every face
-// pencil's flux N1 times, took 104 us FP64 / 80 mixed there against 47 / 36;
-// 30^3 p = 2 42 against 23, 23x19x21 p = 4 66 against 37 (FP64).
-// kAhead: the first face pencil's neighbour values are loaded together with
-// the own ones, one memory round trip less (32^3 p = 3 53 -> 47 us, 256^2
-// p = 3 20.1 -> 17.7); at orders 4 and 5 in 3D, and with the update's terms
-// held too, its registers cost as much as that gains (20^3 p = 5 60 -> 64 us).
-// kEarly: all of the update's sum but the own term is formed before the
-// volume terms, from u and k as they are loaded anyway (RK4 step of 30^3 p = 2
-// 107 -> 103 us, 256^2 p = 1 34.8 -> 32.3); at orders 4 and 5 the 4 N1 sums do
-// not fit beside the rest (20^3 p = 5 276 -> 288 us), so there it comes last.
-template <int DIM, int N1>
-struct AcousticShape {
-    static constexpr int NF = DIM + 1;
-    static constexpr int NP = Pencil<DIM, N1>::NP;
-    static constexpr int NB = Pencil<DIM, N1>::NB;
-    static constexpr int NQ = 2 * (DIM - 1) * (DIM == 3 ? N1 : 1);
-    static constexpr int THREADS = (64 % NP) * 16 <= 64 ? 64 : (128 % NP) * 16 <= 128 ? 128 : 256;
-    static constexpr int EPB = THREADS / NP;
-    // LDS strides (doubles) of a plane and an element: even orders' planes
-    // are a multiple of the 64 banks' period apart without the padding
-    static constexpr int PS = N1 * N1 + (N1 % 2 == 0 ? 2 : 0);
-    static constexpr int ES = (DIM == 3 ? N1 : 1) * PS;
 };
 
 // Pencils of one input vector as loaded (load_raw_n's form).
@@ -599,22 +128,27 @@ __device__ __forceinline__ void add_raw(double c, const double (&x)[NR][N1], boo
 // Stage input of NR pencils at [base + r stride, + N1), in two halves:
 // load_pencils issues the first two input vectors' loads (u, x), mix_pencils
 // forms combine()'s sums from them in u and adds further inputs one by one.
-template <int NR, int N1>
+template <int NR, int N1, int KIND = STAGE_ANY>
 __device__ __forceinline__ void load_pencils(const StageIO& p, int64_t base, int64_t stride, double (&u)[NR][N1],
                                              double (&x)[NR][N1]) {
-    load_raw<NR, N1>(p.in[0], p.in_f32 & 1u, base, stride, u);
-    if (p.n_in > 1) load_raw<NR, N1>(p.in[1], p.in_f32 & 2u, base, stride, x);
+    load_raw<NR, N1>(p.in[0], KIND == STAGE_ANY && (p.in_f32 & 1u), base, stride, u);
+    if (stage_two<KIND>(p)) load_raw<NR, N1>(p.in[1], stage_second_f32<KIND>(p), base, stride, x);
+}
+
+template <int NR, int N1, int KIND = STAGE_ANY>
+__device__ __forceinline__ void mix_two_pencils(const StageIO& p, double (&u)[NR][N1], const double (&x)[NR][N1]) {
+    const bool u32 = KIND == STAGE_ANY && (p.in_f32 & 1u);
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int a = 0; a < N1; ++a) u[r][a] = p.coef[0] * raw_value(u[r][a], u32);
+    if (stage_two<KIND>(p)) add_raw<NR, N1>(p.coef[1], x, stage_second_f32<KIND>(p), u);
 }
 
 template <int NR, int N1>
 __device__ __forceinline__ void mix_pencils(const StageIO& p, int64_t base, int64_t stride, double (&u)[NR][N1],
                                             double (&x)[NR][N1]) {
-    const bool u32 = p.in_f32 & 1u;
-#pragma unroll
-    for (int r = 0; r < NR; ++r)
-#pragma unroll
-        for (int a = 0; a < N1; ++a) u[r][a] = p.coef[0] * raw_value(u[r][a], u32);
-    if (p.n_in > 1) add_raw<NR, N1>(p.coef[1], x, p.in_f32 & 2u, u);
+    mix_two_pencils<NR, N1>(p, u, x);
 #pragma unroll
     for (int i = 2; i < kMaxIn; ++i) {
         if (i >= p.n_in) break;
@@ -714,6 +248,487 @@ __device__ __forceinline__ void store_pencil(const StageIO& p, int64_t o, double
         }
     }
 }
+
+// A neighbour is met only where the flux needs it; F = (2s-1) times the jump
+// (other - own), halved or without the other side as the mode says, which the
+// 1D operator lifts: the terms -(2s-1) ahat_d Mi(idx_d, s) (T_{d,s} - own_{d,s}).
+__device__ __forceinline__ bool face_met(uint32_t m) { return m == MODE_NBR || m == MODE_AVG; }
+__device__ __forceinline__ double face_flux(uint32_t m, int s, double own, double other) {
+    const double h = m == MODE_NONE || m == MODE_NBR ? 1.0 : 0.5;
+    return m == MODE_OWN ? 0.0 : (s ? h : -h) * (other - own);
+}
+
+// The arithmetic of one pencil, shared by every kernel variant so that they
+// agree bit for bit: per direction the one-dimensional operator, its volume
+// part here (x with its faces' fluxes fx), y and z faces by advection_face;
+// then minus ahat_d times each, summed. Row i of s_row: Dr(i, :), Mi(i, 0..1).
+template <int N1>
+__device__ __forceinline__ void advection_rows(const RhsParams& p, double* s_row) {
+    const int i = threadIdx.x / (N1 + 2), j = threadIdx.x % (N1 + 2);
+    if (i < N1) s_row[threadIdx.x] = j < N1 ? p.Dr[i * N1 + j] : p.Mi[i * N1 + j - N1];
+}
+
+template <int DIM, int N1>
+__device__ __forceinline__ void advection_volume(const RhsParams& p, const double (&w)[N1], const double (&fx)[2],
+                                                 const double* sw, const double* s_row, int ib, int ic,
+                                                 double (&t)[DIM][N1]) {
+#pragma unroll
+    for (int a = 0; a < N1; ++a) {
+        double x = 0.0;
+#pragma unroll
+        for (int j = 0; j < N1; ++j) x = fma(p.Dr[a * N1 + j], w[j], x);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) x = fma(p.Mi[a * N1 + s], fx[s], x);
+        t[0][a] = x;
+    }
+#pragma unroll
+    for (int d = 1; d < DIM; ++d) {
+#pragma unroll
+        for (int a = 0; a < N1; ++a) t[d][a] = 0.0;
+#pragma unroll
+        for (int j = 0; j < N1; ++j) {
+            const double dr = s_row[(d == 1 ? ib : ic) * (N1 + 2) + j];
+            const double* row = sw + (d == 1 ? j + N1 * ic : ib + N1 * j) * N1;
+#pragma unroll
+            for (int a = 0; a < N1; ++a) t[d][a] = fma(dr, row[a], t[d][a]);
+        }
+    }
+}
+
+template <int N1>
+__device__ __forceinline__ void advection_face(const double* s_row, int my, int s, const double* flux,
+                                               double (&t)[N1]) {
+    const double mi = s_row[my * (N1 + 2) + N1 + s];
+#pragma unroll
+    for (int a = 0; a < N1; ++a) t[a] = fma(mi, flux[a], t[a]);
+}
+
+template <int DIM, int N1>
+__device__ __forceinline__ void advection_result(const double (&ah)[DIM], const double (&t)[DIM][N1],
+                                                 double (&k)[N1]) {
+#pragma unroll
+    for (int a = 0; a < N1; ++a) {
+        k[a] = -ah[0] * t[0][a];
+#pragma unroll
+        for (int d = 1; d < DIM; ++d) k[a] = fma(-ah[d], t[d][a], k[a]);
+    }
+}
+
+// `tiles` consecutive tiles of EPB elements, from tile t0 * tiles on; one
+// thread per x-pencil, and the same threads once more as one per y/z face
+// pencil (4 N1 an element in 3D, 2 in 2D), so that a face's trace is loaded and
+// its flux formed once and shared through LDS. TILED: the next tile's face
+// data and own pencils are loaded while this tile is computed, and a launch
+// can be sized to fill the GPU in one round. UPD: with the RK update of a
+// step's last stage, all of its sum but the own term formed from the stage
+// input's loads. Threads without a pencil or face work on the tile's first and
+// store nothing.
+//
+// Bound by instruction issue and by the two loads in a row (face data, then the
+// neighbours' values), which a launch of one or two rounds of workgroups cannot
+// hide; hence no decisions per face (an outflow face meets the element itself
+// with coefficient 0), FP64 arithmetic for FP32 stage values too (it issues at
+// the FP32 rate and needs no compensated sums) and a kernel per StageKind. One
+// stage of RK4 (us; before: every pencil of a line loaded and lifted each face
+// trace itself): 32^3 p = 3 14.1 -> 12.2 (4.3 TB/s), with FP32 stage values
+// 11.6 -> 9.4; 61 x 47 x 53 p = 2 26.6 -> 23.9 and 22.5 -> 20.3; 25 x 27 x 26
+// p = 4 17.2 -> 14.5; 301 x 257 p = 3 7.4 -> 6.8. The whole step, its last
+// stage with the update: 66.4 -> 55.6, 54.5 -> 46.5, 115.6 -> 103.2, 96.8 ->
+// 92.4, 76.4 -> 67.0, 37.3 -> 35.2. Reading and writing in memory order through
+// LDS instead of by pencil costs more instructions than it saves (32^3 p = 3
+// 13.3, 61 x 47 x 53 p = 2 27.2).
+template <int DIM, int N1, int KIND, bool UPD, bool TILED>
+__device__ __forceinline__ void advection_tiles(const RhsParams& p, int64_t t0, int tiles) {
+    using S = Pencil<DIM, N1>;
+    constexpr int NB = S::NB, EPB = S::EPB, NF = 2 * DIM;
+    constexpr int NQ = 2 * (DIM - 1) * (DIM == 3 ? N1 : 1);  // y/z face pencils of an element
+    constexpr int NI = (EPB * NQ + kBlock - 1) / kBlock;     // of a thread
+    __shared__ double s_w[EPB * NB];       // stage input
+    __shared__ double s_f[EPB * NQ * N1];  // fluxes
+    __shared__ double s_row[N1 * (N1 + 2)];
+    const int tid = threadIdx.x;
+    const int64_t E = p.n_elem;
+    const int64_t first = TILED ? t0 * tiles : t0;
+    int64_t end = first + 1;
+    if (TILED) {
+        const int64_t n_tiles = (E + EPB - 1) / EPB;
+        end = first + tiles < n_tiles ? first + tiles : n_tiles;
+        if (first >= end) return;
+    }
+    auto item = [&](int k) { return (k + 1) * kBlock <= EPB * NQ || tid + k * kBlock < EPB * NQ; };
+
+    struct Loads {
+        uint2 fx[2], fq[NI];
+        double ah[DIM];
+        double w[1][N1], x[1][N1];
+    };
+    auto fetch = [&](int64_t t, Loads& l) {
+        const int64_t e0 = t * EPB;
+        const int n = E - e0 < EPB ? int(E - e0) : EPB;
+        const uint2* face = p.face + e0 * NF;
+#pragma unroll
+        for (int k = 0; k < NI; ++k)
+            if (item(k)) {
+                const int q = tid + k * kBlock, el = q / NQ < n ? q / NQ : 0;
+                l.fq[k] = face[el * NF + 2 + (DIM == 3 ? q % NQ / N1 : q % NQ)];
+            }
+        const int own = tid < n * S::NP ? tid : 0, le = own / S::NP;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) l.fx[s] = face[le * NF + s];
+        load_pencils<1, N1, KIND>(p.io, e0 * NB + own * N1, 0, l.w, l.x);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) l.ah[d] = p.ahat[d * E + e0 + le];
+    };
+    Loads l;
+    fetch(first, l);
+    advection_rows<N1>(p, s_row);
+
+    for (int64_t t = first; t < end; ++t) {
+        const int64_t e0 = t * EPB;
+        const int n = E - e0 < EPB ? int(E - e0) : EPB;
+        const bool active = tid < n * S::NP;
+        const int own = active ? tid : 0, le = own / S::NP, pc = own % S::NP;
+        const int ib = pc % N1, ic = DIM == 3 ? pc / N1 : 0;
+        const int64_t base = e0 * NB + own * N1;
+        // ---- the neighbours' face pencils and x traces (of the first two inputs)
+        int64_t at[NI], atx[2];
+        int lx[2];
+        double o[NI][1][N1], o1[NI][1][N1], ox[2], ox1[2], cq[NI][2], cx[2][2];
+        auto coef = [](uint32_t c, double (&h)[2]) {
+            h[0] = __hiloint2double(int(c & 0xffff0000u), 0);
+            h[1] = __hiloint2double(int(c << 16), 0);
+        };
+#pragma unroll
+        for (int k = 0; k < NI; ++k)
+            if (item(k)) {
+                const int q = tid + k * kBlock, fi = DIM == 3 ? q % NQ / N1 : q % NQ, j = DIM == 3 ? q % N1 : 0;
+                at[k] = int64_t(l.fq[k].x) * NB + (fi / 2 ? j + N1 * (1 - fi % 2) : (1 - fi % 2) + N1 * j) * N1;
+                load_pencils<1, N1, KIND>(p.io, at[k], 0, o[k], o1[k]);
+                coef(l.fq[k].y, cq[k]);
+            }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int64_t ln = int64_t(l.fx[s].x) - e0;
+            lx[s] = ln >= 0 && ln < n ? int(ln) * NB + pc * N1 + (1 - s) : -1;  // in this block's LDS
+            atx[s] = int64_t(l.fx[s].x) * NB + pc * N1 + (1 - s);
+            if (lx[s] < 0) {
+                const int64_t a1[1] = {atx[s]};
+                double v[1], v1[1];
+                load_two<KIND>(p.io, a1, v, v1);
+                ox[s] = v[0];
+                ox1[s] = v1[0];
+            }
+            coef(l.fx[s].y, cx[s]);
+        }
+        double y[1][N1];
+        if constexpr (UPD) update_partial<1, N1>(p.io, base, 0, l.w, l.x, y);
+        // ---- the sums; further inputs two at a time
+        mix_two_pencils<1, N1, KIND>(p.io, l.w, l.x);
+#pragma unroll
+        for (int k = 0; k < NI; ++k)
+            if (item(k)) mix_two_pencils<1, N1, KIND>(p.io, o[k], o1[k]);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            if (lx[s] < 0) {
+                double v[1][1] = {{ox[s]}}, v1[1][1] = {{ox1[s]}};
+                mix_two_pencils<1, 1, KIND>(p.io, v, v1);
+                ox[s] = v[0][0];
+            }
+        if constexpr (KIND == STAGE_ANY) {
+#pragma unroll 1
+            for (int i = 2; i < p.io.n_in; i += 2) {
+                const bool two = i + 1 < p.io.n_in;
+                const int i1 = two ? i + 1 : i;
+                const double c[2] = {p.io.coef[i], p.io.coef[i1]};
+                const bool f[2] = {((p.io.in_f32 >> i) & 1u) != 0, ((p.io.in_f32 >> i1) & 1u) != 0};
+                const void* in[2] = {p.io.in[i], p.io.in[i1]};
+                double a[2][1][N1], b[2][NI][1][N1], g[2][2][1][1];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (h == 1 && !two) break;
+                    load_raw<1, N1>(in[h], f[h], base, 0, a[h]);
+#pragma unroll
+                    for (int k = 0; k < NI; ++k)
+                        if (item(k)) load_raw<1, N1>(in[h], f[h], at[k], 0, b[h][k]);
+#pragma unroll
+                    for (int s = 0; s < 2; ++s)
+                        if (lx[s] < 0) load_raw<1, 1>(in[h], f[h], atx[s], 0, g[h][s]);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (h == 1 && !two) break;
+                    add_raw<1, N1>(c[h], a[h], f[h], l.w);
+#pragma unroll
+                    for (int k = 0; k < NI; ++k)
+                        if (item(k)) add_raw<1, N1>(c[h], b[h][k], f[h], o[k]);
+#pragma unroll
+                    for (int s = 0; s < 2; ++s)
+                        if (lx[s] < 0) {
+                            double v[1][1] = {{ox[s]}};
+                            add_raw<1, 1>(c[h], g[h][s], f[h], v);
+                            ox[s] = v[0][0];
+                        }
+                }
+            }
+        }
+        double w[N1], ah[DIM];
+#pragma unroll
+        for (int a = 0; a < N1; ++a) w[a] = l.w[0][a];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) ah[d] = l.ah[d];
+        if (TILED && t != first) __syncthreads();  // the previous tile's readers are done
+        if (EPB * S::NP == kBlock || tid < EPB * S::NP) {
+#pragma unroll
+            for (int a = 0; a < N1; ++a) s_w[tid * N1 + a] = w[a];
+        }
+        __syncthreads();
+        if (TILED && t + 1 < end) fetch(t + 1, l);
+
+        // ---- each face pencil's flux, and the volume terms
+#pragma unroll
+        for (int k = 0; k < NI; ++k)
+            if (item(k)) {
+                const int q = tid + k * kBlock, fi = DIM == 3 ? q % NQ / N1 : q % NQ, j = DIM == 3 ? q % N1 : 0;
+                const double* oq = s_w + q / NQ * NB + (fi / 2 ? j + N1 * (fi % 2) : fi % 2 + N1 * j) * N1;
+#pragma unroll
+                for (int a = 0; a < N1; ++a) s_f[q * N1 + a] = fma(cq[k][0], o[k][0][a], -(cq[k][1] * oq[a]));
+            }
+        double tt[DIM][N1], fx[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (lx[s] >= 0) ox[s] = s_w[lx[s]];
+            fx[s] = fma(cx[s][0], ox[s], -(cx[s][1] * w[s]));
+        }
+        advection_volume<DIM, N1>(p, w, fx, s_w + le * NB, s_row, ib, ic, tt);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+#pragma unroll
+            for (int a = 0; a < N1; ++a) form_here(tt[d][a]);
+        __syncthreads();
+#pragma unroll
+        for (int f = 2; f < NF; ++f) {
+            const int q = le * NQ + (DIM == 3 ? (f - 2) * N1 + (f / 2 == 1 ? ic : ib) : f - 2);
+            advection_face<N1>(s_row, f / 2 == 1 ? ib : ic, f % 2, s_f + q * N1, tt[f / 2]);
+        }
+        double k[N1];
+        advection_result<DIM, N1>(ah, tt, k);
+        if (active) {
+            store_pencil<N1>(p.io, base, k);
+            if constexpr (UPD) update_store<N1>(p.io.upd, base, k, y[0]);
+        }
+    }
+}
+
+// Whole RK steps of a small advection mesh in one workgroup: the solution,
+// the stage input, every stage derivative and the per-element face data stay
+// in LDS for all n_steps steps, with workgroup barriers between the phases,
+// so one launch replaces 5 n_steps launches (meshes this small are bound by
+// launch latency, not by HBM). The arithmetic is the graph path's, operation
+// for operation: the stage input as combine() forms it, the RHS by the same
+// sums with the neighbour traces read from LDS, the update as
+// multi_axpy forms it; results are bitwise the same (tested).
+// The one workgroup: 16 wavefronts where the kernel fits in 128 registers,
+// else 8 (256 registers).
+template <int DIM, int N1>
+constexpr int rk_tiny_block() {
+    return (DIM == 2 ? N1 <= 4 : N1 <= 3) ? 1024 : 512;
+}
+
+struct RkTinyParams {
+    RhsParams rhs;          // geometry, tables; io unused
+    double* u;              // [n_dof] solution (read, then written after the last step)
+    void* k[kMaxIn];        // stage vectors (written with the last step's derivatives)
+    int32_t stages;
+    int32_t n_steps;
+    double ca[kMaxIn * kMaxIn];  // dt a_ij, row i
+    double cb[kMaxIn];           // dt b_j
+    uint32_t amask[kMaxIn];      // bit j of row i: a_ij != 0 (the graph path skips zero entries)
+    uint32_t bmask;              // bit j: b_j != 0
+};
+
+// T: the stage derivatives' storage.
+template <int DIM, int N1, typename T>
+__global__ __launch_bounds__((rk_tiny_block<DIM, N1>())) void tensor_advection_rk_tiny(const RkTinyParams p) {
+    constexpr int kTinyBlock = rk_tiny_block<DIM, N1>();
+    using S = Pencil<DIM, N1>;
+    extern __shared__ __align__(16) double dyn[];
+    __shared__ double s_row[N1 * (N1 + 2)];
+    const int64_t E = p.rhs.n_elem, n = E * S::NB;
+    const int st = p.stages;
+    double* su = dyn;                                  // [n] solution
+    double* sw = su + n;                               // [n] stage input
+    uint32_t* smd = reinterpret_cast<uint32_t*>(sw + n);  // [E] upwind modes
+    int32_t* snb = reinterpret_cast<int32_t*>(smd + E);   // [2 DIM][E] neighbours
+    double* sah = reinterpret_cast<double*>(snb + 2 * DIM * E + ((E * (1 + 2 * DIM)) & 1));  // [DIM][E]
+    T* sk = reinterpret_cast<T*>(sah + DIM * E);       // [stages][n] stage derivatives
+    advection_rows<N1>(p.rhs, s_row);
+    for (int64_t i = threadIdx.x; i < n; i += kTinyBlock) su[i] = p.u[i];
+    for (int64_t e = threadIdx.x; e < E; e += kTinyBlock) {
+        smd[e] = p.rhs.mode[e];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) sah[d * E + e] = p.rhs.ahat[d * E + e];
+#pragma unroll
+        for (int f = 0; f < 2 * DIM; ++f) snb[f * E + e] = p.rhs.nbr[f * E + e];
+    }
+    __syncthreads();
+    for (int step = 0; step < p.n_steps; ++step) {
+        for (int i = 0; i < st; ++i) {
+            // stage input: 1 * u, then + (dt a_ij) k_j in order of j
+            for (int64_t q = threadIdx.x; q < n; q += kTinyBlock) {
+                double v = 1.0 * su[q];
+                for (int j = 0; j < i; ++j)
+                    if ((p.amask[i] >> j) & 1u) v = fma(p.ca[i * kMaxIn + j], double(sk[int64_t(j) * n + q]), v);
+                sw[q] = v;
+            }
+            __syncthreads();
+            for (int64_t q = threadIdx.x; q < E * S::NP; q += kTinyBlock) {
+                const int64_t e = q / S::NP;
+                const int pc = int(q % S::NP);
+                double w[N1];
+#pragma unroll
+                for (int a = 0; a < N1; ++a) w[a] = sw[e * S::NB + pc * N1 + a];
+                double ah[DIM];
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) ah[d] = sah[d * E + e];
+                const uint32_t md = smd[e];
+                const double* we = sw + e * S::NB;
+                const int ib = pc % N1, ic = DIM == 3 ? pc / N1 : 0;
+                double fx[2], t[DIM][N1];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const uint32_t m = (md >> (3 * s)) & 7u;
+                    const double o = face_met(m) ? sw[int64_t(snb[s * E + e]) * S::NB + pc * N1 + (1 - s)] : 0.0;
+                    fx[s] = face_flux(m, s, w[s], o);
+                }
+                advection_volume<DIM, N1>(p.rhs, w, fx, we, s_row, ib, ic, t);
+#pragma unroll
+                for (int f = 2; f < 2 * DIM; ++f) {
+                    const uint32_t m = (md >> (3 * f)) & 7u;
+                    const int s = f % 2, k = f / 2 == 1 ? ic : ib;
+                    const int own = f / 2 == 1 ? s + N1 * k : k + N1 * s, nbr = f / 2 == 1 ? (1 - s) + N1 * k : k + N1 * (1 - s);
+                    double flux[N1];
+                    if (face_met(m)) {
+                        const double* o = sw + int64_t(snb[f * E + e]) * S::NB + nbr * N1;
+#pragma unroll
+                        for (int a = 0; a < N1; ++a) flux[a] = face_flux(m, s, we[own * N1 + a], o[a]);
+                    } else {
+#pragma unroll
+                        for (int a = 0; a < N1; ++a) flux[a] = face_flux(m, s, we[own * N1 + a], 0.0);
+                    }
+                    advection_face<N1>(s_row, f / 2 == 1 ? ib : ic, s, flux, t[f / 2]);
+                }
+                double kv[N1];
+                advection_result<DIM, N1>(ah, t, kv);
+#pragma unroll
+                for (int a = 0; a < N1; ++a) sk[int64_t(i) * n + e * S::NB + pc * N1 + a] = T(kv[a]);
+            }
+            __syncthreads();
+        }
+        // update: u + (dt b_j) k_j in order of j
+        for (int64_t q = threadIdx.x; q < n; q += kTinyBlock) {
+            double y = su[q];
+            for (int j = 0; j < st; ++j)
+                if ((p.bmask >> j) & 1u) y = fma(p.cb[j], double(sk[int64_t(j) * n + q]), y);
+            su[q] = y;
+        }
+        __syncthreads();
+    }
+    for (int64_t q = threadIdx.x; q < n; q += kTinyBlock) {
+        p.u[q] = su[q];
+        for (int j = 0; j < st; ++j) static_cast<T*>(p.k[j])[q] = sk[int64_t(j) * n + q];
+    }
+}
+
+// UPD: the RK update fused into this (last) stage, StageIO::upd.
+template <int DIM, int N1, int KIND, bool UPD>
+__global__ __launch_bounds__(kBlock) void tensor_advection_rhs(const RhsParams p) {
+    advection_tiles<DIM, N1, KIND, UPD, false>(p, xcd_block(blockIdx.x, gridDim.x), 1);
+}
+
+template <int DIM, int N1, int KIND>
+__global__ __launch_bounds__(kBlock) void tensor_advection_rhs_tiled(const RhsParams p, int tiles) {
+    advection_tiles<DIM, N1, KIND, false, true>(p, xcd_block(blockIdx.x, gridDim.x), tiles);
+}
+
+// Block b of a batched launch belongs to problem s with off[s] <= b < off[s+1].
+__device__ __forceinline__ int find_problem(const int64_t* off, int n, int64_t b) {
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if (off[mid] <= b) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Many independent problems of one kind in one launch: every block runs the
+// exact code of the single-problem kernel on its own problem's data (UPD:
+// with each problem's fused RK update, StageIO::upd).
+template <int DIM, int N1, bool UPD = false>
+__global__ __launch_bounds__(kBlock) void tensor_advection_rhs_batched(const RhsParams* __restrict__ ps,
+                                                                       const int64_t* __restrict__ off, int n) {
+    const int64_t b = xcd_block(blockIdx.x, gridDim.x);
+    const int s = __builtin_amdgcn_readfirstlane(find_problem(off, n, b));
+    advection_tiles<DIM, N1, STAGE_ANY, UPD, false>(ps[s], b - off[s], 1);
+}
+
+// Acoustic wave system on tensor elements (AcousticWaveLinear_Impl.h:102-283):
+// fields v, s_1..s_dim stored field-major per element. With g_r = sum_d
+// (J^{-1})_{r,d} s_d, the element's own J throughout, and per face (r, s)
+//   F_v = -1/2 (2s-1) (g_r,own - sum_d (J^{-1})_{r,d} s_d,nbr),
+//   F_s = -1/2 (2s-1) (v_own - v_nbr)
+// on internal faces, F_v = -(2s-1) g_r,own and F_s = 0 on reflecting walls,
+//   k_v   =             sum_r [ (Dr along r) g_r + sum_s Mi(:,s) (x) F_v(r,s) ]
+//   k_s_d = (1/c_inv) sum_r (J^{-1})_{r,d} [ (Dr along r) v + sum_s Mi(:,s) (x) F_s(r,s) ].
+// Both brackets are the same one-dimensional operator, applied to g_r and to
+// v; the s fields are only combined from the second at the end. The
+// arithmetic is FP64 in both precisions (an FP64 multiply-add issues at the
+// FP32 rate here); the mixed path differs in the storage of its stage
+// derivatives.
+struct AcousticParams {
+    int64_t n_elem;
+    StageIO io;
+    const double* jinv;   // [dim*dim][n_elem]: (J^{-1})_{r,d} at [(r dim + d) n_elem + e]
+    const double* cinv;   // [n_elem]
+    const int32_t* nbr;   // [2 dim][n_elem], -1 on walls
+    const double* Dr;
+    const double* Mi;
+};
+
+// One thread owns one x-pencil of an element with all its fields; v, g_y and
+// g_z go to LDS for the y and z contractions, and each y or z face pencil's
+// fluxes are formed once, by one of the element's threads (NQ face pencils),
+// and shared through LDS. Nothing but an element's own threads meets at a
+// barrier, so a workgroup is the smallest of 64, 128 and 256 threads that
+// leaves at most one lane in sixteen idle: one wavefront where it can.
+// Sums are explicit multiply-adds: every instance (with and without the
+// update, batched) rounds alike.
+// Bound by memory: 32^3 p = 3 in FP64 reads and writes 201 MB at 4.3 TB/s
+// (a copy of that size reaches 5.4 - 6.9 TB/s). One lane per field and pencil,
+// which applies the derivative of v once per s field and forms every face
+// pencil's flux N1 times, took 104 us FP64 / 80 mixed there against 47 / 36;
+// 30^3 p = 2 42 against 23, 23x19x21 p = 4 66 against 37 (FP64).
+// kAhead: the first face pencil's neighbour values are loaded together with
+// the own ones, one memory round trip less (32^3 p = 3 53 -> 47 us, 256^2
+// p = 3 20.1 -> 17.7); at orders 4 and 5 in 3D, and with the update's terms
+// held too, its registers cost as much as that gains (20^3 p = 5 60 -> 64 us).
+// kEarly: all of the update's sum but the own term is formed before the
+// volume terms, from u and k as they are loaded anyway (RK4 step of 30^3 p = 2
+// 107 -> 103 us, 256^2 p = 1 34.8 -> 32.3); at orders 4 and 5 the 4 N1 sums do
+// not fit beside the rest (20^3 p = 5 276 -> 288 us), so there it comes last.
+template <int DIM, int N1>
+struct AcousticShape {
+    static constexpr int NF = DIM + 1;
+    static constexpr int NP = Pencil<DIM, N1>::NP;
+    static constexpr int NB = Pencil<DIM, N1>::NB;
+    static constexpr int NQ = 2 * (DIM - 1) * (DIM == 3 ? N1 : 1);
+    static constexpr int THREADS = (64 % NP) * 16 <= 64 ? 64 : (128 % NP) * 16 <= 128 ? 128 : 256;
+    static constexpr int EPB = THREADS / NP;
+    // LDS strides (doubles) of a plane and an element: even orders' planes
+    // are a multiple of the 64 banks' period apart without the padding
+    static constexpr int PS = N1 * N1 + (N1 % 2 == 0 ? 2 : 0);
+    static constexpr int ES = (DIM == 3 ? N1 : 1) * PS;
+};
 
 template <int DIM, int N1, bool UPD>
 __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t blk) {
@@ -1574,6 +1589,7 @@ void tensor_operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
         return (2 * s - 1) * ahat[size_t(d) * ne + e] / rownorm[size_t(d) * ne + e];
     };
     std::vector<uint32_t> mode(ne, 0);
+    std::vector<uint2> face(size_t(2) * dim * ne);
     for (int64_t e = 0; e < ne; ++e) {
         uint32_t word = 0;
         for (int f = 0; f < 2 * dim; ++f) {
@@ -1594,9 +1610,15 @@ void tensor_operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
             word |= m << (3 * f);
         }
         mode[e] = word;
+        for (int f = 0; f < 2 * dim; ++f) {
+            const uint32_t m = (word >> (3 * f)) & 7u;
+            face[size_t(e) * 2 * dim + f] = 
+                make_uint2(uint32_t(m == MODE_NBR || m == MODE_AVG ? c->tm.nbr[size_t(f) * ne + e] : e), face_coef(m, f % 2));
+        }
     }
     c->tm.d_geo.upload(ahat, c->stream);
     c->tm.d_mode.upload(mode, c->stream);
+    c->tm.d_face.upload(face, c->stream);
     HGDG_HIP(hipStreamSynchronize(c->stream));
 }
 
@@ -1607,42 +1629,37 @@ static RhsParams advection_params(hgdg_ctx* c, const StageIO& io) {
     p.ahat = c->tm.d_geo.ptr;
     p.nbr = c->tm.d_nbr.ptr;
     p.mode = c->tm.d_mode.ptr;
+    p.face = c->tm.d_face.ptr;
     p.Dr = Dr_ptr(c);
     p.Mi = Mi_ptr(c);
     return p;
 }
 
 static void launch_advection(hgdg_ctx* c, const RhsParams& p, int tiles) {
-    const bool mixed = c->op.precision == HGDG_PREC_MIXED_FP32;
     dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
         constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
         using S = Pencil<DIMc, N1c>;
         const int64_t n_tiles = (c->n_elem + S::EPB - 1) / S::EPB;
-        if (p.io.upd.u != nullptr) {  // the fused RK update runs in the one-tile kernel
-            if (mixed)
-                hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, float, true>), dim3(unsigned(n_tiles)),
+        const bool upd = p.io.upd.u != nullptr;  // the fused RK update runs in the one-tile kernel
+        auto go = [&](auto K) {
+            constexpr int KIND = decltype(K)::value;
+            if (upd)
+                hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, KIND, true>), dim3(unsigned(n_tiles)),
                                    dim3(kBlock), 0, c->stream, p);
+            else if (tiles > 1)
+                hipLaunchKernelGGL((tensor_advection_rhs_tiled<DIMc, N1c, KIND>),
+                                   dim3(unsigned((n_tiles + tiles - 1) / tiles)), dim3(kBlock), 0, c->stream, p,
+                                   tiles);
             else
-                hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, double, true>), dim3(unsigned(n_tiles)),
+                hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, KIND, false>), dim3(unsigned(n_tiles)),
                                    dim3(kBlock), 0, c->stream, p);
-            return;
+        };
+        switch (stage_kind(p.io)) {
+            case STAGE_ONE: go(std::integral_constant<int, STAGE_ONE>{}); break;
+            case STAGE_TWO: go(std::integral_constant<int, STAGE_TWO>{}); break;
+            case STAGE_TWO_MIXED: go(std::integral_constant<int, STAGE_TWO_MIXED>{}); break;
+            default: go(std::integral_constant<int, STAGE_ANY>{}); break;
         }
-        if (tiles > 1) {
-            const int64_t grid = (n_tiles + tiles - 1) / tiles;
-            if (mixed)
-                hipLaunchKernelGGL((tensor_advection_rhs_tiled<DIMc, N1c, float>), dim3(unsigned(grid)), dim3(kBlock),
-                                   0, c->stream, p, tiles);
-            else
-                hipLaunchKernelGGL((tensor_advection_rhs_tiled<DIMc, N1c, double>), dim3(unsigned(grid)),
-                                   dim3(kBlock), 0, c->stream, p, tiles);
-            return;
-        }
-        if (mixed)
-            hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, float>), dim3(unsigned(n_tiles)), dim3(kBlock), 0,
-                               c->stream, p);
-        else
-            hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, double>), dim3(unsigned(n_tiles)), dim3(kBlock), 0,
-                               c->stream, p);
     });
     HGDG_HIP(hipGetLastError());
 }
@@ -1973,6 +1990,7 @@ void tensor_batch_param(hgdg_ctx* c, const StageIO& io, void* out) {
         r.ahat = c->tm.d_geo.ptr;
         r.nbr = c->tm.d_nbr.ptr;
         r.mode = c->tm.d_mode.ptr;
+        r.face = c->tm.d_face.ptr;
         r.Dr = Dr_ptr(c);
         r.Mi = Mi_ptr(c);
         std::memcpy(out, &r, sizeof(r));
@@ -1986,20 +2004,17 @@ void tensor_batch_launch(hipStream_t stream, int kind, int dim, int n1, bool mix
         constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
         const dim3 grid{unsigned(blocks), 1, 1}, block{unsigned(kBlock), 1, 1};
         const dim3 acoustic_block{unsigned(AcousticShape<DIMc, N1c>::THREADS), 1, 1};
-        auto go = [&](auto T_, auto U_) {
-            using Tc = decltype(T_);
-            constexpr bool Uc = decltype(U_)::value;
+        auto go = [&](auto U) {
+            constexpr bool Uc = decltype(U)::value;
             if (kind == HGDG_OP_ACOUSTIC_CENTRAL)
                 hipLaunchKernelGGL((tensor_acoustic_rhs_batched<DIMc, N1c, Uc>), grid, acoustic_block, 0, stream,
                                    static_cast<const AcousticParams*>(params), off, n);
             else
-                hipLaunchKernelGGL((tensor_advection_rhs_batched<DIMc, N1c, Tc, Uc>), grid, block, 0, stream,
+                hipLaunchKernelGGL((tensor_advection_rhs_batched<DIMc, N1c, Uc>), grid, block, 0, stream,
                                    static_cast<const RhsParams*>(params), off, n);
         };
-        if (mixed && upd) go(float{}, std::true_type{});
-        else if (mixed) go(float{}, std::false_type{});
-        else if (upd) go(double{}, std::true_type{});
-        else go(double{}, std::false_type{});
+        if (upd) go(std::true_type{});
+        else go(std::false_type{});
     });
     HGDG_HIP(hipGetLastError());
 }

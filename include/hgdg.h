@@ -61,10 +61,8 @@ enum {
 /* ---- arithmetic of the bulk contractions ------------------------------- */
 enum {
     HGDG_PREC_FP64 = 0,       /* everything FP64 (the parity path)                  */
-    HGDG_PREC_MIXED_FP32 = 1  /* FP32 stage derivatives; FP32 contractions with
-                                 compensated FP32 face sums where they are faster
-                                 (tensor advection), FP64 elsewhere;
-                                 FP64 geometry, state and RK update                 */
+    HGDG_PREC_MIXED_FP32 = 1  /* FP32 storage of the stage derivatives; FP64
+                                 arithmetic, geometry, state and RK update */
 };
 
 /*
