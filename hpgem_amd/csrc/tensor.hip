@@ -258,12 +258,18 @@ __device__ __forceinline__ double face_flux(uint32_t m, int s, double own, doubl
     return m == MODE_OWN ? 0.0 : (s ? h : -h) * (other - own);
 }
 
+__device__ __forceinline__ void face_coef_values(uint32_t c, double& cn, double& co) {
+    cn = __hiloint2double(int(c & 0xffff0000u), 0);
+    co = __hiloint2double(int(c << 16), 0);
+}
+
 // The arithmetic of one pencil, shared by every kernel variant so that they
 // agree bit for bit: per direction the one-dimensional operator, its volume
 // part here (x with its faces' fluxes fx), y and z faces by advection_face;
 // then minus ahat_d times each, summed. Row i of s_row: Dr(i, :), Mi(i, 0..1).
 template <int N1>
 __device__ __forceinline__ void advection_rows(const RhsParams& p, double* s_row) {
+    static_assert(N1 * (N1 + 2) <= 64, "a wavefront's threads");
     const int i = threadIdx.x / (N1 + 2), j = threadIdx.x % (N1 + 2);
     if (i < N1) s_row[threadIdx.x] = j < N1 ? p.Dr[i * N1 + j] : p.Mi[i * N1 + j - N1];
 }
@@ -394,17 +400,13 @@ __device__ __forceinline__ void advection_tiles(const RhsParams& p, int64_t t0, 
         int64_t at[NI], atx[2];
         int lx[2];
         double o[NI][1][N1], o1[NI][1][N1], ox[2], ox1[2], cq[NI][2], cx[2][2];
-        auto coef = [](uint32_t c, double (&h)[2]) {
-            h[0] = __hiloint2double(int(c & 0xffff0000u), 0);
-            h[1] = __hiloint2double(int(c << 16), 0);
-        };
 #pragma unroll
         for (int k = 0; k < NI; ++k)
             if (item(k)) {
                 const int q = tid + k * kBlock, fi = DIM == 3 ? q % NQ / N1 : q % NQ, j = DIM == 3 ? q % N1 : 0;
                 at[k] = int64_t(l.fq[k].x) * NB + (fi / 2 ? j + N1 * (1 - fi % 2) : (1 - fi % 2) + N1 * j) * N1;
                 load_pencils<1, N1, KIND>(p.io, at[k], 0, o[k], o1[k]);
-                coef(l.fq[k].y, cq[k]);
+                face_coef_values(l.fq[k].y, cq[k][0], cq[k][1]);
             }
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -418,7 +420,7 @@ __device__ __forceinline__ void advection_tiles(const RhsParams& p, int64_t t0, 
                 ox[s] = v[0];
                 ox1[s] = v1[0];
             }
-            coef(l.fx[s].y, cx[s]);
+            face_coef_values(l.fx[s].y, cx[s][0], cx[s][1]);
         }
         double y[1][N1];
         if constexpr (UPD) update_partial<1, N1>(p.io, base, 0, l.w, l.x, y);
@@ -636,6 +638,164 @@ __global__ __launch_bounds__((rk_tiny_block<DIM, N1>())) void tensor_advection_r
     for (int64_t q = threadIdx.x; q < n; q += kTinyBlock) {
         p.u[q] = su[q];
         for (int j = 0; j < st; ++j) static_cast<T*>(p.k[j])[q] = sk[int64_t(j) * n + q];
+    }
+}
+
+// The same for meshes with at most one x-pencil a thread: the thread keeps its
+// pencil of the solution, the update's running sum and what it needs of the
+// faces and operators in registers for all steps, and the stage input goes
+// through two LDS buffers in turn, so that a stage has one barrier (a buffer is
+// written again only after the barrier of the other one, which every reader
+// passes later). The last stage derivative is a register too; older ones, where
+// the tableau uses them, are the thread's own values in LDS.
+// Bound by latency (16^2 p = 2: 12 wavefronts' LDS reads and multiply-adds
+// between barriers on one CU). A step of RK4, us, by the kernel above and here:
+// 16^2 p = 2 7.2 and 4.6, 20^2 p = 1 6.0 and 3.1, 10^2 p = 4 10.9 and 6.9, 3^3
+// cells of p = 3 10.3 and 6.1, 3^3 of p = 1 4.5 and 2.2 (a wavefront without work costs
+// as much as one with: only as many are launched as there are pencils). Reading
+// the next stage's tableau entries ahead gained nothing (5.3 against 5.1).
+// Threads: as many as leave every value a register; none for 3D p = 4 and up,
+// where 512 threads spill (3 x 3 x 2 cells of p = 4: 14.5 us a step, no gain).
+template <int DIM, int N1>
+constexpr int rk_pencil_block() {
+    return DIM == 2 ? (N1 <= 3 ? 1024 : 512) : (N1 <= 2 ? 1024 : N1 <= 4 ? 512 : 0);
+}
+
+template <int DIM, int N1, typename T>
+__global__ __launch_bounds__((rk_pencil_block<DIM, N1>())) void tensor_advection_rk_pencil(const RkTinyParams p) {
+    using S = Pencil<DIM, N1>;
+    constexpr int NF = 2 * DIM;
+    extern __shared__ __align__(16) double dyn[];
+    const int n = int(p.rhs.n_elem) * S::NB, st = p.stages;
+    T* sk = reinterpret_cast<T*>(dyn + 2 * n);  // [stages][n]
+    const bool active = threadIdx.x < unsigned(p.rhs.n_elem) * S::NP;
+    const int q = active ? int(threadIdx.x) : 0, e = q / S::NP, pc = q % S::NP;
+    const int ib = pc % N1, ic = DIM == 3 ? pc / N1 : 0;
+    // face f: where its neighbour's values start (x: the one value), and the flux's coefficients
+    int at[NF];
+    uint32_t coef[NF];
+    double ah[DIM];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        const uint2 rec = p.rhs.face[e * NF + f];
+        const int s = f % 2;
+        const int pen = f < 2 ? pc : f < 4 ? (1 - s) + N1 * ic : ib + N1 * (1 - s);
+        at[f] = int(rec.x) * S::NB + pen * N1 + (f < 2 ? 1 - s : 0);
+        coef[f] = rec.y;
+    }
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) ah[d] = p.rhs.ahat[d * p.rhs.n_elem + e];
+    // the rows of the operators of this pencil's y and z index: registers where
+    // they leave no value to spill (2D up to p = 2), else LDS
+    constexpr bool kRows = DIM == 2 && N1 <= 3;
+    __shared__ double s_row[N1 * (N1 + 2)];
+    advection_rows<N1>(p.rhs, s_row);
+    double regs[kRows ? N1 + 2 : 1];
+    if constexpr (kRows) {
+#pragma unroll
+        for (int j = 0; j < N1 + 2; ++j) regs[j] = j < N1 ? p.rhs.Dr[ib * N1 + j] : p.rhs.Mi[ib * N1 + j - N1];
+    }
+    auto row_of = [&](int d, int j) {
+        if constexpr (kRows) return regs[j];
+        else return s_row[(d == 1 ? ib : ic) * (N1 + 2) + j];
+    };
+    double u[N1], kl[N1];
+#pragma unroll
+    for (int a = 0; a < N1; ++a) {
+        u[a] = p.u[q * N1 + a];
+        kl[a] = 0.0;
+    }
+    int buf = 0;
+    for (int step = 0; step < p.n_steps; ++step) {
+        double y[N1];
+#pragma unroll
+        for (int a = 0; a < N1; ++a) y[a] = u[a];
+        for (int i = 0; i < st; ++i) {
+            double w[N1];
+#pragma unroll
+            for (int a = 0; a < N1; ++a) w[a] = 1.0 * u[a];
+            for (uint32_t m = p.amask[i]; m != 0; m &= m - 1) {
+                const int j = __builtin_ctz(m);
+                const double c = p.ca[i * kMaxIn + j];
+                if (j == i - 1) {
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) w[a] = fma(c, kl[a], w[a]);
+                } else {
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) w[a] = fma(c, double(sk[j * n + q * N1 + a]), w[a]);
+                }
+            }
+            double* sw = dyn + buf * n;
+            buf ^= 1;
+            if (active) {
+#pragma unroll
+                for (int a = 0; a < N1; ++a) sw[q * N1 + a] = w[a];
+            }
+            __syncthreads();
+            double fx[2], t[DIM][N1], cn, co;
+            auto face = [&](int f) {
+                if constexpr (!kRows) asm volatile("" : "+v"(coef[f]));  // not unpacked for all stages at once
+                face_coef_values(coef[f], cn, co);
+            };
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                face(s);
+                fx[s] = fma(cn, sw[at[s]], -(co * w[s]));
+            }
+#pragma unroll
+            for (int a = 0; a < N1; ++a) {
+                double x = 0.0;
+#pragma unroll
+                for (int j = 0; j < N1; ++j) x = fma(p.rhs.Dr[a * N1 + j], w[j], x);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) x = fma(p.rhs.Mi[a * N1 + s], fx[s], x);
+                t[0][a] = x;
+            }
+#pragma unroll
+            for (int d = 1; d < DIM; ++d) {
+                double own[2][N1];  // the element's own traces: rows 0 and 1 of the line
+#pragma unroll
+                for (int a = 0; a < N1; ++a) t[d][a] = 0.0;
+#pragma unroll
+                for (int j = 0; j < N1; ++j) {
+                    const double* row = sw + e * S::NB + (d == 1 ? j + N1 * ic : ib + N1 * j) * N1;
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) {
+                        const double v = row[a];
+                        if (j < 2) own[j][a] = v;
+                        t[d][a] = fma(row_of(d, j), v, t[d][a]);
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    face(2 * d + s);
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) {
+                        const double flux = fma(cn, sw[at[2 * d + s] + a], -(co * own[s][a]));
+                        t[d][a] = fma(row_of(d, N1 + s), flux, t[d][a]);
+                    }
+                }
+            }
+            advection_result<DIM, N1>(ah, t, kl);
+            const bool used = (p.bmask >> i) & 1u;
+            const double cb = p.cb[i];
+#pragma unroll
+            for (int a = 0; a < N1; ++a) {
+                const T v = T(kl[a]);
+                if (active) sk[i * n + q * N1 + a] = v;
+                kl[a] = double(v);
+                if (used) y[a] = fma(cb, kl[a], y[a]);
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < N1; ++a) u[a] = y[a];
+    }
+    if (active) {
+#pragma unroll
+        for (int a = 0; a < N1; ++a) {
+            p.u[q * N1 + a] = u[a];
+            for (int j = 0; j < st; ++j) static_cast<T*>(p.k[j])[q * N1 + a] = sk[j * n + q * N1 + a];
+        }
     }
 }
 
@@ -1759,28 +1919,37 @@ bool tensor_rk_tiny(hgdg_ctx* c, int solution, const int* aux, int stages, const
     bool launched = false;
     dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
         constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
-        const void* fn = mixed ? reinterpret_cast<const void*>(&tensor_advection_rk_tiny<DIMc, N1c, float>)
-                               : reinterpret_cast<const void*>(&tensor_advection_rk_tiny<DIMc, N1c, double>);
-        if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) != hipSuccess) {
-            (void)hipGetLastError();  // this device cannot give the LDS: the graph path runs instead
-            return;
+        auto go = [&](auto kernel, int threads, size_t lds) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    int(lds)) != hipSuccess) {
+                (void)hipGetLastError();  // this device cannot give the LDS: the graph path runs instead
+                return false;
+            }
+            // at most kRkTinyChunk steps per launch, so that no launch runs for
+            // long; the solution goes through HBM between launches exactly (FP64)
+            for (int done = 0; done < n_steps; done += kRkTinyChunk) {
+                RkTinyParams q = p;
+                q.n_steps = std::min(kRkTinyChunk, n_steps - done);
+                hipLaunchKernelGGL(kernel, dim3(1), dim3(unsigned(threads)), lds, c->stream, q);
+                HGDG_HIP(hipGetLastError());
+                ++c->rk_fused_launches;
+            }
+            return true;
+        };
+        // one x-pencil a thread where the workgroup has that many threads
+        // (2D p = 2 with RK4: every mesh whose state fits)
+        constexpr int kPencil = rk_pencil_block<DIMc, N1c>(), kTiny = rk_tiny_block<DIMc, N1c>();
+        const size_t lds = size_t(16 * n) + size_t(stages) * size_t(n) * tb;
+        if constexpr (kPencil > 0) {
+            if (E * Pencil<DIMc, N1c>::NP <= kPencil) {
+                const int threads = int((E * Pencil<DIMc, N1c>::NP + 63) / 64 * 64);  // no wavefront without work
+                launched = mixed ? go(tensor_advection_rk_pencil<DIMc, N1c, float>, threads, lds)
+                                 : go(tensor_advection_rk_pencil<DIMc, N1c, double>, threads, lds);
+                return;
+            }
         }
-        constexpr unsigned kThreads = unsigned(rk_tiny_block<DIMc, N1c>());
-        // at most kRkTinyChunk steps per launch, so that no launch runs for
-        // long; the solution goes through HBM between launches exactly (FP64)
-        for (int done = 0; done < n_steps; done += kRkTinyChunk) {
-            RkTinyParams q = p;
-            q.n_steps = std::min(kRkTinyChunk, n_steps - done);
-            if (mixed)
-                hipLaunchKernelGGL((tensor_advection_rk_tiny<DIMc, N1c, float>), dim3(1), dim3(kThreads), bytes,
-                                   c->stream, q);
-            else
-                hipLaunchKernelGGL((tensor_advection_rk_tiny<DIMc, N1c, double>), dim3(1), dim3(kThreads), bytes,
-                                   c->stream, q);
-            HGDG_HIP(hipGetLastError());
-            ++c->rk_fused_launches;
-        }
-        launched = true;
+        launched = mixed ? go(tensor_advection_rk_tiny<DIMc, N1c, float>, kTiny, bytes)
+                         : go(tensor_advection_rk_tiny<DIMc, N1c, double>, kTiny, bytes);
     });
     return launched;
 }

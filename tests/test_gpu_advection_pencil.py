@@ -11,6 +11,7 @@ import pytest
 
 import _oracle as orc
 from _parity import assert_parity, rel
+import hpgem_amd.tableaux
 from hpgem_amd import RK4, HpgemAPIDevice, Mesh
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +56,30 @@ def test_advection_pencil_kernel(n, p, a, periodic):
                 else:
                     assert rel(got, ld) <= 2.0 ** -24 + 1e-12
         dev.close()
+
+
+@pytest.mark.parametrize("n,p,tab,precision", [
+    ([32, 16], 1, "RK4", "fp64"), ([31, 17], 1, "RK4", "mixed"), ([19, 17], 2, "RK3_TVD", "fp64"),
+    ([12, 10], 3, "DORMAND_PRINCE", "mixed"), ([12, 11], 3, "RK4", "fp64"), ([10, 10], 4, "RK4", "fp64"),
+    ([8, 8, 4], 1, "RK2_TVD", "fp64"), ([4, 4, 3], 2, "RK4", "mixed"), ([4, 4, 4], 2, "RK4", "fp64"),
+    ([3, 3, 3], 3, "RK3_TVD", "fp64"), ([3, 3, 3], 1, "RK4", "fp64")])
+def test_one_workgroup_steps_bitwise_equal_graph_replay(n, p, tab, precision):
+    """Steps in one workgroup with one x-pencil a thread, up to its largest
+    number of threads and beyond (the kernel that loops over pencils), against
+    the replayed step graph: the same operations, so the same bits."""
+    print(f"[case] one workgroup n={n} p={p} {tab} {precision}", flush=True)
+    tableau = getattr(hpgem_amd.tableaux, tab)
+    mesh = Mesh.structured(n)
+    a = [1.0, -0.7, 0.3][:len(n)]
+    out = {}
+    for fused in (False, True):
+        dev = HpgemAPIDevice(mesh, p, velocity=a, precision=precision, tableau=tableau, n_extra_vectors=2)
+        dev.setFusedTimeStepping(fused)
+        dev.setTimeIntegrationVector(0, np.random.default_rng(p).standard_normal(dev.n_dof))
+        dev.computeOneTimeStep(0.0, 0.02 / max(n), 5)
+        assert (dev.getFusedTimeStepping()[1] > 0) == fused
+        out[fused] = [dev.getTimeIntegrationVector(v) for v in range(tableau.stages + 1)]
+        dev.close()
+    assert np.all(np.isfinite(out[True][0]))
+    for g, f in zip(out[False], out[True]):
+        np.testing.assert_array_equal(f, g)
