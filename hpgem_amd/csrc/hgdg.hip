@@ -557,7 +557,7 @@ void rk_steps(hgdg_ctx* c, int solution, const int* aux, int stages, const doubl
 // (HpgemAPISimplified::computeErrorAndNormOfUpdate, kernel/Base/
 // HpgemAPISimplified_Impl.h:718-745): err2 = sum over all coefficients of
 // (sum_j dt e_j k_j)^2, norm = sum over elements of the Euclidean norm of the
-// element's solution coefficients. One wavefront per element.
+// element's solution coefficients.
 struct StepNormParams {
     int64_t n_elem;
     const int64_t* off;  // [n_elem + 1] element DOF offsets, or NULL
@@ -567,35 +567,56 @@ struct StepNormParams {
     double c[kMaxIn];
     uint32_t k_f32;
     int32_t n_k;
+    int32_t lanes;       // of an element
     double* partial;     // [blocks][2]
 };
 
+// A group of p.lanes lanes takes an element at a time, all its inputs' loads in
+// flight together. Bound by memory. Lanes by the elements' size and at most
+// kNormBlocks pairs of sums to read back, so that a launch of many small
+// elements neither idles most lanes nor leaves the sum to the host: at 301 x
+// 257 elements of 16, six stage vectors (69 MB), 34.4 -> 17.6 us (one wavefront
+// an element and four elements a block before), and 310 -> 16 KB come back.
+constexpr int64_t kNormBlocks = 1024;
 __global__ __launch_bounds__(kBlock) void step_error_norm(const StepNormParams p) {
     constexpr int W = 64;  // wavefront size on CDNA
     __shared__ double s_part[2][kBlock / W];
-    const int lane = threadIdx.x % W, wave = threadIdx.x / W;
-    const int64_t e = int64_t(blockIdx.x) * (kBlock / W) + wave;
-    double err2 = 0, u2 = 0;
-    if (e < p.n_elem) {
+    const int lane = threadIdx.x % W, wave = threadIdx.x / W, L = p.lanes;
+    const int64_t stride = int64_t(gridDim.x) * kBlock / L;
+    double err = 0, nrm = 0;  // of the group's elements
+    for (int64_t e = (int64_t(blockIdx.x) * kBlock + threadIdx.x) / L; e < p.n_elem; e += stride) {
         const int64_t lo = p.off ? p.off[e] : e * p.block;
         const int64_t hi = p.off ? p.off[e + 1] : lo + p.block;
-        for (int64_t i = lo + lane; i < hi; i += W) {
-            const double v = p.u[i];
-            u2 += v * v;
-            double d = 0;
-            for (int j = 0; j < p.n_k; ++j)
-                d += p.c[j] * (((p.k_f32 >> j) & 1u) ? double(static_cast<const float*>(p.k[j])[i])
-                                                      : static_cast<const double*>(p.k[j])[i]);
-            err2 += d * d;
+        double err2 = 0, u2 = 0;
+        for (int64_t i = lo + threadIdx.x % L; i < hi; i += L) {
+            const int64_t at[1] = {i};
+            double v[1], x[kMaxIn][1], d[1] = {0.0};
+            load_raw_n(p.u, false, at, v);
+#pragma unroll
+            for (int j = 0; j < kMaxIn; ++j)
+                if (j < p.n_k) load_raw_n(p.k[j], (p.k_f32 >> j) & 1u, at, x[j]);
+            u2 = fma(v[0], v[0], u2);
+#pragma unroll
+            for (int j = 0; j < kMaxIn; ++j)
+                if (j < p.n_k) add_raw_n(p.c[j], x[j], (p.k_f32 >> j) & 1u, d);
+            err2 = fma(d[0], d[0], err2);
         }
+        for (int o = L / 2; o > 0; o /= 2) {
+            err2 += __shfl_xor(err2, o, W);
+            u2 += __shfl_xor(u2, o, W);
+        }
+        err += err2;
+        nrm += sqrt(u2);
     }
+    // one lane of each group
+    if (threadIdx.x % L != 0) err = nrm = 0;
     for (int o = W / 2; o > 0; o /= 2) {
-        err2 += __shfl_xor(err2, o, W);
-        u2 += __shfl_xor(u2, o, W);
+        err += __shfl_xor(err, o, W);
+        nrm += __shfl_xor(nrm, o, W);
     }
     if (lane == 0) {
-        s_part[0][wave] = err2;
-        s_part[1][wave] = sqrt(u2);
+        s_part[0][wave] = err;
+        s_part[1][wave] = nrm;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -607,6 +628,14 @@ __global__ __launch_bounds__(kBlock) void step_error_norm(const StepNormParams p
         p.partial[2 * blockIdx.x] = a;
         p.partial[2 * blockIdx.x + 1] = b;
     }
+}
+
+// The lanes of an element (a power of two from 4 to a wavefront, for the mean
+// size) and the launch's workgroups.
+int64_t step_error_grid(const hgdg_ctx* c, StepNormParams& p) {
+    p.lanes = 4;
+    while (p.lanes < 64 && p.lanes * c->n_elem < c->dof) p.lanes *= 2;
+    return std::min(kNormBlocks, (c->n_elem * p.lanes + kBlock - 1) / kBlock);
 }
 
 void step_error_and_norm(hgdg_ctx* c, int solution, const int* aux, int stages, const double* err_coef, double dt,
@@ -624,8 +653,7 @@ void step_error_and_norm(hgdg_ctx* c, int solution, const int* aux, int stages, 
         if (k.is_f32) p.k_f32 |= 1u << p.n_k;
         ++p.n_k;
     }
-    const int64_t per = kBlock / 64;
-    const int64_t grid = (c->n_elem + per - 1) / per;
+    const int64_t grid = step_error_grid(c, p);
     if (c->d_partial.n < size_t(2 * grid)) c->d_partial.alloc(size_t(2 * grid));
     p.partial = c->d_partial.ptr;
     hipLaunchKernelGGL(step_error_norm, dim3(unsigned(grid)), dim3(kBlock), 0, c->stream, p);
@@ -651,7 +679,7 @@ void step_error_and_norm(hgdg_ctx* c, int solution, const int* aux, int stages, 
 // back to the caller's stack. Each GPU holds its own copy of the array (at its
 // own address, looked up once per device when a context is created on it);
 // every call on one GPU shares it, so calls that overlap on one GPU race.
-constexpr int64_t kScratchBlocks = 65536;  // partial pairs: meshes of at most 4 * 65536 elements
+constexpr int64_t kScratchBlocks = 65536;  // partial pairs; meshes of at most 4 * 65536 elements
 constexpr int64_t kScratchMaxElements = 4 * kScratchBlocks;
 static __device__ __align__(256) double scratch[2 * kScratchBlocks + 2];
 constexpr int kMaxDevices = 64;
@@ -734,8 +762,7 @@ int step_error_noalloc(hgdg_ctx* c, int solution, const int* aux, int stages, co
         if (k.is_f32) p.k_f32 |= 1u << p.n_k;
         ++p.n_k;
     }
-    const int64_t per = kBlock / 64;
-    const int64_t grid = (c->n_elem + per - 1) / per;
+    const int64_t grid = c->n_elem > 0 ? step_error_grid(c, p) : 0;
     p.partial = ptr;
     double h[2] = {0.0, 0.0};
     if (grid > 0) {
