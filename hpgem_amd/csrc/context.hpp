@@ -24,6 +24,7 @@ struct TensorMesh {
     DevBuf<int32_t> d_nbr, d_perm;   // d_perm: perm on the device (built on first use)
     DevBuf<double> d_absdet, d_ops;  // d_ops: Dr, Mi, M1 (n1 x n1 each)
     DevBuf<double> d_geo;            // advection: ahat [dim][e]; acoustic: J^{-1} [dim*dim][e], then c_inv [e]
+    DevBuf<int32_t> d_order;         // acoustic: order of the workgroups (empty: in turn)
     DevBuf<uint32_t> d_mode;         // advection: upwind mode, 3 bits per face
     DevBuf<uint2> d_face;            // advection: [e][face] the neighbour met and the flux's coefficients
     bool structured = false;         // periodic unit box built by tensor_structured_upload

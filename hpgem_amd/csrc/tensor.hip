@@ -26,6 +26,8 @@
 #include <array>
 #include <cmath>
 #include <cstring>
+#include <limits>
+#include <numeric>
 #include <string>
 #include <unordered_map>
 
@@ -145,13 +147,13 @@ __device__ __forceinline__ void mix_two_pencils(const StageIO& p, double (&u)[NR
     if (stage_two<KIND>(p)) add_raw<NR, N1>(p.coef[1], x, stage_second_f32<KIND>(p), u);
 }
 
-template <int NR, int N1>
+template <int NR, int N1, int KIND = STAGE_ANY>
 __device__ __forceinline__ void mix_pencils(const StageIO& p, int64_t base, int64_t stride, double (&u)[NR][N1],
                                             double (&x)[NR][N1]) {
-    mix_two_pencils<NR, N1>(p, u, x);
-#pragma unroll
-    for (int i = 2; i < kMaxIn; ++i) {
-        if (i >= p.n_in) break;
+    mix_two_pencils<NR, N1, KIND>(p, u, x);
+    if (KIND != STAGE_ANY) return;
+#pragma unroll 1
+    for (int i = 2; i < p.n_in; ++i) {
         load_raw<NR, N1>(p.in[i], (p.in_f32 >> i) & 1u, base, stride, x);
         add_raw<NR, N1>(p.coef[i], x, (p.in_f32 >> i) & 1u, u);
     }
@@ -853,6 +855,7 @@ struct AcousticParams {
     const int32_t* nbr;   // [2 dim][n_elem], -1 on walls
     const double* Dr;
     const double* Mi;
+    const int32_t* order;  // the workgroup of each place in the launch, or NULL: in turn (acoustic_order)
 };
 
 // One thread owns one x-pencil of an element with all its fields; v, g_y and
@@ -863,7 +866,7 @@ struct AcousticParams {
 // leaves at most one lane in sixteen idle: one wavefront where it can.
 // Sums are explicit multiply-adds: every instance (with and without the
 // update, batched) rounds alike.
-// Bound by memory: 32^3 p = 3 in FP64 reads and writes 201 MB at 4.3 TB/s
+// Bound by memory: 32^3 p = 3 in FP64 reads and writes 201 MB at 4.6 TB/s
 // (a copy of that size reaches 5.4 - 6.9 TB/s). One lane per field and pencil,
 // which applies the derivative of v once per s field and forms every face
 // pencil's flux N1 times, took 104 us FP64 / 80 mixed there against 47 / 36;
@@ -890,7 +893,7 @@ struct AcousticShape {
     static constexpr int ES = (DIM == 3 ? N1 : 1) * PS;
 };
 
-template <int DIM, int N1, bool UPD>
+template <int DIM, int N1, int KIND, bool UPD>
 __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t blk) {
     using S = AcousticShape<DIM, N1>;
     constexpr int NF = S::NF, NB = S::NB, NP = S::NP, NQ = S::NQ;
@@ -929,16 +932,16 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
 #pragma unroll
             for (int d = 0; d < DIM; ++d) J[r][d] = p.jinv[(r * DIM + d) * p.n_elem + e];
         double x[NF][N1];
-        load_pencils<NF, N1>(p.io, base + pc * N1, NB, w, x);
+        load_pencils<NF, N1, KIND>(p.io, base + pc * N1, NB, w, x);
         if constexpr (kEarly) update_partial<NF, N1>(p.io, base + pc * N1, NB, w, x, y);
         if constexpr (kAhead) {
             double xq[NF][N1];
             const int64_t bq = face_pencil(pc, nbq);
-            if (nbq >= 0) load_pencils<NF, N1>(p.io, bq, NB, wq, xq);
-            mix_pencils<NF, N1>(p.io, base + pc * N1, NB, w, x);
-            if (nbq >= 0) mix_pencils<NF, N1>(p.io, bq, NB, wq, xq);
+            if (nbq >= 0) load_pencils<NF, N1, KIND>(p.io, bq, NB, wq, xq);
+            mix_pencils<NF, N1, KIND>(p.io, base + pc * N1, NB, w, x);
+            if (nbq >= 0) mix_pencils<NF, N1, KIND>(p.io, bq, NB, wq, xq);
         } else {
-            mix_pencils<NF, N1>(p.io, base + pc * N1, NB, w, x);
+            mix_pencils<NF, N1, KIND>(p.io, base + pc * N1, NB, w, x);
         }
     } else {
 #pragma unroll
@@ -988,7 +991,9 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
                 int64_t at[NF];
 #pragma unroll
                 for (int f = 0; f < NF; ++f) at[f] = (int64_t(nbx[s]) * NF + f) * NB + pc * N1 + (1 - s);
-                combine_n<NF>(p.io, at, o);
+                double x[NF];
+                load_two<KIND>(p.io, at, o, x);
+                mix_two<KIND>(p.io, at, o, x);
             }
             double gn = 0.0;
 #pragma unroll
@@ -1028,8 +1033,8 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
                     for (int a = 0; a < N1; ++a) o[f][a] = wq[f][a];
             } else {
                 double x[NF][N1];
-                load_pencils<NF, N1>(p.io, face_pencil(q, nb), NB, o, x);
-                mix_pencils<NF, N1>(p.io, face_pencil(q, nb), NB, o, x);
+                load_pencils<NF, N1, KIND>(p.io, face_pencil(q, nb), NB, o, x);
+                mix_pencils<NF, N1, KIND>(p.io, face_pencil(q, nb), NB, o, x);
             }
             const double h = s ? -0.5 : 0.5;
 #pragma unroll
@@ -1121,9 +1126,10 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
 }
 
 // UPD: the RK update fused into this (last) stage, StageIO::upd.
-template <int DIM, int N1, bool UPD = false>
+template <int DIM, int N1, int KIND, bool UPD>
 __global__ __launch_bounds__((AcousticShape<DIM, N1>::THREADS)) void tensor_acoustic_rhs(const AcousticParams p) {
-    acoustic_block<DIM, N1, UPD>(p, xcd_block(blockIdx.x, gridDim.x));
+    const int64_t b = xcd_block(blockIdx.x, gridDim.x);
+    acoustic_block<DIM, N1, KIND, UPD>(p, p.order ? p.order[b] : b);
 }
 
 template <int DIM, int N1, bool UPD = false>
@@ -1131,7 +1137,8 @@ __global__ __launch_bounds__((AcousticShape<DIM, N1>::THREADS)) void tensor_acou
     const AcousticParams* __restrict__ ps, const int64_t* __restrict__ off, int n) {
     const int64_t b = xcd_block(blockIdx.x, gridDim.x);
     const int s = __builtin_amdgcn_readfirstlane(find_problem(off, n, b));
-    acoustic_block<DIM, N1, UPD>(ps[s], b - off[s]);
+    const int32_t* order = ps[s].order;
+    acoustic_block<DIM, N1, STAGE_ANY, UPD>(ps[s], order ? order[b - off[s]] : b - off[s]);
 }
 
 // L2 projection of f(x) = sum_m amp_m sin(2 pi k_m . x) on affine tensor
@@ -1707,6 +1714,39 @@ void tensor_mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     finish_tensor_upload(c);
 }
 
+// The order in which the acoustic kernel's workgroups take the elements of a
+// box too large to go plane by plane: an XCD's share of the launch is a range
+// of planes, a z neighbour is a plane away, and three vectors' planes (two
+// inputs, one output) beyond the 4 MB L2 are read again from farther off. The
+// rows are then taken in columns of as many as fit 1.5 MB, through all planes.
+// Rows and planes are guessed from the numbering (the distances to an
+// element's upper y and z neighbours); a wrong guess changes the order only.
+// RK4 step of 32^3 p = 3 (6.3 MB a plane) 234 -> 220 us, 48^3 p = 2 (6 MB) 437 ->
+// 399; of boxes around the line (23 x 19 planes of p = 4, 5.2 MB) the same.
+static std::vector<int32_t> acoustic_order(const hgdg_ctx* c) {
+    if (c->dim != 3) return {};
+    const int64_t ne = c->n_elem, bytes = 3 * int64_t(sizeof(double)) * c->tm.nb * c->n_fields;
+    int64_t sy = 0, sz = 0;
+    for (int64_t e = ne / 2; e < ne && (sy <= 0 || sz <= sy); ++e) {
+        sy = c->tm.nbr[size_t(3) * ne + e] - e;
+        sz = c->tm.nbr[size_t(5) * ne + e] - e;
+    }
+    if (sy <= 0 || sz <= sy || sz * bytes <= (int64_t(4) << 20)) return {};
+    int64_t epb = 1;
+    dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
+        epb = AcousticShape<decltype(D)::value, decltype(N)::value>::EPB;
+    });
+    const int64_t n = (ne + epb - 1) / epb, rows = std::max<int64_t>(1, (int64_t(3) << 19) / (sy * bytes));
+    if (n > std::numeric_limits<int32_t>::max()) return {};
+    std::vector<int32_t> order(static_cast<size_t>(n));
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+        auto column = [&](int32_t i) { return i * epb % sz / sy / rows; };
+        return column(a) < column(b);
+    });
+    return order;
+}
+
 void tensor_operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
     if (c->tm.general) {
         tensor_general_operator_set(c, op);
@@ -1725,6 +1765,9 @@ void tensor_operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
         c->tm.d_geo.upload(geo, c->stream);
         c->n_fields = dim + 1;
         c->dof = ne * c->tm.nb * c->n_fields;
+        const std::vector<int32_t> order = acoustic_order(c);
+        c->tm.d_order.reset();
+        if (!order.empty()) c->tm.d_order.upload(order, c->stream);
         HGDG_HIP(hipStreamSynchronize(c->stream));
         return;
     }
@@ -1795,13 +1838,23 @@ static RhsParams advection_params(hgdg_ctx* c, const StageIO& io) {
     return p;
 }
 
+template <typename F>
+static void with_stage_kind(const StageIO& io, F&& f) {
+    switch (stage_kind(io)) {
+        case STAGE_ONE: f(std::integral_constant<int, STAGE_ONE>{}); break;
+        case STAGE_TWO: f(std::integral_constant<int, STAGE_TWO>{}); break;
+        case STAGE_TWO_MIXED: f(std::integral_constant<int, STAGE_TWO_MIXED>{}); break;
+        default: f(std::integral_constant<int, STAGE_ANY>{}); break;
+    }
+}
+
 static void launch_advection(hgdg_ctx* c, const RhsParams& p, int tiles) {
     dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
         constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
         using S = Pencil<DIMc, N1c>;
         const int64_t n_tiles = (c->n_elem + S::EPB - 1) / S::EPB;
         const bool upd = p.io.upd.u != nullptr;  // the fused RK update runs in the one-tile kernel
-        auto go = [&](auto K) {
+        with_stage_kind(p.io, [&](auto K) {
             constexpr int KIND = decltype(K)::value;
             if (upd)
                 hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, KIND, true>), dim3(unsigned(n_tiles)),
@@ -1813,13 +1866,7 @@ static void launch_advection(hgdg_ctx* c, const RhsParams& p, int tiles) {
             else
                 hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, KIND, false>), dim3(unsigned(n_tiles)),
                                    dim3(kBlock), 0, c->stream, p);
-        };
-        switch (stage_kind(p.io)) {
-            case STAGE_ONE: go(std::integral_constant<int, STAGE_ONE>{}); break;
-            case STAGE_TWO: go(std::integral_constant<int, STAGE_TWO>{}); break;
-            case STAGE_TWO_MIXED: go(std::integral_constant<int, STAGE_TWO_MIXED>{}); break;
-            default: go(std::integral_constant<int, STAGE_ANY>{}); break;
-        }
+        });
     });
     HGDG_HIP(hipGetLastError());
 }
@@ -1971,16 +2018,22 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
         a.nbr = c->tm.d_nbr.ptr;
         a.Dr = Dr_ptr(c);
         a.Mi = Mi_ptr(c);
+        a.order = c->tm.d_order.ptr;
         dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
             constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
             using S = AcousticShape<DIMc, N1c>;
             const int64_t grid = (c->n_elem + S::EPB - 1) / S::EPB;
-            if (io.upd.u != nullptr)  // the fused RK update of a step's last stage
-                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, true>), dim3(unsigned(grid)), dim3(S::THREADS), 0,
-                                   c->stream, a);
-            else
-                hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c>), dim3(unsigned(grid)), dim3(S::THREADS), 0,
-                                   c->stream, a);
+            with_stage_kind(io, [&](auto K) {
+                // the update at 3D p = 3 is the one form that needs more registers
+                // by its kind (280 against 225: one wavefront a SIMD instead of two)
+                constexpr int KIND = decltype(K)::value, KU = DIMc == 3 && N1c == 4 ? int(STAGE_ANY) : KIND;
+                if (io.upd.u != nullptr)  // the fused RK update of a step's last stage
+                    hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, KU, true>), dim3(unsigned(grid)),
+                                       dim3(S::THREADS), 0, c->stream, a);
+                else
+                    hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, KIND, false>), dim3(unsigned(grid)),
+                                       dim3(S::THREADS), 0, c->stream, a);
+            });
         });
         HGDG_HIP(hipGetLastError());
         return;
@@ -2154,6 +2207,7 @@ void tensor_batch_param(hgdg_ctx* c, const StageIO& io, void* out) {
         a.nbr = c->tm.d_nbr.ptr;
         a.Dr = Dr_ptr(c);
         a.Mi = Mi_ptr(c);
+        a.order = c->tm.d_order.ptr;
         std::memcpy(out, &a, sizeof(a));
     } else {
         RhsParams r{};

@@ -50,3 +50,30 @@ def test_acoustic_pencil_kernel(n, p, periodic):
             else:
                 assert rel(got, ld) <= 2.0 ** -24 + 1e-12
         dev.close()
+
+
+@pytest.mark.parametrize("n,p,precision", [([23, 17, 3], 4, "fp64"), ([21, 11, 2], 5, "mixed"), ([60, 31, 2], 2, "fp64"),
+                                           ([7, 97, 2], 4, "fp64")])
+def test_acoustic_workgroup_order(n, p, precision):
+    """Boxes whose planes pass the L2, whose workgroups are taken in columns of
+    rows, against the same box with its elements in random order (other rows
+    or none): the same operator, so equal within rounding (1e-12, mixed: its
+    storage's 2^-24 more)."""
+    print(f"[case] acoustic order n={n} p={p} {precision}", flush=True)
+    mesh = Mesh.structured(n, periodic=[1, 1, 0])
+    rng = np.random.default_rng(p)
+    E = mesh.n_elements
+    c = 1.0 / rng.uniform(0.5, 2.0, E) ** 2
+    perm = rng.permutation(E)
+    u = rng.standard_normal((E, 4 * (p + 1) ** 3))
+    out = []
+    for order in (np.arange(E), perm):
+        m = Mesh(mesh.shape, np.array(mesh.coords)[order], np.array(mesh.node_ids)[order])
+        dev = HpgemAPIDevice(m, p, precision=precision, kind=OP_ACOUSTIC_CENTRAL, c_inv=c[order], tableau=RK4)
+        dev.setTimeIntegrationVector(0, u[order].ravel())
+        dev.computeOneTimeStep(0.0, 1e-4, 2)
+        dev.computeTimeDerivative([0], [1.0], 1)
+        out.append(np.empty_like(u))
+        out[-1][order] = dev.getTimeIntegrationVector(1).reshape(E, -1)
+        dev.close()
+    assert rel(out[1], out[0]) <= 1e-12 + (2.0 ** -24 if precision == "mixed" else 0.0)
