@@ -34,14 +34,14 @@ N_CELLS = 32
 P = 3
 VELOCITY = [1.0, 0.7, 0.3]
 SEED = 1
-# HBM bytes per launch of tensor_advection_rhs<3,4,T> on this workload, from
+# HBM bytes per launch of tensor_advection_rhs<3,4,KIND,false> on this workload, from
 # `rocprofv3 --pmc FETCH_SIZE` and `--pmc WRITE_SIZE` runs of
 # `bench.py --profile-workload`, each scaled by what the counter reads for a
 # plain copy of one 16 MiB vector (FETCH_SIZE x 1.9979, WRITE_SIZE x 1); the
 # commands and per-kernel figures are in
 # profiles/rhs_kernels_32cube_p3_and_tet24.md. Counters cannot be read from
 # inside this process, so the figure is reported as measured there.
-MEASURED_TRAFFIC = {"double": 58.60e6, "float": 37.46e6}
+MEASURED_TRAFFIC = {"double": 54.81e6, "mixed": 38.04e6}
 # dt = CFL h / |a|. At CFL 0.1 the RK4 step of this p = 3 operator has
 # spectral radius ~1.47 (power iteration on the oracle, 4^3 periodic mesh), so
 # round-off grows ~1e8-fold over 50 steps; 0.05 lies inside the stability
@@ -288,7 +288,7 @@ def run_other_config(name, steps, warmup):
         dt = 0.1 * (1 / 16) / float(np.linalg.norm(vel))
         make = lambda prec: HpgemAPIDevice(mesh, 2, velocity=vel, precision=prec, tableau=RK4, n_extra_vectors=2)
         init = lambda api: api.setInitialSolutionModes(amp, kk)
-        kernel = "tensor_advection_rhs<2,3,{}>"
+        kernel = "tensor_advection_rhs<2,3,{},false>"
     elif name == "hex32_p3_acoustic":
         mesh = Mesh.structured([32, 32, 32])
         c = rng.uniform(0.5, 2.0, size=mesh.n_elements)
@@ -297,7 +297,7 @@ def run_other_config(name, steps, warmup):
         make = lambda prec: HpgemAPIDevice(mesh, 3, precision=prec, kind=OP_ACOUSTIC_CENTRAL, c_inv=cinv,
                                            tableau=RK4, n_extra_vectors=2)
         init = lambda api: api.setInitialSolutionModes([1.0], [[1.0, 2.0, 1.0]], field=0)
-        kernel = "tensor_acoustic_rhs<3,4,{}>"
+        kernel = "tensor_acoustic_rhs<3,4,{},false>"
     else:
         mesh = Mesh.structured([24, 24, 24], periodic=[0, 0, 0], simplices=True)
         orders = rng.integers(1, 5, size=mesh.n_elements).astype(np.int32)
@@ -308,7 +308,7 @@ def run_other_config(name, steps, warmup):
         make = lambda prec: HpgemAPIDevice(mesh, orders, precision=prec, kind=OP_ACOUSTIC_CENTRAL, c_inv=cinv,
                                            tableau=RK4, n_extra_vectors=2)
         init = lambda api: api.setInitialSolutionGaussian(centre, 0.05, 1.0, field=0)
-        kernel = "simplex_acoustic_rhs"
+        kernel = "simplex_acoustic_rhs<{},false>"
     out, finals = {}, {}
     ref = None
     for prec in ("fp64", "mixed"):
@@ -334,7 +334,7 @@ def run_other_config(name, steps, warmup):
         out[prec] = {"gdofs": api.n_dof / (ms * 1e-3) / 1e9, "ms_per_rhs": ms, "bytes_alg_per_rhs": bytes_alg,
                      "achieved_gbs": bytes_alg / (ms * 1e-3) / 1e9,
                      "roofline_frac": bytes_alg / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                     "kernel": kernel.format("double" if prec == "fp64" else "float"),
+                     "kernel": kernel.format("2" if prec == "fp64" else "3"),
                      "rk4_100_steps_ms": run_ms}
         out["dof"], out["elements"], out["faces"], out["dt"] = api.n_dof, api.n_elements, api.n_faces, dt
         if prec == "fp64":
@@ -515,8 +515,8 @@ def main():
     head = gpu["mixed"] if mixed_ok else gpu["fp64"]
     roof = {"bound": "hbm", "achieved": head["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": head["achieved_gbs"] / HBM_PEAK_GBS,
-            "traffic": MEASURED_TRAFFIC["float" if mixed_ok else "double"],
-            "kernel": "tensor_advection_rhs<3,4," + ("float" if mixed_ok else "double") + ">",
+            "traffic": MEASURED_TRAFFIC["mixed" if mixed_ok else "double"],
+            "kernel": "tensor_advection_rhs<3,4," + ("3" if mixed_ok else "2") + ",false>",
             "bytes_alg_per_launch": head["bytes_alg_per_rhs"]}
     out = {
         "metric": METRIC,
@@ -529,7 +529,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32/f64 (f32 contractions and stage derivatives, f64 state, jumps, geometry)" if mixed_ok
+        "dtype": "f32/f64 (f32 stage derivatives, f64 arithmetic, state, geometry)" if mixed_ok
                  else "f64",
         "data": "synthetic (seeded sine modes, L2-projected)",
         "config": {"workload": "3D linear advection, periodic 32^3 hex, p=3, upwind, RK4 stage RHS "

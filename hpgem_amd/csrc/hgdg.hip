@@ -126,6 +126,7 @@ struct PinnedPool {
     std::mutex mu;
     std::vector<double*> kept;
     int64_t users = 0;
+    PinnedPool() { kept.reserve(kPinnedKept); }  // giving a chunk back allocates nothing
 };
 PinnedPool& pinned_pool() {
     static PinnedPool* pool = new PinnedPool;  // never destroyed: the HIP runtime may end before statics do
