@@ -171,6 +171,7 @@ void tensor_project_device(hgdg_ctx* c, Vec& v, int field, int n_modes, const do
                            const double* gauss = nullptr);
 void tensor_operator_set(hgdg_ctx* c, const hgdg_op_desc* op);
 void tensor_rhs(hgdg_ctx* c, const StageIO& io);
+bool tensor_weak_rhs(hgdg_ctx* c, const StageIO& io);  // without the inverse mass; false: no kernel for it
 // n_steps RK steps in one single-workgroup launch when the mesh is small
 // enough for LDS (tensor advection); false: not eligible, nothing launched
 bool tensor_rk_tiny(hgdg_ctx* c, int solution, const int* aux, int stages, const double* a, const double* b,

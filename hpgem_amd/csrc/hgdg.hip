@@ -1081,6 +1081,7 @@ int hgdg_right_hand_side(hgdg_ctx* ctx, const int* in_ids, const double* coeffs,
             hgdg::matrix_rhs(ctx, hgdg::make_io(ctx, in_ids, coeffs, n_in, out_id), false);
             return;
         }
+        if (!ctx->simplex() && hgdg::tensor_weak_rhs(ctx, hgdg::make_io(ctx, in_ids, coeffs, n_in, out_id))) return;
         // r = M k: the fused kernel's k, multiplied back by the block-diagonal mass
         hgdg::launch_rhs(ctx, in_ids, coeffs, n_in, out_id);
         if (ctx->simplex()) hgdg::simplex_mass_apply(ctx, out, false);

@@ -855,6 +855,8 @@ struct AcousticParams {
     const int32_t* nbr;   // [2 dim][n_elem], -1 on walls
     const double* Dr;
     const double* Mi;
+    const double* absdet;  // [n_elem] and
+    const double* M1;      // the 1D mass: MASS only
     const int32_t* order;  // the workgroup of each place in the launch, or NULL: in turn (acoustic_order)
 };
 
@@ -893,7 +895,7 @@ struct AcousticShape {
     static constexpr int ES = (DIM == 3 ? N1 : 1) * PS;
 };
 
-template <int DIM, int N1, int KIND, bool UPD>
+template <int DIM, int N1, int KIND, bool UPD, bool MASS = false>
 __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t blk) {
     using S = AcousticShape<DIM, N1>;
     constexpr int NF = S::NF, NB = S::NB, NP = S::NP, NQ = S::NQ;
@@ -1055,7 +1057,10 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
         }
     }
     __syncthreads();
-    if (!active) return;
+    if constexpr (!MASS) {  // (the mass below meets at barriers: threads without a pencil stay, on the first element)
+        if (!active) return;
+    }
+    const int lr = MASS && le >= S::EPB ? 0 : le;
 
     // ---- per direction: the one-dimensional operator on g_r and on v
     double kv[N1], ks[DIM][N1];
@@ -1079,8 +1084,8 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
 #pragma unroll
     for (int r = 1; r < DIM; ++r) {
         const int my = r == 1 ? ib : ic;
-        const double* sv = s_v + le * S::ES;
-        const double* sg = s_g + ((r - 1) * S::EPB + le) * S::ES;
+        const double* sv = s_v + lr * S::ES;
+        const double* sg = s_g + ((r - 1) * S::EPB + lr) * S::ES;
         double t[N1];
 #pragma unroll
         for (int a = 0; a < N1; ++a) t[a] = 0.0;
@@ -1098,7 +1103,7 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
         for (int s = 0; s < 2; ++s) {
             const double mi = p.Mi[my * N1 + s];
             const int q = DIM == 3 ? ((r - 1) * 2 + s) * N1 + (r == 1 ? ic : ib) : s;
-            const double* f = s_f + (le * NQ + q) * 2 * N1;
+            const double* f = s_f + (lr * NQ + q) * 2 * N1;
 #pragma unroll
             for (int a = 0; a < N1; ++a) {
                 kv[a] = fma(mi, f[a], kv[a]);
@@ -1109,6 +1114,50 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
         for (int d = 0; d < DIM; ++d)
 #pragma unroll
             for (int a = 0; a < N1; ++a) ks[d][a] = fma(J[r][d], t[a], ks[d][a]);
+    }
+    // ---- MASS: the right-hand side itself, M_e times this; c_inv of the s fields'
+    // mass cancels theirs here. Field by field, v's place in LDS for the passes
+    // along y and z.
+    if constexpr (MASS) {
+        const double det = active ? p.absdet[e] : 0.0;
+        auto mass = [&](double (&k)[N1]) {
+            double y[N1];
+#pragma unroll
+            for (int a = 0; a < N1; ++a) {
+                y[a] = 0.0;
+#pragma unroll
+                for (int j = 0; j < N1; ++j) y[a] = fma(p.M1[a * N1 + j], k[j], y[a]);
+            }
+#pragma unroll
+            for (int r = 1; r < DIM; ++r) {
+                __syncthreads();  // the last readers are done
+                if (le < S::EPB) {
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) s_v[le * S::ES + row(ib, ic) + a] = y[a];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int a = 0; a < N1; ++a) y[a] = 0.0;
+#pragma unroll
+                for (int j = 0; j < N1; ++j) {
+                    const double m = p.M1[(r == 1 ? ib : ic) * N1 + j];
+                    const double* x = s_v + lr * S::ES + (r == 1 ? row(j, ic) : row(ib, j));
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) y[a] = fma(m, x[a], y[a]);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < N1; ++a) k[a] = y[a] * det;
+        };
+        mass(kv);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) mass(ks[d]);
+        if (active) {
+            store_pencil<N1>(p.io, base + pc * N1, kv);
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) store_pencil<N1>(p.io, base + pc * N1 + (1 + d) * NB, ks[d]);
+        }
+        return;
     }
     const double ci = 1.0 / p.cinv[e];
     const int64_t o = base + pc * N1;
@@ -1130,6 +1179,17 @@ template <int DIM, int N1, int KIND, bool UPD>
 __global__ __launch_bounds__((AcousticShape<DIM, N1>::THREADS)) void tensor_acoustic_rhs(const AcousticParams p) {
     const int64_t b = xcd_block(blockIdx.x, gridDim.x);
     acoustic_block<DIM, N1, KIND, UPD>(p, p.order ? p.order[b] : b);
+}
+
+// hgdg_right_hand_side: the result times the mass, in one launch instead of this
+// kernel's and tensor_mass's; small meshes are bound by the launches, large ones
+// by the result going through memory twice more. us a call: 48 x 40 p = 2 9.6 ->
+// 6.6, 256^2 p = 3 29 -> 15, 30^3 p = 1 15 -> 7.9, p = 2 34 -> 21, 32^3 p = 3 68 ->
+// 53 (one wavefront a SIMD there), 16^3 p = 5 50 -> 43.
+template <int DIM, int N1>
+__global__ __launch_bounds__((AcousticShape<DIM, N1>::THREADS)) void tensor_acoustic_weak(const AcousticParams p) {
+    const int64_t b = xcd_block(blockIdx.x, gridDim.x);
+    acoustic_block<DIM, N1, STAGE_ANY, false, true>(p, p.order ? p.order[b] : b);
 }
 
 template <int DIM, int N1, bool UPD = false>
@@ -2004,21 +2064,42 @@ bool tensor_rk_tiny(hgdg_ctx* c, int solution, const int* aux, int stages, const
     return launched;
 }
 
+static AcousticParams acoustic_params(hgdg_ctx* c, const StageIO& io) {
+    AcousticParams a{};
+    a.n_elem = c->n_elem;
+    a.io = io;
+    a.jinv = c->tm.d_geo.ptr;
+    a.cinv = c->tm.d_geo.ptr + size_t(c->dim) * c->dim * c->n_elem;
+    a.nbr = c->tm.d_nbr.ptr;
+    a.Dr = Dr_ptr(c);
+    a.Mi = Mi_ptr(c);
+    a.order = c->tm.d_order.ptr;
+    a.absdet = c->tm.d_absdet.ptr;
+    a.M1 = M1_ptr(c);
+    return a;
+}
+
+// hgdg_right_hand_side in one launch, where there is a kernel for it.
+bool tensor_weak_rhs(hgdg_ctx* c, const StageIO& io) {
+    if (c->tm.general || c->op.kind != HGDG_OP_ACOUSTIC_CENTRAL) return false;
+    const AcousticParams a = acoustic_params(c, io);
+    dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
+        constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
+        using S = AcousticShape<DIMc, N1c>;
+        hipLaunchKernelGGL((tensor_acoustic_weak<DIMc, N1c>), dim3(unsigned((c->n_elem + S::EPB - 1) / S::EPB)),
+                           dim3(S::THREADS), 0, c->stream, a);
+    });
+    HGDG_HIP(hipGetLastError());
+    return true;
+}
+
 void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
     if (c->tm.general) {
         tensor_general_rhs(c, io);
         return;
     }
     if (c->op.kind == HGDG_OP_ACOUSTIC_CENTRAL) {
-        AcousticParams a{};
-        a.n_elem = c->n_elem;
-        a.io = io;
-        a.jinv = c->tm.d_geo.ptr;
-        a.cinv = c->tm.d_geo.ptr + size_t(c->dim) * c->dim * c->n_elem;
-        a.nbr = c->tm.d_nbr.ptr;
-        a.Dr = Dr_ptr(c);
-        a.Mi = Mi_ptr(c);
-        a.order = c->tm.d_order.ptr;
+        const AcousticParams a = acoustic_params(c, io);
         dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
             constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
             using S = AcousticShape<DIMc, N1c>;
@@ -2199,15 +2280,7 @@ int64_t tensor_batch_blocks(const hgdg_ctx* c) {
 
 void tensor_batch_param(hgdg_ctx* c, const StageIO& io, void* out) {
     if (c->op.kind == HGDG_OP_ACOUSTIC_CENTRAL) {
-        AcousticParams a{};
-        a.n_elem = c->n_elem;
-        a.io = io;
-        a.jinv = c->tm.d_geo.ptr;
-        a.cinv = c->tm.d_geo.ptr + size_t(c->dim) * c->dim * c->n_elem;
-        a.nbr = c->tm.d_nbr.ptr;
-        a.Dr = Dr_ptr(c);
-        a.Mi = Mi_ptr(c);
-        a.order = c->tm.d_order.ptr;
+        const AcousticParams a = acoustic_params(c, io);
         std::memcpy(out, &a, sizeof(a));
     } else {
         RhsParams r{};

@@ -77,3 +77,29 @@ def test_acoustic_workgroup_order(n, p, precision):
         out[-1][order] = dev.getTimeIntegrationVector(1).reshape(E, -1)
         dev.close()
     assert rel(out[1], out[0]) <= 1e-12 + (2.0 ** -24 if precision == "mixed" else 0.0)
+
+
+@pytest.mark.parametrize("n,p,periodic", CASES)
+def test_acoustic_right_hand_side_in_one_launch(n, p, periodic):
+    """hgdg_right_hand_side (the mass taken in the kernel itself) at the same
+    tiles' edges, FP32 and FP64 inputs, against the oracle."""
+    print(f"[case] acoustic right-hand side n={n} p={p} periodic={periodic}", flush=True)
+    mesh = Mesh.structured(n, periodic=[int(periodic)] * len(n))
+    rng = np.random.default_rng(sum(n) + 2 * p)
+    cinv = 1.0 / rng.uniform(0.5, 2.0, mesh.n_elements) ** 2
+    refs = []
+    for ext in (False, True):
+        P = orc.Problem(mesh.shape, mesh.coords, mesh.node_ids, p, n_fields=len(n) + 1, extended=ext)
+        P.set_acoustic(cinv)
+        refs.append(P)
+    dev = HpgemAPIDevice(mesh, p, kind=OP_ACOUSTIC_CENTRAL, c_inv=cinv, tableau=RK4, n_extra_vectors=2)
+    dev.setStorage(1, "mixed")
+    vecs = [rng.standard_normal(dev.n_dof) for _ in range(3)]
+    vecs[1] = vecs[1].astype(np.float32).astype(np.float64)
+    for i, v in enumerate(vecs):
+        dev.setTimeIntegrationVector(i, v)
+    for m, co in ((1, [1.0]), (2, [1.0, -0.3]), (3, [0.5, 0.2, 1.5])):
+        dev.computeRightHandSide(list(range(m)), co, 3)
+        assert_parity(dev.getTimeIntegrationVector(3), refs[0].right_hand_side(vecs[:m], co),
+                      refs[1].right_hand_side(vecs[:m], co), p, refs[0], f"acoustic right-hand side {n} p={p}")
+    dev.close()
