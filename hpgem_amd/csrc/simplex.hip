@@ -284,7 +284,8 @@ __device__ __forceinline__ void simplex_block(const SimplexParams& p, int64_t fi
             const double pv = __shfl(nv, partner, 64), pg = __shfl(ng, partner, 64);
             if (!in) continue;
             double bv = 0, bg = 0;
-            const int c1 = code[k] >> 6, c2 = m >= 13 ? (rec[k].y >> (m == 13 ? 8 : 10)) & 3 : 0;  // 1: +, 2: -
+            // 1: +, 2: - (m = 15 is no face function: what such a lane has loaded is nobody's)
+            const int c1 = code[k] >> 6, c2 = m >= 13 && m < 15 ? (rec[k].y >> (m == 13 ? 8 : 10)) & 3 : 0;
             if (c1 == 1 || c1 == 2) {
                 bv = c1 == 1 ? nv : -nv;
                 bg = c1 == 1 ? ng : -ng;
