@@ -485,7 +485,10 @@ __global__ __launch_bounds__((GenRhs<DIM, N1, ACOUSTIC>::THREADS)) void tensor_g
             }
             double* out = sc + f * NF * NFP + k;
             if constexpr (!ACOUSTIC) {
-                out[0] = inner ? fma(gf[i][0], own[0], gf[i][1] * nbv[0]) : gf[i][0] * own[0];
+                // a trace the flux does not take is left out, not multiplied by
+                // its factor of zero: it may be infinite or not a number
+                const double fn = inner && gf[i][1] != 0.0 ? gf[i][1] * nbv[0] : 0.0;
+                out[0] = gf[i][0] != 0.0 ? fma(gf[i][0], own[0], fn) : fn;
             } else {
                 // -1/2 n.(s_own - s_nbr) and -1/2 n (v_own - v_nbr), n the own
                 // normal; -n.s_own and nothing on a wall
