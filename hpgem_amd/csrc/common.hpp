@@ -262,32 +262,40 @@ __device__ __forceinline__ void add_raw_n(double c, const double (&x)[K], bool f
 // stages' own combinations without a branch between their loads, or any.
 enum StageKind : int {
     STAGE_ANY = 0,
-    STAGE_ONE = 1,        // one input, FP64
-    STAGE_TWO = 2,        // two, both FP64
-    STAGE_TWO_MIXED = 3,  // two, FP64 and FP32
+    STAGE_ONE = 1,         // one input, FP64
+    STAGE_TWO = 2,         // two, both FP64
+    STAGE_TWO_MIXED = 3,   // two, FP64 and FP32
+    STAGE_MANY = 4,        // three or more, all FP64
+    STAGE_MANY_MIXED = 5,  // three or more, FP64 and then FP32
 };
 inline int stage_kind(const StageIO& p) {
+    const bool mixed = p.in_f32 == (1u << p.n_in) - 2u;
     if (p.n_in == 1 && p.in_f32 == 0) return STAGE_ONE;
-    if (p.n_in == 2 && p.in_f32 == 0) return STAGE_TWO;
-    if (p.n_in == 2 && p.in_f32 == 2) return STAGE_TWO_MIXED;
+    if (p.n_in >= 2 && p.in_f32 == 0) return p.n_in == 2 ? STAGE_TWO : STAGE_MANY;
+    if (p.n_in >= 2 && mixed) return p.n_in == 2 ? STAGE_TWO_MIXED : STAGE_MANY_MIXED;
     return STAGE_ANY;
 }
 
-// Whether there is a second input, and whether it is FP32.
+// Whether there is a second input, whether there may be more, and whether
+// input i > 0 is FP32.
 template <int KIND>
 __device__ __forceinline__ bool stage_two(const StageIO& p) {
     return KIND == STAGE_ANY ? p.n_in > 1 : KIND != STAGE_ONE;
 }
 template <int KIND>
-__device__ __forceinline__ bool stage_second_f32(const StageIO& p) {
-    return KIND == STAGE_ANY ? (p.in_f32 & 2u) != 0 : KIND == STAGE_TWO_MIXED;
+constexpr bool stage_more() {
+    return KIND == STAGE_ANY || KIND == STAGE_MANY || KIND == STAGE_MANY_MIXED;
+}
+template <int KIND>
+__device__ __forceinline__ bool stage_f32(const StageIO& p, int i) {
+    return KIND == STAGE_ANY ? ((p.in_f32 >> i) & 1u) != 0 : KIND == STAGE_TWO_MIXED || KIND == STAGE_MANY_MIXED;
 }
 
 // combine_n in parts: the first two inputs' loads, their sums (in a)
 template <int KIND, int K>
 __device__ __forceinline__ void load_two(const StageIO& p, const int64_t (&idx)[K], double (&a)[K], double (&b)[K]) {
     load_raw_n(p.in[0], KIND == STAGE_ANY && (p.in_f32 & 1u), idx, a);
-    if (stage_two<KIND>(p)) load_raw_n(p.in[1], stage_second_f32<KIND>(p), idx, b);
+    if (stage_two<KIND>(p)) load_raw_n(p.in[1], stage_f32<KIND>(p, 1), idx, b);
 }
 
 template <int KIND, int K>
@@ -298,18 +306,18 @@ __device__ __forceinline__ void mix_first(const StageIO& p, double (&a)[K], cons
     }
 #pragma unroll
     for (int k = 0; k < K; ++k) a[k] = p.coef[0] * a[k];
-    if (stage_two<KIND>(p)) add_raw_n(p.coef[1], b, stage_second_f32<KIND>(p), a);
+    if (stage_two<KIND>(p)) add_raw_n(p.coef[1], b, stage_f32<KIND>(p, 1), a);
 }
 
 // and any further inputs, one by one
 template <int KIND, int K>
 __device__ __forceinline__ void mix_two(const StageIO& p, const int64_t (&idx)[K], double (&a)[K], double (&b)[K]) {
     mix_first<KIND>(p, a, b);
-    if (KIND == STAGE_ANY) {
+    if constexpr (stage_more<KIND>()) {
 #pragma unroll 1
         for (int i = 2; i < p.n_in; ++i) {
-            load_raw_n(p.in[i], (p.in_f32 >> i) & 1u, idx, b);
-            add_raw_n(p.coef[i], b, (p.in_f32 >> i) & 1u, a);
+            load_raw_n(p.in[i], stage_f32<KIND>(p, i), idx, b);
+            add_raw_n(p.coef[i], b, stage_f32<KIND>(p, i), a);
         }
     }
 }

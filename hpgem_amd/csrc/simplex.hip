@@ -1160,11 +1160,13 @@ SimplexParams simplex_params(hgdg_ctx* c, const StageIO& io) {
 using SimplexKernel = void (*)(SimplexParams);
 
 void launch_simplex(hgdg_ctx* c, const SimplexParams& p) {
-    static constexpr SimplexKernel kernels[4][2] = {
+    static constexpr SimplexKernel kernels[6][2] = {
         {&simplex_acoustic_rhs<STAGE_ANY, false>, &simplex_acoustic_rhs<STAGE_ANY, true>},
         {&simplex_acoustic_rhs<STAGE_ONE, false>, &simplex_acoustic_rhs<STAGE_ONE, true>},
         {&simplex_acoustic_rhs<STAGE_TWO, false>, &simplex_acoustic_rhs<STAGE_TWO, true>},
-        {&simplex_acoustic_rhs<STAGE_TWO_MIXED, false>, &simplex_acoustic_rhs<STAGE_TWO_MIXED, true>}};
+        {&simplex_acoustic_rhs<STAGE_TWO_MIXED, false>, &simplex_acoustic_rhs<STAGE_TWO_MIXED, true>},
+        {&simplex_acoustic_rhs<STAGE_ANY, false>, &simplex_acoustic_rhs<STAGE_ANY, true>},
+        {&simplex_acoustic_rhs<STAGE_ANY, false>, &simplex_acoustic_rhs<STAGE_ANY, true>}};
     const int64_t grid = c->sm.n_blocks;
     if (grid > 0)
         hipLaunchKernelGGL(kernels[stage_kind(p.io)][p.io.upd.u != nullptr], dim3(unsigned(grid)), dim3(kBlock), 0,

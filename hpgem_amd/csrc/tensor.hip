@@ -134,7 +134,7 @@ template <int NR, int N1, int KIND = STAGE_ANY>
 __device__ __forceinline__ void load_pencils(const StageIO& p, int64_t base, int64_t stride, double (&u)[NR][N1],
                                              double (&x)[NR][N1]) {
     load_raw<NR, N1>(p.in[0], KIND == STAGE_ANY && (p.in_f32 & 1u), base, stride, u);
-    if (stage_two<KIND>(p)) load_raw<NR, N1>(p.in[1], stage_second_f32<KIND>(p), base, stride, x);
+    if (stage_two<KIND>(p)) load_raw<NR, N1>(p.in[1], stage_f32<KIND>(p, 1), base, stride, x);
 }
 
 template <int NR, int N1, int KIND = STAGE_ANY>
@@ -144,18 +144,19 @@ __device__ __forceinline__ void mix_two_pencils(const StageIO& p, double (&u)[NR
     for (int r = 0; r < NR; ++r)
 #pragma unroll
         for (int a = 0; a < N1; ++a) u[r][a] = p.coef[0] * raw_value(u[r][a], u32);
-    if (stage_two<KIND>(p)) add_raw<NR, N1>(p.coef[1], x, stage_second_f32<KIND>(p), u);
+    if (stage_two<KIND>(p)) add_raw<NR, N1>(p.coef[1], x, stage_f32<KIND>(p, 1), u);
 }
 
 template <int NR, int N1, int KIND = STAGE_ANY>
 __device__ __forceinline__ void mix_pencils(const StageIO& p, int64_t base, int64_t stride, double (&u)[NR][N1],
                                             double (&x)[NR][N1]) {
     mix_two_pencils<NR, N1, KIND>(p, u, x);
-    if (KIND != STAGE_ANY) return;
+    if constexpr (stage_more<KIND>()) {
 #pragma unroll 1
-    for (int i = 2; i < p.n_in; ++i) {
-        load_raw<NR, N1>(p.in[i], (p.in_f32 >> i) & 1u, base, stride, x);
-        add_raw<NR, N1>(p.coef[i], x, (p.in_f32 >> i) & 1u, u);
+        for (int i = 2; i < p.n_in; ++i) {
+            load_raw<NR, N1>(p.in[i], stage_f32<KIND>(p, i), base, stride, x);
+            add_raw<NR, N1>(p.coef[i], x, stage_f32<KIND>(p, i), u);
+        }
     }
 }
 
@@ -438,38 +439,38 @@ __device__ __forceinline__ void advection_tiles(const RhsParams& p, int64_t t0, 
                 mix_two_pencils<1, 1, KIND>(p.io, v, v1);
                 ox[s] = v[0][0];
             }
-        if constexpr (KIND == STAGE_ANY) {
+        constexpr int kStep = 2;
+        if constexpr (stage_more<KIND>()) {
 #pragma unroll 1
-            for (int i = 2; i < p.io.n_in; i += 2) {
-                const bool two = i + 1 < p.io.n_in;
-                const int i1 = two ? i + 1 : i;
-                const double c[2] = {p.io.coef[i], p.io.coef[i1]};
-                const bool f[2] = {((p.io.in_f32 >> i) & 1u) != 0, ((p.io.in_f32 >> i1) & 1u) != 0};
-                const void* in[2] = {p.io.in[i], p.io.in[i1]};
-                double a[2][1][N1], b[2][NI][1][N1], g[2][2][1][1];
+            for (int i = 2; i < p.io.n_in; i += kStep) {
+                double a[kStep][1][N1], b[kStep][NI][1][N1], g[kStep][2][1][1];
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (h == 1 && !two) break;
-                    load_raw<1, N1>(in[h], f[h], base, 0, a[h]);
+                for (int h = 0; h < kStep; ++h) {
+                    if (h > 0 && i + h >= p.io.n_in) break;
+                    const void* in = p.io.in[i + h];
+                    const bool f = stage_f32<KIND>(p.io, i + h);
+                    load_raw<1, N1>(in, f, base, 0, a[h]);
 #pragma unroll
                     for (int k = 0; k < NI; ++k)
-                        if (item(k)) load_raw<1, N1>(in[h], f[h], at[k], 0, b[h][k]);
+                        if (item(k)) load_raw<1, N1>(in, f, at[k], 0, b[h][k]);
 #pragma unroll
                     for (int s = 0; s < 2; ++s)
-                        if (lx[s] < 0) load_raw<1, 1>(in[h], f[h], atx[s], 0, g[h][s]);
+                        if (lx[s] < 0) load_raw<1, 1>(in, f, atx[s], 0, g[h][s]);
                 }
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (h == 1 && !two) break;
-                    add_raw<1, N1>(c[h], a[h], f[h], l.w);
+                for (int h = 0; h < kStep; ++h) {
+                    if (h > 0 && i + h >= p.io.n_in) break;
+                    const double c = p.io.coef[i + h];
+                    const bool f = stage_f32<KIND>(p.io, i + h);
+                    add_raw<1, N1>(c, a[h], f, l.w);
 #pragma unroll
                     for (int k = 0; k < NI; ++k)
-                        if (item(k)) add_raw<1, N1>(c[h], b[h][k], f[h], o[k]);
+                        if (item(k)) add_raw<1, N1>(c, b[h][k], f, o[k]);
 #pragma unroll
                     for (int s = 0; s < 2; ++s)
                         if (lx[s] < 0) {
                             double v[1][1] = {{ox[s]}};
-                            add_raw<1, 1>(c[h], g[h][s], f[h], v);
+                            add_raw<1, 1>(c, g[h][s], f, v);
                             ox[s] = v[0][0];
                         }
                 }
@@ -1898,12 +1899,20 @@ static RhsParams advection_params(hgdg_ctx* c, const StageIO& io) {
     return p;
 }
 
-template <typename F>
+// MANY: with kernels of their own for three and more inputs, as the stages of
+// Dormand-Prince have. By STAGE_ANY each of an input's loads asks for its type
+// and an FP32 value waits in two registers, which costs half the wavefronts:
+// 301 x 257 p = 3 with FP32 stages, 3, 5 and 7 inputs, 10.2, 15.0 and 19.8 us so
+// against 7.3, 9.4 and 11.6 (FP64 11.1, 14.9, 17.8 and 9.0, 12.8, 16.2); 600 x
+// 500 p = 5 82, 119 and 151 against 60, 85 and 107.
+template <bool MANY, typename F>
 static void with_stage_kind(const StageIO& io, F&& f) {
     switch (stage_kind(io)) {
         case STAGE_ONE: f(std::integral_constant<int, STAGE_ONE>{}); break;
         case STAGE_TWO: f(std::integral_constant<int, STAGE_TWO>{}); break;
         case STAGE_TWO_MIXED: f(std::integral_constant<int, STAGE_TWO_MIXED>{}); break;
+        case STAGE_MANY: f(std::integral_constant<int, MANY ? int(STAGE_MANY) : int(STAGE_ANY)>{}); break;
+        case STAGE_MANY_MIXED: f(std::integral_constant<int, MANY ? int(STAGE_MANY_MIXED) : int(STAGE_ANY)>{}); break;
         default: f(std::integral_constant<int, STAGE_ANY>{}); break;
     }
 }
@@ -1914,7 +1923,7 @@ static void launch_advection(hgdg_ctx* c, const RhsParams& p, int tiles) {
         using S = Pencil<DIMc, N1c>;
         const int64_t n_tiles = (c->n_elem + S::EPB - 1) / S::EPB;
         const bool upd = p.io.upd.u != nullptr;  // the fused RK update runs in the one-tile kernel
-        with_stage_kind(p.io, [&](auto K) {
+        with_stage_kind<true>(p.io, [&](auto K) {
             constexpr int KIND = decltype(K)::value;
             if (upd)
                 hipLaunchKernelGGL((tensor_advection_rhs<DIMc, N1c, KIND, true>), dim3(unsigned(n_tiles)),
@@ -2104,7 +2113,7 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
             constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
             using S = AcousticShape<DIMc, N1c>;
             const int64_t grid = (c->n_elem + S::EPB - 1) / S::EPB;
-            with_stage_kind(io, [&](auto K) {
+            with_stage_kind<false>(io, [&](auto K) {
                 // the update at 3D p = 3 is the one form that needs more registers
                 // by its kind (280 against 225: one wavefront a SIMD instead of two)
                 constexpr int KIND = decltype(K)::value, KU = DIMc == 3 && N1c == 4 ? int(STAGE_ANY) : KIND;
