@@ -120,6 +120,7 @@ struct hgdg_ctx {
     hipGraph_t graph2 = nullptr;
     hipGraphExec_t graph2_exec = nullptr;
     hgdg::DevBuf<double> u_spare;
+    hgdg::DevBuf<double> stage_sum;  // [n_dof] a stage's input, where the RHS kernel is given it ready (sum_stage)
     int64_t rk_pair_launches = 0;
     double dt_estimate = 0;  // adaptive stepping: next step size (0 = not started)
     double last_kernel_ms = 0;  // duration of the last assembly kernel (HIP events)

@@ -334,6 +334,7 @@ void mesh_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     c->has_mesh = false;
     c->has_op = false;
     c->vecs.clear();
+    c->stage_sum.reset();
     c->shape = m->shape;
     c->dim = dim;
     c->n_elem = m->n_elements;
@@ -368,7 +369,10 @@ void operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
     c->drop_graph();
     if (c->simplex()) simplex_tune(c);
     else tensor_tune(c);
-    if (old_fields != c->n_fields) c->vecs.clear();  // the field count changed the vector size
+    if (old_fields != c->n_fields) {  // the field count changed the vector size
+        c->vecs.clear();
+        c->stage_sum.reset();
+    }
 }
 
 StageIO make_io(hgdg_ctx* c, const int* in_ids, const double* coeffs, int n_in, int out_id) {
@@ -389,7 +393,88 @@ StageIO make_io(hgdg_ctx* c, const int* in_ids, const double* coeffs, int n_in, 
     return io;
 }
 
-void dispatch_rhs(hgdg_ctx* c, const StageIO& io) {
+// ---- stages of three and more inputs ----------------------------------------
+// The input sum_i coef_i in_i of a stage, once for every value (combine()'s
+// sums, all inputs' loads in flight together).
+struct SumParams {
+    StageIO io;
+    double* sum;
+    int64_t n;
+};
+
+__global__ __launch_bounds__(kBlock) void sum_inputs(const SumParams p) {
+    const int64_t i = 2 * (int64_t(blockIdx.x) * kBlock + threadIdx.x);
+    if (i >= p.n) return;
+    if (i + 1 == p.n) {
+        p.sum[i] = combine(p.io, i);
+        return;
+    }
+    double x[kMaxIn][2];
+#pragma unroll
+    for (int j = 0; j < kMaxIn; ++j) {
+        if (j >= p.io.n_in) break;
+        if ((p.io.in_f32 >> j) & 1u) load_run<2>(static_cast<const float*>(p.io.in[j]) + i, x[j]);
+        else load_run<2>(static_cast<const double*>(p.io.in[j]) + i, x[j]);
+    }
+    double s[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) s[a] = p.io.coef[0] * x[0][a];
+#pragma unroll
+    for (int j = 1; j < kMaxIn; ++j) {
+        if (j >= p.io.n_in) break;
+#pragma unroll
+        for (int a = 0; a < 2; ++a) s[a] = fma(p.io.coef[j], x[j][a], s[a]);
+    }
+    *reinterpret_cast<double2*>(p.sum + i) = make_double2(s[0], s[1]);
+}
+
+// On tetrahedra, whose kernel gathers values here and there, a further input
+// costs more than a pass over memory that sums it in: 20^3 x 5 of order 1..4,
+// 3, 5 and 7 inputs, FP64 75, 94 and 115 us in the kernel and 54, 61 and 68
+// summed first; FP32 stages 73, 87 and 101 against 52, 57 and 59 (2^3 x 5
+// 10.8, 11.6 and 12.6 against 9.9, 10.0 and 10.1). But for small meshes of
+// order 1, where the launch costs more than it saves: 6^3 x 5 7.2, 8.2 and 9.2
+// against 8.1, 9.0 and 9.2 us; 13x11x9 x 5 (103000 values) 12.5 against 9.7.
+bool sums_stages(const hgdg_ctx* c) {
+    return c->simplex() && (c->sm.group_start[1] < c->n_elem || c->n_dof() >= 65536);
+}
+
+// The vector for it, kept for the next stage. None while the stream is being
+// captured or where the memory does not suffice: the RHS kernels then sum.
+bool stage_space(hgdg_ctx* c) {
+    const size_t n = size_t(c->n_dof());
+    if (c->stage_sum.n == n) return true;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    try {
+        c->stage_sum.alloc(n);
+    } catch (const Failure&) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+// io with its inputs summed into one, if it has three or more and the RHS
+// kernel is better off so.
+StageIO sum_stage(hgdg_ctx* c, const StageIO& io) {
+    if (io.n_in < 3 || !sums_stages(c) || !stage_space(c)) return io;
+    const SumParams p{io, c->stage_sum.ptr, c->n_dof()};
+    hipLaunchKernelGGL(sum_inputs, dim3(unsigned((p.n + 2 * kBlock - 1) / (2 * kBlock))), dim3(kBlock), 0, c->stream, p);
+    HGDG_HIP(hipGetLastError());
+    StageIO one = io;
+    one.n_in = 1;
+    one.in[0] = p.sum;
+    one.coef[0] = 1.0;
+    one.in_f32 = 0;
+    return one;
+}
+
+void dispatch_rhs(hgdg_ctx* c, const StageIO& stage) {
+    const StageIO io = sum_stage(c, stage);
     if (c->matrix()) matrix_rhs(c, io, true);
     else if (c->simplex()) simplex_rhs(c, io);
     else tensor_rhs(c, io);
@@ -503,6 +588,9 @@ void rk_steps(hgdg_ctx* c, int solution, const int* aux, int stages, const doubl
     require(n_steps >= 0, HGDG_ERR_ARG, "negative step count");
     check_rk_args(c, solution, aux, stages);
     if (tensor_rk_tiny(c, solution, aux, stages, a, b, dt, n_steps)) return;
+    // a stage that is summed first needs its vector before the capture below
+    for (int i = 0; i < stages && sums_stages(c); ++i)
+        if (i - std::count(a + i * stages, a + i * stages + i, 0.0) >= 2) (void)stage_space(c);
     GraphKey key{solution, std::vector<int>(aux, aux + stages), std::vector<double>(a, a + stages * stages),
                  std::vector<double>(b, b + stages), dt};
     if (c->rk_fused != 0 && rhs_fuses_update(c) && n_steps >= 2) {
