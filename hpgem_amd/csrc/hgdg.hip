@@ -435,8 +435,15 @@ __global__ __launch_bounds__(kBlock) void sum_inputs(const SumParams p) {
 // 10.8, 11.6 and 12.6 against 9.9, 10.0 and 10.1). But for small meshes of
 // order 1, where the launch costs more than it saves: 6^3 x 5 7.2, 8.2 and 9.2
 // against 8.1, 9.0 and 9.2 us; 13x11x9 x 5 (103000 values) 12.5 against 9.7.
-bool sums_stages(const hgdg_ctx* c) {
-    return c->simplex() && (c->sm.group_start[1] < c->n_elem || c->n_dof() >= 65536);
+// Acoustics on cubes of order 5 have no registers for many inputs: 6x7x5, 4, 5
+// and 7 inputs, 11.1, 12.3 and 18.0 us in the kernel and 11.2, 11.2 and 11.4
+// summed first (24^3 168, 199 and 262 against 158, 181 and 220); FP32 stages, 5
+// and 7, 10.8 and 12.4 against 11.6 and 11.9.
+bool sums_stages(const hgdg_ctx* c, int n_in) {
+    if (n_in < 3 || c->matrix() || c->op.kind != HGDG_OP_ACOUSTIC_CENTRAL) return false;
+    if (c->simplex()) return c->sm.group_start[1] < c->n_elem || c->n_dof() >= 65536;
+    return !c->tm.general && c->dim == 3 && c->tm.p == 5 &&
+           n_in >= (c->op.precision == HGDG_PREC_MIXED_FP32 ? 6 : 5);
 }
 
 // The vector for it, kept for the next stage. None while the stream is being
@@ -458,10 +465,9 @@ bool stage_space(hgdg_ctx* c) {
     return true;
 }
 
-// io with its inputs summed into one, if it has three or more and the RHS
-// kernel is better off so.
+// io with its inputs summed into one where the RHS kernel is better off so.
 StageIO sum_stage(hgdg_ctx* c, const StageIO& io) {
-    if (io.n_in < 3 || !sums_stages(c) || !stage_space(c)) return io;
+    if (!sums_stages(c, io.n_in) || !stage_space(c)) return io;
     const SumParams p{io, c->stage_sum.ptr, c->n_dof()};
     hipLaunchKernelGGL(sum_inputs, dim3(unsigned((p.n + 2 * kBlock - 1) / (2 * kBlock))), dim3(kBlock), 0, c->stream, p);
     HGDG_HIP(hipGetLastError());
@@ -589,8 +595,8 @@ void rk_steps(hgdg_ctx* c, int solution, const int* aux, int stages, const doubl
     check_rk_args(c, solution, aux, stages);
     if (tensor_rk_tiny(c, solution, aux, stages, a, b, dt, n_steps)) return;
     // a stage that is summed first needs its vector before the capture below
-    for (int i = 0; i < stages && sums_stages(c); ++i)
-        if (i - std::count(a + i * stages, a + i * stages + i, 0.0) >= 2) (void)stage_space(c);
+    for (int i = 0; i < stages; ++i)
+        if (sums_stages(c, 1 + i - int(std::count(a + i * stages, a + i * stages + i, 0.0)))) (void)stage_space(c);
     GraphKey key{solution, std::vector<int>(aux, aux + stages), std::vector<double>(a, a + stages * stages),
                  std::vector<double>(b, b + stages), dt};
     if (c->rk_fused != 0 && rhs_fuses_update(c) && n_steps >= 2) {

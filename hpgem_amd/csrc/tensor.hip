@@ -878,6 +878,13 @@ struct AcousticParams {
 // the own ones, one memory round trip less (32^3 p = 3 53 -> 47 us, 256^2
 // p = 3 20.1 -> 17.7); at orders 4 and 5 in 3D, and with the update's terms
 // held too, its registers cost as much as that gains (20^3 p = 5 60 -> 64 us).
+// kTogether: of stages of three and more inputs, each is read at once for all
+// that is loaded here, and for the x faces: one memory round trip for it, where
+// pencils and faces summing their inputs each for itself take up to five. us
+// with 3, 5 and 7 inputs by STAGE_ANY and so: 6x7x5 p = 1 6.1, 8.4 and 10.6,
+// 6.0, 6.2 and 6.7; p = 2 6.9, 9.4 and 11.9, 6.1, 6.8 and 8.0; 40x30 p = 4 6.4,
+// 8.3 and 10.3, 6.0, 6.2 and 6.6; 24^3 p = 3 34.8, 59.5 and 84.9, 33.8, 47.9 and
+// 63.8. (At order 5 in 3D a SIMD has one wavefront in any case: kAhead there too.)
 // kEarly: all of the update's sum but the own term is formed before the
 // volume terms, from u and k as they are loaded anyway (RK4 step of 30^3 p = 2
 // 107 -> 103 us, 256^2 p = 1 34.8 -> 32.3); at orders 4 and 5 the 4 N1 sums do
@@ -921,11 +928,23 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
     // ---- own pencil of every field; g_r
     // (kAhead: and the neighbour's pencils of the first face pencil: all loads of
     // both are in flight before any is used)
-    constexpr bool kAhead = !UPD && (DIM == 2 || N1 <= 4);
+    constexpr bool kTogether = (KIND == STAGE_MANY || KIND == STAGE_MANY_MIXED) && !UPD;
+    constexpr bool kAhead = !UPD && (DIM == 2 || N1 <= 4 || (kTogether && N1 == 6));
     double w[NF][N1], J[DIM][DIM], wq[NF][N1];
     constexpr bool kEarly = UPD && N1 <= 4;
     double y[NF][N1];  // kEarly: the update's sum but for this stage's own term
     int32_t nbx[2] = {-1, -1}, nbq = -1;
+    // x faces: a neighbour whose pencil lies in this wavefront (lane srcx) hands
+    // its values over by a lane shuffle, another one's are loaded from atx on
+    auto x_face = [&](int s, int& src, int64_t (&at)[NF]) {
+        const int64_t ln = int64_t(nbx[s]) - blk * S::EPB;
+        const bool here = ln >= 0 && ln < S::EPB && (int(ln) * NP + pc) / 64 == tid / 64;
+        src = here ? (int(ln) * NP + pc) % 64 : tid % 64;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) at[f] = (int64_t(nbx[s]) * NF + f) * NB + pc * N1 + (1 - s);
+        return active && nbx[s] >= 0 && !here;
+    };
+    double ox[2][NF];
     if (active) {
         if (pc < NQ) nbq = p.nbr[(2 + (DIM == 3 ? pc / N1 : pc)) * p.n_elem + e];
 #pragma unroll
@@ -937,7 +956,40 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
         double x[NF][N1];
         load_pencils<NF, N1, KIND>(p.io, base + pc * N1, NB, w, x);
         if constexpr (kEarly) update_partial<NF, N1>(p.io, base + pc * N1, NB, w, x, y);
-        if constexpr (kAhead) {
+        if constexpr (kTogether) {
+            double xq[NF][N1], x1[2][NF];
+            const int64_t bq = face_pencil(pc, nbq);
+            const bool ahead = kAhead && nbq >= 0;
+            bool far[2];
+            int src[2];
+            int64_t at[2][NF];
+            if (ahead) load_pencils<NF, N1, KIND>(p.io, bq, NB, wq, xq);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                far[s] = x_face(s, src[s], at[s]);
+                if (far[s]) load_two<KIND>(p.io, at[s], ox[s], x1[s]);
+            }
+            mix_two_pencils<NF, N1, KIND>(p.io, w, x);
+            if (ahead) mix_two_pencils<NF, N1, KIND>(p.io, wq, xq);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                if (far[s]) mix_first<KIND>(p.io, ox[s], x1[s]);
+#pragma unroll 1
+            for (int i = 2; i < p.io.n_in; ++i) {
+                const bool f32 = stage_f32<KIND>(p.io, i);
+                const double c = p.io.coef[i];
+                load_raw<NF, N1>(p.io.in[i], f32, base + pc * N1, NB, x);
+                if (ahead) load_raw<NF, N1>(p.io.in[i], f32, bq, NB, xq);
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                    if (far[s]) load_raw_n(p.io.in[i], f32, at[s], x1[s]);
+                add_raw<NF, N1>(c, x, f32, w);
+                if (ahead) add_raw<NF, N1>(c, xq, f32, wq);
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                    if (far[s]) add_raw_n(c, x1[s], f32, ox[s]);
+            }
+        } else if constexpr (kAhead) {
             double xq[NF][N1];
             const int64_t bq = face_pencil(pc, nbq);
             if (nbq >= 0) load_pencils<NF, N1, KIND>(p.io, bq, NB, wq, xq);
@@ -977,23 +1029,22 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
         for (int a = 0; a < N1; ++a) s_v[le * S::ES + row(ib, ic) + a] = w[0][a];
     }
 
-    // ---- x faces: one trace value per pencil; a neighbour whose pencil lies
-    // in this wavefront hands it over by a lane shuffle
+    // ---- x faces: one trace value per pencil
     double fvx[2], fsx[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        const int64_t ln = int64_t(nbx[s]) - blk * S::EPB;
-        const bool here = ln >= 0 && ln < S::EPB && (int(ln) * NP + pc) / 64 == tid / 64;
-        const int src = here ? (int(ln) * NP + pc) % 64 : tid % 64;
+        int src;
+        int64_t at[NF];
+        const bool far = x_face(s, src, at);
         double o[NF];
 #pragma unroll
         for (int f = 0; f < NF; ++f) o[f] = __shfl(w[f][1 - s], src, 64);
         fvx[s] = fsx[s] = 0.0;
         if (active && nbx[s] >= 0) {
-            if (!here) {
-                int64_t at[NF];
+            if constexpr (kTogether) {
 #pragma unroll
-                for (int f = 0; f < NF; ++f) at[f] = (int64_t(nbx[s]) * NF + f) * NB + pc * N1 + (1 - s);
+                for (int f = 0; f < NF; ++f) o[f] = far ? ox[s][f] : o[f];
+            } else if (far) {
                 double x[NF];
                 load_two<KIND>(p.io, at, o, x);
                 mix_two<KIND>(p.io, at, o, x);
@@ -2091,6 +2142,10 @@ static AcousticParams acoustic_params(hgdg_ctx* c, const StageIO& io) {
 // hgdg_right_hand_side in one launch, where there is a kernel for it.
 bool tensor_weak_rhs(hgdg_ctx* c, const StageIO& io) {
     if (c->tm.general || c->op.kind != HGDG_OP_ACOUSTIC_CENTRAL) return false;
+    // few cubes of order 5: the passes of the mass, one after another in a few
+    // workgroups, take longer than another launch (6x7x5 14.9 us against 11.4,
+    // 12^3 19.5 against 19.8)
+    if (c->dim == 3 && c->tm.p == 5 && c->n_elem < 1024) return false;
     const AcousticParams a = acoustic_params(c, io);
     dispatch_tensor(c->dim, c->tm.n1, [&](auto D, auto N) {
         constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
@@ -2113,7 +2168,7 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
             constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
             using S = AcousticShape<DIMc, N1c>;
             const int64_t grid = (c->n_elem + S::EPB - 1) / S::EPB;
-            with_stage_kind<false>(io, [&](auto K) {
+            auto launch = [&](auto K) {
                 // the update at 3D p = 3 is the one form that needs more registers
                 // by its kind (280 against 225: one wavefront a SIMD instead of two)
                 constexpr int KIND = decltype(K)::value, KU = DIMc == 3 && N1c == 4 ? int(STAGE_ANY) : KIND;
@@ -2123,7 +2178,14 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
                 else
                     hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, KIND, false>), dim3(unsigned(grid)),
                                        dim3(S::THREADS), 0, c->stream, a);
-            });
+            };
+            // kTogether's registers at 3D p = 2 (177 against 164) leave two
+            // wavefronts a SIMD instead of three, which costs large boxes more
+            // than one further input gains (40^3 76 against 70 us; 24^3 the same)
+            const bool any = io.upd.u != nullptr ||
+                             (DIMc == 3 && N1c == 3 && io.n_in == 3 && c->n_elem > 30 * 30 * 30);
+            if (any) with_stage_kind<false>(io, launch);
+            else with_stage_kind<true>(io, launch);
         });
         HGDG_HIP(hipGetLastError());
         return;

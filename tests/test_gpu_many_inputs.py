@@ -5,6 +5,8 @@ here in long double and rounded once: each of at most eight sums rounds by at
 most eps/2 of a partial sum of at most 6 max|v|, on the way through an operator
 that is linear, so the results differ by at most ~10 eps times the amplification
 that |w| -> |k| already has, below 1e-12 of the largest value."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -109,3 +111,32 @@ def test_steps_of_many_stages(tets, p, precision):
     for other in out[1:]:
         for g, f in zip(out[0], other):
             np.testing.assert_array_equal(f, g)
+
+
+@pytest.mark.parametrize("tets,p", [(True, 0), (False, 2), (False, 5)])
+def test_captured_before_any_other_call(tets, p):
+    """A stage of five inputs captured as the first call of its kind, when no
+    vector for its sum can be allocated: the kernels sum by themselves, and every
+    replay gives what the call gives outside."""
+    print(f"[case] many inputs captured tets={tets} p={p}", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+    mesh = Mesh.structured([4, 3, 3], simplices=tets)
+    rng = np.random.default_rng(p)
+    order = rng.integers(1, 5, mesh.n_elements).astype(np.int32) if tets else p
+    dev = HpgemAPIDevice(mesh, order, kind=OP_ACOUSTIC_CENTRAL, c_inv=rng.uniform(0.5, 2.0, mesh.n_elements), tableau=RK4,
+                         n_extra_vectors=2)
+    graph, run, stream = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p(dev.stream())
+    for v in range(5):
+        dev.setTimeIntegrationVector(v, rng.standard_normal(dev.n_dof))
+    ids, co = list(range(5)), COEFFICIENTS[:5]
+    assert hip.hipStreamBeginCapture(stream, 0) == 0
+    dev.computeTimeDerivative(ids, co, 5)
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+    for _ in range(3):
+        dev.setTimeIntegrationVector(1, rng.standard_normal(dev.n_dof))
+        dev.computeTimeDerivative(ids, co, 6)
+        assert hip.hipGraphLaunch(run, stream) == 0
+        np.testing.assert_array_equal(dev.getTimeIntegrationVector(5), dev.getTimeIntegrationVector(6))
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    dev.close()
