@@ -52,6 +52,7 @@ struct MatParams {
 // a += sum over this thread's columns j = g, g + G, .. < nc of B[i + n j] x[j],
 // B column-major with n rows: consecutive threads (i fast, g slow) read
 // consecutive values.
+template <bool STREAM>
 __device__ __forceinline__ double mat_columns(const double* __restrict__ B, int n, int i, int g, int G, int nc,
                                               const double* x, double a) {
     for (int j0 = g; j0 < nc; j0 += kMatAhead * G) {
@@ -59,7 +60,8 @@ __device__ __forceinline__ double mat_columns(const double* __restrict__ B, int 
 #pragma unroll
         for (int u = 0; u < kMatAhead; ++u) {
             const int j = j0 + u * G;
-            b[u] = j < nc ? __builtin_nontemporal_load(B + (i + int64_t(n) * j)) : 0.0;
+            const double* at = B + (i + int64_t(n) * j);
+            b[u] = j < nc ? (STREAM ? __builtin_nontemporal_load(at) : *at) : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < kMatAhead; ++u) {
@@ -78,16 +80,16 @@ __device__ __forceinline__ double mat_columns(const double* __restrict__ B, int 
 // each, so that every thread streams matrix values and consecutive threads
 // read consecutive ones; the G partial sums of a row meet in LDS. With n > T a
 // thread takes up to four rows of every column.
-// Bound by HBM: every matrix value is read once, with eight loads in flight per
-// thread (non-temporal: nothing of a matrix is read twice). One block at a time
-// behind its own barriers, with n threads of 256, read 1.8 TB/s at n = 27 and
-// 7 blocks a row (5760 elements, 268 MB: 148 us); this form takes 47 us, 5.7
-// TB/s (n = 8: 51 -> 8 us; n = 64, 1680 elements: 151 -> 75).
-template <int T>
+// Bound by memory: every matrix value is read once a launch, with eight loads in
+// flight per thread. One block at a time behind its own barriers, with n threads
+// of 256, read 1.8 TB/s at n = 27 and 7 blocks a row (5760 elements, 268 MB: 148
+// us); this form takes 47 us, 5.7 TB/s (n = 8: 51 -> 8 us; n = 64, 1680 elements:
+// 151 -> 75). STREAM: non-temporal loads, see the launch.
+template <int T, bool STREAM>
 __global__ __launch_bounds__(T) void matrix_rhs(const MatParams p) {
     extern __shared__ double sh[];
     double* red = sh + p.cols;  // [max(T, n)]
-    constexpr int R = T == kMatThreads ? kMatMaxRows / T : 1;  // smaller workgroups only take n <= T
+    constexpr int R = T >= kMatThreads ? kMatMaxRows / T : 1;  // smaller workgroups only take n <= T
     const int64_t e = xcd_block(blockIdx.x, gridDim.x);
     const int64_t o = p.elem_off[e];
     const int n = int(p.elem_off[e + 1] - o);
@@ -104,11 +106,11 @@ __global__ __launch_bounds__(T) void matrix_rhs(const MatParams p) {
         __syncthreads();
         const double* Bj = B + int64_t(n) * j0;
         if (narrow) {
-            if (g < G) acc[0] = mat_columns(Bj, n, i, g, G, m, sh, acc[0]);
+            if (g < G) acc[0] = mat_columns<STREAM>(Bj, n, i, g, G, m, sh, acc[0]);
         } else {
 #pragma unroll
             for (int s = 0; s < R; ++s)
-                if (t + s * T < n) acc[s] = mat_columns(Bj, n, t + s * T, 0, 1, m, sh, acc[s]);
+                if (t + s * T < n) acc[s] = mat_columns<STREAM>(Bj, n, t + s * T, 0, 1, m, sh, acc[s]);
         }
     }
     // the partial sums of a row; afterwards thread t (+ s T) holds row t (+ s T)
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(T) void matrix_rhs(const MatParams p) {
             if (t < n) sh[t] = acc[0];  // every reader of the stage passed gather()'s barrier
             __syncthreads();
             acc[0] = 0.0;
-            if (g < G) acc[0] = mat_columns(Mi, n, i, g, G, n, sh, 0.0);
+            if (g < G) acc[0] = mat_columns<STREAM>(Mi, n, i, g, G, n, sh, 0.0);
             gather();
         } else {
 #pragma unroll
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(T) void matrix_rhs(const MatParams p) {
             __syncthreads();
 #pragma unroll
             for (int s = 0; s < R; ++s)
-                if (t + s * T < n) acc[s] = mat_columns(Mi, n, t + s * T, 0, 1, n, red, 0.0);
+                if (t + s * T < n) acc[s] = mat_columns<STREAM>(Mi, n, t + s * T, 0, 1, n, red, 0.0);
         }
     }
 #pragma unroll
@@ -373,19 +375,33 @@ void matrix_rhs(hgdg_ctx* c, const StageIO& io, bool solve) {
     p.sq_off = c->mat.d_sq_off.ptr;
     p.minv = solve ? c->mat.d_minv.ptr : nullptr;
     p.cols = int32_t(std::max<int64_t>(std::min<int64_t>(c->mat.max_cols, kMatCols), c->mat.max_rows));
-    auto launch = [&](auto T_) {
+    auto launch = [&](auto T_, auto S_) {
         constexpr int T = decltype(T_)::value;
         const size_t lds = sizeof(double) * size_t(p.cols + std::max(T, c->mat.max_rows));
-        hipLaunchKernelGGL((matrix_rhs<T>), dim3(unsigned(c->n_elem)), dim3(T), lds, c->stream, p);
+        hipLaunchKernelGGL((matrix_rhs<T, decltype(S_)::value>), dim3(unsigned(c->n_elem)), dim3(T), lds, c->stream, p);
     };
-    // By the largest block: a workgroup of 64 threads keeps more element rows
-    // in flight where they are short (5760 elements of n = 10: 11.8, 13.9 and
-    // 22.6 us with 64, 128 and 256 threads; n = 27: 47.4, 49.3, 47.9), 128 is
-    // best from there (1680 elements of n = 40: 33.3, 30.3, 33.5; n = 64 alike);
-    // beyond 128 rows the widest form has the most threads on rows.
-    if (c->mat.max_rows <= 32) launch(std::integral_constant<int, 64>{});
-    else if (c->mat.max_rows <= 128) launch(std::integral_constant<int, 128>{});
-    else launch(std::integral_constant<int, kMatThreads>{});
+    // Threads of an element row: 64, 128 or 256 by its rows (5760 elements of n =
+    // 10: 11.8, 13.9 and 22.6 us with 64, 128 and 256 threads; n = 27: 47.4, 49.3,
+    // 47.9; 1680 of n = 40: 33.3, 30.3, 33.5; beyond 128 rows the most threads on
+    // rows). More where few elements leave the chip idle, 2^17 threads in all, but
+    // kMatAhead matrix values for each at least (us with 64 or as many as rows, and so:
+    // 1728 of n = 27 20.8 and 16.0, 512 of n = 125 148 and 87, 216 of n = 64 33 and
+    // 13, 64 of n = 256 273 and 76, 27 of n = 400 754 and 234).
+    const int64_t fill = std::min<int64_t>((int64_t(1) << 17) / c->n_elem, c->mat.max_rows * c->mat.max_cols / kMatAhead);
+    int threads = c->mat.max_rows <= 32 ? 64 : c->mat.max_rows <= 128 ? 128 : kMatThreads;
+    while (threads < fill && threads < kMatMaxRows) threads *= 2;
+    auto go = [&](auto S_) {
+        if (threads == 64) launch(std::integral_constant<int, 64>{}, S_);
+        else if (threads == 128) launch(std::integral_constant<int, 128>{}, S_);
+        else if (threads == 256) launch(std::integral_constant<int, 256>{}, S_);
+        else if (threads == 512) launch(std::integral_constant<int, 512>{}, S_);
+        else launch(std::integral_constant<int, 1024>{}, S_);
+    };
+    // Matrices that the 256 MB cache holds from one stage to the next are read as
+    // usual, larger ones past it (us plain and non-temporal: 64 MB 22 and 28, 216 MB
+    // 34 and 38, 276 MB 234 and 240; 373 MB 75 and 65, 2.1 GB 362 and 319).
+    if ((c->mat.d_pool.n + c->mat.d_minv.n) * sizeof(double) > (size_t(5) << 26)) go(std::true_type{});
+    else go(std::false_type{});
     HGDG_HIP(hipGetLastError());
 }
 
