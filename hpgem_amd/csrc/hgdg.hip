@@ -10,17 +10,15 @@
 #include <sstream>
 #include <cmath>
 #include <cstring>
-#include <exception>
 #include <functional>
 #include <limits>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "context.hpp"
+#include "host_threads.hpp"
 #include "vtk_io.hpp"
 #include "mesh_io.hpp"
 
@@ -296,26 +294,7 @@ static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
         }
         if (done) (void)hipEventDestroy(done);
     };
-    std::vector<std::exception_ptr> failed(static_cast<size_t>(workers));
-    auto guarded = [&](int w) {
-        try {
-            work(w);
-        } catch (...) {
-            failed[size_t(w)] = std::current_exception();
-        }
-    };
-    std::vector<std::thread> threads;
-    threads.reserve(size_t(workers));
-    int started = 1;  // worker 0 is the calling thread
-    try {
-        for (; started < workers; ++started) threads.emplace_back(guarded, started);
-    } catch (const std::system_error&) {  // no more threads: this one does their chunks too
-    }
-    guarded(0);
-    for (int w = started; w < workers; ++w) guarded(w);
-    for (std::thread& t : threads) t.join();
-    for (const std::exception_ptr& f : failed)
-        if (f) std::rethrow_exception(f);
+    on_threads(workers, work);
 }
 
 void host_get(hgdg_ctx* c, Vec& v, double* host) { host_copy(c, v, host, nullptr); }
