@@ -153,7 +153,8 @@ struct PinnedChunk {
             }
         }
         void* p = nullptr;
-        HGDG_HIP(hipHostMalloc(&p, size_t(kChunk) * sizeof(double), hipHostMallocPortable));
+        // coherent whatever HIP_HOST_COHERENT says: the copies wait for events only
+        HGDG_HIP(hipHostMalloc(&p, size_t(kChunk) * sizeof(double), hipHostMallocPortable | hipHostMallocCoherent));
         ptr = static_cast<double*>(p);
     }
     ~PinnedChunk() {
