@@ -113,6 +113,11 @@ void set_storage(hgdg_ctx* c, Vec& v, bool f32) {
 constexpr int64_t kChunk = int64_t(1) << 18;  // doubles per chunk
 constexpr int kCopyThreads = 4;
 constexpr int64_t kThreadedFrom = int64_t(1) << 20;  // doubles: below, one thread is as fast
+// Between these bytes a plain copy is the fastest (us, set and get of 3072 values:
+// 11.7 and 11.3 against 15.2 and 14.5, of 5600 on tetrahedra 12.0 and 12.2 against
+// 17.1 and 15.8; of 10800 15.3 and 16.0 against 16.9 and 16.9; but of 1728 15.7 and
+// 22.1 against 15.3 and 14.2, of 19200 19.0 and 20.4 against 18.4 and 19.0).
+constexpr size_t kWholeFrom = size_t(16) << 10, kWholeTo = size_t(96) << 10;
 
 // The pinned chunks are the process's: allocating one takes about 0.3 ms, too
 // much for a context of its own small vectors. At most kPinnedKept are kept for
@@ -140,6 +145,7 @@ void pinned_user(int change) {
     pool.kept.clear();
 }
 
+struct NoPinnedChunk {};  // there is no pinned memory left
 struct PinnedChunk {
     double* ptr = nullptr;
     PinnedChunk() {
@@ -154,7 +160,10 @@ struct PinnedChunk {
         }
         void* p = nullptr;
         // coherent whatever HIP_HOST_COHERENT says: the copies wait for events only
-        HGDG_HIP(hipHostMalloc(&p, size_t(kChunk) * sizeof(double), hipHostMallocPortable | hipHostMallocCoherent));
+        if (hipHostMalloc(&p, size_t(kChunk) * sizeof(double), hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+            (void)hipGetLastError();
+            throw NoPinnedChunk();
+        }
         ptr = static_cast<double*>(p);
     }
     ~PinnedChunk() {
@@ -209,6 +218,34 @@ __global__ __launch_bounds__(kBlock) void host_copy_elements(const HostCopyParam
     for (int64_t i = threadIdx.x % 64; i < n; i += 64) host_copy_one(p, p.dev[e] + i, h - p.lo + i);
 }
 
+// One copy of the vector as it is stored, permuted (and converted) on the host.
+template <typename T>
+static void host_copy_whole(hgdg_ctx* c, Vec& v, double* out, const double* in) {
+    std::vector<T> dev(static_cast<size_t>(c->n_dof()));
+    auto each = [&](auto&& f) {  // f(position in hpGEM's layout, position in v)
+        if (c->simplex()) {
+            for (size_t e = 0; e + 1 < c->sm.host_off.size(); ++e) {
+                const int64_t h = c->sm.host_off[e], d = c->sm.dof_off[size_t(c->sm.dev_of[e])];
+                for (int64_t i = 0; i < c->sm.host_off[e + 1] - h; ++i) f(h + i, d + i);
+            }
+        } else if (c->matrix()) {
+            for (int64_t i = 0; i < c->n_dof(); ++i) f(i, i);
+        } else {
+            for (int64_t b = 0; b < c->n_dof(); b += c->tm.nb)
+                for (int i = 0; i < c->tm.nb; ++i) f(b + i, b + c->tm.perm[size_t(i)]);
+        }
+    };
+    const size_t bytes = dev.size() * sizeof(T);
+    if (in) {
+        each([&](int64_t h, int64_t d) { dev[size_t(d)] = T(in[h]); });
+        HGDG_HIP(hipMemcpyAsync(v.ptr(), dev.data(), bytes, hipMemcpyHostToDevice, c->stream));
+    } else {
+        HGDG_HIP(hipMemcpyAsync(dev.data(), v.ptr(), bytes, hipMemcpyDeviceToHost, c->stream));
+    }
+    HGDG_HIP(hipStreamSynchronize(c->stream));
+    if (out) each([&](int64_t h, int64_t d) { out[h] = double(dev[size_t(d)]); });
+}
+
 static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
     const int64_t n = c->n_dof();
     HostCopyParams base{};
@@ -243,6 +280,12 @@ static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
         base.nb = uint32_t(tm.nb);
         unit = tm.nb;
     }
+    auto whole = [&] {
+        if (v.is_f32) host_copy_whole<float>(c, v, out, in);
+        else host_copy_whole<double>(c, v, out, in);
+    };
+    const size_t stored = size_t(n) * (v.is_f32 ? sizeof(float) : sizeof(double));
+    if (stored > kWholeFrom && stored <= kWholeTo) return whole();
     // chunk k: unknowns [cut[k], cut[k + 1]); tetrahedra: elements [ecut[k], ecut[k + 1])
     std::vector<int64_t> cut{0}, ecut{0};
     while (cut.back() < n) {
@@ -295,7 +338,11 @@ static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
         }
         if (done) (void)hipEventDestroy(done);
     };
-    on_threads(workers, work);
+    try {
+        on_threads(workers, work);
+    } catch (const NoPinnedChunk&) {
+        whole();
+    }
 }
 
 void host_get(hgdg_ctx* c, Vec& v, double* host) { host_copy(c, v, host, nullptr); }
