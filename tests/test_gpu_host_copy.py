@@ -3,8 +3,9 @@ smaller than a chunk (2^18 unknowns), of exactly one, one unknown or element
 more, several chunks on one thread and on four (from 2^20 unknowns), FP64 and
 FP32 storage, tensor elements (permuted), tetrahedra of mixed order (grouped on
 the device) and matrix operators. What was set comes back bit for bit (rounded
-to FP32 in FP32 storage); a set reaches the unknowns it should: the copy in
-another vector, read element by element, and the unchanged neighbours say so."""
+to FP32 in FP32 storage), and two vectors meet unknown by unknown. Whether each
+unknown reaches its place, which a round trip cannot tell, is compared with the
+oracle's layout in test_gpu_host_layout.py."""
 import numpy as np
 import pytest
 
