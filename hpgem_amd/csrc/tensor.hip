@@ -928,8 +928,8 @@ __device__ __forceinline__ void acoustic_block(const AcousticParams& p, int64_t 
     // ---- own pencil of every field; g_r
     // (kAhead: and the neighbour's pencils of the first face pencil: all loads of
     // both are in flight before any is used)
-    constexpr bool kTogether = (KIND == STAGE_MANY || KIND == STAGE_MANY_MIXED) && !UPD;
-    constexpr bool kAhead = !UPD && (DIM == 2 || N1 <= 4 || (kTogether && N1 == 6));
+    constexpr bool kTogether = KIND == STAGE_MANY || KIND == STAGE_MANY_MIXED;
+    constexpr bool kAhead = (!UPD && (DIM == 2 || N1 <= 4)) || (kTogether && DIM == 3 && N1 == 6);
     double w[NF][N1], J[DIM][DIM], wq[NF][N1];
     constexpr bool kEarly = UPD && N1 <= 4;
     double y[NF][N1];  // kEarly: the update's sum but for this stage's own term
@@ -2168,10 +2168,18 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
             constexpr int DIMc = decltype(D)::value, N1c = decltype(N)::value;
             using S = AcousticShape<DIMc, N1c>;
             const int64_t grid = (c->n_elem + S::EPB - 1) / S::EPB;
+            // kTogether's registers at 3D p = 2 (177 against 164) leave two
+            // wavefronts a SIMD instead of three, which costs large boxes more
+            // than one further input gains (40^3 76 against 70 us; 24^3 the same)
+            const bool many = !(DIMc == 3 && N1c == 3 && io.n_in == 3 && c->n_elem > 30 * 30 * 30);
             auto launch = [&](auto K) {
+                constexpr int KIND = decltype(K)::value;
                 // the update at 3D p = 3 is the one form that needs more registers
-                // by its kind (280 against 225: one wavefront a SIMD instead of two)
-                constexpr int KIND = decltype(K)::value, KU = DIMc == 3 && N1c == 4 ? int(STAGE_ANY) : KIND;
+                // by its kind (280 against 225: one wavefront a SIMD instead of two);
+                // kTogether beside it only where there is one in any case
+                constexpr bool kAny = (DIMc == 3 && N1c == 4) ||
+                                      ((KIND == STAGE_MANY || KIND == STAGE_MANY_MIXED) && !(DIMc == 3 && N1c == 6));
+                constexpr int KU = kAny ? int(STAGE_ANY) : KIND;
                 if (io.upd.u != nullptr)  // the fused RK update of a step's last stage
                     hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, KU, true>), dim3(unsigned(grid)),
                                        dim3(S::THREADS), 0, c->stream, a);
@@ -2179,13 +2187,8 @@ void tensor_rhs(hgdg_ctx* c, const StageIO& io) {
                     hipLaunchKernelGGL((tensor_acoustic_rhs<DIMc, N1c, KIND, false>), dim3(unsigned(grid)),
                                        dim3(S::THREADS), 0, c->stream, a);
             };
-            // kTogether's registers at 3D p = 2 (177 against 164) leave two
-            // wavefronts a SIMD instead of three, which costs large boxes more
-            // than one further input gains (40^3 76 against 70 us; 24^3 the same)
-            const bool any = io.upd.u != nullptr ||
-                             (DIMc == 3 && N1c == 3 && io.n_in == 3 && c->n_elem > 30 * 30 * 30);
-            if (any) with_stage_kind<false>(io, launch);
-            else with_stage_kind<true>(io, launch);
+            if (many) with_stage_kind<true>(io, launch);
+            else with_stage_kind<false>(io, launch);
         });
         HGDG_HIP(hipGetLastError());
         return;
