@@ -113,11 +113,14 @@ void set_storage(hgdg_ctx* c, Vec& v, bool f32) {
 constexpr int64_t kChunk = int64_t(1) << 18;  // doubles per chunk
 constexpr int kCopyThreads = 4;
 constexpr int64_t kThreadedFrom = int64_t(1) << 20;  // doubles: below, one thread is as fast
-// Between these bytes a plain copy is the fastest (us, set and get of 3072 values:
-// 11.7 and 11.3 against 15.2 and 14.5, of 5600 on tetrahedra 12.0 and 12.2 against
-// 17.1 and 15.8; of 10800 15.3 and 16.0 against 16.9 and 16.9; but of 1728 15.7 and
-// 22.1 against 15.3 and 14.2, of 19200 19.0 and 20.4 against 18.4 and 19.0).
-constexpr size_t kWholeFrom = size_t(16) << 10, kWholeTo = size_t(96) << 10;
+// Up to these bytes (as stored) one copy to or from a chunk, permuted by the host,
+// is as fast as the kernel or faster. us, set and get, by the kernel and so: 64
+// values 14.0 and 13.1, 13.7 and 12.9; 3072 14.9 and 14.3, 10.9 and 10.5; 5600 on
+// tetrahedra 16.9 and 15.5, 11.0 and 13.0; 12000 16.7 and 16.9, 14.0 and 14.5; by
+// 19200 the host's permutation takes what the copy saves. (Copied from pageable
+// memory a few of these sizes took 50 us in some processes, with nothing to tell
+// them by.)
+constexpr size_t kWholeTo = size_t(96) << 10;
 
 // The pinned chunks are the process's: allocating one takes about 0.3 ms, too
 // much for a context of its own small vectors. At most kPinnedKept are kept for
@@ -218,10 +221,10 @@ __global__ __launch_bounds__(kBlock) void host_copy_elements(const HostCopyParam
     for (int64_t i = threadIdx.x % 64; i < n; i += 64) host_copy_one(p, p.dev[e] + i, h - p.lo + i);
 }
 
-// One copy of the vector as it is stored, permuted (and converted) on the host.
+// One copy of the vector as it is stored to or from `dev`, permuted (and
+// converted) on the host.
 template <typename T>
-static void host_copy_whole(hgdg_ctx* c, Vec& v, double* out, const double* in) {
-    std::vector<T> dev(static_cast<size_t>(c->n_dof()));
+static void host_copy_whole(hgdg_ctx* c, Vec& v, double* out, const double* in, T* dev) {
     auto each = [&](auto&& f) {  // f(position in hpGEM's layout, position in v)
         if (c->simplex()) {
             for (size_t e = 0; e + 1 < c->sm.host_off.size(); ++e) {
@@ -235,57 +238,21 @@ static void host_copy_whole(hgdg_ctx* c, Vec& v, double* out, const double* in) 
                 for (int i = 0; i < c->tm.nb; ++i) f(b + i, b + c->tm.perm[size_t(i)]);
         }
     };
-    const size_t bytes = dev.size() * sizeof(T);
+    const size_t bytes = size_t(c->n_dof()) * sizeof(T);
     if (in) {
         each([&](int64_t h, int64_t d) { dev[size_t(d)] = T(in[h]); });
-        HGDG_HIP(hipMemcpyAsync(v.ptr(), dev.data(), bytes, hipMemcpyHostToDevice, c->stream));
+        HGDG_HIP(hipMemcpyAsync(v.ptr(), dev, bytes, hipMemcpyHostToDevice, c->stream));
     } else {
-        HGDG_HIP(hipMemcpyAsync(dev.data(), v.ptr(), bytes, hipMemcpyDeviceToHost, c->stream));
+        HGDG_HIP(hipMemcpyAsync(dev, v.ptr(), bytes, hipMemcpyDeviceToHost, c->stream));
     }
     HGDG_HIP(hipStreamSynchronize(c->stream));
     if (out) each([&](int64_t h, int64_t d) { out[h] = double(dev[size_t(d)]); });
 }
 
-static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
+// The chunks, shared by the threads; whole multiples of `unit` (tensor elements'
+// functions).
+static void host_copy_chunks(hgdg_ctx* c, const HostCopyParams& base, int64_t unit, double* out, const double* in) {
     const int64_t n = c->n_dof();
-    HostCopyParams base{};
-    base.v = v.ptr();
-    base.v_f32 = v.is_f32 ? 1 : 0;
-    base.get = out != nullptr ? 1 : 0;
-    int64_t unit = 1;  // chunks are whole multiples of it (tensor elements' functions)
-    if (c->simplex()) {
-        SimplexMesh& sm = c->sm;
-        if (sm.d_io_off.n == 0) {
-            sm.host_off.assign(1, 0);
-            std::vector<int64_t> dev(static_cast<size_t>(c->n_elem));
-            for (int64_t e = 0; e < c->n_elem; ++e) {
-                const int64_t d = sm.dev_of[size_t(e)];
-                dev[size_t(e)] = sm.dof_off[size_t(d)];
-                sm.host_off.push_back(sm.host_off.back() + int64_t(c->n_fields) * tet_nb(sm.order[size_t(d)]));
-            }
-            std::vector<int64_t> both(sm.host_off);
-            both.insert(both.end(), dev.begin(), dev.end());
-            sm.d_io_off.upload(both, c->stream);
-            HGDG_HIP(hipStreamSynchronize(c->stream));
-        }
-        base.off = sm.d_io_off.ptr;
-        base.dev = sm.d_io_off.ptr + c->n_elem + 1;
-    } else if (!c->matrix()) {
-        TensorMesh& tm = c->tm;
-        if (tm.d_perm.n == 0) {
-            tm.d_perm.upload(std::vector<int32_t>(tm.perm.begin(), tm.perm.end()), c->stream);
-            HGDG_HIP(hipStreamSynchronize(c->stream));
-        }
-        base.perm = tm.d_perm.ptr;
-        base.nb = uint32_t(tm.nb);
-        unit = tm.nb;
-    }
-    auto whole = [&] {
-        if (v.is_f32) host_copy_whole<float>(c, v, out, in);
-        else host_copy_whole<double>(c, v, out, in);
-    };
-    const size_t stored = size_t(n) * (v.is_f32 ? sizeof(float) : sizeof(double));
-    if (stored > kWholeFrom && stored <= kWholeTo) return whole();
     // chunk k: unknowns [cut[k], cut[k + 1]); tetrahedra: elements [ecut[k], ecut[k + 1])
     std::vector<int64_t> cut{0}, ecut{0};
     while (cut.back() < n) {
@@ -338,10 +305,58 @@ static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
         }
         if (done) (void)hipEventDestroy(done);
     };
+    on_threads(workers, work);
+}
+
+static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
+    const int64_t n = c->n_dof();
+    HostCopyParams base{};
+    base.v = v.ptr();
+    base.v_f32 = v.is_f32 ? 1 : 0;
+    base.get = out != nullptr ? 1 : 0;
+    int64_t unit = 1;
+    if (c->simplex()) {
+        SimplexMesh& sm = c->sm;
+        if (sm.d_io_off.n == 0) {
+            sm.host_off.assign(1, 0);
+            std::vector<int64_t> dev(static_cast<size_t>(c->n_elem));
+            for (int64_t e = 0; e < c->n_elem; ++e) {
+                const int64_t d = sm.dev_of[size_t(e)];
+                dev[size_t(e)] = sm.dof_off[size_t(d)];
+                sm.host_off.push_back(sm.host_off.back() + int64_t(c->n_fields) * tet_nb(sm.order[size_t(d)]));
+            }
+            std::vector<int64_t> both(sm.host_off);
+            both.insert(both.end(), dev.begin(), dev.end());
+            sm.d_io_off.upload(both, c->stream);
+            HGDG_HIP(hipStreamSynchronize(c->stream));
+        }
+        base.off = sm.d_io_off.ptr;
+        base.dev = sm.d_io_off.ptr + c->n_elem + 1;
+    } else if (!c->matrix()) {
+        TensorMesh& tm = c->tm;
+        if (tm.d_perm.n == 0) {
+            tm.d_perm.upload(std::vector<int32_t>(tm.perm.begin(), tm.perm.end()), c->stream);
+            HGDG_HIP(hipStreamSynchronize(c->stream));
+        }
+        base.perm = tm.d_perm.ptr;
+        base.nb = uint32_t(tm.nb);
+        unit = tm.nb;
+    }
+    auto whole = [&](void* staging) {
+        if (v.is_f32) host_copy_whole(c, v, out, in, static_cast<float*>(staging));
+        else host_copy_whole(c, v, out, in, static_cast<double*>(staging));
+    };
+    const size_t stored = size_t(n) * (v.is_f32 ? sizeof(float) : sizeof(double));
     try {
-        on_threads(workers, work);
-    } catch (const NoPinnedChunk&) {
-        whole();
+        if (stored <= kWholeTo) {
+            const PinnedChunk chunk;
+            whole(chunk.ptr);
+        } else {
+            host_copy_chunks(c, base, unit, out, in);
+        }
+    } catch (const NoPinnedChunk&) {  // pageable memory then
+        std::vector<double> staging((stored + sizeof(double) - 1) / sizeof(double));
+        whole(staging.data());
     }
 }
 
