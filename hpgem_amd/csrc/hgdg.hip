@@ -83,17 +83,33 @@ Vec& vec_at(hgdg_ctx* c, int id) {
     return c->vecs[id];
 }
 
+// An allocation that a call cannot do without. The vector for summed stages, which
+// the kernels can do without, makes room for it.
+template <typename T>
+static void alloc_needed(hgdg_ctx* c, DevBuf<T>& buf, size_t n) {
+    try {
+        buf.alloc(n);
+    } catch (const Failure&) {
+        if (c->stage_sum.n == 0) throw;
+        (void)hipGetLastError();
+        HGDG_HIP(hipStreamSynchronize(c->stream));
+        c->drop_graph();
+        c->stage_sum.reset();
+        buf.alloc(n);
+    }
+}
+
 void set_storage(hgdg_ctx* c, Vec& v, bool f32) {
     if (v.is_f32 == f32 && (f32 ? v.f32 != nullptr : v.f64 != nullptr)) return;
     const size_t n = size_t(c->n_dof());
     if (f32) {
         v.f32.reset(new DevBuf<float>);
-        v.f32->alloc(n);
+        alloc_needed(c, *v.f32, n);
         HGDG_HIP(hipMemsetAsync(v.f32->ptr, 0, n * sizeof(float), c->stream));
         v.f64.reset();
     } else {
         v.f64.reset(new DevBuf<double>);
-        v.f64->alloc(n);
+        alloc_needed(c, *v.f64, n);
         HGDG_HIP(hipMemsetAsync(v.f64->ptr, 0, n * sizeof(double), c->stream));
         v.f32.reset();
     }
@@ -636,19 +652,22 @@ void rk_steps(hgdg_ctx* c, int solution, const int* aux, int stages, const doubl
     require(n_steps >= 0, HGDG_ERR_ARG, "negative step count");
     check_rk_args(c, solution, aux, stages);
     if (tensor_rk_tiny(c, solution, aux, stages, a, b, dt, n_steps)) return;
-    // a stage that is summed first needs its vector before the capture below
-    for (int i = 0; i < stages; ++i)
-        if (sums_stages(c, 1 + i - int(std::count(a + i * stages, a + i * stages + i, 0.0)))) (void)stage_space(c);
     GraphKey key{solution, std::vector<int>(aux, aux + stages), std::vector<double>(a, a + stages * stages),
                  std::vector<double>(b, b + stages), dt};
+    // a stage that is summed first needs its vector before a capture
+    auto before_capture = [&] {
+        for (int i = 0; i < stages; ++i)
+            if (sums_stages(c, 1 + i - int(std::count(a + i * stages, a + i * stages + i, 0.0)))) (void)stage_space(c);
+        HGDG_HIP(hipStreamSynchronize(c->stream));
+    };
     if (c->rk_fused != 0 && rhs_fuses_update(c) && n_steps >= 2) {
         // pairs of steps with the update fused into each last stage: the
         // solution goes to the context's spare vector and back
         double* u0 = vec_at(c, solution).f64->ptr;
-        if (c->u_spare.n != size_t(c->n_dof())) c->u_spare.alloc(size_t(c->n_dof()));
+        if (c->u_spare.n != size_t(c->n_dof())) alloc_needed(c, c->u_spare, size_t(c->n_dof()));
         if (!(c->graph2_valid && c->graph2_key == key && c->graph2_u == u0)) {
             c->drop_graph2();
-            HGDG_HIP(hipStreamSynchronize(c->stream));
+            before_capture();
             HGDG_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             try {
                 enqueue_rk_step_fused(c, solution, aux, stages, a, b, dt, u0, c->u_spare.ptr);
@@ -672,7 +691,7 @@ void rk_steps(hgdg_ctx* c, int solution, const int* aux, int stages, const doubl
     }
     if (!(c->graph_valid && c->graph_key == key)) {
         c->drop_graph();
-        HGDG_HIP(hipStreamSynchronize(c->stream));
+        before_capture();
         HGDG_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         try {
             enqueue_rk_step(c, solution, aux, stages, a, b, dt);
