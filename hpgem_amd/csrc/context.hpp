@@ -37,6 +37,7 @@ struct TensorMesh {
     std::vector<int32_t> ginfo;      // [2 dim][e] neighbour's face, point map, left flag
     DevBuf<double> d_gX, d_gtab, d_gcinv;
     DevBuf<double> d_ggeo, d_gfgeo;  // the RHS kernel's geometry per point and per face point
+    int64_t geo_slab = 0;            // of so many elements at a time; 0: of all
     DevBuf<int32_t> d_gface;         // gnbr then ginfo
 };
 
@@ -190,6 +191,7 @@ void tensor_error_modes(hgdg_ctx* c, const Vec& v, int field, int n_modes, const
 void tensor_general_upload(hgdg_ctx* c, const hgdg_mesh_desc* m);
 void tensor_general_operator_set(hgdg_ctx* c, const hgdg_op_desc* op);
 void tensor_general_rhs(hgdg_ctx* c, const StageIO& io);
+void tensor_general_in_slabs(hgdg_ctx* c, int64_t elements);  // 0: as many as suit
 void tensor_general_mass_apply(hgdg_ctx* c, Vec& v, bool inverse);
 void tensor_general_project(hgdg_ctx* c, Vec& v, int field, int n_modes, const double* amp, const double* k,
                             const double* gauss);

@@ -83,18 +83,20 @@ Vec& vec_at(hgdg_ctx* c, int id) {
     return c->vecs[id];
 }
 
-// An allocation that a call cannot do without. The vector for summed stages, which
-// the kernels can do without, makes room for it.
+// A state vector's allocation. What the kernels can do without, the vector for
+// summed stages and the geometry stored per point, makes room for it.
 template <typename T>
-static void alloc_needed(hgdg_ctx* c, DevBuf<T>& buf, size_t n) {
+static void alloc_vector(hgdg_ctx* c, DevBuf<T>& buf, size_t n) {
     try {
         buf.alloc(n);
     } catch (const Failure&) {
-        if (c->stage_sum.n == 0) throw;
+        const bool stored = c->has_op && !c->matrix() && c->tm.general && c->tm.geo_slab == 0;
+        if (c->stage_sum.n == 0 && !stored) throw;
         (void)hipGetLastError();
         HGDG_HIP(hipStreamSynchronize(c->stream));
         c->drop_graph();
         c->stage_sum.reset();
+        if (stored) tensor_general_in_slabs(c, 0);
         buf.alloc(n);
     }
 }
@@ -104,12 +106,12 @@ void set_storage(hgdg_ctx* c, Vec& v, bool f32) {
     const size_t n = size_t(c->n_dof());
     if (f32) {
         v.f32.reset(new DevBuf<float>);
-        alloc_needed(c, *v.f32, n);
+        alloc_vector(c, *v.f32, n);
         HGDG_HIP(hipMemsetAsync(v.f32->ptr, 0, n * sizeof(float), c->stream));
         v.f64.reset();
     } else {
         v.f64.reset(new DevBuf<double>);
-        alloc_needed(c, *v.f64, n);
+        alloc_vector(c, *v.f64, n);
         HGDG_HIP(hipMemsetAsync(v.f64->ptr, 0, n * sizeof(double), c->stream));
         v.f32.reset();
     }
@@ -523,6 +525,19 @@ bool stage_space(hgdg_ctx* c) {
     return true;
 }
 
+// The spare solution of fused step pairs; without it steps are replayed one by one.
+bool spare_space(hgdg_ctx* c) {
+    const size_t n = size_t(c->n_dof());
+    if (c->u_spare.n == n) return true;
+    try {
+        c->u_spare.alloc(n);
+    } catch (const Failure&) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
 // io with its inputs summed into one where the RHS kernel is better off so.
 StageIO sum_stage(hgdg_ctx* c, const StageIO& io) {
     if (!sums_stages(c, io.n_in) || !stage_space(c)) return io;
@@ -660,11 +675,10 @@ void rk_steps(hgdg_ctx* c, int solution, const int* aux, int stages, const doubl
             if (sums_stages(c, 1 + i - int(std::count(a + i * stages, a + i * stages + i, 0.0)))) (void)stage_space(c);
         HGDG_HIP(hipStreamSynchronize(c->stream));
     };
-    if (c->rk_fused != 0 && rhs_fuses_update(c) && n_steps >= 2) {
+    if (c->rk_fused != 0 && rhs_fuses_update(c) && n_steps >= 2 && spare_space(c)) {
         // pairs of steps with the update fused into each last stage: the
         // solution goes to the context's spare vector and back
         double* u0 = vec_at(c, solution).f64->ptr;
-        if (c->u_spare.n != size_t(c->n_dof())) alloc_needed(c, c->u_spare, size_t(c->n_dof()));
         if (!(c->graph2_valid && c->graph2_key == key && c->graph2_u == u0)) {
             c->drop_graph2();
             before_capture();

@@ -209,12 +209,13 @@ __host__ __device__ __forceinline__ void partner_point(int code, int ka, int kb,
 
 struct GenParams {
     int64_t n_elem;
+    int64_t first, end;    // the elements of this launch
     StageIO io;
     const int32_t* nbr;    // [NFACE][E]
     const int32_t* info;   // [NFACE][E]
     const double* tab;     // NodalOps of the order, packed
-    const double* geo;     // per point, GenRhs::GP numbers [E][GP][NP]
-    const double* fgeo;    // per face point, GenRhs::GF numbers [E][NFACE][GF][NFP]
+    const double* geo;     // per point, GenRhs::GP numbers [E][GP][NP] (where those
+    const double* fgeo;    // of element 0 would be); per face point, GF [E][NFACE][GF][NFP]
     const double* cinv;    // [E] (acoustic)
 };
 
@@ -223,6 +224,8 @@ struct GenParams {
 template <int DIM, int N1, bool ACOUSTIC>
 struct GenRhs {
     using S = GenShape<DIM, N1>;
+    static constexpr int kDim = DIM, kN1 = N1;
+    static constexpr bool kAcoustic = ACOUSTIC;
     static constexpr int NF = ACOUSTIC ? DIM + 1 : 1;
     static constexpr int NP = S::NP, NFP = S::NFP, NFACE = S::NFACE;
     static constexpr int EPB = (64 % NP) * 16 <= 64 ? 64 / NP : (128 % NP) * 16 <= 128 ? 128 / NP : 256 / NP;
@@ -246,10 +249,12 @@ struct GenRhs {
     static constexpr int FC = DIM == 3 ? NBC : NBT;
 };
 
-// The geometry a mesh and an operator fix, once per operator: thread t of
-// element e takes point t and the face points t, t + NP, ..
+// The geometry a mesh and an operator fix, once per operator (or slab by slab
+// before each use, tensor_general_in_slabs): thread t of element e takes point t
+// and the face points t, t + NP, ..
 struct GenGeoParams {
     int64_t n_elem;
+    int64_t first, count;
     const double* X;       // [E][NV][DIM] vertex coordinates
     const int32_t* nbr;
     const int32_t* info;
@@ -265,8 +270,8 @@ __global__ __launch_bounds__(kGenTarget) void tensor_general_geometry(const GenG
     using T = NodalTab<N1>;
     constexpr int NP = G::NP, NFP = G::NFP, NV = G::S::NV, NFACE = G::NFACE;
     const int t = threadIdx.x % NP;
-    const int64_t e = int64_t(blockIdx.x) * G::EPB + threadIdx.x / NP;
-    if (e >= p.n_elem) return;
+    const int64_t at = int64_t(blockIdx.x) * G::EPB + threadIdx.x / NP, e = p.first + at;
+    if (at >= p.count) return;
     const double* tab = p.tab;
     const double* X = p.X + e * NV * DIM;
     const int ii[3] = {t % N1, (t / N1) % N1, DIM == 3 ? t / (N1 * N1) : 0};
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(kGenTarget) void tensor_general_geometry(const GenG
     double W = fabs(det_inv<DIM>(J, Ji));
 #pragma unroll
     for (int d = 0; d < DIM; ++d) W *= tab[T::W + ii[d]];
-    double* geo = p.geo + e * G::GP * NP + t;
+    double* geo = p.geo + at * G::GP * NP + t;
 #pragma unroll
     for (int r = 0; r < DIM; ++r) {
         double ah = 0;
@@ -308,7 +313,7 @@ __global__ __launch_bounds__(kGenTarget) void tensor_general_geometry(const GenG
         double wf = tab[T::W + qa];
         if constexpr (DIM == 3) wf *= tab[T::W + qb];
         const double sgn = left ? 1.0 : -1.0;  // own normal = sgn n
-        double* out = p.fgeo + ((e * NFACE + f) * G::GF) * NFP + k;
+        double* out = p.fgeo + ((at * NFACE + f) * G::GF) * NFP + k;
         if constexpr (ACOUSTIC) {
 #pragma unroll
             for (int d = 0; d < DIM; ++d) out[d * NFP] = sgn * n[d] * wf;
@@ -349,8 +354,8 @@ __global__ __launch_bounds__((GenRhs<DIM, N1, ACOUSTIC>::THREADS)) void tensor_g
     const int le = tid / NP;
     const int t = tid % NP;
     const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const int64_t e = blk * G::EPB + le;
-    const bool ok = e < p.n_elem;
+    const int64_t e = p.first + blk * G::EPB + le;
+    const bool ok = e < p.end;
     const int64_t E = p.n_elem;
     double* sA = lds + le * G::PER + G::A;
     double* sB = lds + le * G::PER + G::B;
@@ -959,6 +964,50 @@ void tensor_general_upload(hgdg_ctx* c, const hgdg_mesh_desc* m) {
     HGDG_HIP(hipStreamSynchronize(c->stream));
 }
 
+namespace {
+
+constexpr int64_t kGeoSlab = 4096;
+
+// f(GenRhs) of the mesh and an operator of this kind
+template <typename F>
+void with_shape(const hgdg_ctx* c, int kind, F&& f) {
+    dispatch_general(c->dim, c->tm.n1, [&](auto D, auto N) {
+        if (kind == HGDG_OP_ACOUSTIC_CENTRAL) f(GenRhs<decltype(D)::value, decltype(N)::value, true>{});
+        else f(GenRhs<decltype(D)::value, decltype(N)::value, false>{});
+    });
+}
+
+void alloc_geometry(hgdg_ctx* c, int kind, int64_t elements) {
+    with_shape(c, kind, [&](auto G_) {
+        using G = decltype(G_);
+        c->tm.d_ggeo.alloc(size_t(elements) * G::GP * G::NP);
+        c->tm.d_gfgeo.alloc(size_t(elements) * G::NFACE * G::GF * G::NFP);
+    });
+}
+
+// The geometry of elements [first, first + count), to the buffers' start.
+void launch_geometry(hgdg_ctx* c, int kind, const double* velocity, int64_t first, int64_t count) {
+    GenGeoParams p{};
+    p.n_elem = c->n_elem;
+    p.first = first;
+    p.count = count;
+    p.X = c->tm.d_gX.ptr;
+    p.nbr = c->tm.d_gface.ptr;
+    p.info = c->tm.d_gface.ptr + size_t(2 * c->dim) * c->n_elem;
+    p.tab = c->tm.d_gtab.ptr;
+    for (int d = 0; d < 3; ++d) p.a[d] = kind == HGDG_OP_ADVECTION_UPWIND && d < c->dim ? velocity[d] : 0.0;
+    p.geo = c->tm.d_ggeo.ptr;
+    p.fgeo = c->tm.d_gfgeo.ptr;
+    with_shape(c, kind, [&](auto G_) {
+        using G = decltype(G_);
+        hipLaunchKernelGGL((tensor_general_geometry<G::kDim, G::kN1, G::kAcoustic>),
+                           dim3(unsigned((count + G::EPB - 1) / G::EPB)), dim3(G::THREADS), 0, c->stream, p);
+    });
+    HGDG_HIP(hipGetLastError());
+}
+
+}  // namespace
+
 void tensor_general_operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
     const int64_t ne = c->n_elem;
     if (op->kind == HGDG_OP_ACOUSTIC_CENTRAL) {
@@ -968,30 +1017,30 @@ void tensor_general_operator_set(hgdg_ctx* c, const hgdg_op_desc* op) {
         c->n_fields = 1;
     }
     c->dof = ne * c->tm.nb * c->n_fields;
-    const bool acoustic = op->kind == HGDG_OP_ACOUSTIC_CENTRAL;
-    GenGeoParams p{};
-    p.n_elem = ne;
-    p.X = c->tm.d_gX.ptr;
-    p.nbr = c->tm.d_gface.ptr;
-    p.info = c->tm.d_gface.ptr + size_t(2 * c->dim) * ne;
-    p.tab = c->tm.d_gtab.ptr;
-    for (int d = 0; d < 3; ++d) p.a[d] = !acoustic && d < c->dim ? op->velocity[d] : 0.0;
-    dispatch_general(c->dim, c->tm.n1, [&](auto D, auto N) {
-        auto build = [&](auto A) {
-            constexpr bool kAc = decltype(A)::value;
-            using G = GenRhs<decltype(D)::value, decltype(N)::value, kAc>;
-            c->tm.d_ggeo.alloc(size_t(ne) * G::GP * G::NP);
-            c->tm.d_gfgeo.alloc(size_t(ne) * G::NFACE * G::GF * G::NFP);
-            p.geo = c->tm.d_ggeo.ptr;
-            p.fgeo = c->tm.d_gfgeo.ptr;
-            hipLaunchKernelGGL((tensor_general_geometry<decltype(D)::value, decltype(N)::value, kAc>),
-                               dim3(unsigned((ne + G::EPB - 1) / G::EPB)), dim3(G::THREADS), 0, c->stream, p);
-        };
-        if (acoustic) build(std::true_type{});
-        else build(std::false_type{});
-    });
-    HGDG_HIP(hipGetLastError());
+    c->tm.geo_slab = 0;
+    try {
+        alloc_geometry(c, op->kind, ne);
+    } catch (const Failure&) {
+        (void)hipGetLastError();
+        c->tm.geo_slab = std::min(ne, kGeoSlab);
+        alloc_geometry(c, op->kind, c->tm.geo_slab);
+        return;
+    }
+    launch_geometry(c, op->kind, op->velocity, 0, ne);
     HGDG_HIP(hipStreamSynchronize(c->stream));
+}
+
+// Gives the stored geometry back but for `elements` at a time, whose geometry
+// each right-hand side forms anew. Of a mesh that nearly fills the card: it takes
+// more than a state vector (3D acoustics 3.5 KB an element against 0.9 at p = 2,
+// 22 against 6.9 at p = 5).
+void tensor_general_in_slabs(hgdg_ctx* c, int64_t elements) {
+    HGDG_HIP(hipStreamSynchronize(c->stream));
+    c->drop_graph();
+    c->tm.d_ggeo.reset();
+    c->tm.d_gfgeo.reset();
+    c->tm.geo_slab = std::min(c->n_elem, elements > 0 ? elements : kGeoSlab);
+    alloc_geometry(c, c->op.kind, c->tm.geo_slab);
 }
 
 void tensor_general_rhs(hgdg_ctx* c, const StageIO& io) {
@@ -1001,21 +1050,21 @@ void tensor_general_rhs(hgdg_ctx* c, const StageIO& io) {
     p.nbr = c->tm.d_gface.ptr;
     p.info = c->tm.d_gface.ptr + size_t(2 * c->dim) * c->n_elem;
     p.tab = c->tm.d_gtab.ptr;
-    p.geo = c->tm.d_ggeo.ptr;
-    p.fgeo = c->tm.d_gfgeo.ptr;
     const bool acoustic = c->op.kind == HGDG_OP_ACOUSTIC_CENTRAL;
     p.cinv = acoustic ? c->tm.d_gcinv.ptr : nullptr;
-    dispatch_general(c->dim, c->tm.n1, [&](auto D, auto N) {
-        auto launch = [&](auto A) {
-            constexpr bool kAc = decltype(A)::value;
-            using G = GenRhs<decltype(D)::value, decltype(N)::value, kAc>;
-            hipLaunchKernelGGL((tensor_general_rhs<decltype(D)::value, decltype(N)::value, kAc>),
-                               dim3(unsigned((c->n_elem + G::EPB - 1) / G::EPB)), dim3(G::THREADS), 0, c->stream, p);
-        };
-        if (acoustic) launch(std::true_type{});
-        else launch(std::false_type{});
-    });
-    HGDG_HIP(hipGetLastError());
+    const int64_t slab = c->tm.geo_slab > 0 ? c->tm.geo_slab : c->n_elem;
+    for (p.first = 0; p.first < c->n_elem; p.first += slab) {
+        p.end = std::min(p.first + slab, c->n_elem);
+        if (c->tm.geo_slab > 0) launch_geometry(c, c->op.kind, c->op.velocity, p.first, p.end - p.first);
+        with_shape(c, c->op.kind, [&](auto G_) {
+            using G = decltype(G_);
+            p.geo = c->tm.d_ggeo.ptr - p.first * G::GP * G::NP;
+            p.fgeo = c->tm.d_gfgeo.ptr - p.first * G::NFACE * G::GF * G::NFP;
+            hipLaunchKernelGGL((tensor_general_rhs<G::kDim, G::kN1, G::kAcoustic>),
+                               dim3(unsigned((p.end - p.first + G::EPB - 1) / G::EPB)), dim3(G::THREADS), 0, c->stream, p);
+        });
+        HGDG_HIP(hipGetLastError());
+    }
 }
 
 void tensor_general_mass_apply(hgdg_ctx* c, Vec& v, bool inverse) {
