@@ -849,9 +849,10 @@ void step_error_and_norm(hgdg_ctx* c, int solution, const int* aux, int stages, 
 // back to the caller's stack. Each GPU holds its own copy of the array (at its
 // own address, looked up once per device when a context is created on it);
 // every call on one GPU shares it, so calls that overlap on one GPU race.
-constexpr int64_t kScratchBlocks = 65536;  // partial pairs; meshes of at most 4 * 65536 elements
-constexpr int64_t kScratchMaxElements = 4 * kScratchBlocks;
-static __device__ __align__(256) double scratch[2 * kScratchBlocks + 2];
+// The limit of elements is the interface's; the launch has at most kNormBlocks
+// workgroups at any size.
+constexpr int64_t kScratchMaxElements = 262144;
+static __device__ __align__(256) double scratch[2 * kNormBlocks + 2];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double* g_scratch[kMaxDevices] = {};  // device address of `scratch` on each device
@@ -912,8 +913,7 @@ int step_error_noalloc(hgdg_ctx* c, int solution, const int* aux, int stages, co
     if (c->vecs[solution].is_f32) return fail_noalloc(HGDG_ERR_ARG, "the solution vector must be stored in FP64");
     if (c->n_elem > kScratchMaxElements)
         return fail_noalloc(HGDG_ERR_UNSUPPORTED,
-                            "hgdg_step_error_noalloc: at most 262144 elements (its fixed scratch array holds "
-                            "65536 partial pairs); use hgdg_step_error for larger meshes");
+                            "hgdg_step_error_noalloc: at most 262144 elements; use hgdg_step_error for larger meshes");
     if (c->device < 0 || c->device >= kMaxDevices || g_scratch[c->device] == nullptr)
         return fail_noalloc(HGDG_ERR_STATE, "no scratch address for this device (create the context with "
                                             "hgdg_ctx_create)");
@@ -937,9 +937,9 @@ int step_error_noalloc(hgdg_ctx* c, int solution, const int* aux, int stages, co
     double h[2] = {0.0, 0.0};
     if (grid > 0) {
         hipLaunchKernelGGL(step_error_norm, dim3(unsigned(grid)), dim3(kBlock), 0, c->stream, p);
-        hipLaunchKernelGGL(reduce_pairs, dim3(1), dim3(kBlock), 0, c->stream, ptr, grid, ptr + 2 * kScratchBlocks);
+        hipLaunchKernelGGL(reduce_pairs, dim3(1), dim3(kBlock), 0, c->stream, ptr, grid, ptr + 2 * kNormBlocks);
         if (hipGetLastError() != hipSuccess) return fail_noalloc(HGDG_ERR_HIP, "kernel launch failed");
-        if (hipMemcpyAsync(h, ptr + 2 * kScratchBlocks, sizeof(h), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+        if (hipMemcpyAsync(h, ptr + 2 * kNormBlocks, sizeof(h), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
             hipStreamSynchronize(c->stream) != hipSuccess)
             return fail_noalloc(HGDG_ERR_HIP, "reading back the reduced sums failed");
     }

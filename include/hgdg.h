@@ -266,7 +266,7 @@ int hgdg_step_error(hgdg_ctx* ctx, int solution, const int* aux_ids, int stages,
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). No counterpart in the reference. It calls no hipMalloc,
  * hipFree or other allocating routine: the per-block partial sums live in a
- * fixed device array of 1 MiB that the library holds on every GPU it runs on
+ * fixed device array of 16 KiB that the library holds on every GPU it runs on
  * until the process ends, reduced on the device, and 16 bytes are read back.
  * Limit: meshes of at most 262144 elements (HGDG_ERR_UNSUPPORTED beyond).
  * All calls on one GPU share that array: calls that overlap on one GPU race.
