@@ -214,6 +214,7 @@ void operator_set(hgdg_ctx* c, const hgdg_op_desc* op);
 void pinned_user(int change);
 void host_get(hgdg_ctx* c, Vec& v, double* host);        // host = v in hpGEM's layout
 void host_set(hgdg_ctx* c, Vec& v, const double* host);  // v = host
+void host_copy_pageable(hgdg_ctx* c, int vec, double* out, const double* in);  // either, where no pinned memory is left
 void state_diff(hgdg_ctx* c, int x, int y, double* l2, double* max_abs);
 
 // matrix_op.hip

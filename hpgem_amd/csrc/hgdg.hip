@@ -124,21 +124,17 @@ void set_storage(hgdg_ctx* c, Vec& v, bool f32) {
 // copies between the chunk and the caller's memory. Large vectors are shared by
 // up to kCopyThreads host threads with a chunk of their own each, so that the
 // transfers run beside the copies, most of whose time is the caller's pages
-// being touched for the first time. 67 MB (32^3 p = 3 acoustic): 100 RK4 steps
-// and reading the state took 34.1 ms with a permutation on the host around a
-// pageable copy, 25.8 so; the copy to fresh memory alone takes 4.9 ms with one
-// thread and 1.6 with four, the transfer 1.3.
+// being touched for the first time. Small vectors go the same way: one copied by
+// hipMemcpyAsync is there 3 us sooner if the stream is idle (3072 values read 10.9
+// and 14.6 us), but 6 later behind a kernel (26.3 and 19.6 after a right-hand side),
+// and after the first such copy each call that steps by graphs takes 25 to 30 us
+// more for good (20 steps of 16x16 p = 1 acoustics 322 -> 349). 67 MB (32^3 p = 3
+// acoustic): 100 RK4 steps and reading the state took 34.1 ms with a permutation on
+// the host around a pageable copy, 25.8 so; the copy to fresh memory alone takes
+// 4.9 ms with one thread and 1.6 with four, the transfer 1.3.
 constexpr int64_t kChunk = int64_t(1) << 18;  // doubles per chunk
 constexpr int kCopyThreads = 4;
 constexpr int64_t kThreadedFrom = int64_t(1) << 20;  // doubles: below, one thread is as fast
-// Up to these bytes (as stored) one copy to or from a chunk, permuted by the host,
-// is as fast as the kernel or faster. us, set and get, by the kernel and so: 64
-// values 14.0 and 13.1, 13.7 and 12.9; 3072 14.9 and 14.3, 10.9 and 10.5; 5600 on
-// tetrahedra 16.9 and 15.5, 11.0 and 13.0; 12000 16.7 and 16.9, 14.0 and 14.5; by
-// 19200 the host's permutation takes what the copy saves. (Copied from pageable
-// memory a few of these sizes took 50 us in some processes, with nothing to tell
-// them by.)
-constexpr size_t kWholeTo = size_t(96) << 10;
 
 // The pinned chunks are the process's: allocating one takes about 0.3 ms, too
 // much for a context of its own small vectors. At most kPinnedKept are kept for
@@ -239,12 +235,30 @@ __global__ __launch_bounds__(kBlock) void host_copy_elements(const HostCopyParam
     for (int64_t i = threadIdx.x % 64; i < n; i += 64) host_copy_one(p, p.dev[e] + i, h - p.lo + i);
 }
 
-// One copy of the vector as it is stored to or from `dev`, permuted (and
-// converted) on the host.
+// Tetrahedra: where the elements' unknowns lie in hpGEM's vector and in v.
+static void host_offsets(hgdg_ctx* c) {
+    SimplexMesh& sm = c->sm;
+    if (sm.d_io_off.n != 0) return;
+    sm.host_off.assign(1, 0);
+    std::vector<int64_t> dev(static_cast<size_t>(c->n_elem));
+    for (int64_t e = 0; e < c->n_elem; ++e) {
+        const int64_t d = sm.dev_of[size_t(e)];
+        dev[size_t(e)] = sm.dof_off[size_t(d)];
+        sm.host_off.push_back(sm.host_off.back() + int64_t(c->n_fields) * tet_nb(sm.order[size_t(d)]));
+    }
+    std::vector<int64_t> both(sm.host_off);
+    both.insert(both.end(), dev.begin(), dev.end());
+    sm.d_io_off.upload(both, c->stream);
+    HGDG_HIP(hipStreamSynchronize(c->stream));
+}
+
+// Where no pinned memory is left: one copy of the vector as it is stored, permuted
+// and converted on the host.
 template <typename T>
-static void host_copy_whole(hgdg_ctx* c, Vec& v, double* out, const double* in, T* dev) {
+static void copy_pageable(hgdg_ctx* c, Vec& v, double* out, const double* in) {
     auto each = [&](auto&& f) {  // f(position in hpGEM's layout, position in v)
         if (c->simplex()) {
+            host_offsets(c);
             for (size_t e = 0; e + 1 < c->sm.host_off.size(); ++e) {
                 const int64_t h = c->sm.host_off[e], d = c->sm.dof_off[size_t(c->sm.dev_of[e])];
                 for (int64_t i = 0; i < c->sm.host_off[e + 1] - h; ++i) f(h + i, d + i);
@@ -256,15 +270,21 @@ static void host_copy_whole(hgdg_ctx* c, Vec& v, double* out, const double* in, 
                 for (int i = 0; i < c->tm.nb; ++i) f(b + i, b + c->tm.perm[size_t(i)]);
         }
     };
-    const size_t bytes = size_t(c->n_dof()) * sizeof(T);
+    std::vector<T> dev(static_cast<size_t>(c->n_dof()));
     if (in) {
         each([&](int64_t h, int64_t d) { dev[size_t(d)] = T(in[h]); });
-        HGDG_HIP(hipMemcpyAsync(v.ptr(), dev, bytes, hipMemcpyHostToDevice, c->stream));
+        HGDG_HIP(hipMemcpyAsync(v.ptr(), dev.data(), dev.size() * sizeof(T), hipMemcpyHostToDevice, c->stream));
     } else {
-        HGDG_HIP(hipMemcpyAsync(dev, v.ptr(), bytes, hipMemcpyDeviceToHost, c->stream));
+        HGDG_HIP(hipMemcpyAsync(dev.data(), v.ptr(), dev.size() * sizeof(T), hipMemcpyDeviceToHost, c->stream));
     }
     HGDG_HIP(hipStreamSynchronize(c->stream));
     if (out) each([&](int64_t h, int64_t d) { out[h] = double(dev[size_t(d)]); });
+}
+
+void host_copy_pageable(hgdg_ctx* c, int vec, double* out, const double* in) {
+    Vec& v = vec_at(c, vec);
+    if (v.is_f32) copy_pageable<float>(c, v, out, in);
+    else copy_pageable<double>(c, v, out, in);
 }
 
 // The chunks, shared by the threads; whole multiples of `unit` (tensor elements'
@@ -335,19 +355,7 @@ static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
     int64_t unit = 1;
     if (c->simplex()) {
         SimplexMesh& sm = c->sm;
-        if (sm.d_io_off.n == 0) {
-            sm.host_off.assign(1, 0);
-            std::vector<int64_t> dev(static_cast<size_t>(c->n_elem));
-            for (int64_t e = 0; e < c->n_elem; ++e) {
-                const int64_t d = sm.dev_of[size_t(e)];
-                dev[size_t(e)] = sm.dof_off[size_t(d)];
-                sm.host_off.push_back(sm.host_off.back() + int64_t(c->n_fields) * tet_nb(sm.order[size_t(d)]));
-            }
-            std::vector<int64_t> both(sm.host_off);
-            both.insert(both.end(), dev.begin(), dev.end());
-            sm.d_io_off.upload(both, c->stream);
-            HGDG_HIP(hipStreamSynchronize(c->stream));
-        }
+        host_offsets(c);
         base.off = sm.d_io_off.ptr;
         base.dev = sm.d_io_off.ptr + c->n_elem + 1;
     } else if (!c->matrix()) {
@@ -360,21 +368,11 @@ static void host_copy(hgdg_ctx* c, Vec& v, double* out, const double* in) {
         base.nb = uint32_t(tm.nb);
         unit = tm.nb;
     }
-    auto whole = [&](void* staging) {
-        if (v.is_f32) host_copy_whole(c, v, out, in, static_cast<float*>(staging));
-        else host_copy_whole(c, v, out, in, static_cast<double*>(staging));
-    };
-    const size_t stored = size_t(n) * (v.is_f32 ? sizeof(float) : sizeof(double));
     try {
-        if (stored <= kWholeTo) {
-            const PinnedChunk chunk;
-            whole(chunk.ptr);
-        } else {
-            host_copy_chunks(c, base, unit, out, in);
-        }
-    } catch (const NoPinnedChunk&) {  // pageable memory then
-        std::vector<double> staging((stored + sizeof(double) - 1) / sizeof(double));
-        whole(staging.data());
+        host_copy_chunks(c, base, unit, out, in);
+    } catch (const NoPinnedChunk&) {
+        if (v.is_f32) copy_pageable<float>(c, v, out, in);
+        else copy_pageable<double>(c, v, out, in);
     }
 }
 

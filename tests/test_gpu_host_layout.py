@@ -2,19 +2,22 @@
 does not take the same way: the right-hand side of what was set, read back and
 compared with the oracle's, which has hpGEM's layout throughout. A wrong
 permutation or offset that set and get share cannot pass, since the operator does
-not commute with it. Vectors of one plain copy (16 to 96 KB as stored), below
-and above it, of several chunks (2^18 unknowns) on one thread and of four threads
+not commute with it. Vectors of a few elements, of several chunks (2^18 unknowns) on one thread and of four threads
 (from 2^20), tensor elements (permuted), tetrahedra of mixed order (regrouped)
 and matrix operators; elements at both sides of every cut are among the compared.
+The same of the library's own copy through pageable memory, which serves where no
+pinned memory is left and no entry point of the interface asks for.
 The oracle runs the same FP64 algorithm as the reference's; the two differ by
 rounding, below 1e-10 of the largest value at these orders (the oracle's own
 mass solves are the larger part), while any misplaced value differs by O(1)."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import _oracle as orc
 from _parity import rel
-from hpgem_amd import OP_ACOUSTIC_CENTRAL, RK4, HpgemAPIDevice, Mesh
+from hpgem_amd import OP_ACOUSTIC_CENTRAL, RK4, HpgemAPIDevice, Mesh, _lib
 from hpgem_amd.api import HpgemAPIMatrixDevice
 
 pytestmark = pytest.mark.gpu
@@ -79,4 +82,33 @@ def test_matrix_operator(blocks, n):
     dev.setTimeIntegrationVector(0, u.ravel())
     dev.computeTimeDerivative([0], [1.0], 1)
     assert rel(dev.getTimeIntegrationVector(1), (scale[:, None] * (u @ a.T)).ravel()) <= 1e-13
+    dev.close()
+
+
+@pytest.mark.parametrize("kind", ["tensor", "tetrahedra", "matrix"])
+def test_pageable(kind):
+    print(f"[case] host layout, pageable, {kind}", flush=True)
+    copy = _lib.load()._ZN4hgdg18host_copy_pageableEP8hgdg_ctxiPdPKd
+    copy.restype, copy.argtypes = None, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    rng = np.random.default_rng(7)
+    if kind == "tensor":
+        dev = HpgemAPIDevice(Mesh.structured([5, 4]), 2, tableau=RK4, velocity=[1.0, 0.7])
+    elif kind == "tetrahedra":
+        mesh = Mesh.structured([2, 2, 3], periodic=[0] * 3, simplices=True)
+        p = rng.integers(1, 5, mesh.n_elements).astype(np.int32)
+        dev = HpgemAPIDevice(mesh, p, kind=OP_ACOUSTIC_CENTRAL, c_inv=np.ones(mesh.n_elements), tableau=RK4)
+    else:
+        dev = HpgemAPIMatrixDevice([np.eye(7)] * 5, [np.eye(7)] * 5, np.zeros((0, 2)), [], tableau=RK4)
+    u, got = rng.standard_normal(dev.n_dof), np.empty(dev.n_dof)
+    for storage in ("fp64", "mixed"):
+        if storage == "mixed":
+            if kind == "matrix":
+                break
+            dev.setStorage(1, "mixed")
+            u = u.astype(np.float32).astype(np.float64)
+        copy(dev.h, 1, None, u.ctypes.data)
+        np.testing.assert_array_equal(dev.getTimeIntegrationVector(1), u)
+        dev.setTimeIntegrationVector(1, -u)
+        copy(dev.h, 1, got.ctypes.data, None)
+        np.testing.assert_array_equal(got, -u)
     dev.close()
