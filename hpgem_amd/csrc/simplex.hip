@@ -158,10 +158,13 @@ __device__ __forceinline__ mfma_d4 mfma_step(double a, double b, mfma_d4 c) {
 // and the fused update's reads are in order.
 //
 // Bound by latency, not by a unit: at 24^3 x 5 elements of order 1..4 a launch
-// takes 71.5 us in FP64 (100.7 before: a launch of 28 us that wrote projected
-// traces of every face, and one of 73 that gathered them, with the matrix units
-// for the derivatives of orders 3 and 4 alone), 69.7 with FP32 stage values (81.1); the bytes of one launch, 92 MB,
-// take 19 us and the matrix instructions keep their units busy for 15 us.
+// takes 72 to 78 us in FP64, as the choice of elements per workgroup turns out
+// (100.7 before: a launch of 28 us that wrote projected traces of every face, and
+// one of 73 that gathered them, with the matrix units for the derivatives of
+// orders 3 and 4 alone), 70 to 76 with FP32 stage values (81.1). Of 78 us the
+// matrix instructions keep their units busy for 15, LDS takes 15, the issue of
+// vector instructions 26; the 125 MB of vectors and geometry take 18 to 23 at a
+// copy's rate (165 MB with what is read more than once, 24 to 31).
 // Whole orders: 31.8 -> 23.3, 53 -> 39.7, 113 -> 66.2 and 179 -> 102.8 us for
 // p = 1..4; 13 x 11 x 9 cells of order 2 (launch-bound, two before) 14.7 ->
 // 10.1 us. Arithmetic is FP64 whatever the stage values' type: the matrix units

@@ -869,11 +869,13 @@ struct AcousticParams {
 // leaves at most one lane in sixteen idle: one wavefront where it can.
 // Sums are explicit multiply-adds: every instance (with and without the
 // update, batched) rounds alike.
-// Bound by memory: 32^3 p = 3 in FP64 reads and writes 201 MB at 4.6 TB/s
-// (a copy of that size reaches 5.4 - 6.9 TB/s). One lane per field and pencil,
-// which applies the derivative of v once per s field and forms every face
-// pencil's flux N1 times, took 104 us FP64 / 80 mixed there against 47 / 36;
-// 30^3 p = 2 42 against 23, 23x19x21 p = 4 66 against 37 (FP64).
+// Bound by memory: 32^3 p = 3 in FP64 takes 44 us for 208 MB of vectors and
+// geometry, 4.7 TB/s; with the z neighbours that come from memory again it is
+// 254 MB at 5.8 TB/s (a copy of that size reaches 5.4 - 6.9). One lane per field
+// and pencil, which applies the derivative of v once per s field and forms every
+// face pencil's flux N1 times, took 104 us FP64 / 80 mixed there against 44 / 33
+// (47 / 36 with the workgroups in plain order, see acoustic_order: so are the next
+// figures); 30^3 p = 2 42 against 23, 23x19x21 p = 4 66 against 37 (FP64).
 // kAhead: the first face pencil's neighbour values are loaded together with
 // the own ones, one memory round trip less (32^3 p = 3 53 -> 47 us, 256^2
 // p = 3 20.1 -> 17.7); at orders 4 and 5 in 3D, and with the update's terms

@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kGenTarget) void tensor_general_geometry(const GenG
 
 // Bound by the LDS reads and barriers of its one-dimensional contractions:
 // every operand but a row of the matrix comes from LDS. The geometry comes
-// from memory (3.5 KB an element at p = 2 in 3D, beside 2.6 KB of state): formed
+// from memory (3.5 KB an element at p = 2 in 3D, where a vector has 0.9): formed
 // from the vertices at every point and face point of every launch, it took 256
 // registers, a third of the LDS for the vertices and most of the time (FP64
 // acoustic, 22x18x20 p = 2: 114 us then, 24 now; 14x12x13 p = 3 70 and 14;
